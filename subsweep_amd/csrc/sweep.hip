@@ -60,6 +60,7 @@
 #include <cstring>
 #include <exception>
 #include <functional>
+#include <limits>
 #include <mutex>
 #include <shared_mutex>
 #include <thread>
@@ -223,7 +224,8 @@ template <typename R>
 struct Flux {
     R* X;                    // D x N, at xidx(d, c)
     const uint32_t* xpos;    // compiled replay: X of (c, d) at the task's schedule position xpos[d*N + c]
-    R* I;                    // D x N
+    R* I;                    // D x N, at iidx(d, c)
+    const uint32_t* ipos;    // direction sweeps: I in X's order (= xpos); else NULL: d*N + c
     R* P;                    // D x Nper
     // After a rotation of the directions (ssw_rotate_directions), the rates
     // that the remap of the state left in place, as offsets to the pull sums:
@@ -233,7 +235,7 @@ struct Flux {
     R* offI;                 // D x N
     R* offP;                 // D x Nper
     const SA<R>* sa;         // N: {source / D in the storage scale, attenuation} (one load per task)
-    double thr;              // threshold in the storage scale
+    R thr;                   // smallest R not below the threshold in the storage scale
     double inv_lref;         // storage scale of rates
     double inv_aref;         // storage scale of areas
 };
@@ -245,6 +247,13 @@ template <typename R>
 __device__ __forceinline__ size_t xidx(const Flux<R>& fl, int64_t N, uint32_t d, uint32_t c) {
     const size_t o = (size_t)d * N + c;
     return fl.xpos ? (size_t)fl.xpos[o] : o;
+}
+
+// Where I of (cell c, direction d) is stored.
+template <typename R>
+__device__ __forceinline__ size_t iidx(const Flux<R>& fl, int64_t N, uint32_t d, uint32_t c) {
+    const size_t o = (size_t)d * N + c;
+    return fl.ipos ? (size_t)fl.ipos[o] : o;
 }
 
 // Descriptor ranges of a grouped launch, one per build pass (the group's
@@ -329,12 +338,12 @@ __device__ __forceinline__ CellIn<R> cell_inputs(const Geo& g, const Flux<R>& fl
 }
 
 // Outgoing rate of a solved task (Site::get_rate + HydrogenOnly::get_outgoing_rate,
-// src/sweep/site.rs:49-56, src/chemistry/hydrogen_only/mod.rs:72-88), stored as X = O / A.
-// X goes to ox, I to oi; returns the stored X.
-template <typename R>
-__device__ __forceinline__ R finish_task(const Flux<R>& fl, size_t ox, size_t oi, R inc, const CellIn<R>& ci,
-                                         R A) {
-    if (fl.offI) {
+// src/sweep/site.rs:49-56, src/chemistry/hydrogen_only/mod.rs:72-88) from its
+// upwind sum `inc`, which is clamped on the way; oi: its place in I. Stored as
+// X = O / A at ox, I at oi.
+template <typename R, bool kOffsets>
+__device__ __forceinline__ R outgoing_rate(const Flux<R>& fl, size_t oi, R& inc, const CellIn<R>& ci) {
+    if (kOffsets && fl.offI) {
         // after a rotation the incoming rate is the remapped rate plus the
         // corrections since, offset + upwind sum; its persistent clamp
         // (Photons::make_positive) sets the offset to -sum, so that the rate
@@ -349,13 +358,18 @@ __device__ __forceinline__ R finish_task(const Flux<R>& fl, size_t ox, size_t oi
         inc = 0;  // Photons::make_positive
     }
     R in = (inc + (R)ci.src) + ci.per;
-    // the threshold in the storage scale is compared in double: in FP32 it is
-    // threshold / lref (e.g. 1e-5 / 2^160), far below the float range
-    R out = ((double)in < fl.thr) ? (R)0 : in * (R)ci.att;
-    const R xv = (A > (R)0) ? out / A : (R)0;
-    fl.X[ox] = xv;
+    // a rate below the threshold; in FP32 the threshold is threshold / lref
+    // (e.g. 1e-5 / 2^160), far below the float range: thr is rounded up, which
+    // leaves the comparison with every float as it is
+    return (in < fl.thr) ? (R)0 : in * (R)ci.att;
+}
+
+template <typename R>
+__device__ __forceinline__ void finish_task(const Flux<R>& fl, size_t ox, size_t oi, R inc, const CellIn<R>& ci,
+                                            R A) {
+    const R out = outgoing_rate<R, true>(fl, oi, inc, ci);
+    fl.X[ox] = (A > (R)0) ? out / A : (R)0;
     fl.I[oi] = inc;
-    return xv;
 }
 
 // The face loop of one task, kLanes lanes per task (one face each), shared by
@@ -459,30 +473,56 @@ __device__ __forceinline__ bool cell_dir(const Geo& g, uint32_t t, uint32_t& c, 
     return (int64_t)c < g.N;
 }
 
-// Per (cell, direction): downwind faces by kind (the byte model) and the
-// number of upwind local faces beyond kPlanes (overflow entries).
-__global__ void k_face_stats(Geo g, unsigned long long* out4, uint32_t* ovf_count) {
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    uint32_t c, d;
-    unsigned long long n[4] = {0, 0, 0, 0};
-    if (cell_dir(g, t, c, d)) {
-        const double dx = g.dirs[3 * d], dy = g.dirs[3 * d + 1], dz = g.dirs[3 * d + 2];
-        uint32_t nup = 0;
-        for (uint32_t f = g.off[c]; f < g.off[c + 1]; f++) {
-            const uint32_t kind = g.nk[f] >> 30;
-            const double dd = fdot(g.geo[f], dx, dy, dz);
-            if (dd > 0.0) n[kind]++;
-            else if (dd < 0.0 && kind == kKindLocal) nup++;
+constexpr int kFluxDirs = 8;    // directions per wave of the kernels that walk the faces of 64 cells
+constexpr int kFluxCells = 64;
+
+// Per (cell, direction): downwind faces by kind (the byte model), the number
+// of upwind local faces beyond kPlanes (overflow entries) and, with `nups`,
+// their number. A wave takes 64 cells and kFluxDirs directions; the counts
+// leave a workgroup with one atomic each (one per wave made the four counters
+// the bound: 4.9 ms on 262144 cells x 84 directions, 0.28 ms like this).
+__global__ void __launch_bounds__(1024) k_face_stats(Geo g, unsigned long long* out4, uint32_t* ovf_count,
+                                                     uint8_t* nups) {
+    __shared__ unsigned long long sum[4];
+    if (threadIdx.x < 4) sum[threadIdx.x] = 0;
+    __syncthreads();
+    const uint32_t lane = threadIdx.x % kFluxCells;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / kFluxCells);
+    const int64_t c = (int64_t)blockIdx.x * kFluxCells + lane;
+    uint32_t n[4] = {0, 0, 0, 0}, nup[kFluxDirs];
+#pragma unroll
+    for (int j = 0; j < kFluxDirs; j++) nup[j] = 0;
+    const uint32_t f1 = c < g.N ? g.off[c + 1] : 0u;
+    for (uint32_t f = c < g.N ? g.off[c] : 0u; f < f1; f++) {
+        const uint32_t kind = g.nk[f] >> 30;
+        const double4 a = g.geo[f];
+#pragma unroll
+        for (int j = 0; j < kFluxDirs; j++) {
+            const int d = (int)w * kFluxDirs + j;
+            if (d >= g.D) break;
+            const double dd = fdot(a, g.dirs[3 * d], g.dirs[3 * d + 1], g.dirs[3 * d + 2]);
+            n[0] += dd > 0.0 && kind == kKindLocal;
+            n[1] += dd > 0.0 && kind == kKindPeriodic;
+            n[2] += dd > 0.0 && kind == kKindBoundary;
+            nup[j] += dd < 0.0 && kind == kKindLocal;
         }
-        const uint32_t extra = nup > (uint32_t)kPlanes ? nup - kPlanes : 0u;
+    }
+#pragma unroll
+    for (int j = 0; j < kFluxDirs; j++) {
+        const int d = (int)w * kFluxDirs + j;
+        if (c >= g.N || d >= g.D) break;
+        const uint32_t extra = nup[j] > (uint32_t)kPlanes ? nup[j] - kPlanes : 0u;
+        n[3] += extra;
         if (ovf_count) ovf_count[(size_t)d * g.N + c] = extra;
-        n[3] = extra;
+        if (nups) nups[(size_t)d * g.N + c] = (uint8_t)nup[j];
     }
     for (int k = 0; k < 4; k++) {
-        unsigned long long v = n[k];
+        uint32_t v = n[k];
         for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o);
-        if (__lane_id() == 0 && v) atomicAdd(&out4[k], v);
+        if (lane == 0 && v) atomicAdd(&sum[k], (unsigned long long)v);
     }
+    __syncthreads();
+    if (threadIdx.x < 4 && sum[threadIdx.x]) atomicAdd(&out4[threadIdx.x], sum[threadIdx.x]);
 }
 
 // Start of the overflow entries (upwind entries q >= kPlanes, in face order)
@@ -607,6 +647,33 @@ __global__ void k_invert(const uint32_t* sorted, uint32_t* xpos, uint32_t n) {
     if (p < n) xpos[sorted[p]] = p;
 }
 
+// The downwind area A of a task from its faces in order: lane l of the 16-lane
+// kernels sums the faces l, l + 16, ..., then their xor butterfly as seen from
+// lane 0.
+struct AreaTree {
+    double part[kLanes];
+    __device__ __forceinline__ AreaTree() {
+#pragma unroll
+        for (int l = 0; l < kLanes; l++) part[l] = 0.0;
+    }
+    __device__ __forceinline__ void add(uint32_t face, double term) {
+#pragma unroll
+        for (int u = 0; u < kLanes; u++)
+            if ((uint32_t)u == face % kLanes) part[u] += term;
+    }
+    __device__ __forceinline__ double total() {
+#pragma unroll
+        for (int m = kLanes / 2; m > 0; m >>= 1) {
+            double nxt[kLanes];
+#pragma unroll
+            for (int l = 0; l < kLanes; l++) nxt[l] = part[l] + part[l ^ m];
+#pragma unroll
+            for (int l = 0; l < kLanes; l++) part[l] = nxt[l];
+        }
+        return part[0];
+    }
+};
+
 // The full schedule from the tasks sorted by (depth, direction, cell): task t =
 // d*N + c at position p of level set k (start b, width W). Compiled: header,
 // A, plane entries and overflow entries, each entry naming the upwind task's
@@ -633,9 +700,7 @@ __global__ void k_schedule(Geo g, double inv_aref, const uint32_t* sorted, const
         return;
     }
     const double dx = g.dirs[3 * d], dy = g.dirs[3 * d + 1], dz = g.dirs[3 * d + 2];
-    double part[kLanes];
-#pragma unroll
-    for (int l = 0; l < kLanes; l++) part[l] = 0.0;
+    AreaTree A;
     uint32_t q = 0;
     const uint32_t os = ovf_start[(size_t)d * g.N + c];
     for (uint32_t f = f0; f < f1; f++) {
@@ -643,11 +708,7 @@ __global__ void k_schedule(Geo g, double inv_aref, const uint32_t* sorted, const
         const uint32_t nk = g.nk[f];
         const double dd = fdot(fa, dx, dy, dz);
         if (dd > 0.0) {
-            const uint32_t l = (f - f0) % kLanes;  // the lane that holds face f in the 16-lane kernels
-            const double term = fa.w * inv_aref * dd;
-#pragma unroll
-            for (int u = 0; u < kLanes; u++)
-                if ((uint32_t)u == l) part[u] += term;
+            A.add(f - f0, fa.w * inv_aref * dd);
         } else if (dd < 0.0 && (nk >> 30) == kKindLocal) {
             Entry<R> e;
             e.nb = xpos[(size_t)d * g.N + (nk & kNbrMask)];
@@ -667,17 +728,8 @@ __global__ void k_schedule(Geo g, double inv_aref, const uint32_t* sorted, const
             q++;
         }
     }
-    // the xor butterfly of the 16-lane kernels, as seen from lane 0
-#pragma unroll
-    for (int m = kLanes / 2; m > 0; m >>= 1) {
-        double nxt[kLanes];
-#pragma unroll
-        for (int l = 0; l < kLanes; l++) nxt[l] = part[l] + part[l ^ m];
-#pragma unroll
-        for (int l = 0; l < kLanes; l++) part[l] = nxt[l];
-    }
     hdr[p] = make_uint4(c | (d << kCellBits), ps, q > (uint32_t)kPlanes ? os : 0u, q);
-    Av[p] = (R)part[0];
+    Av[p] = (R)A.total();
 }
 
 // ---------------------------------------------------------------------------
@@ -947,194 +999,372 @@ __global__ void __launch_bounds__(run_block<R>()) k_sweep_comp_run(Geo g, Flux<R
 // Direction sweeps (compiled replay): the tasks of one direction depend only
 // on tasks of the same direction, so one workgroup per direction solves its
 // direction's whole sweep, level set after level set with a workgroup barrier
-// in between, and no dependency crosses workgroups or launches. The schedule
-// is sorted by (depth, direction, cell), so direction d's tasks of level set k
-// are one range of it: run[d * kmax + k] = {first position b of level set k,
-// its width W (bit 31: wait for all memory operations at the end of this
-// level set), offset of d's tasks in it, their count}; d has levels[d]
-// non-empty level sets, the first ones.
+// in between, and no dependency crosses workgroups or launches.
 //
-// In this mode X is stored in each direction's Kahn order: the task at offset
-// j of d's tasks in level set k has X index d*N + q, q = (d's tasks in level
-// sets before k) + j, and the upwind entries of the schedule name these
-// indices. The workgroup keeps the last kR values it solved in an LDS ring
-// (slot q mod kR), written for the last kR tasks of each level set, so that
-// an upwind value with q >= (end of the current level set) - kR is read from
-// LDS and the barrier between level sets waits for LDS operations only.
-// Older values are read from memory: the host flags a level set for a full
-// wait whenever the level sets since the last flagged one would hold more
-// than kR tasks, so every value older than the ring was stored before a
-// completed wait and barrier.
+// X is stored in each direction's Kahn order (level set, then class of upwind
+// counts, then cell): the q-th task of direction d has X index d*N + q. The
+// last kRing values a workgroup solved sit in an LDS ring (slot q mod kRing).
+// What a task reads of them was known when the schedule was built, so the
+// schedule names LDS words, not tasks, and a level set costs one round of LDS
+// reads between two barriers. Level sets are cut into tiles of up to 64 tasks,
+// the work of one wave, dealt to the waves in turn. A tile's blob, planes of
+// 16 bytes per task and then two lists:
+//   slot planes    8 halfwords per task: {cell | upwind count << 25 (two
+//                  halfwords), periodic source, entries 0-4}, {entries 5-12}
+//   weight planes  {A, weight of entry 0, ...}: 4 (FP32) or 2 (FP64) values
+//   far list       X indices of upwind values that the ring no longer holds
+//                  (and, with kFarPeriodic, P indices of periodic sources)
+//   extra list     weights, then words, of entries past the planes
+// in the order S0 W0 W1 S1 W2 .. (FP64: S0 W0 W1 W2 S1 W3 ..), as many planes
+// as the tile's largest upwind count needs (plane loads past them return 0:
+// word 0, which holds 0, with weight 0). The wave loads the far values itself
+// and puts them, as the extra entries, into a buffer of its own in LDS, whose
+// words the entries name like the ring's. The tile's wave is fixed by its
+// place in the direction, hence so are these words.
 //
-// In a restricted sweep (lvl > 0; the host passes 0 when every cell is
-// active) every task still passes through: a task whose cell is below level
-// lvl is not solved and puts its stored X into the ring. Software pipelined
-// two level sets deep: while level set j is solved, level set j+1's cell
-// inputs, first overflow entries (and level and stored X) and level set
-// j+2's schedule data are loaded. Same arithmetic per task as the other
+// Bound: a level set's chain (barrier, LDS reads, the sum in entry order, one
+// division, LDS write) while the schedule streams past from HBM. A wave loads
+// tile i+2's planes and tile i+1's cell inputs and far values before it waits
+// for tile i's level set, in registers that no copy moves (the loop is
+// unrolled over three sets), so no memory wait enters the chain. One wave per
+// tile instead of one lane per task of a level set keeps 16 x 2 tiles in
+// flight per CU where a level set holds 25 to 400 tasks. The wave that solved
+// a tile passes the level set's end before it stores and loads anything, which
+// else stands between the others and the next level set (0.62 -> 0.42 us per
+// level set of 25 tasks). Per sweep, against one lane per task of a level set
+// with its data two level sets ahead: 25.0 -> 7.1 ms on 2 M clustered cells x
+// 84 directions (1.14 us per level set of 340 tasks, 2.3 TB/s), 2.41 -> 0.77
+// ms on 262144 cells, FP64 2.95 -> 1.1 ms, 1.70 -> 0.39 ms on 23457 cells x 32.
+//
+// Far values: the load for tile i+1 goes out after this wave solved tile i-1;
+// a wave's stores go out before it begins its next tile and are complete when
+// it uses a load issued after them, at most two of its tiles later. So every
+// value more than 5 * kWaves tiles and two level sets behind is in memory, and
+// the ring holds more than that unless a level set is wider than kRing / 4:
+// such directions (`wide`) complete their stores at every barrier and load
+// their far values after it.
+//
+// Waits: every wave passes levels - 1 barriers, whatever tiles it has.
+// A restricted sweep (lvl > 0; the host passes 0 when every cell is active)
+// passes every task: a task whose cell is below level lvl is not solved and
+// puts its stored X into the ring. Same arithmetic per task as the other
 // replays.
-constexpr int kDirBlock = 512;  // lanes of a direction sweep's workgroup
-constexpr uint32_t kDirWait = 0x80000000u;      // run entry: a full wait at the end of this level set
-constexpr uint32_t kDirWidth = 0x7FFFFFFFu;     // run entry: the level set's width
-
-// overflow entries loaded ahead per task (FP32: tasks of up to 18 upwind
-// faces in LDS only; FP64 keeps two, within its registers)
 template <typename R>
-constexpr int dir_ovf() {
-    return sizeof(R) == 4 ? 6 : 2;
-}
-
-template <typename R>
-constexpr uint32_t dir_ring() {
-    return sizeof(R) == 4 ? 32768u : 16384u;  // 128 KiB of LDS
-}
-
-template <typename R>
-__global__ void __launch_bounds__(kDirBlock) k_sweep_dir(Geo g, Flux<R> fl, const uint4* __restrict__ hdr,
-                                                         const R* __restrict__ Av, const Entry<R>* __restrict__ planes,
-                                                         const Entry<R>* __restrict__ ovf,
-                                                         const uint4* __restrict__ runs, int kmax,
-                                                         const uint32_t* __restrict__ levels, int lvl) {
-    constexpr uint32_t kR = dir_ring<R>();
-    constexpr int kDirOvf = dir_ovf<R>();
-    __shared__ R ring[kR];
-    const uint32_t i = threadIdx.x;
-    const uint32_t d = blockIdx.x;
-    const uint4* run = runs + (size_t)d * kmax;
-    const int nl = (int)levels[d];
-    if (nl == 0) return;
-    const int last = nl - 1;
-    const uint32_t dN = d * (uint32_t)g.N;
-    // position in its level set of lane i's task in pass q0 (a valid one for every lane)
-    auto pos = [&](const uint4& r, uint32_t q0) -> uint32_t { return r.z + min(q0 + i, r.w - 1u); };
-    auto ld = [&](TaskS<R>& t, const uint4& r, uint32_t p) {
-        load_task<R>(t, hdr + r.x, Av + r.x, planes + (size_t)kPlanes * r.x, r.y & kDirWidth, p);
-    };
-    // cell inputs, and in a restricted sweep the cell's level and the stored
-    // X (compared and used only when the task is solved, a level set later)
-    struct Pre {
-        CellIn<R> ci;
-        R xold;
-        uint32_t lev;
-        Entry<R> o[kDirOvf];  // the first overflow entries (index clamped to the task's own)
-    };
-    auto pre = [&](const TaskS<R>& t, uint32_t self) -> Pre {
-        Pre q;
-        const uint32_t c = t.h.x & kCellMask;
-        q.ci = cell_inputs<R>(g, fl, c, d, t.h.y);
-        if (t.h.w > (uint32_t)kPlanes) {
-            const uint32_t lastq = t.h.w - kPlanes - 1u;
-#pragma unroll
-            for (int k = 0; k < kDirOvf; k++) q.o[k] = ovf[t.h.z + min((uint32_t)k, lastq)];
-        } else {
-#pragma unroll
-            for (int k = 0; k < kDirOvf; k++) {
-                q.o[k].nb = self;
-                q.o[k].w = (R)0;
-            }
-        }
-        if (lvl > 0) {
-            q.lev = g.level[c];
-            q.xold = fl.X[self];
-        } else {
-            q.lev = 0;
-            q.xold = (R)0;
-        }
-        return q;
-    };
-    // an upwind value: from the ring when it holds it, else from memory
-    auto up = [&](uint32_t nb, uint32_t hi) -> R {
-        const uint32_t qu = nb - dN;
-        return (qu + kR >= hi) ? ring[qu & (kR - 1u)] : fl.X[nb];
-    };
-    // the task's upwind sum in entry order, its stores, and its ring slot.
-    // Waves whose tasks find every upwind value in the ring (and have at most
-    // kDirOvf overflow entries, loaded a level set ahead) read LDS only, so
-    // that no wait on memory loads (which would also wait for the loads of
-    // the next level sets) enters the chain; other waves take the slow path.
-    auto solve = [&](const TaskS<R>& t, const Pre& pr, uint32_t self, uint32_t hi, bool lane) {
-        const uint32_t nup = t.h.w;
-        bool near = nup <= (uint32_t)(kPlanes + kDirOvf);
-#pragma unroll
-        for (int q = 0; q < kPlanes; q++)
-            near = near && ((uint32_t)q >= nup || (t.e[q].nb - dN) + kR >= hi);
-#pragma unroll
-        for (int k = 0; k < kDirOvf; k++) near = near && (pr.o[k].nb - dN) + kR >= hi;
-        R x[kPlanes];
-        R inc = 0;
-        if (__ballot(!near) == 0ull) {
-#pragma unroll
-            for (int q = 0; q < kPlanes; q++) x[q] = ring[(((uint32_t)q < nup ? t.e[q].nb : self) - dN) & (kR - 1u)];
-            R xo[kDirOvf];
-#pragma unroll
-            for (int k = 0; k < kDirOvf; k++) xo[k] = ring[(pr.o[k].nb - dN) & (kR - 1u)];
-#pragma unroll
-            for (int q = 0; q < kPlanes; q++) inc += ((uint32_t)q < nup) ? t.e[q].w * x[q] : (R)0;
-#pragma unroll
-            for (int k = 0; k < kDirOvf; k++)  // overflow entries, in entry order
-                if ((uint32_t)(kPlanes + k) < nup) inc += pr.o[k].w * xo[k];
-        } else {
-#pragma unroll
-            for (int q = 0; q < kPlanes; q++) x[q] = up((uint32_t)q < nup ? t.e[q].nb : self, hi);
-#pragma unroll
-            for (int q = 0; q < kPlanes; q++) inc += ((uint32_t)q < nup) ? t.e[q].w * x[q] : (R)0;
-            for (uint32_t q = kPlanes; q < nup; q++) {  // overflow entries, in entry order
-                const Entry<R> o = ovf[t.h.z + q - kPlanes];
-                inc += o.w * up(o.nb, hi);
-            }
-        }
-        if (lane) {
-            const bool act = pr.lev >= (uint32_t)lvl;
-            const R xv = act ? finish_task<R>(fl, self, (size_t)d * g.N + (t.h.x & kCellMask), inc, pr.ci, t.A)
-                             : pr.xold;
-            const uint32_t qs = self - dN;
-            if (qs + kR >= hi) ring[qs & (kR - 1u)] = xv;
-        }
-    };
-    // level sets j (r0), j+1 (r1), j+2 (r2) and their first q (past the last
-    // level set the entries repeat the last one)
-    uint4 r0 = run[0], r1 = run[min(1, last)], r2 = run[min(2, last)];
-    uint32_t qs0 = 0;
-    uint32_t qs1 = last >= 1 ? r0.w : 0u;
-    uint32_t qs2 = last >= 2 ? qs1 + r1.w : qs1;
-    uint32_t p0 = pos(r0, 0), p1 = pos(r1, 0);
-    TaskS<R> t0, t1;
-    ld(t0, r0, p0);
-    ld(t1, r1, p1);
-    Pre c0 = pre(t0, dN + qs0 + (p0 - r0.z));
-    for (int j = 0; j < nl; j++) {
-        const Pre c1 = pre(t1, dN + qs1 + (p1 - r1.z));
-        const uint32_t p2 = pos(r2, 0);
-        TaskS<R> t2;
-        ld(t2, r2, p2);
-        const uint4 r3 = run[min(j + 3, last)];
-        const uint32_t hi = qs0 + r0.w;
-        solve(t0, c0, dN + qs0 + (p0 - r0.z), hi, i < r0.w);
-        for (uint32_t q0 = kDirBlock; q0 < r0.w; q0 += kDirBlock) {  // wide level sets: further passes
-            const uint32_t pq = pos(r0, q0);
-            const uint32_t self = dN + qs0 + (pq - r0.z);
-            TaskS<R> t;
-            ld(t, r0, pq);
-            solve(t, pre(t, self), self, hi, q0 + i < r0.w);
-        }
-        if (r0.y & kDirWait) {  // every store so far complete before the barrier
-            __builtin_amdgcn_s_waitcnt(0);
-            __syncthreads();
-        } else {  // LDS operations only
-            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        }
-        r0 = r1;
-        p0 = p1;
-        t0 = t1;
-        c0 = c1;
-        qs0 = qs1;
-        r1 = r2;
-        p1 = p2;
-        t1 = t2;
-        qs1 = qs2;
-        qs2 = (j + 3 <= last) ? qs2 + r2.w : qs2;
-        r2 = r3;
+struct DirShape {
+    static constexpr int kWaves = sizeof(R) == 4 ? 16 : 12;  // FP64: 168 VGPRs a wave
+    static constexpr uint32_t kRing = sizeof(R) == 4 ? 32768u : 16384u;  // 128 KiB
+    static constexpr int kPer = 16 / (int)sizeof(R);                     // values per weight plane
+    static constexpr int kWPlanes = sizeof(R) == 4 ? 4 : 7;              // A and 13 weights
+    static constexpr int kS1 = sizeof(R) == 4 ? 3 : 4;                   // place of the second slot plane
+    static constexpr uint32_t kRingAt = 64;                              // words 0-63: 0
+    static constexpr uint32_t kBufs = kRingAt + kRing;
+    static constexpr uint32_t kBuf = 256 + 512 / (uint32_t)sizeof(R);    // 128 far, 128 weights, 128 words of 4 bytes
+    static constexpr uint32_t kWords = kBufs + kWaves * kBuf;
+    // planes that hold up to n entries
+    __host__ __device__ static constexpr uint32_t planes(uint32_t n) {
+        if (sizeof(R) == 4) return n <= 3 ? 2u : n <= 5 ? 3u : n <= 7 ? 4u : n <= 11 ? 5u : 6u;
+        return n <= 1 ? 2u : n <= 3 ? 3u : n <= 5 ? 4u : n <= 7 ? 6u : n <= 9 ? 7u : n <= 11 ? 8u : 9u;
     }
+    // place of weight plane j
+    __host__ __device__ static constexpr uint32_t wplane(uint32_t j) { return j + 1 < (uint32_t)kS1 ? j + 1 : j + 2; }
+};
+constexpr uint32_t kDirEntries = 13;           // entries in the planes; a task with more has 12 there and the rest
+                                               // in the extra list from the position that entry 12's word gives
+constexpr uint32_t kDirCap = 64;               // far and extra entries of a tile of more than one task
+constexpr uint32_t kFarPeriodic = 0x80000000u;
+constexpr int kStream = 2;                     // non-temporal: the schedule is read once per sweep and leaves the L2
+                                               // to the cells' lines (13.8 -> 12.9 ms per sweep on 2 M cells)
+
+// Classes of upwind counts by which a level set's tasks are sorted, so that a
+// tile's tasks need about the same planes.
+__host__ __device__ __forceinline__ uint32_t dir_class(uint32_t nup) {
+    return (nup > 5) + (nup > 7) + (nup > 9) + (nup > 11);
+}
+
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// A tile, 32 bytes: blob offset in 16-byte units (two words), first q, end of
+// the level set's q, level set, tasks | far << 8 | extra << 16 | planes << 24.
+struct DirTile {
+    uint64_t off;
+    uint32_t q0, hi, k, cnt, nfar, nex, np;
+};
+
+template <typename R>
+struct DirRegs {
+    u32x4 s[2];
+    uint32_t w[14 * sizeof(R) / 4];  // A and 13 weights (a register that nothing reads would be taken for another
+                                     // use while its load is still on the way, and waited for)
+    uint32_t far;     // far list entry of this lane
+    R exw;            // extra entry of this lane
+    uint32_t exs;
+    SA<R> sa;         // one tile ahead: cell inputs, far value
+    R fv;
+    R off, xold;      // general variant only
+    uint32_t lev;
+    DirTile t;
+};
+
+template <typename R, bool kGeneral>
+__global__ void __launch_bounds__(64 * DirShape<R>::kWaves) k_sweep_dir(Geo g, Flux<R> fl,
+                                                                        const uint4* __restrict__ blob,
+                                                                        const uint4* __restrict__ tiles,
+                                                                        const uint4* __restrict__ dirs,
+                                                                        const SA<R>* __restrict__ sas,
+                                                                        const uint8_t* __restrict__ levs, int lvl) {
+    using S = DirShape<R>;
+    constexpr uint32_t kRing = S::kRing;
+    __shared__ R lds[S::kWords];
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t d = blockIdx.x;
+    const uint4 di = dirs[d];  // first tile, tiles, level sets, wide
+    const uint32_t ntiles = di.y, levels = di.z;
+    const bool wide = di.w != 0;
+    const uint32_t dN = d * (uint32_t)g.N;
+    R* const buf = lds + S::kBufs + w * S::kBuf;
+    uint32_t* const bufs = reinterpret_cast<uint32_t*>(buf + 256);
+    if (threadIdx.x < 64) lds[threadIdx.x] = (R)0;
+    __syncthreads();
+
+    // descriptor of the wave's i-th tile, as vector loads (scalar ones would
+    // be waited for at the barriers); past the last tile it reads the last one
+    uint4 da, db;
+    auto fetch = [&](uint32_t i) {
+        uint32_t at = 2u * (di.x + min(w + i * S::kWaves, ntiles - 1u));
+        asm volatile("" : "+v"(at));
+        da = tiles[at];
+        db = tiles[at + 1u];
+    };
+    auto uni = [](uint32_t v) -> uint32_t { return __builtin_amdgcn_readfirstlane(v); };
+    auto decode = [&](DirTile& t, uint32_t i) {
+        const bool any = w + i * S::kWaves < ntiles;
+        const uint32_t c = any ? uni(db.y) : 0u;
+        t.off = (uint64_t)uni(da.x) | ((uint64_t)uni(da.y) << 32);
+        t.q0 = uni(da.z);
+        t.hi = uni(da.w);
+        t.k = uni(db.x);
+        t.cnt = c & 255u;
+        t.nfar = (c >> 8) & 255u;
+        t.nex = (c >> 16) & 255u;
+        t.np = c >> 24;
+    };
+    auto rsrc = [&](const uint4* p, uint32_t bytes) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4*>(p), 0, (int)bytes, 0x00027000);
+    };
+    auto ex_units = [](uint32_t nex) { return (nex * (uint32_t)sizeof(R) + 15u) / 16u; };
+    // the planes and lists of a tile (loads past them return 0)
+    auto load = [&](DirRegs<R>& T) {
+        const DirTile& t = T.t;
+        const uint4* p = blob + t.off;
+        const auto rp = rsrc(p, t.np * t.cnt * 16u);
+        const uint32_t o = min(lane, max(t.cnt, 1u) - 1u) * 16u, st = t.cnt * 16u;
+        T.s[0] = __builtin_amdgcn_raw_buffer_load_b128(rp, o, 0, kStream);
+        p += t.np * t.cnt;
+        T.far = __builtin_amdgcn_raw_buffer_load_b32(rsrc(p, t.nfar * 4u), lane * 4u, 0, kStream);
+        __builtin_amdgcn_sched_barrier(0);  // loads return in order: what is needed first goes out first
+#pragma unroll
+        for (int j = 0; j < S::kWPlanes; j++) {
+            if (j + 1 == S::kS1) T.s[1] = __builtin_amdgcn_raw_buffer_load_b128(rp, o + S::kS1 * st, 0, kStream);
+            if (sizeof(R) == 4 && j == S::kWPlanes - 1) {
+                const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(rp, o + S::wplane(j) * st, 0, kStream);
+                T.w[4 * j] = v.x;
+                T.w[4 * j + 1] = v.y;
+            } else {
+                const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rp, o + S::wplane(j) * st, 0, kStream);
+#pragma unroll
+                for (int m = 0; m < 4; m++) T.w[4 * j + m] = v[m];
+            }
+        }
+        p += (t.nfar + 3u) / 4u;
+        if constexpr (sizeof(R) == 4) {
+            T.exw = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc(p, t.nex * 4u), lane * 4u, 0, kStream));
+        } else {
+            const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(rsrc(p, t.nex * 8u), lane * 8u, 0, kStream);
+            T.exw = __hiloint2double((int)v.y, (int)v.x);
+        }
+        p += ex_units(t.nex);
+        T.exs = __builtin_amdgcn_raw_buffer_load_b32(rsrc(p, t.nex * 4u), lane * 4u, 0, kStream);
+    };
+    auto far_value = [&](uint32_t at) -> R {
+        const R* src = (at & kFarPeriodic) ? fl.P : fl.X;
+        return src[at & ~kFarPeriodic];
+    };
+    auto pre = [&](DirRegs<R>& T) {
+        const uint32_t p = dN + T.t.q0 + min(lane, max(T.t.cnt, 1u) - 1u);
+        T.sa = sas[p];
+        T.fv = far_value(T.far);
+        if (kGeneral) {
+            T.off = fl.offI ? fl.offI[(size_t)d * g.N + (T.s[0].x & kCellMask)] : (R)0;
+            T.lev = lvl > 0 ? levs[p] : 0u;
+            T.xold = lvl > 0 ? fl.X[p] : (R)0;
+        }
+    };
+    uint32_t at_level = 0;
+    auto pass_to = [&](uint32_t k) {
+        while (at_level < k) {
+            if (wide) __builtin_amdgcn_s_waitcnt(0);
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            at_level++;
+        }
+    };
+    auto slot = [&](const DirRegs<R>& T, int e) -> uint32_t {  // entry e's LDS word (-1: the periodic source's)
+        const int h = e + 3;
+        const uint32_t v = T.s[h / 8][(h % 8) / 2];
+        return (h & 1) ? v >> 16 : v & 0xFFFFu;
+    };
+    auto weight = [&](const DirRegs<R>& T, int i) -> R {  // 0: A, 1 + e: entry e's
+        if constexpr (sizeof(R) == 4) return __uint_as_float(T.w[i]);
+        else return __hiloint2double((int)T.w[2 * i + 1], (int)T.w[2 * i]);
+    };
+    // next: level set of the wave's next tile (its own, if it has none)
+    auto solve = [&](DirRegs<R>& T, uint32_t next) {
+        const DirTile& t = T.t;
+        if (t.cnt == 0) return;
+        // the wave's buffer, before it waits for the level set (far values of a
+        // wide direction after it); each load in a branch of its own, so that
+        // no wait for it enters the others
+        if (t.nex) {
+            buf[128u + lane] = T.exw;
+            bufs[lane] = T.exs;
+            if (t.nex > 64u) {  // one task with more than 64 entries
+                const uint4* p = blob + t.off + t.np * t.cnt + (t.nfar + 3u) / 4u;
+                if (64u + lane < t.nex) {
+                    buf[192u + lane] = reinterpret_cast<const R*>(p)[64u + lane];
+                    bufs[64u + lane] = reinterpret_cast<const uint32_t*>(p + ex_units(t.nex))[64u + lane];
+                }
+            }
+        }
+        const uint32_t hdr = T.s[0].x, q = t.q0 + lane;
+        const bool more = (hdr >> kCellBits) > kDirEntries;
+        uint32_t at[kDirEntries + 1];  // LDS words of the periodic source and the entries
+#pragma unroll
+        for (int e = 0; e <= (int)kDirEntries; e++)
+            at[e] = (e == (int)kDirEntries && more) ? 0u : slot(T, e - 1);
+        if (sizeof(R) == 4) {  // formed before the barrier (FP64 has no registers for them)
+#pragma unroll
+            for (int e = 0; e <= (int)kDirEntries; e++) asm volatile("" : "+v"(at[e]));
+        }
+        if (wide) {
+            pass_to(t.k);
+            for (uint32_t j = 0; j < t.nfar; j += 64u) {
+                const uint32_t* list = reinterpret_cast<const uint32_t*>(blob + t.off + t.np * t.cnt);
+                if (j + lane < t.nfar) buf[j + lane] = far_value(list[j + lane]);
+            }
+        } else {
+            buf[lane] = T.fv;
+            if (t.nfar > 64u) {
+                const uint32_t* list = reinterpret_cast<const uint32_t*>(blob + t.off + t.np * t.cnt);
+                if (64u + lane < t.nfar) buf[64u + lane] = far_value(list[64u + lane]);
+            }
+            pass_to(t.k);
+        }
+        // all reads in one batch: those past the planes read word 0
+        R x[kDirEntries + 1];
+#pragma unroll
+        for (int e = 0; e <= (int)kDirEntries; e++) x[e] = lds[at[e]];
+        R inc = 0;
+#pragma unroll
+        for (int e = 0; e < (int)kDirEntries; e++) inc += weight(T, 1 + e) * x[1 + e];
+        if (t.nex && more) {
+            const uint32_t nup = hdr >> kCellBits;
+            const uint32_t first = slot(T, (int)kDirEntries - 1) - (kDirEntries - 1u);
+            for (uint32_t e0 = kDirEntries - 1u; e0 < nup; e0 += 4u) {  // four reads in flight
+                R v[4], y[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const uint32_t e = first + min(e0 + j, nup - 1u);
+                    v[j] = buf[128u + e];
+                    y[j] = lds[bufs[e]];
+                }
+#pragma unroll
+                for (int j = 0; j < 4; j++) inc += e0 + j < nup ? v[j] * y[j] : (R)0;
+            }
+        }
+        CellIn<R> ci;
+        ci.src = T.sa.x;
+        ci.att = T.sa.y;
+        ci.per = x[0];
+        ci.off = kGeneral ? T.off : (R)0;
+        const R A = weight(T, 0);
+        const size_t oi = (size_t)d * g.N + (hdr & kCellMask);
+        bool act = lane < t.cnt;
+        R xv;
+        if (kGeneral) {
+            const bool lev = T.lev >= (uint32_t)lvl;
+            if (act && lev) {
+                const R out = outgoing_rate<R, true>(fl, oi, inc, ci);
+                xv = (A > (R)0) ? out / A : (R)0;
+            } else {
+                xv = T.xold;
+            }
+            if (act && q + kRing >= t.hi) lds[S::kRingAt + (q & (kRing - 1u))] = xv;
+            act = act && lev;
+        } else {
+            const R out = outgoing_rate<R, false>(fl, oi, inc, ci);
+            xv = (A > (R)0) ? out / A : (R)0;
+            if (act && q + kRing >= t.hi) lds[S::kRingAt + (q & (kRing - 1u))] = xv;
+        }
+        // the level set's end before anything that does not belong to it: the
+        // stores and the next tiles' loads run beside the next level set
+        if (!wide && next > t.k) pass_to(t.k + 1u);
+        if (act) {
+            fl.X[dN + q] = xv;
+            fl.I[dN + q] = inc;
+        }
+    };
+    // iteration i: tile i+2's planes, tile i+1's inputs, tile i
+    DirRegs<R> T0, T1, T2;
+    fetch(0);
+    decode(T0.t, 0);
+    load(T0);
+    fetch(1);
+    decode(T1.t, 1);
+    fetch(2);
+    __builtin_amdgcn_sched_barrier(0);  // as in the loop: its waits count the loads after a fetch
+    load(T1);
+    __builtin_amdgcn_sched_barrier(0);
+    pre(T0);
+    __builtin_amdgcn_sched_barrier(0);
+    auto step = [&](DirRegs<R>& a, DirRegs<R>& b, DirRegs<R>& c, uint32_t i) {
+        decode(c.t, i + 2);
+        fetch(i + 3);
+        __builtin_amdgcn_sched_barrier(0);
+        load(c);
+        __builtin_amdgcn_sched_barrier(0);
+        pre(b);
+        __builtin_amdgcn_sched_barrier(0);
+        solve(a, b.t.cnt ? b.t.k : a.t.k);
+    };
+    const uint32_t mine = ntiles > w ? (ntiles - w + S::kWaves - 1u) / S::kWaves : 0u;
+    for (uint32_t i = 0; i < mine; i += 3) {
+        step(T0, T1, T2, i);
+        step(T1, T2, T0, i + 1);
+        step(T2, T0, T1, i + 2);
+    }
+    pass_to(levels - 1u);
+}
+
+// The inputs of a direction sweep in X's order, before each sweep: every
+// task's {source, attenuation} and, in a restricted sweep, its cell's level.
+// Their gathers cost a CU one line at a time (44 ns per 64 tasks); here all
+// CUs share them, in the sweep itself only the D that run it. With I stored in
+// X's order likewise (chemistry gathers it), a sweep of 262144 cells x 84
+// directions went from 1.24 to 0.90 ms, and one of 2 M clustered cells
+// from 12.1 to 8.3 ms, these passes included (the gather in k_chemistry adds
+// 1.4 ms there).
+template <typename R>
+__global__ void __launch_bounds__(kBlock) k_dir_inputs(const uint32_t* __restrict__ cell, const SA<R>* __restrict__ sa,
+                                                       const uint8_t* __restrict__ level, SA<R>* __restrict__ sas,
+                                                       uint8_t* __restrict__ levs, uint32_t n) {
+    // a die takes consecutive positions: the level sets that cross the same
+    // cells' lines share its L2
+    const uint32_t p = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
+    if (p >= n) return;
+    const uint32_t c = cell[p];
+    sas[p] = sa[c];
+    if (levs) levs[p] = level[c];
 }
 
 // The lowest timestep level of the cells (direction sweeps: a restricted
@@ -1147,31 +1377,237 @@ __global__ void k_min_level(const uint8_t* __restrict__ level, int64_t n, uint32
     if (__lane_id() == 0) atomicMin(out, m);
 }
 
-// X index of every task in the direction sweeps' order: the task at position
-// p of level set k (sorted[p] = d*N + c) goes to d*N + qstart + (p - b_k - off)
-// with oq[k*D + d] = {off, qstart} of d's tasks in k.
-__global__ void k_invert_dir(const uint32_t* __restrict__ sorted, const uint32_t* __restrict__ fstart, int kmax,
-                             const uint2* __restrict__ oq, uint32_t N, uint32_t D, uint32_t* __restrict__ xpos,
-                             uint32_t n) {
-    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n) return;
-    int a = 0, bb = kmax - 1;  // level set of position p
-    while (a < bb) {
-        const int m = (a + bb + 1) >> 1;
-        if (fstart[m] <= p) a = m;
-        else bb = m - 1;
-    }
-    const uint32_t t = sorted[p];
-    const uint32_t d = t / N;
-    const uint2 v = oq[(size_t)a * D + d];
-    xpos[t] = d * N + v.y + (p - fstart[a] - v.x);
+// --- the direction sweeps' schedule, built once per grid ----------------------
+
+// Sort key of every task t = d*N + c: direction, level set, class.
+__global__ void k_dir_keys(const uint32_t* __restrict__ depth, const uint8_t* __restrict__ nup, uint32_t N,
+                           uint32_t kmax, uint32_t n, uint32_t* __restrict__ key, uint32_t* __restrict__ val) {
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= n) return;
+    key[t] = ((t / N * kmax + depth[t]) << 3) | dir_class(nup[t]);
+    val[t] = t;
 }
 
-// Tasks per (level set, direction): cnt[depth[t] * D + t / N] for every task t = d*N + c.
-__global__ void k_dir_counts(const uint32_t* __restrict__ depth, uint32_t N, uint32_t D, uint32_t n,
-                             uint32_t* __restrict__ cnt) {
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) atomicAdd(&cnt[(size_t)depth[t] * D + t / N], 1u);
+// First position of every (direction, level set) in the sorted keys
+// (start[d * kmax + k], which starts as kNone), the X index of every task, and
+// the cell at every X index.
+__global__ void k_dir_starts(const uint32_t* __restrict__ key, const uint32_t* __restrict__ sorted, uint32_t n,
+                             uint32_t N, uint32_t* __restrict__ start, uint32_t* __restrict__ xpos,
+                             uint32_t* __restrict__ cell) {
+    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= n) return;
+    const uint32_t k = key[p] >> 3;
+    if (p == 0 || (key[p - 1] >> 3) != k) start[k] = p;
+    xpos[sorted[p]] = p;
+    cell[p] = sorted[p] % N;
+}
+
+// End position of level set k of direction d in the sorted order (the level
+// sets of a direction are its first ones, without gaps).
+__device__ __forceinline__ uint32_t dir_level_end(const uint32_t* start, uint32_t d, uint32_t k, uint32_t kmax,
+                                                  uint32_t N) {
+    const uint32_t e = k + 1 < kmax ? start[d * kmax + k + 1] : kNone;
+    return e != kNone ? e : (d + 1u) * N;
+}
+
+// Groups of up to 64 consecutive tasks of one level set: {first position,
+// tasks, end of the level set, level set} at first[d * kmax + k] ...
+__global__ void k_dir_groups(const uint32_t* __restrict__ start, const uint32_t* __restrict__ first, uint32_t N,
+                             uint32_t D, uint32_t kmax, uint4* __restrict__ groups) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= D * kmax || start[i] == kNone) return;
+    const uint32_t k = i % kmax, e = dir_level_end(start, i / kmax, k, kmax, N);
+    uint32_t j = first[i];
+    for (uint32_t p = start[i]; p < e; p += 64u) groups[j++] = make_uint4(p, min(64u, e - p), e, k);
+}
+
+// Entries of every task that its far list names: upwind values older than the
+// ring at the end of the task's level set, and the periodic source. A wave
+// takes 64 cells and kFluxDirs directions, as k_fluxes does.
+template <typename R>
+__global__ void __launch_bounds__(1024) k_dir_far(Geo g, const uint32_t* __restrict__ xpos,
+                                                  const uint32_t* __restrict__ depth,
+                                                  const uint32_t* __restrict__ start, uint32_t kmax,
+                                                  uint8_t* __restrict__ nfar) {
+    const uint32_t lane = threadIdx.x % kFluxCells;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / kFluxCells);
+    const int64_t c0 = (int64_t)blockIdx.x * kFluxCells + lane;
+    if (c0 >= g.N) return;
+    const uint32_t c = (uint32_t)c0, N = (uint32_t)g.N;
+    uint32_t hi[kFluxDirs], n[kFluxDirs];
+#pragma unroll
+    for (int j = 0; j < kFluxDirs; j++) {
+        const uint32_t d = min(w * kFluxDirs + j, (uint32_t)g.D - 1u);
+        hi[j] = dir_level_end(start, d, depth[(size_t)d * N + c], kmax, N);
+        n[j] = (g.Nper && g.pslot[c] != kNone) ? 1u : 0u;
+    }
+    for (uint32_t f = g.off[c]; f < g.off[c + 1]; f++) {
+        const double4 a = g.geo[f];
+        const uint32_t nk = g.nk[f];
+        if ((nk >> 30) != kKindLocal) continue;
+#pragma unroll
+        for (int j = 0; j < kFluxDirs; j++) {
+            const uint32_t d = min(w * kFluxDirs + j, (uint32_t)g.D - 1u);
+            if (fdot(a, g.dirs[3 * d], g.dirs[3 * d + 1], g.dirs[3 * d + 2]) < 0.0 &&
+                xpos[(size_t)d * N + (nk & kNbrMask)] + DirShape<R>::kRing < hi[j])
+                n[j]++;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < kFluxDirs; j++)
+        if ((int)(w * kFluxDirs) + j < g.D) nfar[(size_t)(w * kFluxDirs + j) * N + c] = (uint8_t)n[j];
+}
+
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v) {  // inclusive
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t u = (uint32_t)__shfl_up((int)v, o);
+        if ((int)__lane_id() >= o) v += u;
+    }
+    return v;
+}
+
+// The tiles of one group, one wave: consecutive tasks while their far and
+// extra entries stay within kDirCap (a task with more is a tile of its own).
+// Calls tile(first lane, tasks, far, extra, planes, units) for each.
+template <typename R, typename F>
+__device__ __forceinline__ void dir_tiles(uint32_t cnt, uint32_t nup, uint32_t far, uint32_t pf, uint32_t pe, F tile) {
+    const uint32_t lane = __lane_id();
+    uint32_t a = 0;
+    while (a < cnt) {
+        const uint32_t bf = a ? (uint32_t)__shfl((int)pf, a - 1) : 0u, be = a ? (uint32_t)__shfl((int)pe, a - 1) : 0u;
+        const unsigned long long over =
+            __ballot(lane > a && lane < cnt && (pf - bf > kDirCap || pe - be > kDirCap));
+        const uint32_t e = over ? (uint32_t)__ffsll((long long)over) - 1u : cnt;
+        const uint32_t nf = (uint32_t)__shfl((int)pf, e - 1) - bf, ne = (uint32_t)__shfl((int)pe, e - 1) - be;
+        const uint32_t np = DirShape<R>::planes(wave_max(lane >= a && lane < e ? nup : 0u));
+        const uint32_t units = np * (e - a) + (nf + 3u) / 4u + (ne * (uint32_t)sizeof(R) + 15u) / 16u + (ne + 3u) / 4u;
+        tile(a, e - a, bf, nf, be, ne, np, units);
+        a = e;
+    }
+}
+
+__device__ __forceinline__ uint32_t dir_extra(uint32_t nup) { return nup > kDirEntries ? nup - (kDirEntries - 1u) : 0u; }
+
+// Tiles and blob units of every group, one wave per group.
+template <typename R>
+__global__ void __launch_bounds__(kBlock) k_dir_tile_count(const uint4* __restrict__ groups, uint32_t ng,
+                                                           const uint32_t* __restrict__ sorted,
+                                                           const uint8_t* __restrict__ nups,
+                                                           const uint8_t* __restrict__ nfars, uint32_t* __restrict__ gt,
+                                                           uint64_t* __restrict__ gu) {
+    const uint32_t i = blockIdx.x * (kBlock / 64) + threadIdx.x / 64, lane = __lane_id();
+    if (i >= ng) return;
+    const uint4 G = groups[i];
+    const uint32_t t = sorted[G.x + min(lane, G.y - 1u)];
+    const uint32_t nup = nups[t], far = lane < G.y ? nfars[t] : 0u;
+    uint32_t nt = 0;
+    uint64_t nu = 0;
+    dir_tiles<R>(G.y, nup, far, wave_scan(far), wave_scan(lane < G.y ? dir_extra(nup) : 0u),
+                 [&](uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t units) {
+                     nt++;
+                     nu += units;
+                 });
+    if (lane == 0) {
+        gt[i] = nt;
+        gu[i] = nu;
+    }
+}
+
+// The tiles and their blobs, one wave per group, one lane per task; the
+// entries in face order, A as the 16-lane kernels form it. tfirst[d]: first
+// tile of direction d (a tile's wave is its place in the direction mod
+// kWaves).
+template <typename R>
+__global__ void __launch_bounds__(kBlock) k_dir_tile_fill(Geo g, double inv_aref, const uint4* __restrict__ groups,
+                                                          uint32_t ng, const uint32_t* __restrict__ sorted,
+                                                          const uint8_t* __restrict__ nups,
+                                                          const uint8_t* __restrict__ nfars,
+                                                          const uint32_t* __restrict__ xpos,
+                                                          const uint32_t* __restrict__ ts, const uint64_t* __restrict__ us,
+                                                          const uint32_t* __restrict__ tfirst, uint4* __restrict__ blob,
+                                                          uint4* __restrict__ tiles) {
+    using S = DirShape<R>;
+    const uint32_t i = blockIdx.x * (kBlock / 64) + threadIdx.x / 64, lane = __lane_id();
+    if (i >= ng) return;
+    const uint4 G = groups[i];
+    const uint32_t t = sorted[G.x + min(lane, G.y - 1u)];
+    const uint32_t N = (uint32_t)g.N, d = t / N, c = t - d * N, dN = d * N;
+    const uint32_t nup = nups[t], far = lane < G.y ? nfars[t] : 0u;
+    const uint32_t pf = wave_scan(far), pe = wave_scan(lane < G.y ? dir_extra(nup) : 0u);
+    uint32_t tile = ts[i];
+    uint64_t off = us[i];
+    const double dx = g.dirs[3 * d], dy = g.dirs[3 * d + 1], dz = g.dirs[3 * d + 2];
+    dir_tiles<R>(G.y, nup, far, pf, pe, [&](uint32_t a, uint32_t cnt, uint32_t bf, uint32_t nf, uint32_t be, uint32_t ne,
+                                            uint32_t np, uint32_t units) {
+        uint4* const base = blob + off;
+        if (lane == 0) {
+            tiles[2 * (size_t)tile] = make_uint4((uint32_t)off, (uint32_t)(off >> 32), G.x + a - dN, G.z - dN);
+            tiles[2 * (size_t)tile + 1] = make_uint4(G.w, cnt | (nf << 8) | (ne << 16) | (np << 24), 0u, 0u);
+        }
+        if (lane >= a && lane < a + cnt) {
+            const uint32_t li = lane - a;
+            const uint32_t buf = S::kBufs + ((tile - tfirst[d]) % S::kWaves) * S::kBuf;
+            uint32_t* const flist = reinterpret_cast<uint32_t*>(base + np * cnt);
+            R* const exw = reinterpret_cast<R*>(base + np * cnt + (nf + 3u) / 4u);
+            uint32_t* const exs = reinterpret_cast<uint32_t*>(base + np * cnt + (nf + 3u) / 4u +
+                                                              (ne * (uint32_t)sizeof(R) + 15u) / 16u);
+            uint32_t fp = pf - far - bf, ep = pe - dir_extra(nup) - be;
+            const uint32_t inplane = nup > kDirEntries ? kDirEntries - 1u : kDirEntries;
+            auto put_slot = [&](uint32_t h, uint32_t v) {  // halfword h of the slot planes
+                reinterpret_cast<uint16_t*>(base + (h < 8 ? 0u : S::kS1 * cnt) + li)[h % 8] = (uint16_t)v;
+            };
+            auto put_weight = [&](uint32_t j, R v) {
+                reinterpret_cast<R*>(base + S::wplane(j / S::kPer) * cnt + li)[j % S::kPer] = v;
+            };
+            const uint32_t hdr = c | (nup << kCellBits);
+            put_slot(0, hdr & 0xFFFFu);
+            put_slot(1, hdr >> 16);
+            const uint32_t ps = g.pslot[c];
+            if (g.Nper && ps != kNone) {
+                flist[fp] = kFarPeriodic | (uint32_t)((size_t)d * g.Nper + ps);
+                put_slot(2, buf + fp++);
+            } else {
+                put_slot(2, 0u);
+            }
+            AreaTree A;
+            uint32_t q = 0;
+            const uint32_t f0 = g.off[c], f1 = g.off[c + 1];
+            for (uint32_t f = f0; f < f1; f++) {
+                const double4 fa = g.geo[f];
+                const uint32_t nk = g.nk[f];
+                const double dd = fdot(fa, dx, dy, dz);
+                if (dd > 0.0) {
+                    A.add(f - f0, fa.w * inv_aref * dd);
+                } else if (dd < 0.0 && (nk >> 30) == kKindLocal) {
+                    const R wt = (R)(fa.w * inv_aref * -dd);
+                    const uint32_t x = xpos[(size_t)dN + (nk & kNbrMask)];
+                    uint32_t at = S::kRingAt + ((x - dN) & (S::kRing - 1u));
+                    if (x + S::kRing < G.z) {
+                        flist[fp] = x;
+                        at = buf + fp++;
+                    }
+                    if (q < inplane) {
+                        put_slot(3 + q, at);
+                        put_weight(1 + q, wt);
+                    } else {
+                        exw[ep + q - inplane] = wt;
+                        exs[ep + q - inplane] = at;
+                    }
+                    q++;
+                }
+            }
+            put_weight(0, (R)A.total());
+            // the rest of the tile's planes: word 0, weight 0
+            const bool two = np > (uint32_t)S::kS1;
+            const uint32_t nw = (np - (two ? 2u : 1u)) * S::kPer;
+            for (uint32_t e = min(q, inplane); e < (two ? 13u : 5u); e++) put_slot(3 + e, 0u);
+            for (uint32_t e = min(q, inplane); e + 1 < nw; e++) put_weight(1 + e, (R)0);
+            if (nup > kDirEntries) put_slot(3 + kDirEntries - 1u, ep);
+        }
+        tile++;
+        off += units;
+    });
 }
 
 // ---------------------------------------------------------------------------
@@ -1485,7 +1921,7 @@ struct GroupJob {
     R* P;
     R* offI;
     const SA<R>* sa;
-    double thr;
+    R thr;
     const uint4* hdr;
     const R* A;
     const Entry<R>* planes;
@@ -1523,6 +1959,7 @@ __global__ void __launch_bounds__(E) k_sweep_group_pack(const PackArgs<R> a) {
     Flux<R> fl{};
     fl.X = J.X;
     fl.I = J.I;
+    fl.ipos = nullptr;
     fl.P = J.P;
     fl.offI = J.offI;
     fl.sa = J.sa;
@@ -1675,7 +2112,9 @@ __device__ __forceinline__ void wave_count(bool pred, unsigned long long* counte
 // attenuation of the updated cell for the next sweep.
 template <typename R>
 __global__ void k_chemistry(Geo g, Flux<R> fl, ChemArgs ca, int lvl) {
-    int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    // a die takes consecutive cells: where I is gathered (direction sweeps),
+    // they share its lines in the die's L2
+    int64_t c = (int64_t)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     if (c == 0) g.need[lvl] = 0;  // the active-set list of this sweep level is current
     if (c >= g.N) return;
     int lev = g.level[c];
@@ -1690,8 +2129,9 @@ __global__ void k_chemistry(Geo g, Flux<R> fl, ChemArgs ca, int lvl) {
     const bool has_p = ps != kNone && fl.P;
     const double src = ca.src[c];
     double rate = 0.0;
+#pragma unroll 6
     for (int d = 0; d < g.D; d++) {
-        const double inc = (double)fl.I[(size_t)d * g.N + c] * ca.lref;
+        const double inc = (double)fl.I[iidx(fl, g.N, (uint32_t)d, (uint32_t)c)] * ca.lref;
         // current periodic source (k_periodic ran after the sweep)
         const double per = has_p ? (double)fl.P[(size_t)d * g.Nper + ps] * ca.lref : 0.0;
         rate += (inc + src) + per;  // sum over d of Site::get_rate, in direction order
@@ -1745,8 +2185,9 @@ __global__ void k_chem_outputs(Geo g, Flux<R> fl, ChemArgs ca, int which, double
     const bool has_p = ps != kNone && fl.P;
     const double src = ca.src[c];
     double rate = 0.0;
+#pragma unroll 6
     for (int d = 0; d < g.D; d++) {
-        const double inc = (double)fl.I[(size_t)d * g.N + c] * ca.lref;
+        const double inc = (double)fl.I[iidx(fl, g.N, (uint32_t)d, (uint32_t)c)] * ca.lref;
         const double per = has_p ? (double)fl.P[(size_t)d * g.Nper + ps] * ca.lref : 0.0;
         rate += (inc + src) + per;  // Site::get_rate (src/sweep/site.rs:53-56)
     }
@@ -1787,9 +2228,6 @@ __global__ void k_levels(Geo g, const double* change_ts, uint8_t* level, double 
 // order (wave after wave through LDS). Photon rate of 262144 cells x 84
 // directions: 9.2 ms with one thread per cell and its directions one after the
 // other, 2.46 ms like this.
-constexpr int kFluxDirs = 8;
-constexpr int kFluxCells = 64;
-
 template <typename R, bool kAll>
 __global__ void __launch_bounds__(1024) k_fluxes(Geo g, Flux<R> fl, double lref, double* I_out, double* O_out,
                                                  double* P_out, double* photon_rate, const uint32_t* rate_idx) {
@@ -1863,11 +2301,11 @@ __global__ void __launch_bounds__(1024) k_fluxes(Geo g, Flux<R> fl, double lref,
 // (262144 cells x 84 directions FP32: 88 MB; the pull takes 2.46 ms).
 template <typename R>
 __global__ void k_rate_sum(Geo g, Flux<R> fl, double lref, double* photon_rate, const uint32_t* rate_idx) {
-    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t c = (int64_t)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     if (c >= g.N) return;
     double total = 0.0;
 #pragma unroll 12
-    for (int d = 0; d < g.D; d++) total += (double)fl.I[(size_t)d * g.N + c] * lref;
+    for (int d = 0; d < g.D; d++) total += (double)fl.I[iidx(fl, g.N, (uint32_t)d, (uint32_t)c)] * lref;
     photon_rate[rate_idx ? rate_idx[c] : c] = total;
 }
 
@@ -1900,7 +2338,7 @@ __global__ void k_rotate_state(Geo g, Flux<R> fl, const double* __restrict__ kep
     const R o = (R)(out * fl.inv_lref);
     fl.X[xidx(fl, g.N, d, c)] = (Ar > (R)0) ? o / Ar : (R)0;
     const size_t oi = (size_t)d * g.N + c;
-    fl.I[oi] = (R)(inc * fl.inv_lref);
+    fl.I[iidx(fl, g.N, d, c)] = (R)(inc * fl.inv_lref);
     fl.offI[oi] = (R)(inc * fl.inv_lref);
     const uint32_t ps = g.pslot[c];
     if (ps != kNone && fl.P) {
@@ -2025,9 +2463,15 @@ struct ssw_sweep {
     bool graphs_on = true;                          // capture replays as graphs
     bool narrow_runs = true;                        // runs of narrow level sets in one workgroup
     bool dir_sweeps = false;                        // full sweeps: one workgroup per direction
-    uint4* d_dirrun = nullptr;                      // direction sweeps' run table (D x kmax)
-    uint32_t* d_dirlev = nullptr;                   // direction sweeps: level sets per direction
-    std::vector<uint2> dir_oq;                      // direction sweeps: {offset, first q} per (level set, direction)
+    // direction sweeps' schedule: tiles, their blobs, and per direction {first
+    // tile, tiles, level sets, wide}; the cell of every task in X's order, and
+    // in that order the cell inputs of the running sweep (k_dir_inputs); the
+    // upwind counts the build starts from
+    uint4 *d_dirblob = nullptr, *d_dirtiles = nullptr, *d_dirinfo = nullptr;
+    uint32_t* d_dircell = nullptr;
+    void* d_dirsa = nullptr;
+    uint8_t* d_dirlev = nullptr;
+    uint8_t* d_nup = nullptr;
     int group_request = kGroupLevels;               // level sets per grouped launch (1: off)
     int group_block = kGroupT;                      // grouped replay: root tasks per workgroup
     // grouped replay of full sweeps (compiled): per group of level sets its
@@ -2239,13 +2683,16 @@ Flux<R> make_flux(ssw_sweep* s) {
     f.X = (R*)s->d_X;
     f.xpos = s->compiled ? s->d_xpos : nullptr;
     f.I = (R*)s->d_I;
+    f.ipos = s->d_dirinfo ? s->d_xpos : nullptr;
     f.P = (R*)s->d_P;
     f.offI = (R*)s->d_offI;
     f.offP = (R*)s->d_offP;
     f.sa = (const SA<R>*)s->d_sa;
     f.inv_lref = 1.0 / s->lref;
     f.inv_aref = 1.0 / s->aref;
-    f.thr = s->p.significant_rate_threshold * f.inv_lref;
+    const double thr = s->p.significant_rate_threshold * f.inv_lref;
+    f.thr = (R)thr;
+    if ((double)f.thr < thr) f.thr = std::nextafter(f.thr, std::numeric_limits<R>::infinity());
     return f;
 }
 
@@ -2493,7 +2940,7 @@ int plan_replay(ssw_sweep* s, int lvl) {
     std::vector<uint4>& tab = s->runtab[lvl];
     plan.clear();
     tab.clear();
-    if (s->d_dirrun) {  // direction sweeps: one launch, restricted sweeps included
+    if (s->d_dirinfo) {  // direction sweeps: one launch, restricted sweeps included
         plan.push_back({0, s->kmax, 0u, 2});
         dfree(s, s->d_runtab[lvl]);
         return SSW_OK;
@@ -2773,71 +3220,133 @@ int build_groups(ssw_sweep* s) {
     s->groups.clear();
     s->group_tasks = 0;
     s->group_fallback = false;
-    if (!s->compiled || s->group_request < 2 || s->d_dirrun) return SSW_OK;  // direction sweeps need no cones
+    if (!s->compiled || s->group_request < 2 || s->d_dirinfo) return SSW_OK;  // direction sweeps need no cones
     return s->fp32 ? build_groups_t<float>(s) : build_groups_t<double>(s);
 }
 
-// The run table of the direction sweeps from every task's depth: per
-// direction d and level set k, {first position of k, width of k, offset of
-// d's tasks in k, their count}, and d's number of level sets (its tasks of
-// depth k exist for every k below its deepest, since a task of depth k has an
-// upwind task of depth k - 1 in its own direction).
-int build_dir_runs(ssw_sweep* s, const uint32_t* d_depth) {
-    const size_t DN = (size_t)s->D * s->N;
-    const size_t KD = (size_t)s->kmax * s->D;
-    uint32_t* d_cnt = nullptr;
-    Defer cleanup{[&] { dfree(s, d_cnt); }};
-    TRY(dalloc(s, &d_cnt, KD));
-    k_fill_u32<<<grid_for((int64_t)KD), kBlock, 0, s->stream>>>(d_cnt, 0u, (int64_t)KD);
-    k_dir_counts<<<grid_for((int64_t)DN), kBlock, 0, s->stream>>>(d_depth, (uint32_t)s->N, (uint32_t)s->D,
-                                                                  (uint32_t)DN, d_cnt);
+// The direction sweeps' schedule from every task's depth and upwind count:
+// tasks sorted by (direction, level set, class, cell), groups of 64 of a level
+// set, their tiles counted, placed and written. Takes d_depth (freed as soon as
+// it is no longer needed).
+template <typename R>
+int build_dir_schedule_t(ssw_sweep* s, uint32_t*& d_depth) {
+    using S = DirShape<R>;
+    const size_t DN = (size_t)s->D * s->N, KD = (size_t)s->kmax * s->D;
+    const uint32_t N = (uint32_t)s->N, D = (uint32_t)s->D, kmax = (uint32_t)s->kmax;
+    uint32_t *key = nullptr, *key2 = nullptr, *val = nullptr, *val2 = nullptr, *sorted = nullptr, *start = nullptr,
+             *first = nullptr, *gt = nullptr, *ts = nullptr, *at = nullptr, *tf = nullptr;
+    uint64_t *gu = nullptr, *us = nullptr;
+    uint8_t *tmp = nullptr, *nfar = nullptr;
+    uint4* groups = nullptr;
+    Defer cleanup{[&] {
+        for (uint32_t** p : {&key, &key2, &val, &val2, &sorted, &start, &first, &gt, &ts, &at, &tf}) dfree(s, *p);
+        dfree(s, gu);
+        dfree(s, us);
+        dfree(s, tmp);
+        dfree(s, nfar);
+        dfree(s, groups);
+        dfree(s, s->d_nup);
+    }};
+    Geo g = make_geo(s);
+    for (uint32_t** p : {&key, &key2, &val, &val2}) TRY(dalloc(s, p, DN));
+    k_dir_keys<<<grid_for((int64_t)DN), kBlock, 0, s->stream>>>(d_depth, s->d_nup, N, kmax, (uint32_t)DN, key, val);
+    int bits = 3;  // keys below D * kmax * 8 < 2^32 (kmax <= 2^22 + 1, D <= 127)
+    while (bits < 32 && (KD >> (bits - 3))) bits++;
+    hipcub::DoubleBuffer<uint32_t> kb(key, key2), vb(val, val2);
+    size_t tb = 0;
+    HIP_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, kb, vb, (int)DN, 0, bits, s->stream));
+    TRY(dalloc(s, &tmp, tb));
+    HIP_TRY(hipcub::DeviceRadixSort::SortPairs(tmp, tb, kb, vb, (int)DN, 0, bits, s->stream));
+    TRY(dalloc(s, &start, KD));
+    TRY(dalloc(s, &s->d_xpos, DN));
+    k_fill_u32<<<grid_for((int64_t)KD), kBlock, 0, s->stream>>>(start, kNone, (int64_t)KD);
+    TRY(dalloc(s, &s->d_dircell, DN));
+    k_dir_starts<<<grid_for((int64_t)DN), kBlock, 0, s->stream>>>(kb.Current(), vb.Current(), (uint32_t)DN, N, start,
+                                                                  s->d_xpos, s->d_dircell);
     HIP_TRY(hipGetLastError());
-    std::vector<uint32_t> cnt(KD);
-    HIP_TRY(hipMemcpyAsync(cnt.data(), d_cnt, KD * 4, hipMemcpyDeviceToHost, s->stream));
+    std::vector<uint32_t> hs(KD);
+    HIP_TRY(hipMemcpyAsync(hs.data(), start, KD * 4, hipMemcpyDeviceToHost, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
-    const std::vector<uint32_t>& fs = s->full_start;
-    std::vector<uint4> run(KD, make_uint4(0, 0, 0, 0));
-    std::vector<uint32_t> lev(s->D, 0), qs(s->D, 0);
-    s->dir_oq.assign(KD, make_uint2(0, 0));
-    for (int k = 0; k < s->kmax; k++) {
-        uint32_t off = 0;
-        for (int d = 0; d < s->D; d++) {
-            const uint32_t c = cnt[(size_t)k * s->D + d];
-            run[(size_t)d * s->kmax + k] = make_uint4(fs[k], fs[k + 1] - fs[k], off, c);
-            s->dir_oq[(size_t)k * s->D + d] = make_uint2(off, qs[d]);
-            if (c) {
-                if (lev[d] != (uint32_t)k) return fail(SSW_ERR_HIP, "direction sweeps: a direction skips a level set");
-                lev[d] = (uint32_t)k + 1;
-            }
-            off += c;
-            qs[d] += c;
+    sorted = vb.Current();  // owned by exactly one pointer
+    if (sorted == val) val = nullptr;
+    else val2 = nullptr;
+    dfree(s, tmp);
+    for (uint32_t** p : {&key, &key2, &val, &val2}) dfree(s, *p);
+    // level sets and widest level set of every direction, and the first group
+    // of every (direction, level set)
+    std::vector<uint32_t> hf(KD), at0(D + 1);
+    std::vector<uint4> info(D);
+    uint32_t ng = 0;
+    for (uint32_t d = 0; d < D; d++) {
+        at0[d] = ng;
+        uint32_t k = 0, widest = 0;
+        for (; k < kmax && hs[(size_t)d * kmax + k] != kNone; k++) {
+            const uint32_t b = hs[(size_t)d * kmax + k];
+            const uint32_t e = k + 1 < kmax && hs[(size_t)d * kmax + k + 1] != kNone ? hs[(size_t)d * kmax + k + 1]
+                                                                                     : (d + 1) * N;
+            if (e <= b) return fail(SSW_ERR_HIP, "direction sweeps: level set starts out of order");
+            widest = std::max(widest, e - b);
+            hf[(size_t)d * kmax + k] = ng;
+            ng += (e - b + 63) / 64;
         }
-        if (off != fs[k + 1] - fs[k]) return fail(SSW_ERR_HIP, "direction sweeps: level set counts differ");
-        if (off > kDirWidth) return fail(SSW_ERR_INVALID, "direction sweeps: a level set is too wide");
+        for (uint32_t j = k; j < kmax; j++)
+            if (hs[(size_t)d * kmax + j] != kNone) return fail(SSW_ERR_HIP, "direction sweeps: a direction skips a level set");
+        info[d] = make_uint4(0, 0, k, widest > S::kRing / 4 ? 1u : 0u);
     }
-    // full waits (kDirWait): at the end of level set k - 1 whenever the
-    // level sets since the last wait, k included, would hold more tasks than
-    // the LDS ring, so that every upwind value older than the ring was stored
-    // before a completed wait and barrier
-    const uint64_t ring = s->fp32 ? dir_ring<float>() : dir_ring<double>();
-    for (int d = 0; d < s->D; d++) {
-        uint64_t acc = 0;
-        for (uint32_t k = 0; k < lev[d]; k++) {
-            const uint64_t c = run[(size_t)d * s->kmax + k].w;
-            if (k > 0 && acc + c > ring) {
-                run[(size_t)d * s->kmax + k - 1].y |= kDirWait;
-                acc = 0;
-            }
-            acc += c;
-        }
+    at0[D] = ng;
+    TRY(dalloc(s, &first, KD));
+    TRY(dalloc(s, &groups, ng));
+    HIP_TRY(hipMemcpyAsync(first, hf.data(), KD * 4, hipMemcpyHostToDevice, s->stream));
+    k_dir_groups<<<grid_for((int64_t)KD), kBlock, 0, s->stream>>>(start, first, N, D, kmax, groups);
+    TRY(dalloc(s, &nfar, DN));
+    const unsigned nb = (unsigned)((s->N + kFluxCells - 1) / kFluxCells);
+    k_dir_far<R><<<nb, kFluxCells * ((D + kFluxDirs - 1) / kFluxDirs), 0, s->stream>>>(g, s->d_xpos, d_depth, start,
+                                                                                      kmax, nfar);
+    TRY(dalloc(s, &gt, (size_t)ng + 1));
+    TRY(dalloc(s, &ts, (size_t)ng + 1));
+    TRY(dalloc(s, &gu, (size_t)ng + 1));
+    TRY(dalloc(s, &us, (size_t)ng + 1));
+    HIP_TRY(hipMemsetAsync(gt + ng, 0, 4, s->stream));
+    HIP_TRY(hipMemsetAsync(gu + ng, 0, 8, s->stream));
+    const unsigned gb = (unsigned)((ng + kBlock / 64 - 1) / (kBlock / 64));
+    k_dir_tile_count<R><<<gb, kBlock, 0, s->stream>>>(groups, ng, sorted, s->d_nup, nfar, gt, gu);
+    HIP_TRY(hipGetLastError());
+    size_t t1 = 0, t2 = 0;
+    HIP_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, t1, gt, ts, (int)ng + 1, s->stream));
+    HIP_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, t2, gu, us, (int)ng + 1, s->stream));
+    TRY(dalloc(s, &tmp, std::max(t1, t2)));
+    HIP_TRY(hipcub::DeviceScan::ExclusiveSum(tmp, t1, gt, ts, (int)ng + 1, s->stream));
+    HIP_TRY(hipcub::DeviceScan::ExclusiveSum(tmp, t2, gu, us, (int)ng + 1, s->stream));
+    TRY(dalloc(s, &at, (size_t)D + 1));
+    TRY(dalloc(s, &tf, (size_t)D + 1));
+    HIP_TRY(hipMemcpyAsync(at, at0.data(), ((size_t)D + 1) * 4, hipMemcpyHostToDevice, s->stream));
+    k_gather_u32<<<grid_for(D + 1), kBlock, 0, s->stream>>>(ts, at, tf, D + 1);
+    HIP_TRY(hipGetLastError());
+    std::vector<uint32_t> htf(D + 1);
+    uint64_t units = 0;
+    HIP_TRY(hipMemcpyAsync(htf.data(), tf, ((size_t)D + 1) * 4, hipMemcpyDeviceToHost, s->stream));
+    HIP_TRY(hipMemcpyAsync(&units, us + ng, 8, hipMemcpyDeviceToHost, s->stream));
+    HIP_TRY(hipStreamSynchronize(s->stream));
+    for (uint32_t d = 0; d < D; d++) {
+        info[d].x = htf[d];
+        info[d].y = htf[d + 1] - htf[d];
     }
-    TRY(dalloc(s, &s->d_dirrun, KD));
-    TRY(dalloc(s, &s->d_dirlev, (size_t)s->D));
-    HIP_TRY(hipMemcpyAsync(s->d_dirrun, run.data(), KD * sizeof(uint4), hipMemcpyHostToDevice, s->stream));
-    HIP_TRY(hipMemcpyAsync(s->d_dirlev, lev.data(), (size_t)s->D * 4, hipMemcpyHostToDevice, s->stream));
+    dfree(s, d_depth);
+    dfree(s, tmp);
+    TRY(dalloc(s, (uint8_t**)&s->d_dirsa, DN * sizeof(SA<R>)));
+    if (s->p.num_timestep_levels > 1) TRY(dalloc(s, &s->d_dirlev, DN));
+    TRY(dalloc(s, &s->d_dirblob, (size_t)units));
+    TRY(dalloc(s, &s->d_dirtiles, 2 * (size_t)htf[D]));
+    TRY(dalloc(s, &s->d_dirinfo, (size_t)D));
+    HIP_TRY(hipMemcpyAsync(s->d_dirinfo, info.data(), D * sizeof(uint4), hipMemcpyHostToDevice, s->stream));
+    k_dir_tile_fill<R><<<gb, kBlock, 0, s->stream>>>(g, 1.0 / s->aref, groups, ng, sorted, s->d_nup, nfar, s->d_xpos, ts,
+                                                     us, tf, s->d_dirblob, s->d_dirtiles);
+    HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(s->stream));
     return SSW_OK;
 }
+
+int init_replay(ssw_sweep* s);
 
 // The full schedule, once per grid: Kahn layering of the whole graph, each
 // task's depth, a stable sort by depth of the tasks in (direction, cell)
@@ -2866,8 +3375,11 @@ int build_schedule(ssw_sweep* s) {
                                                                                                   d_depth);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(s->stream));
-    if (s->compiled && s->dir_sweeps) TRY(build_dir_runs(s, d_depth));
     dfree(s, s->d_flat);
+    if (s->compiled && s->dir_sweeps) {
+        TRY(s->fp32 ? build_dir_schedule_t<float>(s, d_depth) : build_dir_schedule_t<double>(s, d_depth));
+        return init_replay(s);
+    }
     TRY(dalloc(s, &d_keys, DN));
     TRY(dalloc(s, &d_vals, DN));
     TRY(dalloc(s, &d_vals2, DN));
@@ -2897,22 +3409,7 @@ int build_schedule(ssw_sweep* s) {
     const double inv_aref = 1.0 / s->aref;
     if (s->compiled) {
         TRY(dalloc(s, &s->d_xpos, DN));
-        if (s->d_dirrun) {  // direction sweeps: X in each direction's Kahn order
-            uint2* d_oq = nullptr;
-            Defer free_oq{[&] { dfree(s, d_oq); }};
-            TRY(dalloc(s, &d_oq, s->dir_oq.size()));
-            HIP_TRY(hipMemcpyAsync(d_oq, s->dir_oq.data(), s->dir_oq.size() * sizeof(uint2), hipMemcpyHostToDevice,
-                                   s->stream));
-            k_invert_dir<<<grid_for((int64_t)DN), kBlock, 0, s->stream>>>(d_sorted, s->d_fstart, s->kmax, d_oq,
-                                                                         (uint32_t)s->N, (uint32_t)s->D, s->d_xpos,
-                                                                         (uint32_t)DN);
-            HIP_TRY(hipGetLastError());
-            HIP_TRY(hipStreamSynchronize(s->stream));
-            s->dir_oq.clear();
-            s->dir_oq.shrink_to_fit();
-        } else {
-            k_invert<<<grid_for((int64_t)DN), kBlock, 0, s->stream>>>(d_sorted, s->d_xpos, (uint32_t)DN);
-        }
+        k_invert<<<grid_for((int64_t)DN), kBlock, 0, s->stream>>>(d_sorted, s->d_xpos, (uint32_t)DN);
         TRY(dalloc(s, &s->d_hdr, DN));
         TRY(dalloc(s, (uint8_t**)&s->d_A, DN * real_size(s)));
         TRY(dalloc(s, (uint8_t**)&s->d_planes, (size_t)kPlanes * DN * entry_size(s)));
@@ -2958,6 +3455,12 @@ int build_schedule(ssw_sweep* s) {
                                              s->stream));
     TRY(dalloc(s, (uint8_t**)&s->d_scan_tmp, s->scan_tmp_bytes));
     HIP_TRY(hipStreamSynchronize(s->stream));
+    return init_replay(s);
+}
+
+// Empty active-set lists, plans and graphs, the cones of the grouped replay,
+// and the full sweep's plan.
+int init_replay(ssw_sweep* s) {
     const int L = s->p.num_timestep_levels;
     for (uint32_t*& p : s->d_idx) dfree(s, p);
     s->d_idx.assign(L, nullptr);
@@ -3055,7 +3558,7 @@ int make_group_list(ssw_sweep* s, int lvl) {
 }
 
 int make_list(ssw_sweep* s, int lvl) {
-    if (s->d_dirrun) {  // direction sweeps pass every task and test its level: no list
+    if (s->d_dirinfo) {  // direction sweeps pass every task and test its level: no list
         uint32_t* d_min = nullptr;
         Defer free_min{[&] { dfree(s, d_min); }};
         TRY(dalloc(s, &d_min, 1));
@@ -3121,8 +3624,18 @@ void launch_item_t(ssw_sweep* s, const Geo& g, const Flux<R>& fl, int lvl, const
     const uint32_t* idx = all ? nullptr : s->d_idx[lvl];
     const Entry<R>* ovf = (const Entry<R>*)s->d_ovf;
     if (it.group == 2) {  // direction sweeps: one workgroup per direction
-        k_sweep_dir<R><<<s->D, kDirBlock, 0, st>>>(g, fl, s->d_hdr, (const R*)s->d_A, (const Entry<R>*)s->d_planes,
-                                                    ovf, s->d_dirrun, s->kmax, s->d_dirlev, all ? 0 : lvl);
+        constexpr int lanes = 64 * DirShape<R>::kWaves;
+        const int at = all ? 0 : lvl;
+        const uint32_t DN = (uint32_t)(s->D * s->N);
+        SA<R>* sas = (SA<R>*)s->d_dirsa;
+        k_dir_inputs<R><<<grid_for(DN), kBlock, 0, st>>>(s->d_dircell, fl.sa, g.level, sas, at ? s->d_dirlev : nullptr,
+                                                         DN);
+        if (at == 0 && !fl.offI)
+            k_sweep_dir<R, false><<<s->D, lanes, 0, st>>>(g, fl, s->d_dirblob, s->d_dirtiles, s->d_dirinfo, sas,
+                                                          s->d_dirlev, 0);
+        else
+            k_sweep_dir<R, true><<<s->D, lanes, 0, st>>>(g, fl, s->d_dirblob, s->d_dirtiles, s->d_dirinfo, sas,
+                                                         s->d_dirlev, at);
         return;
     }
     if (it.group) {
@@ -3792,8 +4305,13 @@ void free_grid(ssw_sweep* s) {
     dfree(s, s->d_cnt);
     dfree(s, s->d_level);
     dfree(s, s->d_fstart);
-    dfree(s, s->d_dirrun);
+    dfree(s, s->d_dirblob);
+    dfree(s, s->d_dirtiles);
+    dfree(s, s->d_dirinfo);
+    dfree(s, s->d_dircell);
+    dfree(s, s->d_dirsa);
     dfree(s, s->d_dirlev);
+    dfree(s, s->d_nup);
     dfree(s, s->d_recs);
     dfree(s, s->d_hdr);
     dfree(s, s->d_A);
@@ -3879,7 +4397,11 @@ int build_direction_graph(ssw_sweep* s, bool choose_mode) {
     HIP_TRY(hipMemsetAsync(d_stats, 0, 5 * 8, s->stream));
     Geo g = make_geo(s);
     if (choose_mode) k_check_mirror<<<grid_for(n), kBlock, 0, s->stream>>>(g, d_stats);
-    k_face_stats<<<grid_for((int64_t)DN), kBlock, 0, s->stream>>>(g, d_stats + 1, s->d_cnt);
+    const bool dir = s->dir_sweeps && (choose_mode ? s->mode_request != SSW_TRANSPORT_MODE_GEOMETRIC : s->compiled);
+    if (dir) TRY(dalloc(s, &s->d_nup, DN));
+    k_face_stats<<<(unsigned)((n + kFluxCells - 1) / kFluxCells),
+                   kFluxCells * ((s->D + kFluxDirs - 1) / kFluxDirs), 0, s->stream>>>(g, d_stats + 1, s->d_cnt,
+                                                                                      s->d_nup);
     HIP_TRY(hipGetLastError());
     unsigned long long hb[5] = {0, 0, 0, 0, 0};
     HIP_TRY(hipMemcpyAsync(hb, d_stats, sizeof(hb), hipMemcpyDeviceToHost, s->stream));
@@ -3891,7 +4413,7 @@ int build_direction_graph(ssw_sweep* s, bool choose_mode) {
     for (int k = 0; k < 3; k++) s->dw[k] = (double)hb[k + 1] / ((double)n * s->D);
     s->ovf_total = (int64_t)hb[4];
     if (!choose_mode) {
-        if (s->compiled) TRY(setup_overflow(s, s->d_cnt));
+        if (s->compiled && !dir) TRY(setup_overflow(s, s->d_cnt));
         return build_schedule(s);
     }
     // transport mode: compiled when, at its peak (schedule arrays, overflow
@@ -3909,7 +4431,8 @@ int build_direction_graph(ssw_sweep* s, bool choose_mode) {
     if (s->mode_request == SSW_TRANSPORT_MODE_COMPILED) s->compiled = true;
     else if (s->mode_request == SSW_TRANSPORT_MODE_GEOMETRIC) s->compiled = false;
     else s->compiled = (double)comp_need <= 0.85 * (double)free_b;
-    if (s->compiled) TRY(setup_overflow(s, s->d_cnt));
+    if (!s->compiled) dfree(s, s->d_nup);
+    if (s->compiled && !dir) TRY(setup_overflow(s, s->d_cnt));
     return build_schedule(s);
 }
 
@@ -4604,19 +5127,25 @@ int ssw_download_transport(ssw_sweep* s, void* X, void* I) {
     const size_t m = (size_t)DN * real_size(s);
     uint8_t* dtmp = nullptr;
     Defer cleanup{[&] { dfree(s, dtmp); }};
-    if (X && s->compiled) {  // X is stored in schedule-position order
-        TRY(dalloc(s, &dtmp, m));
-        if (s->fp32)
-            k_gather_x<float><<<grid_for(DN), kBlock, 0, s->stream>>>((const float*)s->d_X, s->d_xpos,
-                                                                      (float*)dtmp, DN);
-        else
-            k_gather_x<double><<<grid_for(DN), kBlock, 0, s->stream>>>((const double*)s->d_X, s->d_xpos,
-                                                                       (double*)dtmp, DN);
-        HIP_TRY(hipGetLastError());
-    }
-    if (X) HIP_TRY(hipMemcpyAsync(X, dtmp ? (void*)dtmp : s->d_X, m, hipMemcpyDeviceToHost, s->stream));
-    if (I) HIP_TRY(hipMemcpyAsync(I, s->d_I, m, hipMemcpyDeviceToHost, s->stream));
-    HIP_TRY(hipStreamSynchronize(s->stream));
+    // X, and in direction sweeps I, is stored in schedule-position order
+    auto get = [&](void* out, const void* in, bool ordered) -> int {
+        if (!out) return SSW_OK;
+        if (ordered) {
+            if (!dtmp) TRY(dalloc(s, &dtmp, m));
+            if (s->fp32)
+                k_gather_x<float><<<grid_for(DN), kBlock, 0, s->stream>>>((const float*)in, s->d_xpos, (float*)dtmp, DN);
+            else
+                k_gather_x<double><<<grid_for(DN), kBlock, 0, s->stream>>>((const double*)in, s->d_xpos, (double*)dtmp,
+                                                                           DN);
+            HIP_TRY(hipGetLastError());
+            in = dtmp;
+        }
+        HIP_TRY(hipMemcpyAsync(out, in, m, hipMemcpyDeviceToHost, s->stream));
+        HIP_TRY(hipStreamSynchronize(s->stream));
+        return SSW_OK;
+    };
+    TRY(get(X, s->d_X, s->compiled));
+    TRY(get(I, s->d_I, s->d_dirinfo != nullptr));
     dfree(s, dtmp);
     for (void* a : {X, I}) {
         if (!a) continue;
@@ -4697,7 +5226,12 @@ int save_t(ssw_sweep* s, uint8_t* buf) {
         HIP_TRY(hipGetLastError());
     }
     HIP_TRY(hipMemcpyAsync(X, tmp ? (void*)tmp : s->d_X, DN * sizeof(R), hipMemcpyDeviceToHost, s->stream));
-    HIP_TRY(hipMemcpyAsync(I, s->d_I, DN * sizeof(R), hipMemcpyDeviceToHost, s->stream));
+    if (s->d_dirinfo) {  // I in X's order
+        HIP_TRY(hipStreamSynchronize(s->stream));
+        k_gather_x<R><<<grid_for(DN), kBlock, 0, s->stream>>>((const R*)s->d_I, s->d_xpos, tmp, DN);
+        HIP_TRY(hipGetLastError());
+    }
+    HIP_TRY(hipMemcpyAsync(I, s->d_dirinfo ? (void*)tmp : s->d_I, DN * sizeof(R), hipMemcpyDeviceToHost, s->stream));
     std::vector<R> Pd((size_t)s->D * s->Nper);
     if (s->Nper)
         HIP_TRY(hipMemcpyAsync(Pd.data(), s->d_P, Pd.size() * sizeof(R), hipMemcpyDeviceToHost, s->stream));
@@ -4774,7 +5308,13 @@ int load_t(ssw_sweep* s, const uint8_t* buf) {
     } else {
         HIP_TRY(hipMemcpyAsync(s->d_X, X.data(), DN * sizeof(R), hipMemcpyHostToDevice, s->stream));
     }
-    HIP_TRY(hipMemcpyAsync(s->d_I, I.data(), DN * sizeof(R), hipMemcpyHostToDevice, s->stream));
+    if (s->d_dirinfo) {  // I in X's order
+        HIP_TRY(hipMemcpyAsync(tmp, I.data(), DN * sizeof(R), hipMemcpyHostToDevice, s->stream));
+        k_scatter_x<R><<<grid_for(DN), kBlock, 0, s->stream>>>((R*)s->d_I, s->d_xpos, tmp, DN);
+        HIP_TRY(hipGetLastError());
+    } else {
+        HIP_TRY(hipMemcpyAsync(s->d_I, I.data(), DN * sizeof(R), hipMemcpyHostToDevice, s->stream));
+    }
     if (s->Nper)
         HIP_TRY(hipMemcpyAsync(s->d_P, Pd.data(), Pd.size() * sizeof(R), hipMemcpyHostToDevice, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
@@ -4856,7 +5396,7 @@ int ssw_get_info(ssw_sweep* s, ssw_info* info) {
     info->replay_block = s->rec_block;
     info->graph_replay = s->graphs_on ? 1 : 0;
     info->narrow_runs = (s->compiled && s->narrow_runs) ? 1 : 0;
-    info->direction_sweeps = s->d_dirrun ? 1 : 0;
+    info->direction_sweeps = s->d_dirinfo ? 1 : 0;
     info->group_levels = s->groups.empty() ? 1 : s->group_request;
     info->group_fallback = s->group_fallback ? 1 : 0;
     info->group_tasks = s->group_tasks;
