@@ -70,48 +70,50 @@ struct Cell {
 };
 
 // --- rate fits (hydrogen_only/mod.rs:161-302) ---------------------------------
-SSW_HD double fit_collision(double t) {
-    return sqrt(t) / (1.0 + sqrt(t / 1e5)) * exp(-157809.1 / t);
+// The fits take the exponentials and powers they contain as arguments, so that
+// a solver step gathers them and evaluates them together (transcendentals
+// below): they are nearly all of its time, and on the device the lanes of a
+// quad share them.
+SSW_HD double fit_collision(double t, double e) {  // e = exp(-157809.1 / t)
+    return sqrt(t) / (1.0 + sqrt(t / 1e5)) * e;
 }
-SSW_HD double fit_collision_dt(double t) {
+SSW_HD double fit_collision_dt(double t, double e) {
     const double k1 = 1.0 / 1e5, k2 = 157809.1;
     double s = sqrt(k1 * t);
-    return (exp(-k2 / t) * (k1 * k2 * t + 0.5 * s * (2.0 * k2 + t))) /
+    return (e * (k1 * k2 * t + 0.5 * s * (2.0 * k2 + t))) /
            (sqrt(powi(t, 3)) * s * powi(s + 1.0, 2));
 }
-SSW_HD double alpha_b(double T) {
-    double l = 315614.0 / T;
-    return (2.753e-14 * pow(l, 1.5) / pow(1.0 + pow(l / 2.74, 0.407), 2.242)) * kCm3PerS;
-}
-SSW_HD double alpha_b_dt(double T) {
+// alpha_B: l15 = l^1.5, w = (1 + (l / 2.74)^0.407)^2.242 with l = 315614 / T
+SSW_HD double alpha_b(double l15, double w) { return (2.753e-14 * l15 / w) * kCm3PerS; }
+// p = (k1 l)^0.407, w = (p + 1)^(-3.242)
+SSW_HD double alpha_b_dt(double T, double p, double w) {
     double l = 315614.0 / T;
     double dl = -315614.0 / (T * T);
-    const double k1 = 1.0 / 2.74, k2 = 0.407, k3 = 2.242;
-    double p = pow(k1 * l, k2);
-    double d = -sqrt(l) * pow(p + 1.0, -k3 - 1.0) * (k2 * k3 * p - 1.5 * p - 1.5);
+    const double k2 = 0.407, k3 = 2.242;
+    double d = -sqrt(l) * w * (k2 * k3 * p - 1.5 * p - 1.5);
     return ((2.753e-14 * d) * kCm3PerS) * dl;
 }
-SSW_HD double recomb_cooling(double T) {
-    double l = 315614.0 / T;
-    return (3.435e-30 * T * pow(l, 1.97) / pow(1.0 + pow(l / 2.25, 0.376), 3.72)) * kErgCm3PerS;
+// l197 = l^1.97, w = (1 + (l / 2.25)^0.376)^3.72
+SSW_HD double recomb_cooling(double T, double l197, double w) {
+    return (3.435e-30 * T * l197 / w) * kErgCm3PerS;
 }
-SSW_HD double recomb_cooling_dt(double T) {
-    const double k1 = 315614.0, k2 = 1.97, k3 = 0.376, k4 = 3.72, k5 = 2.25;
-    double q = pow(k1 / (k5 * T), k3);
-    double v = pow(1.0 + q, -1.0 - k4) * (1.0 - 1.0 * k2 + (1.0 - 1.0 * k2 + k3 * k4) * q) * pow(k1 / T, k2);
+// q = (k1 / (k5 T))^0.376, w = (1 + q)^(-4.72)
+SSW_HD double recomb_cooling_dt(double l197, double q, double w) {
+    const double k2 = 1.97, k3 = 0.376, k4 = 3.72;
+    double v = w * (1.0 - 1.0 * k2 + (1.0 - 1.0 * k2 + k3 * k4) * q) * l197;
     return ((3.435e-30 * v) * kErgCm3PerS) / 1.0;
 }
-SSW_HD double beta_ci(double T) { return (5.85e-11 * fit_collision(T)) * kCm3PerS; }
-SSW_HD double beta_ci_dt(double T) { return ((5.85e-11 * fit_collision_dt(T)) * kCm3PerS) / 1.0; }
-SSW_HD double ci_cooling(double T) { return (1.27e-21 * fit_collision(T)) * kErgCm3PerS; }
-SSW_HD double ci_cooling_dt(double T) { return ((1.27e-21 * fit_collision_dt(T)) * kErgCm3PerS) / 1.0; }
-SSW_HD double ce_cooling(double T) {
-    return (7.5e-19 / (1.0 + sqrt(T / 1e5)) * exp(-118348.0 / T)) * kErgCm3PerS;
+SSW_HD double beta_ci(double T, double e) { return (5.85e-11 * fit_collision(T, e)) * kCm3PerS; }
+SSW_HD double beta_ci_dt(double T, double e) { return ((5.85e-11 * fit_collision_dt(T, e)) * kCm3PerS) / 1.0; }
+SSW_HD double ci_cooling(double T, double e) { return (1.27e-21 * fit_collision(T, e)) * kErgCm3PerS; }
+SSW_HD double ci_cooling_dt(double T, double e) { return ((1.27e-21 * fit_collision_dt(T, e)) * kErgCm3PerS) / 1.0; }
+SSW_HD double ce_cooling(double T, double e) {  // e = exp(-118348 / T)
+    return (7.5e-19 / (1.0 + sqrt(T / 1e5)) * e) * kErgCm3PerS;
 }
-SSW_HD double ce_cooling_dt(double T) {
+SSW_HD double ce_cooling_dt(double T, double e) {
     const double k1 = 7.5e-19, k2 = 118348.0, k3 = 1.0 / 1e5;
     double s = sqrt(k3 * T);
-    double v = (k1 * exp(-k2 / T) * (k2 * k3 * T - 0.5 * k3 * powi(T, 2) + k2 * s)) /
+    double v = (k1 * e * (k2 * k3 * T - 0.5 * k3 * powi(T, 2) + k2 * s)) /
                (powi(T, 2) * s * powi(1.0 + s, 2));
     return (v * kErgCm3PerS) / 1.0;
 }
@@ -132,41 +134,125 @@ SSW_HD double n_hii(const Cell& c) { return n_h(c) * c.x; }
 SSW_HD double n_hi(const Cell& c) { return n_h(c) * (1.0 - c.x); }
 SSW_HD double mu(const Cell& c) { return 1.0 / (c.x + 1.0); }
 
-SSW_HD double cooling(const Cell& c) {
+// Powers and exponentials of up to four argument pairs at once: one after the
+// other, or (Quad) one per lane of a quad.
+struct Serial {
+    template <int kN>
+    SSW_HD void powers(const double (&b)[kN], const double (&e)[kN], double (&out)[kN]) const {
+#pragma unroll
+        for (int i = 0; i < kN; i++) out[i] = pow(b[i], e[i]);
+    }
+    template <int kN>
+    SSW_HD void exps(const double (&a)[kN], double (&out)[kN]) const {
+#pragma unroll
+        for (int i = 0; i < kN; i++) out[i] = exp(a[i]);
+    }
+};
+
+#if defined(__HIPCC__)
+// The four lanes of a quad hold the same cell: each evaluates one of the
+// arguments and all get the results (the same calls, so the same bits).
+struct Quad {
+    template <int kI>
+    static __device__ __forceinline__ double from(double v) {  // lane kI's value, on every lane of the quad
+        const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), kI * 0x55, 0xF, 0xF, true);
+        const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), kI * 0x55, 0xF, 0xF, true);
+        return __hiloint2double(hi, lo);
+    }
+    template <int kN>
+    static __device__ __forceinline__ double mine(const double (&a)[kN]) {
+        const unsigned r = threadIdx.x & 3u;
+        double v = a[0];
+#pragma unroll
+        for (int i = 1; i < kN; i++) v = r == (unsigned)i ? a[i] : v;
+        return v;
+    }
+    template <int kN>
+    static __device__ __forceinline__ void share(double v, double (&out)[kN]) {
+        static_assert(kN <= 4, "one argument per lane of a quad");
+        out[0] = from<0>(v);
+        if constexpr (kN > 1) out[1] = from<1>(v);
+        if constexpr (kN > 2) out[2] = from<2>(v);
+        if constexpr (kN > 3) out[3] = from<3>(v);
+    }
+    template <int kN>
+    __device__ __forceinline__ void powers(const double (&b)[kN], const double (&e)[kN], double (&out)[kN]) const {
+        share(pow(mine(b), mine(e)), out);
+    }
+    template <int kN>
+    __device__ __forceinline__ void exps(const double (&a)[kN], double (&out)[kN]) const {
+        share(exp(mine(a)), out);
+    }
+};
+#endif
+
+// What the temperature's step takes: cooling and its derivative at T, and the
+// transmitted fraction of the cell (the ionised fraction's step has it too).
+struct HeatRates {
+    double ce, ci, pass;    // exp(-118348 / T), exp(-157809.1 / T), exp(-n_HI sigma L)
+    double l197, w, q, wd;  // recomb_cooling's and recomb_cooling_dt's powers
+};
+struct IonRates {
+    double ci;              // exp(-157809.1 / T)
+    double l15, w, p, wd;   // alpha_b's and alpha_b_dt's powers
+};
+
+template <typename Ev>
+SSW_HD HeatRates heat_rates(const Cell& c, const Ev& ev) {
+    const double l = 315614.0 / c.T;
+    const double k1 = 315614.0, k4 = 3.72, k5 = 2.25;
+    double p[3], w[2], e[3];
+    ev.template powers<3>({l, l / 2.25, k1 / (k5 * c.T)}, {1.97, 0.376, 0.376}, p);
+    ev.template powers<2>({1.0 + p[1], 1.0 + p[2]}, {3.72, -1.0 - k4}, w);
+    ev.template exps<3>({-118348.0 / c.T, -157809.1 / c.T, -n_hi(c) * kSigma * c.len}, e);
+    return {e[0], e[1], e[2], p[0], w[0], p[2], w[1]};
+}
+template <typename Ev>
+SSW_HD IonRates ion_rates(const Cell& c, const Ev& ev) {
+    const double l = 315614.0 / c.T;
+    const double k1 = 1.0 / 2.74, k3 = 2.242;
+    double p[3], w[2], e[1];
+    ev.template powers<3>({l, l / 2.74, k1 * l}, {1.5, 0.407, 0.407}, p);
+    ev.template powers<2>({1.0 + p[1], p[2] + 1.0}, {2.242, -k3 - 1.0}, w);
+    ev.template exps<1>({-157809.1 / c.T}, e);
+    return {e[0], p[0], w[0], p[2], w[1]};
+}
+
+SSW_HD double cooling(const Cell& c, const HeatRates& r) {
     double ne = n_hii(c), n0 = n_hi(c), n1 = n_hii(c);
-    double coll = (ce_cooling(c.T) + ci_cooling(c.T)) * ne * n0;
-    double rec = recomb_cooling(c.T) * ne * n1;
+    double coll = (ce_cooling(c.T, r.ce) + ci_cooling(c.T, r.ci)) * ne * n0;
+    double rec = recomb_cooling(c.T, r.l197, r.w) * ne * n1;
     double br = brems_cooling(c.T) * ne * n1;
     double co = compton_cooling(c.T, c.a) * ne;
     return coll + rec + br + co;
 }
-SSW_HD double cooling_dt(const Cell& c) {
+SSW_HD double cooling_dt(const Cell& c, const HeatRates& r) {
     double ne = n_hii(c), n0 = n_hi(c), n1 = n_hii(c);
-    double coll = (ce_cooling_dt(c.T) + ci_cooling_dt(c.T)) * ne * n0;
-    double rec = recomb_cooling_dt(c.T) * ne * n1;
+    double coll = (ce_cooling_dt(c.T, r.ce) + ci_cooling_dt(c.T, r.ci)) * ne * n0;
+    double rec = recomb_cooling_dt(r.l197, r.q, r.wd) * ne * n1;
     double br = brems_cooling_dt(c.T) * ne * n1;
     double co = compton_cooling_dt(c.a) * ne;
     return coll + rec + br + co;
 }
-SSW_HD double newly_ionized(const Cell& c, double dt) {  // :312-319
-    double absorbed = 1.0 - exp(-n_hi(c) * kSigma * c.len);
+SSW_HD double newly_ionized(const Cell& c, double dt, double pass) {  // :312-319
+    double absorbed = 1.0 - pass;
     double photons = dt * c.rate;
     return photons * absorbed;
 }
-SSW_HD double delta_temperature(const Cell& c, double dt) {  // :304-310
+SSW_HD double delta_temperature(const Cell& c, double dt, const HeatRates& r) {  // :304-310
     double k = (kGamma - 1.0) * kProtonMass / (c.rho * kBoltzmann);
-    double heat = newly_ionized(c, dt) / c.vol * (kPhotonEnergy - kRydberg) / dt;  // photoheating_rate
-    double lam = heat - cooling(c);
-    double dlam = -cooling_dt(c);
+    double heat = newly_ionized(c, dt, r.pass) / c.vol * (kPhotonEnergy - kRydberg) / dt;  // photoheating_rate
+    double lam = heat - cooling(c, r);
+    double dlam = -cooling_dt(c, r);
     double m = mu(c);
     return k * m * lam * dt / (1.0 - k * m * dlam * dt);
 }
-SSW_HD double delta_ionized(const Cell& c, double dt) {  // :334-354 (Rosdahl+15 A23)
+SSW_HD double delta_ionized(const Cell& c, double dt, const IonRates& r, double pass) {  // :334-354 (Rosdahl+15 A23)
     double nh = n_h(c);
     double ne = n_hii(c);
-    double al = alpha_b(c.T), dal = alpha_b_dt(c.T);
-    double be = beta_ci(c.T), dbe = beta_ci_dt(c.T);
-    double gam = newly_ionized(c, dt) / (n_hi(c) * c.vol) / dt;  // photoionization_rate
+    double al = alpha_b(r.l15, r.w), dal = alpha_b_dt(c.T, r.p, r.wd);
+    double be = beta_ci(c.T, r.ci), dbe = beta_ci_dt(c.T, r.ci);
+    double gam = newly_ionized(c, dt, pass) / (n_hi(c) * c.vol) / dt;  // photoionization_rate
     double cc = be * ne + gam;
     double m = mu(c);
     double dd = al * ne;
@@ -183,20 +269,22 @@ SSW_HD double delta_ionized(const Cell& c, double dt) {  // :334-354 (Rosdahl+15
 // evaluated with the fixed timestep of :15-19 (1 yr = 3.15576e7 s,
 // src/units/mod.rs:48) on the state after the step, without a floor
 constexpr double kYear = 3.15576e7;
-SSW_HD double photoionization_rate(const Cell& c, double dt) {  // hydrogen_only/mod.rs:327-332
-    return newly_ionized(c, dt) / (n_hi(c) * c.vol) / dt;
+SSW_HD double photoionization_rate(const Cell& c, double dt, double pass) {  // hydrogen_only/mod.rs:327-332
+    return newly_ionized(c, dt, pass) / (n_hi(c) * c.vol) / dt;
 }
-SSW_HD double photoheating_rate(const Cell& c, double dt) {  // :321-325
-    return newly_ionized(c, dt) / c.vol * (kPhotonEnergy - kRydberg) / dt;
+SSW_HD double photoheating_rate(const Cell& c, double dt, double pass) {  // :321-325
+    return newly_ionized(c, dt, pass) / c.vol * (kPhotonEnergy - kRydberg) / dt;
 }
 // which: 0 PhotoionizationRate, 1 HeatingRate (photoheating - cooling),
 // 2 RecombinationRate (alpha_B n_e x), 3 CollisionalIonizationRate (beta n_e (1 - x))
 SSW_HD double chemistry_output(const Cell& c, int which) {
+    const HeatRates h = heat_rates(c, Serial());
+    const IonRates i = ion_rates(c, Serial());
     switch (which) {
-        case 0: return photoionization_rate(c, kYear);
-        case 1: return photoheating_rate(c, kYear) - cooling(c);
-        case 2: return alpha_b(c.T) * n_hii(c) * c.x;
-        default: return beta_ci(c.T) * n_hii(c) * (1.0 - c.x);
+        case 0: return photoionization_rate(c, kYear, h.pass);
+        case 1: return photoheating_rate(c, kYear, h.pass) - cooling(c, h);
+        case 2: return alpha_b(i.l15, i.w) * n_hii(c) * c.x;
+        default: return beta_ci(c.T, i.ci) * n_hii(c) * (1.0 - c.x);
     }
 }
 
@@ -225,11 +313,13 @@ SSW_HD bool accept(double& value, double change, double safety, double dt, doubl
 }
 
 // try_timestep_update (:371-392)
-SSW_HD bool try_step(Cell& c, const Floor& f, double dt, double safety, double& ts, int& proc) {
-    double dT = delta_temperature(c, dt);
+template <typename Ev>
+SSW_HD bool try_step(Cell& c, const Floor& f, double dt, double safety, double& ts, int& proc, const Ev& ev) {
+    const HeatRates h = heat_rates(c, ev);
+    double dT = delta_temperature(c, dt, h);
     double tsT;
     if (!accept(c.T, dT, safety, dt, tsT)) return false;
-    double dx = delta_ionized(c, dt);
+    double dx = delta_ionized(c, dt, ion_rates(c, ev), h.pass);
     double tsx;
     if (!accept(c.x, dx, safety, dt, tsx)) return false;
     clamp_state(c, f);
@@ -243,40 +333,60 @@ SSW_HD bool try_step(Cell& c, const Floor& f, double dt, double safety, double& 
     return true;
 }
 
+// A cell's walk through its sub-steps: the pending second halves (bit =
+// depth), the current depth and step, and the timescale and process of the
+// last accepted step.
+struct Walk {
+    uint64_t lo = 0, hi = 0;
+    int depth = 0;
+    double dt = 0.0, ts = 0.0;
+    int proc = kProcTemperature;
+    bool failed = false;
+};
+
+// One attempt of perform_timestep (:394-441); true when the walk has ended,
+// with its timescale in w.ts (dt0 / 10 and w.failed on depth overflow).
+template <typename Ev>
+SSW_HD bool walk_step(Cell& c, const Floor& f, double dt0, double safety, Walk& w, const Ev& ev) {
+    clamp_state(c, f);
+    double T0 = c.T, x0 = c.x;
+    if (w.depth > kMaxDepth) {
+        w.failed = true;
+        w.proc = kProcTemperature;
+        w.ts = dt0 / 10.0;
+        return true;
+    }
+    if (try_step(c, f, w.dt, safety, w.ts, w.proc, ev)) {
+        if (w.lo == 0 && w.hi == 0) return true;
+        if (w.hi) {
+            w.depth = 127 - __builtin_clzll(w.hi);
+            w.hi &= ~(1ull << (w.depth - 64));
+        } else {
+            w.depth = 63 - __builtin_clzll(w.lo);
+            w.lo &= ~(1ull << w.depth);
+        }
+        w.dt = dt0;
+        for (int k = 0; k < w.depth; k++) w.dt = w.dt / 2.0;
+    } else {
+        c.T = T0;
+        c.x = x0;
+        w.depth += 1;
+        if (w.depth < 64) w.lo |= 1ull << w.depth;
+        else w.hi |= 1ull << (w.depth - 64);
+        w.dt = w.dt / 2.0;
+    }
+    return false;
+}
+
 // perform_timestep (:394-441). Returns the timescale; *failed on depth overflow.
 SSW_HD double perform_timestep(Cell& c, const Floor& f, double dt0, double safety, int& proc, bool& failed) {
-    uint64_t pend_lo = 0, pend_hi = 0;  // pending second halves, bit = depth
-    int depth = 0;
-    double dt = dt0;
-    double ts = 0.0;
-    failed = false;
-    for (;;) {
-        clamp_state(c, f);
-        double T0 = c.T, x0 = c.x;
-        if (depth > kMaxDepth) {
-            failed = true;
-            proc = kProcTemperature;
-            return dt0 / 10.0;
-        }
-        if (try_step(c, f, dt, safety, ts, proc)) {
-            if (pend_lo == 0 && pend_hi == 0) return ts;
-            if (pend_hi) {
-                depth = 127 - __builtin_clzll(pend_hi);
-                pend_hi &= ~(1ull << (depth - 64));
-            } else {
-                depth = 63 - __builtin_clzll(pend_lo);
-                pend_lo &= ~(1ull << depth);
-            }
-        } else {
-            c.T = T0;
-            c.x = x0;
-            depth += 1;
-            if (depth < 64) pend_lo |= 1ull << depth;
-            else pend_hi |= 1ull << (depth - 64);
-        }
-        dt = dt0;
-        for (int k = 0; k < depth; k++) dt = dt / 2.0;
+    Walk w;
+    w.dt = dt0;
+    while (!walk_step(c, f, dt0, safety, w, Serial())) {
     }
+    proc = w.proc;
+    failed = w.failed;
+    return w.ts;
 }
 
 }  // namespace ssw

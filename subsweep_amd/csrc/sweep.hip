@@ -2059,11 +2059,13 @@ __global__ void k_gather_u32(const uint32_t* __restrict__ src, const uint32_t* _
 // sweep: the chemistry of the sweep reads it (the reference's periodic
 // corrections have all arrived when update_chemistry runs), and the next
 // sweep's transport reads it as the value at its start (X does not change in
-// between). Thread t handles (periodic cell t / D, direction t % D).
+// between). Thread t handles (periodic cell t / D, direction t % D). The first
+// one empties the queue of the chemistry that follows.
 template <typename R>
-__global__ void k_periodic(Geo g, Flux<R> fl) {
-    if (fl.P == nullptr) return;
+__global__ void k_periodic(Geo g, Flux<R> fl, uint32_t* queue) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t == 0) queue[0] = queue[1] = 0u;
+    if (fl.P == nullptr) return;
     const uint32_t s = t / (uint32_t)g.D;
     const uint32_t d = t - s * (uint32_t)g.D;
     if ((int64_t)s >= g.Nper) return;
@@ -2099,6 +2101,7 @@ struct ChemArgs {
     unsigned long long* failures;
     unsigned long long* active;
     unsigned long long* limiting;  // [3] TimescaleCounter: temperature, ionisation fraction, photon rate
+    uint32_t* queue;         // {cells queued, cells taken beyond the first ones}, then the queued cells
 };
 
 // Adds the number of lanes with `pred` to *counter with one atomic per wave
@@ -2108,10 +2111,50 @@ __device__ __forceinline__ void wave_count(bool pred, unsigned long long* counte
     if (m && __lane_id() == __ffsll((long long)__ballot(1)) - 1) atomicAdd(counter, (unsigned long long)__popcll(m));
 }
 
-// update_chemistry (src/sweep/mod.rs:549-574) for the active cells, then the
-// attenuation of the updated cell for the next sweep.
+// The cell of c for the solver, at summed rate `rate`.
+__device__ __forceinline__ ssw::Cell solver_cell(const ChemArgs& ca, int64_t c, double rate) {
+    ssw::Cell cell;
+    cell.x = ca.x[c];
+    cell.T = ca.T[c];
+    cell.rho = ca.rho[c];
+    cell.vol = ca.vol[c];
+    cell.len = ca.size[c];
+    cell.rate = rate;
+    cell.a = ca.scale_factor;
+    return cell;
+}
+
+// The end of a cell's update: state, timescales, process counts (lanes with
+// `own` only) and the attenuation for the next sweep.
 template <typename R>
-__global__ void k_chemistry(Geo g, Flux<R> fl, ChemArgs ca, int lvl) {
+__device__ __forceinline__ void finish_chemistry(const ChemArgs& ca, int64_t c, const ssw::Cell& cell, double rate_ts,
+                                                 const ssw::Walk& w, bool own) {
+    // Timescale::min (src/chemistry/timescale.rs:32-38): a tie goes to the chemistry
+    const bool rate_limits = rate_ts < w.ts;
+    const double change = rate_limits ? rate_ts : w.ts;
+    // TimescaleCounter::count (src/chemistry/timescale.rs:80-87)
+    const int process = rate_limits ? 2 : w.proc;
+    const bool counted = own && change < ca.max_ts;
+    wave_count(counted && process == 0, &ca.limiting[0]);
+    wave_count(counted && process == 1, &ca.limiting[1]);
+    wave_count(counted && process == 2, &ca.limiting[2]);
+    wave_count(own && w.failed, ca.failures);
+    const R att = (R)ssw::non_absorbed_fraction(cell.rho, cell.x, cell.len);
+    if (!own) return;
+    ca.x[c] = cell.x;
+    ca.T[c] = cell.T;
+    ca.species_ts[c] = w.ts;
+    ca.change_ts[c] = change;
+    ((SA<R>*)ca.sa)[c].y = att;
+}
+
+// update_chemistry (src/sweep/mod.rs:549-574) for the active cells, then the
+// attenuation of the updated cell for the next sweep. One lane per cell for
+// the rate and the first attempt of the solver; cells whose full step is
+// rejected go to the queue of k_chemistry_tail, else a wave would last as long
+// as its slowest cell's sub-steps, one after the other.
+template <typename R>
+__global__ void __launch_bounds__(kBlock) k_chemistry(Geo g, Flux<R> fl, ChemArgs ca, int lvl) {
     // a die takes consecutive cells: where I is gathered (direction sweeps),
     // they share its lines in the die's L2
     int64_t c = (int64_t)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
@@ -2144,33 +2187,65 @@ __global__ void k_chemistry(Geo g, Flux<R> fl, ChemArgs ca, int lvl) {
     }
     ca.prev_rate[c] = rate;
     const double rate_ts = dt / rel;
-    ssw::Cell cell;
-    cell.x = ca.x[c];
-    cell.T = ca.T[c];
-    cell.rho = ca.rho[c];
-    cell.vol = ca.vol[c];
-    cell.len = ca.size[c];
-    cell.rate = rate;
-    cell.a = ca.scale_factor;
-    ssw::Floor fl0{ca.prevent_cooling != 0, cell.T, cell.x};
-    int proc = 0;
-    bool failed = false;
-    double used = ssw::perform_timestep(cell, fl0, dt, ca.safety, proc, failed);
-    if (failed) atomicAdd(ca.failures, 1ull);
-    ca.x[c] = cell.x;
-    ca.T[c] = cell.T;
-    ca.species_ts[c] = used;
-    // Timescale::min (src/chemistry/timescale.rs:32-38): a tie goes to the chemistry
-    const bool rate_limits = rate_ts < used;
-    const double change = rate_limits ? rate_ts : used;
-    ca.change_ts[c] = change;
-    // TimescaleCounter::count (src/chemistry/timescale.rs:80-87)
-    const int process = rate_limits ? 2 : proc;
-    const bool counted = change < ca.max_ts;
-    wave_count(counted && process == 0, &ca.limiting[0]);
-    wave_count(counted && process == 1, &ca.limiting[1]);
-    wave_count(counted && process == 2, &ca.limiting[2]);
-    ((SA<R>*)ca.sa)[c].y = (R)ssw::non_absorbed_fraction(cell.rho, cell.x, cell.len);
+    ssw::Cell cell = solver_cell(ca, c, rate);
+    const ssw::Floor floor{ca.prevent_cooling != 0, cell.T, cell.x};
+    ssw::Walk w;
+    w.dt = dt;
+    const bool done = ssw::walk_step(cell, floor, dt, ca.safety, w, ssw::Serial());
+    const unsigned long long m = __ballot(!done);
+    if (m) {  // queued, with the photon rate's timescale in change_ts
+        uint32_t at = 0;
+        const int leader = __ffsll((long long)__ballot(1)) - 1;
+        if ((int)__lane_id() == leader) at = atomicAdd(&ca.queue[0], (uint32_t)__popcll(m));
+        at = (uint32_t)__shfl((int)at, leader);
+        if (!done) {
+            ca.queue[2 + at + (uint32_t)__popcll(m & ((1ull << __lane_id()) - 1ull))] = (uint32_t)c;
+            ca.change_ts[c] = rate_ts;
+        }
+    }
+    if (done) finish_chemistry<R>(ca, c, cell, rate_ts, w, true);
+}
+
+// The queued cells' sub-steps, from the first rejection on. Bound: the chain
+// of one cell's sub-steps (up to a few hundred near a source), each mostly its
+// powers (0.4 us each). So a quad of lanes takes a cell and shares them, two
+// rounds of them before the temperature's step and two before the ionised
+// fraction's instead of eleven powers, and a quad that has finished its cell
+// takes the next one while the others of its wave go on. Chemistry of 262144
+// cells with 64 sources: 1.04 -> 0.60 ms (0.19 + 0.41), of 32768 cells in the
+// first two steps 1.96 -> 1.33 ms a step.
+template <typename R>
+__global__ void __launch_bounds__(64) k_chemistry_tail(Geo g, ChemArgs ca) {
+    const uint32_t n = ca.queue[0], first = gridDim.x * 16u;
+    const bool lead = (threadIdx.x & 3u) == 0;
+    uint32_t i = blockIdx.x * 16u + threadIdx.x / 4u;
+    int64_t c = 0;
+    double dt = 0.0;
+    ssw::Cell cell{};
+    ssw::Floor floor{};
+    ssw::Walk w;
+    bool have = false;
+    for (;;) {
+        if (!have && i < n) {
+            c = ca.queue[2 + i];
+            dt = ca.max_ts * ssw::powi(0.5, g.level[c]);
+            cell = solver_cell(ca, c, ca.prev_rate[c]);
+            floor = ssw::Floor{ca.prevent_cooling != 0, cell.T, cell.x};
+            w = ssw::Walk();
+            w.depth = 1;  // the full step was rejected: its two halves are pending
+            w.lo = 2;
+            w.dt = dt / 2.0;
+            have = true;
+        }
+        if (__ballot(have) == 0ull) break;
+        if (have && ssw::walk_step(cell, floor, dt, ca.safety, w, ssw::Quad())) {
+            finish_chemistry<R>(ca, c, cell, ca.change_ts[c], w, lead);
+            have = false;
+            uint32_t next = 0;
+            if (lead) next = atomicAdd(&ca.queue[1], 1u);
+            i = first + (uint32_t)__builtin_amdgcn_mov_dpp((int)next, 0, 0xF, 0xF, true);
+        }
+    }
 }
 
 // The optional chemistry outputs (src/sweep/chemistry_output.rs:25-67) of
@@ -2575,6 +2650,7 @@ struct ssw_sweep {
     void* d_sa = nullptr;                           // SA<R>: {transport source / D, attenuation}
     double *d_sts = nullptr, *d_prev = nullptr, *d_change = nullptr;
     unsigned long long* d_active = nullptr;
+    uint32_t* d_chemq = nullptr;                    // k_chemistry's queue (ChemArgs::queue)
     unsigned long long* d_limit = nullptr;          // [3] limiting processes of the last step
     uint8_t* d_level = nullptr;
     void *d_X = nullptr, *d_I = nullptr, *d_P = nullptr;
@@ -3771,7 +3847,18 @@ ChemArgs chem_args(ssw_sweep* s) {
     ca.failures = s->d_fail;
     ca.active = s->d_active;
     ca.limiting = s->d_limit;
+    ca.queue = s->d_chemq;
     return ca;
+}
+
+// The periodic sources and the chemistry after a sweep at level lvl. The tail
+// gets a wave per 16 cells, at most two per SIMD (its quads take further cells
+// as they finish); waves that find no queued cell end at once.
+template <typename R>
+void launch_chemistry(ssw_sweep* s, const Geo& g, const Flux<R>& fl, const ChemArgs& ca, int lvl, hipStream_t st) {
+    k_periodic<R><<<grid_for(std::max<int64_t>(s->Nper, 1) * s->D), kBlock, 0, st>>>(g, fl, ca.queue);
+    k_chemistry<R><<<grid_for(s->N), kBlock, 0, st>>>(g, fl, ca, lvl);
+    k_chemistry_tail<R><<<(unsigned)std::min<int64_t>((s->N + 15) / 16, 2048), 64, 0, st>>>(g, ca);
 }
 
 // ssw_sweep::rates_current after the sweeps of `order`.
@@ -3790,7 +3877,6 @@ int run_step(ssw_sweep* s, double* elapsed) {
     s->rates_current = false;  // an error below leaves a partly swept state
     k_fill_u32<<<1, 2, 0, s->stream>>>((uint32_t*)s->d_active, 0u, 2);
     k_fill_u32<<<1, 6, 0, s->stream>>>((uint32_t*)s->d_limit, 0u, 6);
-    const unsigned gper = grid_for(std::max<int64_t>(s->Nper, 1) * s->D);
     const unsigned gcells = grid_for(s->N);
     s->sweeps_last = 0;
     s->builds_last = 0;
@@ -3839,8 +3925,7 @@ int run_step(ssw_sweep* s, double* elapsed) {
         HIP_TRY(hipGetLastError());
         s->replays[lvl]++;
         hipEvent_t a = s->timing ? mark() : nullptr;
-        k_periodic<R><<<gper, kBlock, 0, s->stream>>>(g, fl);
-        k_chemistry<R><<<gcells, kBlock, 0, s->stream>>>(g, fl, ca, lvl);
+        launch_chemistry<R>(s, g, fl, ca, lvl, s->stream);
         if (s->timing) ch.push_back({a, mark()});
         s->sweeps_last++;
     }
@@ -3987,8 +4072,7 @@ void packed_item(ssw_sweep* s, const Geo& g, int lvl, const ssw_sweep::ReplayIte
 template <typename R>
 void batch_chemistry(ssw_sweep* s, const Geo& g, int lvl, hipStream_t st) {
     const Flux<R> fl = make_flux<R>(s);
-    k_periodic<R><<<grid_for(std::max<int64_t>(s->Nper, 1) * s->D), kBlock, 0, st>>>(g, fl);
-    k_chemistry<R><<<grid_for(s->N), kBlock, 0, st>>>(g, fl, chem_args(s), lvl);
+    launch_chemistry<R>(s, g, fl, chem_args(s), lvl, st);
 }
 
 // Graphs of packed sweeps, keyed by (uid, epoch, sweep level) of every
@@ -4262,6 +4346,7 @@ void free_state(ssw_sweep* s) {
     dfree(s, s->d_sts);
     dfree(s, s->d_prev);
     dfree(s, s->d_change);
+    dfree(s, s->d_chemq);
     dfree(s, s->d_X);
     dfree(s, s->d_I);
     dfree(s, s->d_P);
@@ -4831,6 +4916,7 @@ int ssw_upload_state(ssw_sweep* s, const double* density, const double* xhii, co
     TRY(dalloc(s, &s->d_sts, n));
     TRY(dalloc(s, &s->d_prev, n));
     TRY(dalloc(s, &s->d_change, n));
+    TRY(dalloc(s, &s->d_chemq, (size_t)n + 2));
     TRY(dalloc(s, (uint8_t**)&s->d_X, (size_t)s->D * n * es));
     TRY(dalloc(s, (uint8_t**)&s->d_I, (size_t)s->D * n * es));
     if (s->Nper) TRY(dalloc(s, (uint8_t**)&s->d_P, (size_t)s->D * s->Nper * es));
@@ -5480,7 +5566,7 @@ int64_t ssw_estimate_device_bytes(const ssw_sweep_parameters* p, int64_t n, int6
     int64_t build = std::max(DN * 20 + ostart, std::max(DN * 16 + ostart, sched + DN * 4 + ostart));
     if (comp) build = std::max(build, sched + grp + DN * 5);
     // afterwards: schedule, active-set (or group) lists, state, the photon-rate download
-    const int64_t run = sched + lists + n * 8 * 9 + 2 * DN * rs + D * num_periodic_cells * rs + n * 8;
+    const int64_t run = sched + lists + n * 8 * 9 + n * 4 + 2 * DN * rs + D * num_periodic_cells * rs + n * 8;
     const int64_t b = grid + std::max(build, run);
     return b + b / 20 + (1 << 20);
 }
