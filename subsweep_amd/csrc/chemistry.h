@@ -275,17 +275,15 @@ SSW_HD double photoionization_rate(const Cell& c, double dt, double pass) {  // 
 SSW_HD double photoheating_rate(const Cell& c, double dt, double pass) {  // :321-325
     return newly_ionized(c, dt, pass) / c.vol * (kPhotonEnergy - kRydberg) / dt;
 }
-// which: 0 PhotoionizationRate, 1 HeatingRate (photoheating - cooling),
-// 2 RecombinationRate (alpha_B n_e x), 3 CollisionalIonizationRate (beta n_e (1 - x))
-SSW_HD double chemistry_output(const Cell& c, int which) {
+// PhotoionizationRate, HeatingRate (photoheating - cooling), RecombinationRate
+// (alpha_B n_e x), CollisionalIonizationRate (beta n_e (1 - x))
+SSW_HD void chemistry_outputs(const Cell& c, double (&out)[4]) {
     const HeatRates h = heat_rates(c, Serial());
     const IonRates i = ion_rates(c, Serial());
-    switch (which) {
-        case 0: return photoionization_rate(c, kYear, h.pass);
-        case 1: return photoheating_rate(c, kYear, h.pass) - cooling(c, h);
-        case 2: return alpha_b(i.l15, i.w) * n_hii(c) * c.x;
-        default: return beta_ci(c.T, i.ci) * n_hii(c) * (1.0 - c.x);
-    }
+    out[0] = photoionization_rate(c, kYear, h.pass);
+    out[1] = photoheating_rate(c, kYear, h.pass) - cooling(c, h);
+    out[2] = alpha_b(i.l15, i.w) * n_hii(c) * c.x;
+    out[3] = beta_ci(c.T, i.ci) * n_hii(c) * (1.0 - c.x);
 }
 
 struct Floor {

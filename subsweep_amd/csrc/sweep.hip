@@ -2251,10 +2251,11 @@ __global__ void __launch_bounds__(64) k_chemistry_tail(Geo g, ChemArgs ca) {
 // The optional chemistry outputs (src/sweep/chemistry_output.rs:25-67) of
 // every cell: Sweep::get_solver (src/sweep/mod.rs:612-632) with the rate
 // summed over directions in direction order as in update_chemistry, the
-// current x and T, and no floor; output `which` of ssw::chemistry_output.
+// current x and T, and no floor (an output that is NULL is left out).
 template <typename R>
-__global__ void k_chem_outputs(Geo g, Flux<R> fl, ChemArgs ca, int which, double* out) {
-    int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void __launch_bounds__(64) k_chem_outputs(Geo g, Flux<R> fl, ChemArgs ca, double* out0, double* out1,
+                                                     double* out2, double* out3) {
+    int64_t c = (int64_t)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     if (c >= g.N) return;
     const uint32_t ps = g.pslot[c];
     const bool has_p = ps != kNone && fl.P;
@@ -2274,7 +2275,12 @@ __global__ void k_chem_outputs(Geo g, Flux<R> fl, ChemArgs ca, int which, double
     cell.len = ca.size[c];
     cell.rate = rate;
     cell.a = ca.scale_factor;
-    out[c] = ssw::chemistry_output(cell, which);
+    double out[4];
+    ssw::chemistry_outputs(cell, out);
+    if (out0) out0[c] = out[0];
+    if (out1) out1[c] = out[1];
+    if (out2) out2[c] = out[2];
+    if (out3) out3[c] = out[3];
 }
 
 // update_timestep_levels (src/sweep/mod.rs:576-589) for all cells. Marks the
@@ -2458,6 +2464,25 @@ __global__ void k_to_caller(const T* __restrict__ src, const uint32_t* __restric
     if (i < n) dst[idx[i]] = src[i];
 }
 
+// Outputs of up to 6 per-cell arrays for the caller's cells [j0, j0 + n) into
+// pinned host memory, in the caller's order (perm: internal cell of each
+// caller's cell; NULL: the same): consecutive lanes write consecutive values
+// over the bus, and the scattered side of the permutation stays in HBM.
+struct OutputArrays {
+    const double* a[6];
+    const uint8_t* level;
+    int n;
+};
+__global__ void __launch_bounds__(kBlock) k_stage_outputs(OutputArrays src, const uint32_t* __restrict__ perm,
+                                                          uint32_t j0, uint32_t n, uint32_t stride,
+                                                          double* __restrict__ out) {
+    const uint32_t j = blockIdx.x * kBlock + threadIdx.x;
+    if (j >= n) return;
+    const uint32_t i = perm ? perm[j0 + j] : j0 + j;
+    for (int k = 0; k < src.n; k++) out[(size_t)k * stride + j] = src.a[k][i];
+    if (src.level) reinterpret_cast<uint8_t*>(out + (size_t)src.n * stride)[j] = src.level[i];
+}
+
 // Direction-major copy of X from the schedule-position order.
 template <typename R>
 __global__ void k_gather_x(const R* X, const uint32_t* xpos, R* out, int64_t n) {
@@ -2594,7 +2619,8 @@ struct ssw_sweep {
     std::vector<double> pos;
     std::vector<uint32_t> perm, inv;
     bool permuted = false;
-    uint32_t* d_inv = nullptr;                      // inv on the device (permuted grids only)
+    uint32_t *d_inv = nullptr, *d_perm = nullptr;   // inv and perm on the device (permuted grids only)
+    bool downloaded = false;                        // later downloads go through the pinned staging
     uint32_t *d_off = nullptr, *d_nk = nullptr, *d_pslot = nullptr, *d_pcells = nullptr;
     std::vector<uint32_t> h_pcells;                 // internal cell of each periodic slot
     uint32_t *d_pfoff = nullptr, *d_pfidx = nullptr;
@@ -2650,6 +2676,7 @@ struct ssw_sweep {
     void* d_sa = nullptr;                           // SA<R>: {transport source / D, attenuation}
     double *d_sts = nullptr, *d_prev = nullptr, *d_change = nullptr;
     unsigned long long* d_active = nullptr;
+    double* d_photon = nullptr;                     // photon rates of a download (internal order)
     uint32_t* d_chemq = nullptr;                    // k_chemistry's queue (ChemArgs::queue)
     unsigned long long* d_limit = nullptr;          // [3] limiting processes of the last step
     uint8_t* d_level = nullptr;
@@ -4337,6 +4364,114 @@ int step_batch(ssw_sweep* const* hs, int n, double* elapsed) {
     return SSW_OK;
 }
 
+// Pinned host memory through which downloads pass, one for the process:
+// kernels write the outputs into it in the caller's order, chunk by chunk, and
+// host threads copy finished chunks on into the caller's arrays (whose pages
+// are usually touched there for the first time: 5 GB/s on one thread). Made at
+// a handle's second download, freed with the last handle; a download that
+// finds it in use by another thread takes the plain path. Results of 262144
+// cells: 1.8 -> 0.27 ms, of 1000 cells 0.10 -> 0.03 ms (six
+// copies of 25 us each before).
+constexpr uint32_t kStageCells = 49152;             // cells of a chunk
+constexpr int kStageChunks = 16;
+constexpr size_t kStageChunkBytes = (size_t)kStageCells * (6 * 8 + 1);
+constexpr int kStageThreads = 6;
+struct Staging {
+    std::mutex mu;
+    uint8_t* host = nullptr;
+    int device = -1;
+    std::vector<hipEvent_t> done;
+    void free() {
+        if (host) (void)hipHostFree(host);
+        host = nullptr;
+        for (hipEvent_t e : done) (void)hipEventDestroy(e);
+        done.clear();
+    }
+    bool make(int dev) {
+        if (host) return device == dev;
+        std::shared_lock<std::shared_mutex> lock(g_capture_mu);
+        device = dev;
+        if (hipHostMalloc((void**)&host, kStageChunkBytes * kStageChunks, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            host = nullptr;
+            return false;
+        }
+        for (int k = 0; k < kStageChunks; k++) {
+            hipEvent_t e;
+            if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+                (void)hipGetLastError();
+                free();
+                return false;
+            }
+            done.push_back(e);
+        }
+        return true;
+    }
+};
+Staging g_staging;
+
+// The device arrays `src` (and levels) into the host arrays `dst` in the
+// caller's cell order. Plain path: one copy per array, permuted on the host.
+int fetch_outputs(ssw_sweep* s, const std::vector<const double*>& src, const std::vector<double*>& dst,
+                  const uint8_t* d_level, uint8_t* level) {
+    const int64_t n = s->N;
+    std::unique_lock<std::mutex> lock(g_staging.mu, std::try_to_lock);
+    if (!s->downloaded || !lock.owns_lock() || !g_staging.make(s->device)) {
+        s->downloaded = true;
+        for (size_t k = 0; k < src.size(); k++)
+            HIP_TRY(hipMemcpyAsync(dst[k], src[k], n * 8, hipMemcpyDeviceToHost, s->stream));
+        if (level) HIP_TRY(hipMemcpyAsync(level, d_level, n, hipMemcpyDeviceToHost, s->stream));
+        HIP_TRY(hipStreamSynchronize(s->stream));
+        for (double* a : dst) to_caller(s, a, 1);
+        if (level) to_caller(s, level, 1);
+        return SSW_OK;
+    }
+    OutputArrays oa{};
+    oa.n = (int)src.size();
+    for (int k = 0; k < oa.n; k++) oa.a[k] = src[k];
+    oa.level = level ? d_level : nullptr;
+    for (int64_t r0 = 0; r0 < n; r0 += (int64_t)kStageCells * kStageChunks) {
+        const int chunks = (int)std::min<int64_t>(kStageChunks, (n - r0 + kStageCells - 1) / kStageCells);
+        auto first = [&](int c) { return r0 + (int64_t)c * kStageCells; };
+        auto cells = [&](int c) { return std::min<int64_t>(kStageCells, n - first(c)); };
+        auto copy = [&](int c) {
+            const uint8_t* st = g_staging.host + (size_t)c * kStageChunkBytes;
+            for (int k = 0; k < oa.n; k++)
+                std::memcpy(dst[k] + first(c), st + (size_t)k * kStageCells * 8, (size_t)cells(c) * 8);
+            if (level) std::memcpy(level + first(c), st + (size_t)oa.n * kStageCells * 8, (size_t)cells(c));
+        };
+        for (int c = 0; c < chunks; c++) {
+            k_stage_outputs<<<grid_for(cells(c)), kBlock, 0, s->stream>>>(
+                oa, s->permuted ? s->d_perm : nullptr, (uint32_t)first(c), (uint32_t)cells(c), kStageCells,
+                (double*)(g_staging.host + (size_t)c * kStageChunkBytes));
+            HIP_TRY(hipGetLastError());
+            if (chunks > 1) HIP_TRY(hipEventRecord(g_staging.done[c], s->stream));
+        }
+        if (chunks == 1) {
+            HIP_TRY(hipStreamSynchronize(s->stream));
+            copy(0);
+            continue;
+        }
+        std::atomic<int> next{0};
+        std::atomic<bool> failed{false};
+        auto work = [&] {
+            for (int c = next++; c < chunks; c = next++) {
+                if (hipEventSynchronize(g_staging.done[c]) != hipSuccess) failed = true;
+                copy(c);
+            }
+        };
+        std::vector<std::thread> th;
+        try {
+            for (int k = 1; k < std::min(kStageThreads, chunks); k++) th.emplace_back(work);
+        } catch (const std::exception&) {  // no thread to spare: fewer
+        }
+        work();
+        for (std::thread& t : th) t.join();
+        if (failed) return fail(SSW_ERR_HIP, "a download's kernel failed");
+    }
+    return SSW_OK;
+}
+
 void free_state(ssw_sweep* s) {
     dfree(s, s->d_rho);
     dfree(s, s->d_x);
@@ -4347,6 +4482,7 @@ void free_state(ssw_sweep* s) {
     dfree(s, s->d_prev);
     dfree(s, s->d_change);
     dfree(s, s->d_chemq);
+    dfree(s, s->d_photon);
     dfree(s, s->d_X);
     dfree(s, s->d_I);
     dfree(s, s->d_P);
@@ -4376,6 +4512,7 @@ void free_grid(ssw_sweep* s) {
     s->groups.clear();
     dfree(s, s->d_off);
     dfree(s, s->d_inv);
+    dfree(s, s->d_perm);
     dfree(s, s->d_geo);
     dfree(s, s->d_nk);
     dfree(s, s->d_vol);
@@ -4682,7 +4819,11 @@ void ssw_destroy(ssw_sweep* s) {
         (void)hipStreamDestroy(s->stream);
     }
     delete s;
-    g_live_handles--;
+    if (--g_live_handles == 0) {
+        std::lock_guard<std::mutex> lock(g_staging.mu);
+        std::shared_lock<std::shared_mutex> alloc(g_capture_mu);
+        if (g_live_handles == 0) g_staging.free();
+    }
 }
 
 int ssw_set_transport_mode(ssw_sweep* s, int32_t mode) {
@@ -4861,7 +5002,9 @@ int ssw_upload_grid(ssw_sweep* s, int64_t n, const int64_t* off, const int32_t* 
     TRY(dalloc(s, &s->d_cnt, DN));
     if (s->permuted) {
         TRY(dalloc(s, &s->d_inv, n));
+        TRY(dalloc(s, &s->d_perm, n));
         HIP_TRY(hipMemcpyAsync(s->d_inv, s->inv.data(), n * 4, hipMemcpyHostToDevice, s->stream));
+        HIP_TRY(hipMemcpyAsync(s->d_perm, s->perm.data(), n * 4, hipMemcpyHostToDevice, s->stream));
     }
     HIP_TRY(hipMemcpyAsync(s->d_off, off32.data(), (n + 1) * 4, hipMemcpyHostToDevice, s->stream));
     HIP_TRY(hipMemcpyAsync(s->d_geo, geo.data(), F * sizeof(double4), hipMemcpyHostToDevice, s->stream));
@@ -5049,31 +5192,24 @@ int ssw_synchronize(ssw_sweep* s) {
 int ssw_download(ssw_sweep* s, double* x, double* T, double* sts, double* photon, uint8_t* level, double* change) {
     if (!s) return fail(SSW_ERR_INVALID, "null handle");
     if (!s->have_state) return fail(SSW_ERR_INVALID, "ssw_upload_state must be called first");
-    const int64_t n = s->N;
-    if (x) HIP_TRY(hipMemcpyAsync(x, s->d_x, n * 8, hipMemcpyDeviceToHost, s->stream));
-    if (T) HIP_TRY(hipMemcpyAsync(T, s->d_T, n * 8, hipMemcpyDeviceToHost, s->stream));
-    if (sts) HIP_TRY(hipMemcpyAsync(sts, s->d_sts, n * 8, hipMemcpyDeviceToHost, s->stream));
-    if (change) HIP_TRY(hipMemcpyAsync(change, s->d_change, n * 8, hipMemcpyDeviceToHost, s->stream));
-    if (level) HIP_TRY(hipMemcpyAsync(level, s->d_level, n, hipMemcpyDeviceToHost, s->stream));
+    std::vector<const double*> src;
+    std::vector<double*> dst;
+    auto want = [&](const double* d, double* h) {
+        if (!h) return;
+        src.push_back(d);
+        dst.push_back(h);
+    };
+    want(s->d_x, x);
+    want(s->d_T, T);
+    want(s->d_sts, sts);
+    want(s->d_change, change);
     if (photon) {
-        double* d_pr = nullptr;
-        Defer cleanup{[&] { dfree(s, d_pr); }};
-        TRY(dalloc(s, &d_pr, n));
-        Geo g = make_geo(s);
-        launch_photon_rate(s, g, d_pr, nullptr);
+        if (!s->d_photon) TRY(dalloc(s, &s->d_photon, s->N));
+        launch_photon_rate(s, make_geo(s), s->d_photon, nullptr);
         HIP_TRY(hipGetLastError());
-        HIP_TRY(hipMemcpyAsync(photon, d_pr, n * 8, hipMemcpyDeviceToHost, s->stream));
-        HIP_TRY(hipStreamSynchronize(s->stream));
-        dfree(s, d_pr);
+        want(s->d_photon, photon);
     }
-    HIP_TRY(hipStreamSynchronize(s->stream));
-    if (x) to_caller(s, x, 1);
-    if (T) to_caller(s, T, 1);
-    if (sts) to_caller(s, sts, 1);
-    if (change) to_caller(s, change, 1);
-    if (level) to_caller(s, level, 1);
-    if (photon) to_caller(s, photon, 1);
-    return SSW_OK;
+    return fetch_outputs(s, src, dst, s->d_level, level);
 }
 
 int ssw_download_noalloc(ssw_sweep* s, double* x, double* T, double* sts, double* photon, uint8_t* level,
@@ -5112,22 +5248,24 @@ int ssw_download_chemistry_outputs(ssw_sweep* s, double* photoionization, double
     double* outs[4] = {photoionization, heating, recombination, collisional_ionization};
     double* d_out = nullptr;
     Defer cleanup{[&] { dfree(s, d_out); }};
-    TRY(dalloc(s, &d_out, n));
+    TRY(dalloc(s, &d_out, 4 * n));
+    double* d[4];
+    std::vector<const double*> src;
+    std::vector<double*> dst;
+    for (int k = 0; k < 4; k++) {
+        d[k] = outs[k] ? d_out + k * n : nullptr;
+        if (!outs[k]) continue;
+        src.push_back(d[k]);
+        dst.push_back(outs[k]);
+    }
+    if (src.empty()) return SSW_OK;
     const Geo g = make_geo(s);
     const ChemArgs ca = chem_args(s);
-    for (int k = 0; k < 4; k++) {
-        if (!outs[k]) continue;
-        if (s->fp32)
-            k_chem_outputs<float><<<grid_for(n), kBlock, 0, s->stream>>>(g, make_flux<float>(s), ca, k, d_out);
-        else
-            k_chem_outputs<double><<<grid_for(n), kBlock, 0, s->stream>>>(g, make_flux<double>(s), ca, k, d_out);
-        HIP_TRY(hipGetLastError());
-        HIP_TRY(hipMemcpyAsync(outs[k], d_out, n * 8, hipMemcpyDeviceToHost, s->stream));
-        HIP_TRY(hipStreamSynchronize(s->stream));
-        to_caller(s, outs[k], 1);
-    }
-    dfree(s, d_out);
-    return SSW_OK;
+    const unsigned nb = (unsigned)((n + 63) / 64);
+    if (s->fp32) k_chem_outputs<float><<<nb, 64, 0, s->stream>>>(g, make_flux<float>(s), ca, d[0], d[1], d[2], d[3]);
+    else k_chem_outputs<double><<<nb, 64, 0, s->stream>>>(g, make_flux<double>(s), ca, d[0], d[1], d[2], d[3]);
+    HIP_TRY(hipGetLastError());
+    return fetch_outputs(s, src, dst, nullptr, nullptr);
 }
 
 int ssw_download_counts(ssw_sweep* s, int32_t lvl, uint32_t* counts) {
@@ -5553,7 +5691,7 @@ int64_t ssw_estimate_device_bytes(const ssw_sweep_parameters* p, int64_t n, int6
     // held from the grid upload on: grid arrays (with the caller-order map of
     // a permuted grid), level starts, chunk table
     const int64_t grid = (n + 1) * 4 + F * 32 + F * 4 + n * 16 + n * 4 + num_periodic_cells * 8 + F * 4 + n +
-                         (n + 4) * 4 + n * 4 + DN / kChunk * 40 + (1 << 20);
+                         (n + 4) * 4 + n * 8 + DN / kChunk * 40 + (1 << 20);
     const int64_t sched = comp ? DN * (16 + rs + kPlanes * es + 4) + ovf : DN * 16;  // compiled: + positions
     // compiled replay with the default grouped replay (4 level sets, 64 roots):
     // group lists instead of active-set lists, and the cone build's scratch
@@ -5565,8 +5703,9 @@ int64_t ssw_estimate_device_bytes(const ssw_sweep_parameters* p, int64_t n, int6
     const int64_t ostart = comp ? DN * 4 + ovf : 0;
     int64_t build = std::max(DN * 20 + ostart, std::max(DN * 16 + ostart, sched + DN * 4 + ostart));
     if (comp) build = std::max(build, sched + grp + DN * 5);
-    // afterwards: schedule, active-set (or group) lists, state, the photon-rate download
-    const int64_t run = sched + lists + n * 8 * 9 + n * 4 + 2 * DN * rs + D * num_periodic_cells * rs + n * 8;
+    // afterwards: schedule, active-set (or group) lists, state, the photon-rate
+    // and the optional outputs' downloads
+    const int64_t run = sched + lists + n * 8 * 9 + n * 4 + 2 * DN * rs + D * num_periodic_cells * rs + n * 40;
     const int64_t b = grid + std::max(build, run);
     return b + b / 20 + (1 << 20);
 }
