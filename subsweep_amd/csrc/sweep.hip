@@ -81,12 +81,11 @@ constexpr uint32_t kKindPeriodic = 1;
 constexpr uint32_t kKindBoundary = 2;
 constexpr uint32_t kNbrMask = 0x3FFFFFFFu;
 constexpr uint32_t kNone = 0xFFFFFFFFu;
-constexpr int kLanes = 16;                 // lanes per task in the build / geometric kernels
+constexpr int kLanes = 16;                 // lanes per task in the geometric kernels
 constexpr int kTasksPerBlock = kBlock / kLanes;
 constexpr uint32_t kCellBits = 25;         // task record: cell index bits
 constexpr uint32_t kCellMask = (1u << kCellBits) - 1u;
 constexpr int kMaxFaces = 127;             // faces per cell
-constexpr int kQueueCap = kTasksPerBlock * kMaxFaces;
 constexpr int kPlanes = 12;                // upwind entries per task held in planes
 static_assert(kPlanes % 2 == 0, "FP32 plane entries are stored in pairs");
 constexpr int kChunk = 4096;               // compaction chunk (tasks, within one level set)
@@ -200,9 +199,6 @@ struct Geo {
     const double4* pgeo;     // {normal, area} of each of them
     const uint32_t* pnb;     // and its neighbour
     int64_t Nper;
-    uint4* flat;             // Kahn layering: task records in level order (D*N)
-    uint32_t* lstart;        // Kahn layering: level starts
-    uint32_t* ctr;           // Kahn layering: 3 rotating append counters
     uint32_t* cnt;           // D x N missing-upwind counters
     uint32_t* need;          // L: the active set of a sweep level changed
 };
@@ -294,20 +290,6 @@ __device__ __forceinline__ uint4 task_record(uint32_t c, uint32_t f0, uint32_t f
     return make_uint4(c | ((f1 - f0) << kCellBits), f0, d, ps);
 }
 
-// Appends `rec` for every lane with `pred` at dst[*counter ...], one atomic per
-// wave; lanes outside the current control flow take no part.
-__device__ __forceinline__ void wave_append(bool pred, uint4 rec, uint32_t* counter, uint4* dst) {
-    unsigned long long m = __ballot(pred);
-    if (m == 0ull) return;
-    unsigned long long act = __ballot(1);
-    int leader = __ffsll((long long)act) - 1;
-    int lane = __lane_id();
-    uint32_t base = 0;
-    if (lane == leader) base = atomicAdd(counter, (uint32_t)__popcll(m));
-    base = __shfl(base, leader);
-    if (pred) dst[base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = rec;
-}
-
 __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, o));
@@ -373,18 +355,14 @@ __device__ __forceinline__ void finish_task(const Flux<R>& fl, size_t ox, size_t
     fl.I[oi] = inc;
 }
 
-// The face loop of one task, kLanes lanes per task (one face each), shared by
-// the Kahn build and the geometric replay. Lane `sub` handles faces sub,
-// sub + kLanes, ...; the loop runs to the longest face list of the wave so
-// that every lane takes part in the shuffles. The upwind sum is accumulated
-// in face order on every lane of the group; A is the xor-butterfly over the
-// lanes' partial sums.
-//   kTransport  gather the upwind X and sum
-//   kBuild      decrement the downwind neighbours' counters and queue the
-//               tasks that become ready into the block queue `sq`
-template <typename R, bool kTransport, bool kBuild>
+// The face loop of one task of the geometric replay, kLanes lanes per task
+// (one face each). Lane `sub` handles faces sub, sub + kLanes, ...; the loop
+// runs to the longest face list of the wave so that every lane takes part in
+// the shuffles. The upwind sum is accumulated in face order on every lane of
+// the group; A is the xor-butterfly over the lanes' partial sums.
+template <typename R>
 __device__ __forceinline__ void task_faces(const Geo& g, const Flux<R>& fl, bool valid, uint4 r, uint32_t sub,
-                                           uint32_t nfmax, double& A_out, R& inc_out, uint4* sq, uint32_t* sq_n) {
+                                           uint32_t nfmax, double& A_out, R& inc_out) {
     const uint32_t nf = valid ? (r.x >> kCellBits) : 0u;
     const uint32_t d = r.z;
     const double dx = g.dirs[3 * d], dy = g.dirs[3 * d + 1], dz = g.dirs[3 * d + 2];
@@ -408,29 +386,11 @@ __device__ __forceinline__ void task_faces(const Geo& g, const Flux<R>& fl, bool
         // and for boundary faces), so the gathers and the neighbour loads are
         // unconditional and issue together; the products are selected after.
         const R w = up ? (R)(a.w * fl.inv_aref * -dd) : (R)0;
-        const R xv = kTransport ? fl.X[dN + nb] : (R)0;
+        const R xv = fl.X[dN + nb];
         const R v = up ? w * xv : (R)0;
-        bool ready = false;
-        uint4 rec = make_uint4(0, 0, 0, 0);
-        if (kBuild) {
-            const uint32_t f0n = g.off[nb], f1n = g.off[nb + 1], psn = g.pslot[nb];
-            if (down && local) ready = atomicSub(&g.cnt[dN + nb], 1u) == 1u;
-            rec = task_record(nb, f0n, f1n, d, psn);
-        }
         if (down) A += a.w * fl.inv_aref * dd;
-        if (kTransport) {
 #pragma unroll
-            for (int l = 0; l < kLanes; l++) inc += __shfl(v, gbase + l);
-        }
-        if (kBuild) {
-            const unsigned long long m = __ballot(ready);
-            if (m) {
-                uint32_t b = 0;
-                if (lane == 0) b = atomicAdd(sq_n, (uint32_t)__popcll(m));
-                b = __shfl(b, 0);
-                if (ready) sq[b + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = rec;
-            }
-        }
+        for (int l = 0; l < kLanes; l++) inc += __shfl(v, gbase + l);
     }
 #pragma unroll
     for (int m = kLanes / 2; m > 0; m >>= 1) A += __shfl_xor(A, m, kLanes);
@@ -542,98 +502,108 @@ __global__ void k_overflow(Geo g, const uint32_t* ovf_count, uint32_t* ovf_start
 // Kahn layering (once per grid for the full graph; on demand for a restricted
 // active set, for the parity hook)
 
-// Resets the append counters and the first level start.
-__global__ void k_kahn_reset(Geo g) {
-    if (threadIdx.x < 3) g.ctr[threadIdx.x] = 0;
-    if (threadIdx.x == 0) g.lstart[0] = 0;
-}
-
-// init_counts (src/sweep/mod.rs:346-386) + get_initial_tasks (:388-398) for the
-// active set {level >= lvl}: counts the active local upwind neighbours of every
-// active (cell, direction) and queues the tasks with count 0 as level set 0
-// (unless only_counts). Thread t handles (cell t / D, direction t % D).
-__global__ void k_count(Geo g, int lvl, int only_counts) {
+// init_counts (src/sweep/mod.rs:346-386) for the active set {level >= lvl}:
+// the active local upwind neighbours of every active (cell, direction), kNone
+// for inactive cells. Thread t handles (cell t / D, direction t % D).
+__global__ void k_count(Geo g, int lvl) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     uint32_t c, d;
-    const bool in = cell_dir(g, t, c, d);
-    const bool active = in && g.level[c] >= lvl;
-    uint32_t n = 0, f0 = 0, f1 = 0;
+    if (!cell_dir(g, t, c, d)) return;
+    uint32_t n = 0;
+    const bool active = g.level[c] >= lvl;
     if (active) {
         const double dx = g.dirs[3 * d], dy = g.dirs[3 * d + 1], dz = g.dirs[3 * d + 2];
-        f0 = g.off[c];
-        f1 = g.off[c + 1];
-        for (uint32_t f = f0; f < f1; f++) {
+        for (uint32_t f = g.off[c]; f < g.off[c + 1]; f++) {
             const uint32_t nk = g.nk[f];
             if ((nk >> 30) != kKindLocal) continue;
             if (!(fdot(g.geo[f], dx, dy, dz) < 0.0)) continue;
             if (g.level[nk & kNbrMask] >= lvl) n++;
         }
     }
-    if (in) g.cnt[(size_t)d * g.N + c] = active ? n : kNone;
-    if (only_counts) return;
-    const bool ready = active && n == 0;
-    wave_append(ready, ready ? task_record(c, f0, f1, d, g.pslot[c]) : make_uint4(0, 0, 0, 0), &g.ctr[0], g.flat);
+    g.cnt[(size_t)d * g.N + c] = active ? n : kNone;
 }
 
-// Level set k+1 of the layering from level set k: kLanes lanes per task
-// decrement the counters of the local downwind neighbours (an inactive
-// neighbour's counter starts at 0xFFFFFFFF and never reaches 0); the tasks that
-// become ready are gathered per block in LDS and appended with one atomic per
-// block (handle_local_neighbour, src/sweep/mod.rs:487-503).
-__global__ void __launch_bounds__(kBlock) k_kahn(Geo g, int k) {
-    __shared__ uint4 sq[kQueueCap];
-    __shared__ uint32_t sq_n, sq_base, sq_cnt;
-    uint32_t* ls = g.lstart;
-    uint32_t* ctr = g.ctr;
-    const uint32_t beg = ls[k];
-    const uint32_t end = beg + ctr[k % 3];
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        ls[k + 1] = end;
-        ctr[(k + 2) % 3] = 0;
-    }
-    if (beg >= end) return;
-    uint32_t* next_ctr = ctr + (k + 1) % 3;
-    const uint32_t sub = threadIdx.x % kLanes;
-    const uint32_t stride = gridDim.x * kTasksPerBlock;
-    Flux<float> fl{};
-    if (threadIdx.x == 0) sq_n = 0;
+// The level sets of every direction from its counters (handle_local_neighbour,
+// src/sweep/mod.rs:487-503): one workgroup per direction, since no dependency
+// crosses directions. The tasks of a level set decrement their local downwind
+// neighbours' counters, 8 lanes a task, two faces each; a counter that reaches
+// 0 queues its task for the next level set. Writes depth[d*N + c] of active
+// tasks, adds each level set's tasks to hist[k], and their number and the
+// direction's level sets to totals = {tasks, most level sets}.
+// Bound: the chain of a level set (queue, face range, faces, counters, one
+// barrier). With kLds the counters lie in LDS as bytes (at most 127 upwind
+// faces; an inactive cell's byte starts at 255 and never reaches 0), up to
+// kLayerCells cells; else they are decremented in memory. The queues are in
+// LDS, longer ones go on in `spill` (2 N entries a direction). A launch for
+// every level set of all directions took 5 to 30 us a level set: 32768 cells x
+// 84 directions 4.5 -> 1.3 ms, 262144 cells 23 -> 9.8 ms, 2 M clustered 184 ->
+// 113 ms, 12167 cells x 32 1.9 -> 0.73 ms.
+constexpr uint32_t kLayerQueue = 2048;
+constexpr uint32_t kLayerCells = 139264;  // 136 KiB of LDS beside the queues
+template <bool kLds>
+__global__ void __launch_bounds__(1024) k_layers(Geo g, uint32_t kcap, uint32_t* __restrict__ depth, uint32_t* spill,
+                                                 uint32_t* hist, uint32_t* totals) {
+    __shared__ uint32_t queue[2][kLayerQueue];
+    __shared__ uint32_t len[2];
+    __shared__ uint32_t bytes[kLds ? kLayerCells / 4 : 1];
+    const uint32_t d = blockIdx.x, N = (uint32_t)g.N, tid = threadIdx.x;
+    const size_t dN = (size_t)d * N;
+    const double dx = g.dirs[3 * d], dy = g.dirs[3 * d + 1], dz = g.dirs[3 * d + 2];
+    uint32_t* const cnt = g.cnt + dN;
+    auto push = [&](uint32_t which, uint32_t c) {
+        const uint32_t i = atomicAdd(&len[which], 1u);
+        if (i < kLayerQueue) queue[which][i] = c;
+        else spill[2 * dN + (size_t)which * N + i] = c;
+    };
+    if (tid < 2) len[tid] = 0;
     __syncthreads();
-    for (uint32_t i0 = beg + blockIdx.x * kTasksPerBlock; i0 < end; i0 += stride) {
-        const uint32_t i = i0 + threadIdx.x / kLanes;
-        const bool valid = i < end;
-        const uint4 r = valid ? g.flat[i] : make_uint4(0, 0, 0, 0);
-        const uint32_t nfmax = wave_max(valid ? (r.x >> kCellBits) : 0u);
-        double A;
-        float inc;
-        task_faces<float, false, true>(g, fl, valid, r, sub, nfmax, A, inc, sq, &sq_n);
-        // flush the block queue into level set k+1
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            const uint32_t n = sq_n;
-            sq_cnt = n;
-            sq_base = n ? atomicAdd(next_ctr, n) : 0u;
-            sq_n = 0;
+    for (uint32_t c0 = 4 * tid; c0 < N; c0 += 4096) {  // level set 0
+        uint32_t word = 0;
+        for (uint32_t u = 0; u < 4 && c0 + u < N; u++) {
+            const uint32_t n = cnt[c0 + u];
+            word |= min(n, 255u) << (8 * u);
+            if (n == 0) push(0, c0 + u);
+        }
+        if (kLds) bytes[c0 / 4] = word;
+    }
+    __syncthreads();
+    uint32_t total = 0, k = 0;
+    for (;; k++) {
+        const uint32_t cur = k & 1u, n = len[cur];
+        if (n == 0 || k >= kcap) break;
+        if (tid == 0) atomicAdd(&hist[k], n);
+        total += n;
+        for (uint32_t i = tid / 8; i < n; i += 128) {
+            const uint32_t c = i < kLayerQueue ? queue[cur][i] : spill[2 * dN + (size_t)cur * N + i];
+            const uint32_t sub = tid % 8, f1 = g.off[c + 1];
+            if (sub == 0) depth[dN + c] = k;
+            for (uint32_t f = g.off[c] + sub; f < f1; f += 16) {
+                const uint32_t h = f + 8 < f1 ? f + 8 : f;
+                const double4 a[2] = {g.geo[f], g.geo[h]};
+                const uint32_t nk[2] = {g.nk[f], g.nk[h]};
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    if ((u && h == f) || (nk[u] >> 30) != kKindLocal || !(fdot(a[u], dx, dy, dz) > 0.0)) continue;
+                    const uint32_t nb = nk[u] & kNbrMask;
+                    bool ready;
+                    if (kLds) {
+                        const uint32_t sh = 8 * (nb & 3u);
+                        ready = ((atomicSub(&bytes[nb / 4], 1u << sh) >> sh) & 255u) == 1u;
+                    } else {
+                        ready = __hip_atomic_fetch_sub(&cnt[nb], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) ==
+                                1u;
+                    }
+                    if (ready) push(cur ^ 1u, nb);
+                }
+            }
         }
         __syncthreads();
-        const uint32_t n = sq_cnt, b = end + sq_base;
-        for (uint32_t t = threadIdx.x; t < n; t += kBlock) g.flat[b + t] = sq[t];
+        if (tid == 0) len[cur] = 0;
         __syncthreads();
     }
-}
-
-// Kahn depth of every task of a layering: entry i of the level-major array is
-// in level set k with lstart[k] <= i < lstart[k+1].
-__global__ void k_scatter_depth(Geo g, int kmax, uint32_t* depth) {
-    const uint32_t total = g.lstart[kmax];
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x) {
-        int a = 0, b = kmax - 1;  // last k with lstart[k] <= i
-        while (a < b) {
-            int m = (a + b + 1) >> 1;
-            if (g.lstart[m] <= i) a = m;
-            else b = m - 1;
-        }
-        const uint4 r = g.flat[i];
-        depth[(size_t)r.z * g.N + (r.x & kCellMask)] = (uint32_t)a;
+    if (tid == 0) {
+        atomicAdd(&totals[0], total);
+        atomicMax(&totals[1], k);
     }
 }
 
@@ -811,7 +781,7 @@ __global__ void __launch_bounds__(kBlock) k_sweep_rec(Geo g, Flux<R> fl, const u
     const uint32_t nfmax = wave_max(valid ? (r.x >> kCellBits) : 0u);
     double A;
     R inc;
-    task_faces<R, true, false>(g, fl, valid, r, sub, nfmax, A, inc, nullptr, nullptr);
+    task_faces<R>(g, fl, valid, r, sub, nfmax, A, inc);
     if (valid && sub == 0) finish_task<R>(fl, (size_t)d * g.N + c, (size_t)d * g.N + c, inc, ci, (R)A);
 }
 
@@ -2659,11 +2629,8 @@ struct ssw_sweep {
     double aref = 1.0;
     double dw[3] = {0, 0, 0};
     int64_t ovf_total = 0;
-    // Kahn layering scratch (full graph at upload, restricted sets for the
-    // hooks): flat and cnt are held only while a layering or count runs
-    uint4* d_flat = nullptr;
-    uint32_t *d_lstart = nullptr, *d_ctr = nullptr, *d_cnt = nullptr, *d_need = nullptr;
-    int kcap = 0;
+    // upwind counters, held only while a layering or a count runs
+    uint32_t *d_cnt = nullptr, *d_need = nullptr;
     // full schedule
     int kmax = 0;
     std::vector<uint32_t> full_start;               // kmax + 1 level starts
@@ -2803,9 +2770,6 @@ Geo make_geo(ssw_sweep* s) {
     g.pgeo = s->d_pgeo;
     g.pnb = s->d_pnb;
     g.Nper = s->Nper;
-    g.flat = s->d_flat;
-    g.lstart = s->d_lstart;
-    g.ctr = s->d_ctr;
     g.cnt = s->d_cnt;
     g.need = s->d_need;
     return g;
@@ -2976,75 +2940,48 @@ void drop_all_lists(ssw_sweep* s) {
     for (int l = 0; l < (int)s->list_ok.size(); l++) drop_list(s, l);
 }
 
-// The layering scratch: counters (cnt) and, with `flat`, the level-major task
-// records of a layering.
-int ensure_layering_scratch(ssw_sweep* s, bool flat = true) {
-    const size_t DN = (size_t)s->D * s->N;
-    if (!s->d_cnt) TRY(dalloc(s, &s->d_cnt, DN));
-    if (flat && !s->d_flat) TRY(dalloc(s, &s->d_flat, DN));
-    return SSW_OK;
-}
-
-void release_layering_scratch(ssw_sweep* s) {
-    dfree(s, s->d_flat);
-    dfree(s, s->d_cnt);
-}
-
-// Kahn layering of the active set {level >= lvl} into the scratch records:
-// counting, then one launch per level set until the queue is empty. The
-// launches go out in batches of kKahnBatch level sets between host reads of
-// the level starts (a launch past the last level set finds it empty and only
-// repeats its start); the grid of a batch is sized from the last width read.
+// Kahn layering of the active set {level >= lvl}: every active task's depth
+// into d_depth, the number of level sets and, with `starts`, where each of
+// them starts in level order. The upwind counters are freed again.
 // `expected` active tasks must all be placed, else the graph has a cycle.
-constexpr int kKahnBatch = 32;
-
-int kahn_layering(ssw_sweep* s, int lvl, int64_t expected, int* depth_out, std::vector<uint32_t>* starts) {
-    Geo g = make_geo(s);
-    k_kahn_reset<<<1, 64, 0, s->stream>>>(g);
-    k_count<<<grid_for((int64_t)s->N * s->D), kBlock, 0, s->stream>>>(g, lvl, 0);
+int kahn_layering(ssw_sweep* s, int lvl, int64_t expected, uint32_t* d_depth, int* depth_out,
+                  std::vector<uint32_t>* starts) {
+    const size_t DN = (size_t)s->D * s->N;
+    const uint32_t kcap = (uint32_t)std::min<int64_t>(s->N + 1, 1 << 22);
+    uint32_t *spill = nullptr, *hist = nullptr;  // hist: totals, then the level sets' tasks
+    Defer cleanup{[&] {
+        dfree(s, spill);
+        dfree(s, hist);
+        dfree(s, s->d_cnt);
+    }};
+    if (!s->d_cnt) TRY(dalloc(s, &s->d_cnt, DN));
+    TRY(dalloc(s, &spill, 2 * DN));
+    TRY(dalloc(s, &hist, (size_t)kcap + 2));
+    const Geo g = make_geo(s);
+    k_fill_u32<<<grid_for((int64_t)kcap + 2), kBlock, 0, s->stream>>>(hist, 0u, (int64_t)kcap + 2);
+    k_count<<<grid_for((int64_t)DN), kBlock, 0, s->stream>>>(g, lvl);
+    if (s->N <= (int64_t)kLayerCells)
+        k_layers<true><<<s->D, 1024, 0, s->stream>>>(g, kcap, d_depth, spill, hist + 2, hist);
+    else
+        k_layers<false><<<s->D, 1024, 0, s->stream>>>(g, kcap, d_depth, spill, hist + 2, hist);
     HIP_TRY(hipGetLastError());
-    if (starts) starts->assign(1, 0u);
-    uint32_t c3[3];
-    HIP_TRY(hipMemcpyAsync(c3, s->d_ctr, sizeof(c3), hipMemcpyDeviceToHost, s->stream));
+    uint32_t totals[2] = {0, 0};
+    HIP_TRY(hipMemcpyAsync(totals, hist, sizeof(totals), hipMemcpyDeviceToHost, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
-    if (c3[0] == 0) {
-        if (expected != 0)
-            return fail(SSW_ERR_CYCLE, "dependency cycle: " + std::to_string(expected) +
-                                           " cell-direction pairs never become ready");
-        k_kahn<<<1, kBlock, 0, s->stream>>>(g, 0);  // no active task: one empty level set
-        HIP_TRY(hipGetLastError());
-        if (starts) starts->push_back(0u);
-        *depth_out = 1;
-        return SSW_OK;
+    if ((int64_t)totals[0] != expected) {
+        if (totals[1] >= kcap) return fail(SSW_ERR_CYCLE, "level-set depth exceeds its bound");
+        return fail(SSW_ERR_CYCLE, "dependency cycle: " + std::to_string(expected - (int64_t)totals[0]) +
+                                       " cell-direction pairs never become ready");
     }
-    uint32_t hint = c3[0], prev = 0;
-    std::vector<uint32_t> part(kKahnBatch);
-    for (int k = 0;;) {
-        const int kend = std::min(k + kKahnBatch, s->kcap - 1);
-        if (k >= kend) return fail(SSW_ERR_CYCLE, "level-set depth exceeds its bound");
-        const unsigned blocks =
-            (unsigned)std::max<int64_t>(1, std::min<int64_t>(16384, (2 * (int64_t)hint + kTasksPerBlock - 1) /
-                                                                        kTasksPerBlock));
-        for (int kk = k; kk < kend; kk++) k_kahn<<<blocks, kBlock, 0, s->stream>>>(g, kk);
-        HIP_TRY(hipGetLastError());
-        HIP_TRY(hipMemcpyAsync(part.data(), s->d_lstart + k + 1, (size_t)(kend - k) * 4, hipMemcpyDeviceToHost,
-                               s->stream));
+    *depth_out = (int)std::max(1u, totals[1]);  // no active task: one empty level set
+    if (starts) {
+        std::vector<uint32_t> h((size_t)*depth_out);
+        HIP_TRY(hipMemcpyAsync(h.data(), hist + 2, h.size() * 4, hipMemcpyDeviceToHost, s->stream));
         HIP_TRY(hipStreamSynchronize(s->stream));
-        for (int kk = k; kk < kend; kk++) {
-            const uint32_t cur = part[kk - k];
-            if (cur == prev) {  // level set kk is empty: the layering ended with kk level sets
-                if ((int64_t)prev != expected)
-                    return fail(SSW_ERR_CYCLE, "dependency cycle: " + std::to_string(expected - (int64_t)prev) +
-                                                   " cell-direction pairs never become ready");
-                *depth_out = std::max(1, kk);
-                return SSW_OK;
-            }
-            if (starts) starts->push_back(cur);
-            hint = cur - prev;
-            prev = cur;
-        }
-        k = kend;
+        starts->assign(1, 0u);
+        for (uint32_t v : h) starts->push_back(starts->back() + v);
     }
+    return SSW_OK;
 }
 
 // Device bytes of the grouped replay for DN tasks, n cells and L timestep
@@ -3488,13 +3425,6 @@ int init_replay(ssw_sweep* s);
 // chunk table of the compaction.
 int build_schedule(ssw_sweep* s) {
     const size_t DN = (size_t)s->D * s->N;
-    s->kcap = (int)std::min<int64_t>(s->N + 2, 1 << 22);
-    TRY(dalloc(s, &s->d_lstart, (size_t)s->kcap + 2));
-    TRY(ensure_layering_scratch(s));
-    int depth = 0;
-    TRY(kahn_layering(s, 0, (int64_t)DN, &depth, &s->full_start));
-    s->kmax = depth;
-    dfree(s, s->d_cnt);
     // sort the tasks by depth, stable over t = d*N + c (double-buffered: four
     // DN-word arrays and a small temporary)
     uint32_t *d_depth = nullptr, *d_keys = nullptr, *d_vals = nullptr, *d_vals2 = nullptr, *d_sorted = nullptr;
@@ -3504,12 +3434,8 @@ int build_schedule(ssw_sweep* s) {
         dfree(s, d_tmp);
     }};
     TRY(dalloc(s, &d_depth, DN));
+    TRY(kahn_layering(s, 0, (int64_t)DN, d_depth, &s->kmax, &s->full_start));
     Geo g = make_geo(s);
-    k_scatter_depth<<<grid_for(std::min<int64_t>((int64_t)DN, 1 << 22)), kBlock, 0, s->stream>>>(g, s->kmax,
-                                                                                                  d_depth);
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(s->stream));
-    dfree(s, s->d_flat);
     if (s->compiled && s->dir_sweeps) {
         TRY(s->fp32 ? build_dir_schedule_t<float>(s, d_depth) : build_dir_schedule_t<double>(s, d_depth));
         return init_replay(s);
@@ -4554,9 +4480,6 @@ void free_grid(ssw_sweep* s) {
     dfree(s, s->d_pfoff);
     dfree(s, s->d_pnb);
     dfree(s, s->d_pgeo);
-    dfree(s, s->d_flat);
-    dfree(s, s->d_lstart);
-    dfree(s, s->d_ctr);
     dfree(s, s->d_cnt);
     dfree(s, s->d_level);
     dfree(s, s->d_fstart);
@@ -5036,7 +4959,6 @@ int ssw_upload_grid(ssw_sweep* s, int64_t n, const int64_t* off, const int32_t* 
     TRY(dalloc(s, &s->d_pnb, std::max<size_t>(1, pnb.size())));
     TRY(dalloc(s, &s->d_pgeo, std::max<size_t>(1, pgeo.size())));
     TRY(dalloc(s, &s->d_level, n));
-    TRY(dalloc(s, &s->d_ctr, 3));
     TRY(dalloc(s, &s->d_cnt, DN));
     if (s->permuted) {
         TRY(dalloc(s, &s->d_inv, n));
@@ -5311,14 +5233,14 @@ int ssw_download_counts(ssw_sweep* s, int32_t lvl, uint32_t* counts) {
     if (!s || !counts) return fail(SSW_ERR_INVALID, "null argument");
     if (!s->have_grid) return fail(SSW_ERR_INVALID, "ssw_upload_grid must be called first");
     if (lvl < 0 || lvl >= s->p.num_timestep_levels) return fail(SSW_ERR_INVALID, "sweep_level out of range");
-    Defer cleanup{[&] { release_layering_scratch(s); }};
-    TRY(ensure_layering_scratch(s, false));
-    Geo g = make_geo(s);
-    k_count<<<grid_for((int64_t)s->N * s->D), kBlock, 0, s->stream>>>(g, lvl, 1);
+    Defer cleanup{[&] { dfree(s, s->d_cnt); }};
+    if (!s->d_cnt) TRY(dalloc(s, &s->d_cnt, (size_t)s->D * s->N));
+    const Geo g = make_geo(s);
+    k_count<<<grid_for((int64_t)s->N * s->D), kBlock, 0, s->stream>>>(g, lvl);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipMemcpyAsync(counts, s->d_cnt, (size_t)s->D * s->N * 4, hipMemcpyDeviceToHost, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
-    release_layering_scratch(s);
+    dfree(s, s->d_cnt);
     to_caller(s, counts, s->D);
     return SSW_OK;
 }
@@ -5327,8 +5249,7 @@ int ssw_download_levelsets(ssw_sweep* s, int32_t lvl, uint32_t* depth) {
     if (!s || !depth) return fail(SSW_ERR_INVALID, "null argument");
     if (!s->have_grid) return fail(SSW_ERR_INVALID, "ssw_upload_grid must be called first");
     if (lvl < 0 || lvl >= s->p.num_timestep_levels) return fail(SSW_ERR_INVALID, "sweep_level out of range");
-    // Kahn layering of the restricted graph in the scratch records (the replay
-    // schedule is not touched)
+    // Kahn layering of the restricted graph (the replay schedule is not touched)
     std::vector<uint8_t> lev(s->N);
     HIP_TRY(hipMemcpyAsync(lev.data(), s->d_level, s->N, hipMemcpyDeviceToHost, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
@@ -5336,22 +5257,14 @@ int ssw_download_levelsets(ssw_sweep* s, int32_t lvl, uint32_t* depth) {
     for (uint8_t v : lev) active += v >= lvl;
     int k = 0;
     uint32_t* d_depth = nullptr;
-    Defer cleanup{[&] {
-        dfree(s, d_depth);
-        release_layering_scratch(s);
-    }};
-    TRY(ensure_layering_scratch(s));
-    TRY(kahn_layering(s, lvl, active * s->D, &k, nullptr));
+    Defer cleanup{[&] { dfree(s, d_depth); }};
     const int64_t DN = (int64_t)s->D * s->N;
     TRY(dalloc(s, &d_depth, (size_t)DN));
     k_fill_u32<<<grid_for(DN), kBlock, 0, s->stream>>>(d_depth, kNone, DN);
-    Geo g = make_geo(s);
-    k_scatter_depth<<<grid_for(std::min<int64_t>(DN, 1 << 22)), kBlock, 0, s->stream>>>(g, k, d_depth);
-    HIP_TRY(hipGetLastError());
+    TRY(kahn_layering(s, lvl, active * s->D, d_depth, &k, nullptr));
     HIP_TRY(hipMemcpyAsync(depth, d_depth, (size_t)DN * 4, hipMemcpyDeviceToHost, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
     dfree(s, d_depth);
-    release_layering_scratch(s);
     to_caller(s, depth, s->D);
     return SSW_OK;
 }

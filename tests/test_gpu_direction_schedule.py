@@ -14,6 +14,7 @@ to the grouped replay (X, I, fields) on grids made by hand:
 import numpy as np
 import pytest
 
+from oracle.oracle import OracleSweep
 from subsweep_amd import Sweep, SweepParameters
 from subsweep_amd.grid import Grid
 
@@ -98,3 +99,18 @@ def test_tiles_bitwise_equal_grouped(name, precision, hip_available):
             assert np.array_equal(ra.ionized_hydrogen_fraction, rb.ionized_hydrogen_fraction)
             assert np.array_equal(ra.photon_rate, rb.photon_rate) and np.array_equal(ra.level, rb.level)
         assert np.count_nonzero(a.transport_state()[1]) > n // 2 or n == 1
+
+
+@pytest.mark.parametrize("name", ["tiny1", "tiny65", "hub115", "slab110", "slab190"])
+def test_level_sets_equal_the_oracles(name, hip_available):
+    # counters in LDS and (slab190: 144400 cells) in memory, level sets that
+    # fit in the queues and ones that go on in memory
+    grid, dirs = CASES[name]()
+    n = grid.num_cells
+    state = (np.full(n, 1e-27), np.full(n, 1e-10), np.full(n, 1e4), np.full(n, 1e48))
+    p = SweepParameters(directions=dirs, num_timestep_levels=2, max_timestep=1e-3 * MYR)
+    o = OracleSweep(p, grid, *state)
+    with Sweep(p, grid, *state) as s:
+        for lvl in range(2):
+            assert np.array_equal(s.counts(lvl), o.counts(lvl)) and np.array_equal(s.levelsets(lvl), o.levelsets(lvl))
+    o.close()
