@@ -2026,6 +2026,45 @@ __global__ void k_gather_u32(const uint32_t* __restrict__ src, const uint32_t* _
 // ---------------------------------------------------------------------------
 // per-sweep kernels
 
+struct ChemArgs {
+    double* rho;
+    double* x;
+    double* T;
+    double* src;             // source per direction bin (SI)
+    void* sa;                // SA<R>[N], .y: attenuation of the next sweep
+    double* species_ts;
+    double* prev_rate;
+    double* change_ts;
+    const double* vol;
+    const double* size;
+    double max_ts;
+    double thr;
+    double safety;
+    double scale_factor;
+    int prevent_cooling;
+    double lref;             // storage scale of I (rate = I * lref)
+    unsigned long long* failures;
+    unsigned long long* active;
+    unsigned long long* limiting;  // [3] TimescaleCounter: temperature, ionisation fraction, photon rate
+    uint32_t* queue;         // {cells queued, cells taken beyond the first ones}, then the queued cells
+};
+
+// The arguments of the kernels after a sweep, for one handle, or for the
+// handles of a packed step (one per blockIdx.y).
+template <typename R>
+struct ChemJob {
+    Geo g;
+    Flux<R> fl;
+    ChemArgs ca;
+    int lvl;
+};
+constexpr int kChemJobs = 4;
+template <typename R, int kJobs>
+struct ChemJobs {
+    ChemJob<R> job[kJobs];
+    __device__ __forceinline__ const ChemJob<R>& mine() const { return job[kJobs > 1 ? blockIdx.y : 0]; }
+};
+
 // Periodic source of every periodic cell from the current X, after each
 // sweep: the chemistry of the sweep reads it (the reference's periodic
 // corrections have all arrived when update_chemistry runs), and the next
@@ -2039,9 +2078,12 @@ __global__ void k_gather_u32(const uint32_t* __restrict__ src, const uint32_t* _
 // 108, 47 and 29. The first
 // thread empties the queue of the chemistry that follows.
 constexpr int kPerDirs = 2;
-template <typename R>
-__global__ void __launch_bounds__(kBlock) k_periodic(Geo g, Flux<R> fl, uint32_t* queue) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) queue[0] = queue[1] = 0u;
+template <typename R, int kJobs>
+__global__ void __launch_bounds__(kBlock) k_periodic(const ChemJobs<R, kJobs> jobs) {
+    const ChemJob<R>& J = jobs.mine();
+    const Geo& g = J.g;
+    const Flux<R>& fl = J.fl;
+    if (blockIdx.x == 0 && threadIdx.x == 0) J.ca.queue[0] = J.ca.queue[1] = 0u;
     if (fl.P == nullptr) return;
     const uint32_t dblocks = ((uint32_t)g.D + kPerDirs - 1u) / kPerDirs;
     const uint32_t w = __builtin_amdgcn_readfirstlane((blockIdx.x * kBlock + threadIdx.x) / 64u);
@@ -2079,29 +2121,6 @@ __global__ void __launch_bounds__(kBlock) k_periodic(Geo g, Flux<R> fl, uint32_t
     for (int j = 0; j < kPerDirs; j++)
         if (d0 + j < (uint32_t)g.D) fl.P[(size_t)(d0 + j) * g.Nper + s] = acc[j];
 }
-
-struct ChemArgs {
-    double* rho;
-    double* x;
-    double* T;
-    double* src;             // source per direction bin (SI)
-    void* sa;                // SA<R>[N], .y: attenuation of the next sweep
-    double* species_ts;
-    double* prev_rate;
-    double* change_ts;
-    const double* vol;
-    const double* size;
-    double max_ts;
-    double thr;
-    double safety;
-    double scale_factor;
-    int prevent_cooling;
-    double lref;             // storage scale of I (rate = I * lref)
-    unsigned long long* failures;
-    unsigned long long* active;
-    unsigned long long* limiting;  // [3] TimescaleCounter: temperature, ionisation fraction, photon rate
-    uint32_t* queue;         // {cells queued, cells taken beyond the first ones}, then the queued cells
-};
 
 // Adds the number of lanes with `pred` to *counter with one atomic per wave
 // (lanes outside the current control flow take no part).
@@ -2152,11 +2171,18 @@ __device__ __forceinline__ void finish_chemistry(const ChemArgs& ca, int64_t c, 
 // the rate and the first attempt of the solver; cells whose full step is
 // rejected go to the queue of k_chemistry_tail, else a wave would last as long
 // as its slowest cell's sub-steps, one after the other.
-template <typename R>
-__global__ void __launch_bounds__(kBlock) k_chemistry(Geo g, Flux<R> fl, ChemArgs ca, int lvl) {
+template <typename R, int kJobs>
+__global__ void __launch_bounds__(kBlock) k_chemistry(const ChemJobs<R, kJobs> jobs) {
+    const ChemJob<R>& J = jobs.mine();
+    const Geo& g = J.g;
+    const Flux<R>& fl = J.fl;
+    const ChemArgs& ca = J.ca;
+    const int lvl = J.lvl;
+    const uint32_t nb = (uint32_t)((g.N + kBlock - 1) / kBlock);
+    if (blockIdx.x >= nb) return;  // another handle's cells are more
     // a die takes consecutive cells: where I is gathered (direction sweeps),
     // they share its lines in the die's L2
-    int64_t c = (int64_t)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    int64_t c = (int64_t)xcd_block(blockIdx.x, nb) * kBlock + threadIdx.x;
     if (c == 0) g.need[lvl] = 0;  // the active-set list of this sweep level is current
     if (c >= g.N) return;
     int lev = g.level[c];
@@ -2213,8 +2239,10 @@ __global__ void __launch_bounds__(kBlock) k_chemistry(Geo g, Flux<R> fl, ChemArg
 // takes the next one while the others of its wave go on. Chemistry of 262144
 // cells with 64 sources: 1.04 -> 0.60 ms (0.19 + 0.41), of 32768 cells in the
 // first two steps 1.96 -> 1.33 ms a step.
-template <typename R>
-__global__ void __launch_bounds__(64) k_chemistry_tail(Geo g, ChemArgs ca) {
+template <typename R, int kJobs>
+__global__ void __launch_bounds__(64) k_chemistry_tail(const ChemJobs<R, kJobs> jobs) {
+    const Geo& g = jobs.mine().g;
+    const ChemArgs& ca = jobs.mine().ca;
     const uint32_t n = ca.queue[0], first = gridDim.x * 16u;
     const bool lead = (threadIdx.x & 3u) == 0;
     uint32_t i = blockIdx.x * 16u + threadIdx.x / 4u;
@@ -2672,10 +2700,10 @@ struct ssw_sweep {
     double *d_rho = nullptr, *d_x = nullptr, *d_T = nullptr, *d_src = nullptr;
     void* d_sa = nullptr;                           // SA<R>: {transport source / D, attenuation}
     double *d_sts = nullptr, *d_prev = nullptr, *d_change = nullptr;
+    // of the last step: chemistry updates, then the 3 limiting processes' counts
     unsigned long long* d_active = nullptr;
     double* d_photon = nullptr;                     // photon rates of a download (internal order)
     uint32_t* d_chemq = nullptr;                    // k_chemistry's queue (ChemArgs::queue)
-    unsigned long long* d_limit = nullptr;          // [3] limiting processes of the last step
     uint8_t* d_level = nullptr;
     void *d_X = nullptr, *d_I = nullptr, *d_P = nullptr;
     void *d_offI = nullptr, *d_offP = nullptr;      // rate offsets after a rotation (Flux::offI / offP)
@@ -3830,20 +3858,28 @@ ChemArgs chem_args(ssw_sweep* s) {
     ca.lref = s->lref;
     ca.failures = s->d_fail;
     ca.active = s->d_active;
-    ca.limiting = s->d_limit;
+    ca.limiting = s->d_active + 1;
     ca.queue = s->d_chemq;
     return ca;
 }
 
-// The periodic sources and the chemistry after a sweep at level lvl. The tail
-// gets a wave per 16 cells, at most two per SIMD (its quads take further cells
-// as they finish); waves that find no queued cell end at once.
-template <typename R>
-void launch_chemistry(ssw_sweep* s, const Geo& g, const Flux<R>& fl, const ChemArgs& ca, int lvl, hipStream_t st) {
-    const int64_t pwaves = (s->Nper + 63) / 64 * ((s->D + kPerDirs - 1) / kPerDirs);
-    k_periodic<R><<<grid_for(64 * pwaves), kBlock, 0, st>>>(g, fl, ca.queue);
-    k_chemistry<R><<<grid_for(s->N), kBlock, 0, st>>>(g, fl, ca, lvl);
-    k_chemistry_tail<R><<<(unsigned)std::min<int64_t>((s->N + 15) / 16, 2048), 64, 0, st>>>(g, ca);
+// The periodic sources and the chemistry of n handles (at most kChemJobs) after
+// their sweeps. The tail gets a wave per 16 cells, at most two per SIMD (its
+// quads take further cells as they finish); waves that find no queued cell end
+// at once.
+template <typename R, int kJobs>
+void launch_chemistry(const ChemJob<R>* j, int n, hipStream_t st) {
+    ChemJobs<R, kJobs> a;
+    int64_t pw = 0, cells = 0;
+    for (int k = 0; k < n; k++) {
+        a.job[k] = j[k];
+        const Geo& g = j[k].g;
+        pw = std::max(pw, (g.Nper + 63) / 64 * ((g.D + kPerDirs - 1) / kPerDirs));
+        cells = std::max(cells, g.N);
+    }
+    k_periodic<R, kJobs><<<dim3(grid_for(64 * pw), n), kBlock, 0, st>>>(a);
+    k_chemistry<R, kJobs><<<dim3(grid_for(cells), n), kBlock, 0, st>>>(a);
+    k_chemistry_tail<R, kJobs><<<dim3((unsigned)std::min<int64_t>((cells + 15) / 16, 2048), n), 64, 0, st>>>(a);
 }
 
 // ssw_sweep::rates_current after the sweeps of `order`.
@@ -3860,8 +3896,7 @@ int run_step(ssw_sweep* s, double* elapsed) {
     const std::vector<int> order = s->ts.sweep_order();
     const int L = s->p.num_timestep_levels;
     s->rates_current = false;  // an error below leaves a partly swept state
-    k_fill_u32<<<1, 2, 0, s->stream>>>((uint32_t*)s->d_active, 0u, 2);
-    k_fill_u32<<<1, 6, 0, s->stream>>>((uint32_t*)s->d_limit, 0u, 6);
+    k_fill_u32<<<1, 8, 0, s->stream>>>((uint32_t*)s->d_active, 0u, 8);
     const unsigned gcells = grid_for(s->N);
     s->sweeps_last = 0;
     s->builds_last = 0;
@@ -3910,7 +3945,8 @@ int run_step(ssw_sweep* s, double* elapsed) {
         HIP_TRY(hipGetLastError());
         s->replays[lvl]++;
         hipEvent_t a = s->timing ? mark() : nullptr;
-        launch_chemistry<R>(s, g, fl, ca, lvl, s->stream);
+        const ChemJob<R> job{g, fl, ca, lvl};
+        launch_chemistry<R, 1>(&job, 1, s->stream);
         if (s->timing) ch.push_back({a, mark()});
         s->sweeps_last++;
     }
@@ -4054,10 +4090,16 @@ void packed_item(ssw_sweep* s, const Geo& g, int lvl, const ssw_sweep::ReplayIte
     launch_item_t<R>(s, g, make_flux<R>(s), lvl, it, st);
 }
 
+// The chemistry of a packed sweep's handles of one precision, kChemJobs to a
+// launch: a handle's sub-steps are a chain of their own, and one launch after
+// the other would add them up.
 template <typename R>
-void batch_chemistry(ssw_sweep* s, const Geo& g, int lvl, hipStream_t st) {
-    const Flux<R> fl = make_flux<R>(s);
-    launch_chemistry<R>(s, g, fl, chem_args(s), lvl, st);
+void batch_chemistry(const std::vector<ChemJob<R>>& jobs, hipStream_t st) {
+    for (size_t k = 0; k < jobs.size(); k += kChemJobs) {
+        const int n = (int)std::min<size_t>(kChemJobs, jobs.size() - k);
+        if (n == 1) launch_chemistry<R, 1>(&jobs[k], 1, st);
+        else launch_chemistry<R, kChemJobs>(&jobs[k], n, st);
+    }
 }
 
 // Graphs of packed sweeps, keyed by (uid, epoch, sweep level) of every
@@ -4139,8 +4181,7 @@ int step_pack(BatchSweep* bs, int n, double* elapsed) {
         HIP_TRY(hipStreamWaitEvent(st, s->sync_ev, 0));
     }
     for (int h = 0; h < n; h++) {
-        k_fill_u32<<<1, 2, 0, st>>>((uint32_t*)bs[h].s->d_active, 0u, 2);
-        k_fill_u32<<<1, 6, 0, st>>>((uint32_t*)bs[h].s->d_limit, 0u, 6);
+        k_fill_u32<<<1, 8, 0, st>>>((uint32_t*)bs[h].s->d_active, 0u, 8);
     }
     size_t sweeps = 0;
     for (int h = 0; h < n; h++) sweeps = std::max(sweeps, bs[h].order.size());
@@ -4148,8 +4189,8 @@ int step_pack(BatchSweep* bs, int n, double* elapsed) {
     for (int h = 0; h < n; h++) graphs = graphs && bs[h].s->graphs_on;
     const int dev = bs[0].s->device;
     for (size_t i = 0; i < sweeps; i++) {
-        // sweep i of every handle: the t-th plan items together, then each
-        // handle's periodic sources and chemistry
+        // sweep i of every handle: the t-th plan items together, then the
+        // handles' periodic sources and chemistry together
         const std::function<void()> enqueue = [&]() {
             Packs pk;
             size_t items = 0;
@@ -4168,12 +4209,16 @@ int step_pack(BatchSweep* bs, int n, double* elapsed) {
                 }
                 pk.flush(st);
             }
+            std::vector<ChemJob<float>> jf;
+            std::vector<ChemJob<double>> jd;
             for (int h = 0; h < n; h++) {
                 BatchSweep& b = bs[h];
                 if (i >= b.order.size()) continue;
-                if (b.s->fp32) batch_chemistry<float>(b.s, b.g, b.order[i], st);
-                else batch_chemistry<double>(b.s, b.g, b.order[i], st);
+                if (b.s->fp32) jf.push_back({b.g, make_flux<float>(b.s), chem_args(b.s), b.order[i]});
+                else jd.push_back({b.g, make_flux<double>(b.s), chem_args(b.s), b.order[i]});
             }
+            batch_chemistry<float>(jf, st);
+            batch_chemistry<double>(jd, st);
         };
         bool done = false;
         if (graphs) {
@@ -4740,16 +4785,14 @@ int ssw_create(const ssw_sweep_parameters* params, ssw_sweep** out) {
     int r = dalloc(s, &s->d_dirs, dirs.size());
     if (r == SSW_OK) r = dalloc(s, &s->d_need, (size_t)p.num_timestep_levels);
     if (r == SSW_OK) r = dalloc(s, &s->d_fail, 1);
-    if (r == SSW_OK) r = dalloc(s, &s->d_active, 1);
-    if (r == SSW_OK) r = dalloc(s, &s->d_limit, 3);
+    if (r == SSW_OK) r = dalloc(s, &s->d_active, 4);
     if (r != SSW_OK) {
         ssw_destroy(s);
         return r;
     }
     if (hipMemcpyAsync(s->d_dirs, dirs.data(), dirs.size() * 8, hipMemcpyHostToDevice, s->stream) != hipSuccess ||
         hipMemsetAsync(s->d_fail, 0, 8, s->stream) != hipSuccess ||
-        hipMemsetAsync(s->d_active, 0, 8, s->stream) != hipSuccess ||
-        hipMemsetAsync(s->d_limit, 0, 24, s->stream) != hipSuccess || hipStreamSynchronize(s->stream) != hipSuccess) {
+        hipMemsetAsync(s->d_active, 0, 32, s->stream) != hipSuccess || hipStreamSynchronize(s->stream) != hipSuccess) {
         ssw_destroy(s);
         return fail(SSW_ERR_HIP, "initialisation of the handle's device memory failed");
     }
@@ -4767,7 +4810,6 @@ void ssw_destroy(ssw_sweep* s) {
     dfree(s, s->d_need);
     dfree(s, s->d_fail);
     dfree(s, s->d_active);
-    dfree(s, s->d_limit);
     for (hipEvent_t e : s->ev) (void)hipEventDestroy(e);
     if (s->sync_ev) (void)hipEventDestroy(s->sync_ev);
     if (s->stream) {
@@ -5040,8 +5082,7 @@ int ssw_upload_state(ssw_sweep* s, const double* density, const double* xhii, co
     HIP_TRY(hipMemsetAsync(s->d_I, 0, (size_t)s->D * n * es, s->stream));
     if (s->Nper) HIP_TRY(hipMemsetAsync(s->d_P, 0, (size_t)s->D * s->Nper * es, s->stream));
     HIP_TRY(hipMemsetAsync(s->d_fail, 0, 8, s->stream));
-    HIP_TRY(hipMemsetAsync(s->d_active, 0, 8, s->stream));
-    HIP_TRY(hipMemsetAsync(s->d_limit, 0, 24, s->stream));
+    HIP_TRY(hipMemsetAsync(s->d_active, 0, 32, s->stream));
     std::vector<uint8_t> lev(n, (uint8_t)(L - 1));  // src/sweep/mod.rs:206
     HIP_TRY(hipMemcpyAsync(s->d_level, lev.data(), n, hipMemcpyHostToDevice, s->stream));
     if (s->fp32)
@@ -5593,7 +5634,7 @@ int ssw_get_info(ssw_sweep* s, ssw_info* info) {
         unsigned long long f = 0, a = 0, lim[3] = {0, 0, 0};
         HIP_TRY(hipMemcpyAsync(&f, s->d_fail, 8, hipMemcpyDeviceToHost, s->stream));
         HIP_TRY(hipMemcpyAsync(&a, s->d_active, 8, hipMemcpyDeviceToHost, s->stream));
-        HIP_TRY(hipMemcpyAsync(lim, s->d_limit, 24, hipMemcpyDeviceToHost, s->stream));
+        HIP_TRY(hipMemcpyAsync(lim, s->d_active + 1, 24, hipMemcpyDeviceToHost, s->stream));
         HIP_TRY(hipStreamSynchronize(s->stream));
         info->chemistry_failures = (int64_t)f;
         info->updates_last_step = (int64_t)a * s->D;
