@@ -93,6 +93,7 @@ constexpr int kRunBlock = 1024;            // workgroup of a run of narrow level
 constexpr int kGroupT = 64;                // grouped replay: root tasks per workgroup (default; 64 or 128)
 constexpr int kGroupLevels = 4;            // grouped replay: level sets per group (default)
 constexpr int kConeCap = 3072;             // grouped replay build: cone members / pending entries per workgroup
+constexpr int kConeThreads = 256;
 constexpr int kSortCap = 4096;             // grouped replay build: entries of one level set sorted in LDS
 constexpr int kMaxGroup = 8;               // grouped replay: level sets per group
 constexpr uint32_t kNarrowGroup = 2048;    // grouped replay: level sets this narrow go kMaxGroup to a group
@@ -1438,6 +1439,9 @@ __device__ __forceinline__ uint32_t wave_scan(uint32_t v) {  // inclusive
     return v;
 }
 
+// 16-byte units of n values of b bytes.
+__host__ __device__ __forceinline__ uint32_t units16(uint32_t n, uint32_t b) { return (n * b + 15u) / 16u; }
+
 // The tiles of one group, one wave: consecutive tasks while their far and
 // extra entries stay within kDirCap (a task with more is a tile of its own).
 // Calls tile(first lane, tasks, far, extra, planes, units) for each.
@@ -1452,7 +1456,7 @@ __device__ __forceinline__ void dir_tiles(uint32_t cnt, uint32_t nup, uint32_t f
         const uint32_t e = over ? (uint32_t)__ffsll((long long)over) - 1u : cnt;
         const uint32_t nf = (uint32_t)__shfl((int)pf, e - 1) - bf, ne = (uint32_t)__shfl((int)pe, e - 1) - be;
         const uint32_t np = DirShape<R>::planes(wave_max(lane >= a && lane < e ? nup : 0u));
-        const uint32_t units = np * (e - a) + (nf + 3u) / 4u + (ne * (uint32_t)sizeof(R) + 15u) / 16u + (ne + 3u) / 4u;
+        const uint32_t units = np * (e - a) + units16(nf, 4) + units16(ne, sizeof(R)) + units16(ne, 4);
         tile(a, e - a, bf, nf, be, ne, np, units);
         a = e;
     }
@@ -1485,6 +1489,72 @@ __global__ void __launch_bounds__(kBlock) k_dir_tile_count(const uint4* __restri
     }
 }
 
+// Writes task li of a tile of cnt tasks and np planes at `base`: header,
+// entries in face order, A as the 16-lane kernels form it. word(x) gives the
+// LDS word that holds the upwind X of index x, or kNone: then x goes to the
+// far list (at position fp on) and the entry names that place in the wave's
+// buffer (word `buf` on). Entries past the planes go to the extra list (at
+// position ep on).
+template <typename R, typename W>
+__device__ __forceinline__ void fill_task(const Geo& g, double inv_aref, uint32_t c, uint32_t d, uint32_t nup,
+                                          const uint32_t* __restrict__ xpos, uint4* base, uint32_t np, uint32_t cnt,
+                                          uint32_t li, uint32_t* flist, uint32_t fp, uint32_t buf, R* exw,
+                                          uint32_t* exs, uint32_t ep, W word) {
+    using S = DirShape<R>;
+    const uint32_t inplane = nup > kDirEntries ? kDirEntries - 1u : kDirEntries;
+    auto put_slot = [&](uint32_t h, uint32_t v) {  // halfword h of the slot planes
+        reinterpret_cast<uint16_t*>(base + (h < 8 ? 0u : S::kS1 * cnt) + li)[h % 8] = (uint16_t)v;
+    };
+    auto put_weight = [&](uint32_t j, R v) {
+        reinterpret_cast<R*>(base + S::wplane(j / S::kPer) * cnt + li)[j % S::kPer] = v;
+    };
+    const double dx = g.dirs[3 * d], dy = g.dirs[3 * d + 1], dz = g.dirs[3 * d + 2];
+    const uint32_t hdr = c | (nup << kCellBits);
+    put_slot(0, hdr & 0xFFFFu);
+    put_slot(1, hdr >> 16);
+    const uint32_t ps = g.pslot[c];
+    if (g.Nper && ps != kNone) {
+        flist[fp] = kFarPeriodic | (uint32_t)((size_t)d * g.Nper + ps);
+        put_slot(2, buf + fp++);
+    } else {
+        put_slot(2, 0u);
+    }
+    AreaTree A;
+    uint32_t q = 0;
+    const uint32_t f0 = g.off[c], f1 = g.off[c + 1];
+    for (uint32_t f = f0; f < f1; f++) {
+        const double4 fa = g.geo[f];
+        const uint32_t nk = g.nk[f];
+        const double dd = fdot(fa, dx, dy, dz);
+        if (dd > 0.0) {
+            A.add(f - f0, fa.w * inv_aref * dd);
+        } else if (dd < 0.0 && (nk >> 30) == kKindLocal) {
+            const R wt = (R)(fa.w * inv_aref * -dd);
+            const uint32_t x = xpos[(size_t)d * g.N + (nk & kNbrMask)];
+            uint32_t at = word(x);
+            if (at == kNone) {
+                flist[fp] = x;
+                at = buf + fp++;
+            }
+            if (q < inplane) {
+                put_slot(3 + q, at);
+                put_weight(1 + q, wt);
+            } else {
+                exw[ep + q - inplane] = wt;
+                exs[ep + q - inplane] = at;
+            }
+            q++;
+        }
+    }
+    put_weight(0, (R)A.total());
+    // the rest of the tile's planes: word 0, weight 0
+    const bool two = np > (uint32_t)S::kS1;
+    const uint32_t nw = (np - (two ? 2u : 1u)) * S::kPer;
+    for (uint32_t e = min(q, inplane); e < (two ? 13u : 5u); e++) put_slot(3 + e, 0u);
+    for (uint32_t e = min(q, inplane); e + 1 < nw; e++) put_weight(1 + e, (R)0);
+    if (nup > kDirEntries) put_slot(3 + kDirEntries - 1u, ep);
+}
+
 // The tiles and their blobs, one wave per group, one lane per task; the
 // entries in face order, A as the 16-lane kernels form it. tfirst[d]: first
 // tile of direction d (a tile's wave is its place in the direction mod
@@ -1508,7 +1578,6 @@ __global__ void __launch_bounds__(kBlock) k_dir_tile_fill(Geo g, double inv_aref
     const uint32_t pf = wave_scan(far), pe = wave_scan(lane < G.y ? dir_extra(nup) : 0u);
     uint32_t tile = ts[i];
     uint64_t off = us[i];
-    const double dx = g.dirs[3 * d], dy = g.dirs[3 * d + 1], dz = g.dirs[3 * d + 2];
     dir_tiles<R>(G.y, nup, far, pf, pe, [&](uint32_t a, uint32_t cnt, uint32_t bf, uint32_t nf, uint32_t be, uint32_t ne,
                                             uint32_t np, uint32_t units) {
         uint4* const base = blob + off;
@@ -1517,64 +1586,15 @@ __global__ void __launch_bounds__(kBlock) k_dir_tile_fill(Geo g, double inv_aref
             tiles[2 * (size_t)tile + 1] = make_uint4(G.w, cnt | (nf << 8) | (ne << 16) | (np << 24), 0u, 0u);
         }
         if (lane >= a && lane < a + cnt) {
-            const uint32_t li = lane - a;
             const uint32_t buf = S::kBufs + ((tile - tfirst[d]) % S::kWaves) * S::kBuf;
-            uint32_t* const flist = reinterpret_cast<uint32_t*>(base + np * cnt);
-            R* const exw = reinterpret_cast<R*>(base + np * cnt + (nf + 3u) / 4u);
-            uint32_t* const exs = reinterpret_cast<uint32_t*>(base + np * cnt + (nf + 3u) / 4u +
-                                                              (ne * (uint32_t)sizeof(R) + 15u) / 16u);
-            uint32_t fp = pf - far - bf, ep = pe - dir_extra(nup) - be;
-            const uint32_t inplane = nup > kDirEntries ? kDirEntries - 1u : kDirEntries;
-            auto put_slot = [&](uint32_t h, uint32_t v) {  // halfword h of the slot planes
-                reinterpret_cast<uint16_t*>(base + (h < 8 ? 0u : S::kS1 * cnt) + li)[h % 8] = (uint16_t)v;
-            };
-            auto put_weight = [&](uint32_t j, R v) {
-                reinterpret_cast<R*>(base + S::wplane(j / S::kPer) * cnt + li)[j % S::kPer] = v;
-            };
-            const uint32_t hdr = c | (nup << kCellBits);
-            put_slot(0, hdr & 0xFFFFu);
-            put_slot(1, hdr >> 16);
-            const uint32_t ps = g.pslot[c];
-            if (g.Nper && ps != kNone) {
-                flist[fp] = kFarPeriodic | (uint32_t)((size_t)d * g.Nper + ps);
-                put_slot(2, buf + fp++);
-            } else {
-                put_slot(2, 0u);
-            }
-            AreaTree A;
-            uint32_t q = 0;
-            const uint32_t f0 = g.off[c], f1 = g.off[c + 1];
-            for (uint32_t f = f0; f < f1; f++) {
-                const double4 fa = g.geo[f];
-                const uint32_t nk = g.nk[f];
-                const double dd = fdot(fa, dx, dy, dz);
-                if (dd > 0.0) {
-                    A.add(f - f0, fa.w * inv_aref * dd);
-                } else if (dd < 0.0 && (nk >> 30) == kKindLocal) {
-                    const R wt = (R)(fa.w * inv_aref * -dd);
-                    const uint32_t x = xpos[(size_t)dN + (nk & kNbrMask)];
-                    uint32_t at = S::kRingAt + ((x - dN) & (S::kRing - 1u));
-                    if (x + S::kRing < G.z) {
-                        flist[fp] = x;
-                        at = buf + fp++;
-                    }
-                    if (q < inplane) {
-                        put_slot(3 + q, at);
-                        put_weight(1 + q, wt);
-                    } else {
-                        exw[ep + q - inplane] = wt;
-                        exs[ep + q - inplane] = at;
-                    }
-                    q++;
-                }
-            }
-            put_weight(0, (R)A.total());
-            // the rest of the tile's planes: word 0, weight 0
-            const bool two = np > (uint32_t)S::kS1;
-            const uint32_t nw = (np - (two ? 2u : 1u)) * S::kPer;
-            for (uint32_t e = min(q, inplane); e < (two ? 13u : 5u); e++) put_slot(3 + e, 0u);
-            for (uint32_t e = min(q, inplane); e + 1 < nw; e++) put_weight(1 + e, (R)0);
-            if (nup > kDirEntries) put_slot(3 + kDirEntries - 1u, ep);
+            uint4* const lists = base + np * cnt;
+            uint4* const extra = lists + units16(nf, 4);
+            fill_task<R>(g, inv_aref, c, d, nup, xpos, base, np, cnt, lane - a, reinterpret_cast<uint32_t*>(lists),
+                         pf - far - bf, buf, reinterpret_cast<R*>(extra),
+                         reinterpret_cast<uint32_t*>(extra + units16(ne, sizeof(R))), pe - dir_extra(nup) - be,
+                         [&](uint32_t x) {
+                             return x + S::kRing < G.z ? kNone : S::kRingAt + ((x - dN) & (S::kRing - 1u));
+                         });
         }
         tile++;
         off += units;
@@ -1610,23 +1630,64 @@ __device__ void lds_sort(uint32_t* a, uint32_t n2) {
         }
 }
 
-// Appends the upwind schedule positions in [lo, hi) of the task at position
-// P (level set starting at b, width W) to cand.
-template <typename R>
-__device__ void push_upwind(const uint4* hdr, const Entry<R>* planes, const Entry<R>* ovf, uint32_t P, uint32_t b,
-                            uint32_t W, uint32_t lo, uint32_t hi, uint32_t* cand, uint32_t* ncand, uint32_t* over) {
-    const uint4 h = hdr[P];
-    for (uint32_t q = 0; q < h.w; q++) {
-        const Entry<R>* base = planes + (size_t)kPlanes * b;
-        uint32_t v;
-        if (q >= (uint32_t)kPlanes) v = ovf[h.z + q - kPlanes].nb;
-        else if constexpr (sizeof(R) == 4) v = base[plane_off<R>(q, W, P - b)].nb;
-        else v = reinterpret_cast<const uint32_t*>(base)[plane_nb_off(q, W, P - b)];
-        if (v < lo || v >= hi) continue;
+// Cone build: the upwind tasks of every task as schedule positions, task P's
+// at up[uoff[P] ..] in face order (uoff the prefix sums of k_up_count). A wave
+// per 64 cells and kFluxDirs directions reads each face once for all of them.
+__global__ void k_up_count(const uint32_t* __restrict__ sorted, const uint8_t* __restrict__ nups, uint32_t n,
+                           uint64_t* __restrict__ cnt) {
+    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p <= n) cnt[p] = p < n ? nups[sorted[p]] : 0u;
+}
+
+__global__ void __launch_bounds__(1024) k_up_fill(Geo g, const uint32_t* __restrict__ xpos,
+                                                  const uint64_t* __restrict__ uoff, uint32_t* __restrict__ up) {
+    const uint32_t N = (uint32_t)g.N, lane = threadIdx.x % kFluxCells;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / kFluxCells);
+    const uint32_t c = blockIdx.x * kFluxCells + lane;
+    if (c >= N) return;
+    uint64_t at[kFluxDirs];
+#pragma unroll
+    for (int j = 0; j < kFluxDirs; j++)
+        at[j] = uoff[xpos[(size_t)min(w * kFluxDirs + j, (uint32_t)g.D - 1u) * N + c]];
+    for (uint32_t f = g.off[c]; f < g.off[c + 1]; f++) {
+        const double4 a = g.geo[f];
+        const uint32_t nk = g.nk[f];
+        if ((nk >> 30) != kKindLocal) continue;
+#pragma unroll
+        for (int j = 0; j < kFluxDirs; j++) {
+            const uint32_t d = w * kFluxDirs + j;
+            if (d < (uint32_t)g.D && fdot(a, g.dirs[3 * d], g.dirs[3 * d + 1], g.dirs[3 * d + 2]) < 0.0)
+                up[at[j]++] = xpos[(size_t)d * N + (nk & kNbrMask)];
+        }
+    }
+}
+
+// Calls use(x) for the upwind positions x of the task at position P, eight
+// loads in flight.
+template <typename F>
+__device__ __forceinline__ void each_upwind(const uint64_t* __restrict__ uoff, const uint32_t* __restrict__ up,
+                                            uint32_t P, F use) {
+    const uint64_t e0 = uoff[P], e1 = uoff[P + 1];
+    for (uint64_t e = e0; e < e1; e += 8u) {
+        uint32_t v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = up[min(e + j, e1 - 1u)];
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            if (e + j < e1) use(v[j]);
+    }
+}
+
+// Appends the upwind schedule positions in [lo, hi) of the task at position P
+// to cand.
+__device__ void push_upwind(const uint64_t* uoff, const uint32_t* up, uint32_t P, uint32_t lo, uint32_t hi,
+                            uint32_t* cand, uint32_t* ncand, uint32_t* over) {
+    each_upwind(uoff, up, P, [&](uint32_t v) {
+        if (v < lo || v >= hi) return;
         const uint32_t k = atomicAdd(ncand, 1u);
         if (k < (uint32_t)kConeCap) cand[k] = v;
         else *over = 1u;
-    }
+    });
 }
 
 // Workgroup descriptor of the grouped replay, two uint4: {list offset, level
@@ -1637,27 +1698,27 @@ __device__ __forceinline__ uint32_t desc_count(const uint4& d0, const uint4& d1,
     return (ph & 1) ? (w >> 16) : (w & 0xFFFFu);
 }
 
-// One workgroup per block of at most T roots of one level set j of a group
+// One workgroup per block of at most 128 roots of one level set j of a group
 // starting at level set k0, meta[block] = {k0, j, first root, roots}: its cone
 // per level set (sorted, unique), written with the roots to the task list,
 // level set k0 first, and its descriptor. Members and roots are marked done
 // in todo. Roots are roots[first + r] or, without a root list, positions
 // first + r. Pending upwind entries are kept per level set: those of level
 // set i are taken out when i is processed.
-template <typename R, int T>
-__global__ void __launch_bounds__(T) k_cone(const uint4* hdr, const Entry<R>* planes, const Entry<R>* ovf,
+__global__ void __launch_bounds__(kConeThreads) k_cone(const uint64_t* uoff, const uint32_t* up,
                                             const uint32_t* fstart, const uint4* meta, const uint32_t* roots,
                                             uint8_t* todo, uint32_t* list, uint32_t list_cap, uint32_t* cursor,
                                             uint4* desc, uint32_t* fail) {
     __shared__ uint32_t candA[kConeCap], candB[kConeCap], tmp[kSortCap], memb[kConeCap];
     __shared__ uint32_t ncand, nkeep, ntmp, nmemb, over, base;
-    __shared__ uint32_t cnt[kMaxGroup], psum[T];
+    __shared__ uint32_t cnt[kMaxGroup], psum[kConeThreads / 64];
     uint32_t* cand = candA;
     uint32_t* keep = candB;
     const uint32_t tid = threadIdx.x;
     const uint4 mb = meta[blockIdx.x];
     const int k0 = (int)mb.x, j = (int)mb.y;
-    const uint32_t n = min((uint32_t)T, mb.w);
+    const uint32_t n = mb.w;  // at most kConeThreads
+    constexpr uint32_t T = kConeThreads;
     if (tid == 0) {
         ncand = 0;
         nmemb = 0;
@@ -1669,12 +1730,11 @@ __global__ void __launch_bounds__(T) k_cone(const uint4* hdr, const Entry<R>* pl
     uint32_t root = 0;
     if (tid < n) {
         root = roots ? roots[mb.z + tid] : mb.z + tid;
-        push_upwind<R>(hdr, planes, ovf, root, fstart[j], fstart[j + 1] - fstart[j], lo, fstart[j], cand, &ncand,
-                       &over);
+        push_upwind(uoff, up, root, lo, fstart[j], cand, &ncand, &over);
     }
     __syncthreads();
     for (int i = j - 1; i >= k0; i--) {
-        const uint32_t bi = fstart[i], ei = fstart[i + 1];
+        const uint32_t bi = fstart[i];
         if (tid == 0) {
             ntmp = 0;
             nkeep = 0;
@@ -1684,7 +1744,7 @@ __global__ void __launch_bounds__(T) k_cone(const uint4* hdr, const Entry<R>* pl
         const uint32_t nc = min(ncand, (uint32_t)kConeCap);
         for (uint32_t c = tid; c < nc; c += T) {
             const uint32_t v = cand[c];
-            if (v >= bi) tmp[atomicAdd(&ntmp, 1u)] = v;  // v < ei: entries are below the level sets done
+            if (v >= bi) tmp[atomicAdd(&ntmp, 1u)] = v;  // entries are below the level sets done
             else keep[atomicAdd(&nkeep, 1u)] = v;
         }
         __syncthreads();
@@ -1705,22 +1765,22 @@ __global__ void __launch_bounds__(T) k_cone(const uint4* hdr, const Entry<R>* pl
         const uint32_t c0 = min(nt, tid * per), c1 = min(nt, c0 + per);
         uint32_t u = 0;
         for (uint32_t c = c0; c < c1; c++) u += (c == 0 || tmp[c] != tmp[c - 1]) ? 1u : 0u;
-        psum[tid] = u;
+        const uint32_t incl = wave_scan(u);
+        if (tid % 64u == 63u) psum[tid / 64u] = incl;
         __syncthreads();
+        uint32_t before = incl - u, all = 0;
+        for (uint32_t l = 0; l < T / 64u; l++) {
+            if (l < tid / 64u) before += psum[l];
+            all += psum[l];
+        }
         if (tid == 0) {
-            uint32_t s = 0;
-            for (int l = 0; l < T; l++) {
-                const uint32_t x = psum[l];
-                psum[l] = s;
-                s += x;
-            }
-            cnt[i - k0] = s;
-            if (nmemb + s > (uint32_t)kConeCap) over = 1u;
+            cnt[i - k0] = all;
+            if (nmemb + all > (uint32_t)kConeCap) over = 1u;
         }
         __syncthreads();
         if (over) break;
         const uint32_t m0 = nmemb;
-        uint32_t w = m0 + psum[tid];
+        uint32_t w = m0 + before;
         for (uint32_t c = c0; c < c1; c++)
             if (c == 0 || tmp[c] != tmp[c - 1]) memb[w++] = tmp[c];
         __syncthreads();
@@ -1729,7 +1789,7 @@ __global__ void __launch_bounds__(T) k_cone(const uint4* hdr, const Entry<R>* pl
         const uint32_t m1 = nmemb;
         if (i > k0)
             for (uint32_t c = m0 + tid; c < m1; c += T)
-                push_upwind<R>(hdr, planes, ovf, memb[c], bi, ei - bi, lo, bi, cand, &ncand, &over);
+                push_upwind(uoff, up, memb[c], lo, bi, cand, &ncand, &over);
         __syncthreads();
     }
     if (over) {
@@ -1815,93 +1875,203 @@ __global__ void k_permute_desc(const uint4* in, const uint32_t* perm, uint4* out
     out[2 * i + 1] = in[2 * perm[i] + 1];
 }
 
-// Grouped replay of the level sets k0 .. k0+phases-1 with E lanes per
-// workgroup: workgroup w solves the tasks of its descriptor, level set by
-// level set, barrier in between. Each lane's first task of every level set is
-// read from the list up front, and the next level set's schedule data is
-// loaded while the current level set's gathers are in flight; loads are
-// unconditional (lanes without a task read the level set's first position)
-// so that the waits stay exact. Tasks beyond the first E of a level set are
-// solved without this overlap.
-// PH > 0: the group has exactly PH level sets (known at compile time, so no
-// list entry is read and no schedule data is prefetched for a level set past
-// the group's last); PH = 0: phases level sets, at most kMaxGroup.
-template <typename R, int E, int PH>
-__device__ __forceinline__ void group_body(const Geo& g, const Flux<R>& fl, const uint4* __restrict__ hdr,
-                                           const R* __restrict__ Av, const Entry<R>* __restrict__ planes,
-                                           const Entry<R>* __restrict__ ovf, const uint32_t* __restrict__ fstart,
-                                           int k0, int phases, const uint4* __restrict__ desc,
-                                           const uint32_t* __restrict__ list, uint32_t list_len, const PassTab& pt,
-                                           uint32_t blk) {
-    constexpr int MaxPh = PH > 0 ? PH : kMaxGroup;
-    if constexpr (PH > 0) phases = PH;
-    const uint32_t w = pass_item(pt, blk);
-    const uint4 d0 = desc[2 * w], d1 = desc[2 * w + 1];
-    const uint32_t tid = threadIdx.x;
-    uint32_t n[MaxPh], off[MaxPh], bb[MaxPh], WW[MaxPh], P[MaxPh];
+// Grouped replay of a group of level sets: one workgroup per cone, compiled
+// into tiles like a direction's (k_sweep_dir): up to 64 tasks of one level
+// set, planes whose entries name LDS words, a far list. Here the LDS holds one
+// word per task of the cone, so that X passes between the group's level sets
+// through LDS, and everything older than the group is in memory when the
+// launch starts: it is on the far list, whose loads go out with the tile's
+// cell inputs. A wave takes a tile (tile i the wave i mod waves, which fixes
+// the words of its buffer), loads all it needs, and waits for its level set
+// only then: every wave passes level sets - 1 barriers, whatever tiles it has.
+// Bound by the chain of a launch: descriptor, planes and far list, far values,
+// then per level set a barrier, the LDS reads, the sum and a division. With
+// planes in schedule order and upwind values gathered from memory, every level
+// set ended with a store, a wait for it and a gather: a launch of 8 level sets
+// took 14.6 us in the captured sweep of 32768 cells x 16 directions FP64 (6.1 us
+// like this), one of 4 level sets 9.4 us on 117649 cells x 64 directions FP32
+// (5.1 us).
+//   tile  {blob offset (48 bits), LDS word of its first task (16 bits), tasks |
+//         planes << 7 | extra << 11 | far << 19, level set in the cone | level
+//         sets << 8 | tiles of the cone << 16}
+//   blob  planes, {X index, I index} of the tasks, far list, extra weights,
+//         extra words
+// The first `waves` tiles of cone b are at tiles[b * waves] (those it does not
+// have without tasks), the others from tiles[more[b]] on: no load has to
+// return before a wave's first descriptor is on its way.
+// A restricted sweep runs the cones with active tasks; a task whose cell is
+// below level lvl is not solved and puts its stored X into its word.
+template <typename R>
+struct ConeShape {
+    static constexpr uint32_t kAt = 64;                                         // words 0-63: 0
+    static constexpr uint32_t kFar = 512;                                       // far entries of a tile
+    static constexpr uint32_t kBuf = kFar + 128 + 512 / (uint32_t)sizeof(R);    // far, extra weights, extra words
+    static constexpr int waves(int roots) { return roots == 32 ? 4 : roots == 64 ? 8 : 16; }
+    static size_t bytes(int roots, uint32_t cone) { return sizeof(R) * (kAt + cone + (size_t)waves(roots) * kBuf); }
+};
+
+template <typename R, int kWaves, bool kGeneral>
+__device__ __forceinline__ void cone_body(const Geo& g, const Flux<R>& fl, const uint4* __restrict__ blob,
+                                          const uint4* __restrict__ tiles, const uint32_t* __restrict__ more,
+                                          uint32_t cone, uint32_t words, int lvl) {
+    using S = DirShape<R>;
+    using K = ConeShape<R>;
+    extern __shared__ double cone_lds[];
+    R* const lds = reinterpret_cast<R*>(cone_lds);
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    R* const buf = lds + K::kAt + words + w * K::kBuf;
+    uint32_t* const bufs = reinterpret_cast<uint32_t*>(buf + K::kFar + 128);
+    uint4 t = tiles[(size_t)cone * kWaves + w];
+    lds[lane] = (R)0;  // by every wave, before its own reads
+    auto uni = [](uint32_t v) -> uint32_t { return __builtin_amdgcn_readfirstlane(v); };
+    auto rsrc = [&](const uint4* p, uint32_t bytes) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4*>(p), 0, (int)bytes, 0x00027000);
+    };
+    uint32_t at_level = 0;
+    auto pass_to = [&](uint32_t k) {  // every wave passes level sets - 1 barriers
+        while (at_level < k) {
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            at_level++;
+        }
+    };
+    const uint32_t levels = (uni(t.w) >> 8) & 255u, n = uni(t.w) >> 16;
+    for (uint32_t i = w; i < n; i += kWaves) {
+        if (i >= kWaves) t = tiles[(size_t)more[cone] + i - kWaves];
+        const uint64_t off = (uint64_t)uni(t.x) | ((uint64_t)(uni(t.y) & 0xFFFFu) << 32);
+        const uint32_t word0 = uni(t.y) >> 16, k = uni(t.w) & 255u, pk = uni(t.z);
+        const uint32_t cnt = pk & 127u, np = (pk >> 7) & 15u, nex = (pk >> 11) & 255u, nfar = pk >> 19;
+        const uint32_t li = min(lane, cnt - 1u), st = cnt * 16u;
+        const uint4* p = blob + off;
+        const auto rp = rsrc(p, np * st);
+        const u32x4 s0 = __builtin_amdgcn_raw_buffer_load_b128(rp, li * 16u, 0, 0);
+        p += np * cnt;
+        const uint2 at = reinterpret_cast<const uint2*>(p)[li];
+        const uint32_t xi = at.x, oi = at.y;
+        p += units16(cnt, 8);
+        uint32_t far[K::kFar / 64];
+        const auto rf = rsrc(p, nfar * 4u);
 #pragma unroll
-    for (int ph = 0; ph < MaxPh; ph++) {
-        n[ph] = desc_count(d0, d1, ph);
-        off[ph] = ph == 0 ? d0.x : off[ph - 1] + n[ph - 1];
-        const int k = k0 + min(ph, phases - 1);
-        bb[ph] = fstart[k];
-        WW[ph] = fstart[k + 1] - bb[ph];
-        const uint32_t v = list[min(off[ph] + tid, list_len - 1u)];
-        P[ph] = (ph < phases && tid < n[ph]) ? v : bb[ph];
-    }
-    TaskS<R> cur;
-    load_task<R>(cur, hdr + bb[0], Av + bb[0], planes + (size_t)kPlanes * bb[0], WW[0], P[0] - bb[0]);
+        for (int j = 0; j < (int)(K::kFar / 64); j++) {
+            far[j] = 0;
+            if (nfar > 64u * j) far[j] = __builtin_amdgcn_raw_buffer_load_b32(rf, (lane + 64u * j) * 4u, 0, 0);
+        }
+        const u32x4 s1 = __builtin_amdgcn_raw_buffer_load_b128(rp, li * 16u + S::kS1 * st, 0, 0);
+        uint32_t wt[4 * S::kWPlanes];
 #pragma unroll
-    for (int ph = 0; ph < MaxPh; ph++) {
-        if (ph < phases) {
-            TaskG<R> G;
-            issue_task<R>(G, g, fl, cur, ovf, P[ph]);
-            TaskS<R> nxt;
-            const int q = ph + 1 < MaxPh ? ph + 1 : ph;
-            if (PH == 0 || ph + 1 < MaxPh)
-                load_task<R>(nxt, hdr + bb[q], Av + bb[q], planes + (size_t)kPlanes * bb[q], WW[q], P[q] - bb[q]);
-            if (tid < n[ph]) finish_task_c<R>(g, fl, cur, G, ovf, P[ph]);
-            for (uint32_t i = tid + E; i < n[ph]; i += E)
-                comp_task<R>(g, fl, hdr + bb[ph], Av + bb[ph], planes + (size_t)kPlanes * bb[ph], ovf, bb[ph],
-                             WW[ph], list[off[ph] + i] - bb[ph]);
-            __syncthreads();
-            if (PH == 0 || ph + 1 < MaxPh) cur = nxt;
+        for (int j = 0; j < S::kWPlanes; j++) {
+            const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rp, li * 16u + S::wplane(j) * st, 0, 0);
+#pragma unroll
+            for (int m = 0; m < 4; m++) wt[4 * j + m] = v[m];
+        }
+        p += units16(nfar, 4);
+        const uint32_t hdr = s0.x, c = hdr & kCellMask, nup = hdr >> kCellBits;
+        const SA<R> sa = fl.sa[c];
+        R off_i = 0, xold = 0;
+        uint32_t lev = 0;
+        if (kGeneral) {
+            if (fl.offI) off_i = fl.offI[oi];
+            if (lvl > 0) {
+                lev = g.level[c];
+                xold = fl.X[xi];
+            }
+        }
+        R fv[K::kFar / 64];
+#pragma unroll
+        for (int j = 0; j < (int)(K::kFar / 64); j++) {
+            fv[j] = (R)0;
+            if (nfar > 64u * j) {
+                const R* src = (far[j] & kFarPeriodic) ? fl.P : fl.X;
+                fv[j] = src[far[j] & ~kFarPeriodic];
+            }
+        }
+        for (uint32_t e = lane; e < nex; e += 64u) {
+            buf[K::kFar + e] = reinterpret_cast<const R*>(p)[e];
+            bufs[e] = reinterpret_cast<const uint32_t*>(p + units16(nex, sizeof(R)))[e];
+        }
+#pragma unroll
+        for (int j = 0; j < (int)(K::kFar / 64); j++)
+            if (nfar > 64u * j) buf[64u * j + lane] = fv[j];
+        const bool more = nup > kDirEntries;
+        auto half = [&](int h) -> uint32_t {
+            const uint32_t v = h < 8 ? s0[(h % 8) / 2] : s1[(h % 8) / 2];
+            return (h & 1) ? v >> 16 : v & 0xFFFFu;
+        };
+        auto weight = [&](int m) -> R {
+            if constexpr (sizeof(R) == 4) return __uint_as_float(wt[m]);
+            else return __hiloint2double((int)wt[2 * m + 1], (int)wt[2 * m]);
+        };
+        pass_to(k);
+        R x[kDirEntries + 1];
+#pragma unroll
+        for (int e = 0; e <= (int)kDirEntries; e++) x[e] = lds[(e == (int)kDirEntries && more) ? 0u : half(e + 2)];
+        R inc = 0;
+#pragma unroll
+        for (int e = 0; e < (int)kDirEntries; e++) inc += weight(1 + e) * x[1 + e];
+        if (nex && more) {
+            const uint32_t first = half((int)kDirEntries + 2) - (kDirEntries - 1u);
+            for (uint32_t e0 = kDirEntries - 1u; e0 < nup; e0 += 4u) {
+                R v[4], y[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const uint32_t e = first + min(e0 + j, nup - 1u);
+                    v[j] = buf[K::kFar + e];
+                    y[j] = lds[bufs[e]];
+                }
+#pragma unroll
+                for (int j = 0; j < 4; j++) inc += e0 + j < nup ? v[j] * y[j] : (R)0;
+            }
+        }
+        const CellIn<R> ci{sa.x, sa.y, x[0], off_i};
+        const R A = weight(0);
+        bool act = lane < cnt && (!kGeneral || lev >= (uint32_t)lvl);
+        R xv = xold;
+        if (act) {
+            const R out = outgoing_rate<R, kGeneral>(fl, oi, inc, ci);
+            xv = (A > (R)0) ? out / A : (R)0;
+        }
+        if (lane < cnt) lds[word0 + lane] = xv;
+        // a wave's last tile: its level set's end before its stores
+        if (i + kWaves >= n) pass_to(min(k + 1u, levels - 1u));
+        if (act) {
+            fl.X[xi] = xv;
+            fl.I[oi] = inc;
         }
     }
+    pass_to(levels - 1u);
 }
 
-template <typename R, int E, int PH>
-__global__ void __launch_bounds__(E) k_sweep_group(Geo g, Flux<R> fl, const uint4* __restrict__ hdr,
-                                                   const R* __restrict__ Av, const Entry<R>* __restrict__ planes,
-                                                   const Entry<R>* __restrict__ ovf,
-                                                   const uint32_t* __restrict__ fstart, int k0, int phases,
-                                                   const uint4* __restrict__ desc, const uint32_t* __restrict__ list,
-                                                   uint32_t list_len, PassTab pt) {
-    group_body<R, E, PH>(g, fl, hdr, Av, planes, ovf, fstart, k0, phases, desc, list, list_len, pt, blockIdx.x);
+template <typename R, int kWaves, bool kGeneral>
+__global__ void __launch_bounds__(64 * kWaves) k_sweep_cone(Geo g, Flux<R> fl, const uint4* __restrict__ blob,
+                                                            const uint4* __restrict__ tiles,
+                                                            const uint32_t* __restrict__ more,
+                                                            const uint32_t* __restrict__ sel, uint32_t cone0,
+                                                            uint32_t words, int lvl,
+                                                            PassTab pt) {
+    const uint32_t b = pass_item(pt, blockIdx.x);
+    cone_body<R, kWaves, kGeneral>(g, fl, blob, tiles, more, cone0 + (sel ? sel[b] : b), words, lvl);
 }
 
 // One problem's grouped launch inside a packed launch: everything the grouped
 // kernel reads of its handle, and its workgroups [start, start + blocks) of
 // the packed grid (start a multiple of kXcds, so that the die-aware order of
-// its descriptors holds as in a launch of its own).
+// its cones holds as in a launch of its own).
 template <typename R>
 struct GroupJob {
-    int64_t N, Nper;
+    int64_t N;
     R* X;
     R* I;
     R* P;
     R* offI;
     const SA<R>* sa;
     R thr;
-    const uint4* hdr;
-    const R* A;
-    const Entry<R>* planes;
-    const Entry<R>* ovf;
-    const uint32_t* fstart;
-    const uint4* desc;
-    const uint32_t* list;
-    uint32_t list_len;
-    int k0, phases;
+    const uint8_t* level;
+    const uint4* blob;
+    const uint4* tiles;
+    const uint32_t* more;
+    const uint32_t* sel;
+    uint32_t cone0, words;
+    int lvl;
     uint32_t start, blocks;
     PassTab pt;
 };
@@ -1915,106 +2085,186 @@ struct PackArgs {
 };
 
 // Grouped launches of up to kMaxPack problems in one launch: workgroup b runs
-// the job whose range holds it, as k_sweep_group would run it alone.
-template <typename R, int E, int PH>
-__global__ void __launch_bounds__(E) k_sweep_group_pack(const PackArgs<R> a) {
+// the job whose range holds it, as k_sweep_cone would run it alone.
+template <typename R, int kWaves, bool kGeneral>
+__global__ void __launch_bounds__(64 * kWaves) k_sweep_cone_pack(const PackArgs<R> a) {
     int j = 0;
     for (int k = 1; k < a.n; k++)
         if (blockIdx.x >= a.job[k].start) j = k;
     const GroupJob<R>& J = a.job[j];
-    const uint32_t b = blockIdx.x - J.start;
-    if (b >= J.blocks) return;  // padding up to the next job's die-aligned start
+    const uint32_t i = blockIdx.x - J.start;
+    if (i >= J.blocks) return;  // padding up to the next job's die-aligned start
     Geo g{};
     g.N = J.N;
-    g.Nper = J.Nper;
+    g.level = J.level;
     Flux<R> fl{};
     fl.X = J.X;
     fl.I = J.I;
-    fl.ipos = nullptr;
     fl.P = J.P;
     fl.offI = J.offI;
     fl.sa = J.sa;
     fl.thr = J.thr;
-    group_body<R, E, PH>(g, fl, J.hdr, J.A, J.planes, J.ovf, J.fstart, J.k0, J.phases, J.desc, J.list, J.list_len,
-                         J.pt, b);
+    const uint32_t b = pass_item(J.pt, i);
+    cone_body<R, kWaves, kGeneral>(g, fl, J.blob, J.tiles, J.more, J.cone0 + (J.sel ? J.sel[b] : b), J.words, J.lvl);
 }
 
-// The grouped replay of a restricted sweep (active set {level >= lvl}):
-// workgroup w filters descriptor w's task list to the active tasks, in order,
-// into the same place of list_out, and, if any is left, writes its filtered
-// descriptor to desc_tmp[w] and kept[w] = 1 (k_place_desc then packs the kept
-// descriptors of each group in order), so that a launch starts only
-// workgroups with active tasks; the active tasks and the kept descriptors of
-// each group are summed into gcount and gblocks (gmap: group of each
-// descriptor). The cones of the full graph contain the active cones, so every
-// dependency of an active task inside a launch stays inside its workgroup;
-// the workgroups of a launch are independent, so their order is free.
-__global__ void __launch_bounds__(kBlock) k_group_compact(Geo g, const uint4* __restrict__ hdr, int lvl,
-                                                          const uint4* __restrict__ desc_in,
-                                                          const uint32_t* __restrict__ list_in,
-                                                          const uint32_t* __restrict__ gmap, uint32_t ndesc,
-                                                          uint4* desc_tmp, uint32_t* kept, uint32_t* list_out,
-                                                          uint32_t* gcount, uint32_t* gblocks) {
-    const uint32_t w = blockIdx.x;
-    if (w >= ndesc) return;
-    __shared__ uint32_t wave_tot[kBlock / 64];
-    const uint4 d0 = desc_in[2 * w], d1 = desc_in[2 * w + 1];
-    uint32_t m[kMaxGroup];
-    const int lane = __lane_id(), wv = threadIdx.x / 64;
-    uint32_t src = d0.x, dst = d0.x;
-    for (int ph = 0; ph < kMaxGroup; ph++) {
-        const uint32_t n = desc_count(d0, d1, ph);
-        const uint32_t base = dst;
-        for (uint32_t p0 = 0; p0 < n; p0 += kBlock) {
-            const uint32_t i = p0 + threadIdx.x;
-            uint32_t P = 0;
-            bool act = false;
-            if (i < n) {
-                P = list_in[src + i];
-                act = g.level[hdr[P].x & kCellMask] >= lvl;
+// Tiles of every cone: counted (kFill = false, one wave each: the tiles past
+// the first `waves` and blob units of each cone, the far entries of each task
+// of the list, and the largest cone of each group into words) or written (four
+// waves each, a tile the wave). gk0[gmap[cone]]: first level set of the cone's
+// group.
+template <typename R, bool kFill>
+__global__ void __launch_bounds__(kFill ? 256 : 64) k_cone_tiles(
+    Geo g, double inv_aref, const uint32_t* __restrict__ sorted, const uint32_t* __restrict__ xpos,
+    const uint64_t* __restrict__ uoff, const uint32_t* __restrict__ up, const uint32_t* __restrict__ fstart,
+    const uint8_t* __restrict__ nups, uint8_t* __restrict__ fars, const uint4* __restrict__ desc,
+    const uint32_t* __restrict__ list, const uint32_t* __restrict__ gmap, const uint32_t* __restrict__ gk0,
+    uint32_t* __restrict__ ct, uint64_t* __restrict__ cu, uint32_t* __restrict__ words,
+    const uint32_t* __restrict__ ts, const uint64_t* __restrict__ us, uint32_t waves, uint4* __restrict__ blob,
+    uint4* __restrict__ tiles, uint32_t* __restrict__ more) {
+    using K = ConeShape<R>;
+    extern __shared__ uint32_t memb[];  // kFill: the cone's tasks
+    __shared__ uint32_t fs[kMaxGroup + 1], zs[kMaxGroup + 1];
+    const uint32_t w = blockIdx.x, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint4 d0 = desc[2 * (size_t)w], d1 = desc[2 * (size_t)w + 1];
+    const uint32_t k0 = gk0[gmap[w]], levels = d0.y, N = (uint32_t)g.N;
+    uint32_t total = 0;
+    for (uint32_t ph = 0; ph < levels; ph++) total += desc_count(d0, d1, (int)ph);
+    if (kFill) {
+        if (threadIdx.x == 0)
+            for (uint32_t ph = 0, z = 0; ph <= levels; ph++) {
+                fs[ph] = fstart[k0 + ph];
+                zs[ph] = z;
+                z += ph < levels ? desc_count(d0, d1, (int)ph) : 0u;
             }
-            const unsigned long long bal = __ballot(act);
-            if (lane == 0) wave_tot[wv] = (uint32_t)__popcll(bal);
-            __syncthreads();
-            uint32_t before = 0, all = 0;
-            for (int k = 0; k < kBlock / 64; k++) {
-                if (k < wv) before += wave_tot[k];
-                all += wave_tot[k];
+        for (uint32_t i = threadIdx.x; i < total; i += blockDim.x) memb[i] = list[d0.x + i];
+        __syncthreads();
+    }
+    const uint32_t lo = fstart[k0], cone = d0.x;
+    uint32_t seg = 0, nt = 0, all = 0;
+    uint64_t off = kFill ? us[w] : 0;
+    const uint32_t more0 = kFill ? gridDim.x * waves + ts[w] : 0u;
+    if (kFill) all = waves + ts[w + 1] - ts[w];  // the tiles, if more than `waves`
+    for (uint32_t ph = 0; ph < levels; ph++) {
+        const uint32_t m = desc_count(d0, d1, (int)ph);
+        for (uint32_t b = 0; b < m; b += 64u) {
+            const uint32_t n = min(64u, m - b), at = cone + seg + b + min(lane, n - 1u), P = list[at];
+            const uint32_t t = sorted[P], nup = nups[t];
+            uint32_t far = 0;
+            if (lane < n) {
+                if (kFill) {
+                    far = fars[at];
+                } else {
+                    far = (g.Nper && g.pslot[t % N] != kNone) ? 1u : 0u;
+                    each_upwind(uoff, up, P, [&](uint32_t x) { far += x < lo ? 1u : 0u; });
+                    fars[at] = (uint8_t)far;
+                }
             }
-            if (act) list_out[dst + before + (uint32_t)__popcll(bal & ((1ull << lane) - 1ull))] = P;
-            dst += all;
-            __syncthreads();
+            const uint32_t ex = lane < n ? dir_extra(nup) : 0u, pf = wave_scan(far), pe = wave_scan(ex);
+            for (uint32_t a = 0; a < n;) {
+                const uint32_t bf = a ? (uint32_t)__shfl((int)pf, a - 1) : 0u;
+                const uint32_t be = a ? (uint32_t)__shfl((int)pe, a - 1) : 0u;
+                const unsigned long long over =
+                    __ballot(lane > a && lane < n && (pf - bf > K::kFar || pe - be > kDirCap));
+                const uint32_t e = over ? (uint32_t)__ffsll((long long)over) - 1u : n, cnt = e - a;
+                const uint32_t nf = (uint32_t)__shfl((int)pf, e - 1) - bf, ne = (uint32_t)__shfl((int)pe, e - 1) - be;
+                const uint32_t np = DirShape<R>::planes(wave_max(lane >= a && lane < e ? nup : 0u));
+                if (kFill && nt % (blockDim.x / 64u) == wave) {
+                    uint4* const base = blob + off;
+                    uint2* const at2 = reinterpret_cast<uint2*>(base + np * cnt);
+                    uint4* const lists = base + np * cnt + units16(cnt, 8);
+                    uint4* const extra = lists + units16(nf, 4);
+                    if (lane == 0)
+                        tiles[nt < waves ? w * (size_t)waves + nt : (size_t)more0 + nt - waves] = make_uint4(
+                            (uint32_t)off, (uint32_t)(off >> 32) | ((K::kAt + seg + b + a) << 16),
+                            cnt | (np << 7) | (ne << 11) | (nf << 19), ph | (levels << 8) | (all << 16));
+                    if (lane >= a && lane < e) {
+                        at2[lane - a] = make_uint2(P, t);
+                        fill_task<R>(g, inv_aref, t % N, t / N, nup, xpos, base, np, cnt, lane - a,
+                                     reinterpret_cast<uint32_t*>(lists), pf - far - bf,
+                                     K::kAt + words[gmap[w]] + (nt % waves) * K::kBuf, reinterpret_cast<R*>(extra),
+                                     reinterpret_cast<uint32_t*>(extra + units16(ne, sizeof(R))), pe - ex - be,
+                                     [&](uint32_t x) {
+                                         if (x < lo) return kNone;
+                                         uint32_t q = 0;  // its level set, then its place there
+                                         while (fs[q + 1] <= x) q++;
+                                         uint32_t z0 = zs[q], z1 = zs[q + 1];
+                                         while (z1 - z0 > 1) {
+                                             const uint32_t z = (z0 + z1) / 2;
+                                             if (memb[z] <= x) z0 = z;
+                                             else z1 = z;
+                                         }
+                                         return K::kAt + z0;
+                                     });
+                    }
+                }
+                off += np * cnt + units16(cnt, 8) + units16(nf, 4) + units16(ne, sizeof(R)) + units16(ne, 4);
+                nt++;
+                a = e;
+            }
         }
-        m[ph] = dst - base;
-        src += n;
+        seg += m;
+    }
+    if (!kFill) {
+        if (lane == 0) {
+            ct[w] = nt > waves ? nt - waves : 0u;
+            cu[w] = off;
+            atomicMax(&words[gmap[w]], total);
+        }
+        return;
+    }
+    // the number of tiles, now known, in the descriptors of a cone that has no
+    // more than `waves`; the places it does not use
+    if (all > waves) {
+        if (threadIdx.x == 0) more[w] = more0;
+        return;
+    }
+    __syncthreads();
+    if (threadIdx.x < waves) {
+        uint4* const t = tiles + w * (size_t)waves + threadIdx.x;
+        if (threadIdx.x < nt) t->w = (t->w & 0xFFFFu) | (nt << 16);
+        else *t = make_uint4(0u, 0u, 0u, (levels << 8) | (nt << 16));
+    }
+}
+
+// The grouped replay of a restricted sweep (active set {level >= lvl}): a wave
+// per cone counts its active tasks; cones that have some are kept (k_place_cone
+// then packs each group's in order), and the active tasks and kept cones of
+// each group are summed into gcount and gblocks (gmap: group of each cone).
+__global__ void __launch_bounds__(64) k_cone_active(Geo g, int lvl, const uint4* __restrict__ blob,
+                                                    const uint4* __restrict__ tiles,
+                                                    const uint32_t* __restrict__ more, uint32_t waves,
+                                                    const uint32_t* __restrict__ gmap, uint32_t* kept,
+                                                    uint32_t* gcount, uint32_t* gblocks) {
+    const uint32_t tn = tiles[blockIdx.x * (size_t)waves].w >> 16;
+    uint32_t n = 0;
+    for (uint32_t i = 0; i < tn; i++) {
+        const uint4 t = tiles[i < waves ? blockIdx.x * (size_t)waves + i : (size_t)more[blockIdx.x] + i - waves];
+        const uint32_t cnt = t.z & 127u;
+        const uint32_t hdr = blob[((uint64_t)t.x | ((uint64_t)(t.y & 0xFFFFu) << 32)) + min(threadIdx.x, cnt - 1u)].x;
+        n += (uint32_t)__popcll(__ballot(threadIdx.x < cnt && g.level[hdr & kCellMask] >= lvl));
     }
     if (threadIdx.x == 0) {
-        uint32_t total = 0;
-        for (int k = 0; k < kMaxGroup; k++) total += m[k];
-        kept[w] = total ? 1u : 0u;
-        if (total) {
-            const uint32_t gr = gmap[w];
-            atomicAdd(&gcount[gr], total);
-            atomicAdd(&gblocks[gr], 1u);
-            desc_tmp[2 * w] = make_uint4(d0.x, d0.y, m[0] | (m[1] << 16), m[2] | (m[3] << 16));
-            desc_tmp[2 * w + 1] = make_uint4(m[4] | (m[5] << 16), m[6] | (m[7] << 16), 0u, 0u);
+        kept[blockIdx.x] = n ? 1u : 0u;
+        if (n) {
+            atomicAdd(&gcount[gmap[blockIdx.x]], n);
+            atomicAdd(&gblocks[gmap[blockIdx.x]], 1u);
         }
     }
 }
 
-// Packs the kept filtered descriptors: descriptor w of group g (whose
-// descriptors start at gbase[g]) goes to gbase[g] + (pos[w] - pos[gbase[g]]),
-// pos the exclusive prefix sum of kept, so each group's kept descriptors keep
-// their order (and with it the pass ranges of the die-aware launch order).
-__global__ void k_place_desc(const uint4* __restrict__ desc_tmp, const uint32_t* __restrict__ kept,
-                             const uint32_t* __restrict__ pos, const uint32_t* __restrict__ gmap,
-                             const uint32_t* __restrict__ gbase, uint4* desc_out, uint32_t ndesc) {
+// Packs the kept cones: cone w of group g (whose cones start at gbase[g]) goes
+// to place pos[w] - pos[gbase[g]] of the group (pos the exclusive prefix sum
+// of kept), so each group's kept cones keep their order (and with it the pass
+// ranges of the die-aware launch order). sel holds cones counted from the
+// group's first.
+__global__ void k_place_cone(const uint32_t* __restrict__ kept, const uint32_t* __restrict__ pos,
+                             const uint32_t* __restrict__ gmap, const uint32_t* __restrict__ gbase, uint32_t* sel,
+                             uint32_t n) {
     const uint32_t w = blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= ndesc || !kept[w]) return;
+    if (w >= n || !kept[w]) return;
     const uint32_t b = gbase[gmap[w]];
-    const uint32_t o = b + (pos[w] - pos[b]);
-    desc_out[2 * o] = desc_tmp[2 * w];
-    desc_out[2 * o + 1] = desc_tmp[2 * w + 1];
+    sel[b + (pos[w] - pos[b])] = w - b;
 }
 
 __global__ void k_gather_u32(const uint32_t* __restrict__ src, const uint32_t* __restrict__ idx, uint32_t* out,
@@ -2602,40 +2852,37 @@ struct ssw_sweep {
     int group_request = kGroupLevels;               // level sets per grouped launch (1: off)
     int group_block = kGroupT;                      // grouped replay: root tasks per workgroup
     // grouped replay of full sweeps (compiled): per group of level sets its
-    // first level set, level-set count and workgroup descriptors
+    // first level set, level-set count and cones
     struct Group {
         int k0, levels;
         uint32_t desc0, ndesc;
-        PassTab passes;  // descriptor ranges of the build passes, relative to desc0
+        PassTab passes;  // cone ranges of the build passes, relative to desc0
+        uint32_t words;  // tasks of its largest cone
     };
     std::vector<Group> groups;
-    uint4* d_gdesc = nullptr;
-    uint32_t* d_glist = nullptr;
-    uint32_t* d_gmap = nullptr;                     // group of each descriptor
+    uint4 *d_coneblob = nullptr, *d_conetiles = nullptr;
+    uint32_t* d_conemore = nullptr;
+    uint32_t* d_gmap = nullptr;                     // group of each cone
     uint32_t ndesc = 0;
-    // restricted sweeps (level >= 1): filtered descriptors and lists, active
-    // tasks per group
-    std::vector<uint4*> d_gdesc_l;
-    std::vector<uint32_t*> d_glist_l;
+    // restricted sweeps (level >= 1): kept cones, active tasks per group
+    std::vector<uint32_t*> d_gsel_l;
     uint32_t* d_gcount = nullptr;
-    uint32_t* d_gbase = nullptr;                    // first descriptor of each group
+    uint32_t* d_gbase = nullptr;                    // first cone of each group
     uint32_t* d_gblocks = nullptr;                  // restricted sweep: workgroups with active tasks per group
-    // global descriptor index of every pass boundary of every group (group
+    // global cone index of every pass boundary of every group (group
     // gi's npass + 1 boundaries from pbound_start[gi]); per restricted sweep
-    // level the pass ranges of each group's kept descriptors
+    // level the pass ranges of each group's kept cones
     uint32_t* d_pbound = nullptr;
     std::vector<uint32_t> pbound_start;
-    // restricted sweeps' filter scratch, held from the cone build on: filtered
-    // descriptors in place, kept flags, their prefix sum, the pass bounds'
-    // packed positions and the scan's temporary storage
-    uint4* d_gf_desc = nullptr;
+    // restricted sweeps' filter scratch, held from the cone build on: kept
+    // flags, their prefix sum, the pass bounds' packed positions and the scan's
+    // temporary storage
     uint32_t *d_gf_kept = nullptr, *d_gf_pos = nullptr, *d_gf_pbval = nullptr;
     uint8_t* d_gf_scan = nullptr;
     size_t gf_scan_bytes = 0;
     std::vector<std::vector<PassTab>> gpass_l;
     std::vector<std::vector<uint32_t>> gcount, gblocks;
     int64_t group_tasks = 0;                        // tasks solved per full sweep by the grouped replay
-    uint32_t glist_len = 0;                         // entries of the grouped replay's task list
     bool group_fallback = false;                    // groups requested but a cone did not fit
     bool compiled = false;
     // grid
@@ -3090,14 +3337,21 @@ int plan_replay(ssw_sweep* s, int lvl) {
     return SSW_OK;
 }
 
+// A kernel of the grouped replay by roots per workgroup and whether it is a
+// restricted sweep or has offsets.
+#define SSW_CONE_KERNEL(name, R, roots, general)                                       \
+    ((roots) == 32 ? ((general) ? name<R, 4, true> : name<R, 4, false>)                \
+     : (roots) == 64 ? ((general) ? name<R, 8, true> : name<R, 8, false>)              \
+                     : ((general) ? name<R, 16, true> : name<R, 16, false>))
+
 // The grouped replay of full sweeps (compiled replay, group_request >= 2):
 // groups of m consecutive level sets; in each group, from its last level set
 // down to its first, the level set's tasks in no cone yet become roots, in
-// blocks of kGroupT, whose cones are built (k_cone). If a cone exceeds the
-// LDS capacity or the task list its bound, full sweeps keep the per-level
-// replay (no groups).
+// blocks of kGroupT, whose cones are built (k_cone) and compiled into tiles
+// (k_cone_tiles). If a cone exceeds the LDS capacity or the task list its
+// bound, there are no groups, and sweeps keep the per-level replay.
 template <typename R>
-int build_groups_t(ssw_sweep* s) {
+int build_groups_t(ssw_sweep* s, const uint32_t* sorted) {
     const int m = s->group_request;
     const size_t DN = (size_t)s->D * s->N;
     const std::vector<uint32_t>& fs = s->full_start;
@@ -3119,7 +3373,7 @@ int build_groups_t(ssw_sweep* s) {
             if (narrow) mk = kMaxGroup;
         }
         const int lv = std::min(s->kmax, k0 + mk) - k0;
-        s->groups.push_back({k0, lv, 0u, 0u, PassTab{}});
+        s->groups.push_back({k0, lv, 0u, 0u, PassTab{}, 0u});
         mmax = std::max(mmax, lv);
         k0 += mk;
     }
@@ -3133,18 +3387,42 @@ int build_groups_t(ssw_sweep* s) {
     }
     uint8_t *todo = nullptr, *flags = nullptr, *lvlflag = nullptr, *tmp = nullptr;
     uint32_t *roots = nullptr, *ctl = nullptr, *bounds = nullptr, *perm = nullptr;  // ctl: cursor, fail, selected
+    uint32_t *list = nullptr, *k0s = nullptr, *words = nullptr, *ct = nullptr, *ts = nullptr;
+    uint64_t *cu = nullptr, *us = nullptr, *ucnt = nullptr, *uoff = nullptr;
+    uint32_t* up = nullptr;
+    uint8_t* fars = nullptr;
     int* lv = nullptr;
-    uint4 *meta = nullptr, *desc_rm = nullptr;
+    uint4 *meta = nullptr, *desc_rm = nullptr, *desc = nullptr;
     Defer cleanup{[&] {
         for (uint8_t** p : {&todo, &flags, &lvlflag, &tmp}) dfree(s, *p);
-        for (uint32_t** p : {&roots, &ctl, &bounds, &perm}) dfree(s, *p);
+        for (uint32_t** p : {&roots, &ctl, &bounds, &perm, &list, &k0s, &words, &ct, &ts}) dfree(s, *p);
+        for (uint64_t** p : {&cu, &us, &ucnt, &uoff}) dfree(s, *p);
+        dfree(s, up);
+        dfree(s, fars);
         dfree(s, lv);
-        dfree(s, meta);
-        dfree(s, desc_rm);
+        for (uint4** p : {&meta, &desc_rm, &desc}) dfree(s, *p);
     }};
+    const Geo g = make_geo(s);
+    // every task's upwind positions
+    TRY(dalloc(s, &ucnt, DN + 1));
+    TRY(dalloc(s, &uoff, DN + 1));
+    k_up_count<<<grid_for((int64_t)DN + 1), kBlock, 0, s->stream>>>(sorted, s->d_nup, (uint32_t)DN, ucnt);
+    size_t ub = 0;
+    HIP_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, ub, ucnt, uoff, (int)(DN + 1), s->stream));
+    TRY(dalloc(s, &tmp, ub));
+    HIP_TRY(hipcub::DeviceScan::ExclusiveSum(tmp, ub, ucnt, uoff, (int)(DN + 1), s->stream));
+    uint64_t nup_all = 0;
+    HIP_TRY(hipMemcpyAsync(&nup_all, uoff + DN, 8, hipMemcpyDeviceToHost, s->stream));
+    HIP_TRY(hipStreamSynchronize(s->stream));
+    dfree(s, tmp);
+    dfree(s, ucnt);
+    TRY(dalloc(s, &up, std::max<size_t>(1, (size_t)nup_all)));
+    k_up_fill<<<(unsigned)((s->N + kFluxCells - 1) / kFluxCells),
+                kFluxCells * ((s->D + kFluxDirs - 1) / kFluxDirs), 0, s->stream>>>(g, s->d_xpos, uoff, up);
+    HIP_TRY(hipGetLastError());
     TRY(dalloc(s, &todo, DN));
     TRY(dalloc(s, &ctl, 3));
-    TRY(dalloc(s, &s->d_glist, list_cap));
+    TRY(dalloc(s, &list, list_cap));
     TRY(dalloc(s, &desc_rm, 2 * desc_cap));
     HIP_TRY(hipMemsetAsync(todo, 1, DN, s->stream));
     HIP_TRY(hipMemsetAsync(ctl, 0, 12, s->stream));
@@ -3159,9 +3437,6 @@ int build_groups_t(ssw_sweep* s) {
                                               ctl + 2, (int)DN, s->stream));
         TRY(dalloc(s, &tmp, tb));
     }
-    const uint4* hdr = s->d_hdr;
-    const Entry<R>* planes = (const Entry<R>*)s->d_planes;
-    const Entry<R>* ovf = (const Entry<R>*)s->d_ovf;
     // blocks of group g in pass r: [rstart[r][g], rstart[r][g] + rcount[r][g]) of the pass-major descriptors
     std::vector<std::vector<uint32_t>> rstart(mmax, std::vector<uint32_t>(ng, 0u)), rcount(rstart);
     uint32_t ndesc = 0;
@@ -3220,15 +3495,8 @@ int build_groups_t(ssw_sweep* s) {
         TRY(dalloc(s, &meta, hmeta.size()));
         HIP_TRY(hipMemcpyAsync(meta, hmeta.data(), hmeta.size() * sizeof(uint4), hipMemcpyHostToDevice, s->stream));
         const unsigned nb = (unsigned)hmeta.size();
-        if (T == 32)
-            k_cone<R, 32><<<nb, 32, 0, s->stream>>>(hdr, planes, ovf, s->d_fstart, meta, rl, todo, s->d_glist,
-                                                    (uint32_t)list_cap, ctl, desc_rm + 2 * (size_t)ndesc, ctl + 1);
-        else if (T == 64)
-            k_cone<R, 64><<<nb, 64, 0, s->stream>>>(hdr, planes, ovf, s->d_fstart, meta, rl, todo, s->d_glist,
-                                                    (uint32_t)list_cap, ctl, desc_rm + 2 * (size_t)ndesc, ctl + 1);
-        else
-            k_cone<R, 128><<<nb, 128, 0, s->stream>>>(hdr, planes, ovf, s->d_fstart, meta, rl, todo, s->d_glist,
-                                                      (uint32_t)list_cap, ctl, desc_rm + 2 * (size_t)ndesc, ctl + 1);
+        k_cone<<<nb, kConeThreads, 0, s->stream>>>(uoff, up, s->d_fstart, meta, rl, todo, list, (uint32_t)list_cap, ctl,
+                                                   desc_rm + 2 * (size_t)ndesc, ctl + 1);
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipStreamSynchronize(s->stream));  // meta is reallocated by the next pass
         ndesc += nb;
@@ -3247,8 +3515,6 @@ int build_groups_t(ssw_sweep* s) {
     dfree(s, todo);
     if (hctl[1] != 0) {  // a cone or the list did not fit: per-level replay
         s->groups.clear();
-        dfree(s, desc_rm);
-        dfree(s, s->d_glist);
         s->group_fallback = true;
         return SSW_OK;
     }
@@ -3267,18 +3533,7 @@ int build_groups_t(ssw_sweep* s) {
         gr.ndesc = (uint32_t)hperm.size() - gr.desc0;
         gr.passes.off[gr.passes.n] = gr.ndesc;
     }
-    TRY(dalloc(s, &s->d_gdesc, 2 * std::max<size_t>(1, ndesc)));
-    TRY(dalloc(s, &perm, std::max<size_t>(1, ndesc)));
-    if (ndesc) {
-        HIP_TRY(hipMemcpyAsync(perm, hperm.data(), hperm.size() * 4, hipMemcpyHostToDevice, s->stream));
-        k_permute_desc<<<grid_for(ndesc), kBlock, 0, s->stream>>>(desc_rm, perm, s->d_gdesc, ndesc);
-        HIP_TRY(hipGetLastError());
-    }
-    HIP_TRY(hipStreamSynchronize(s->stream));
-    dfree(s, perm);
-    dfree(s, desc_rm);
     s->group_tasks = hctl[0];
-    s->glist_len = std::max<uint32_t>(1u, hctl[0]);
     s->ndesc = ndesc;
     std::vector<uint32_t> gmap(std::max<uint32_t>(1u, ndesc), 0u);
     for (size_t i = 0; i < s->groups.size(); i++)
@@ -3301,26 +3556,100 @@ int build_groups_t(ssw_sweep* s) {
     if (pb.empty()) pb.push_back(0u);
     TRY(dalloc(s, &s->d_pbound, pb.size()));
     HIP_TRY(hipMemcpyAsync(s->d_pbound, pb.data(), pb.size() * 4, hipMemcpyHostToDevice, s->stream));
-    if (s->p.num_timestep_levels > 1 && ndesc) {  // restricted sweeps filter the cones
+    if (s->p.num_timestep_levels > 1) {  // restricted sweeps filter the cones
         s->gf_scan_bytes = 0;
         HIP_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, s->gf_scan_bytes, s->d_gf_kept, s->d_gf_pos, (int)ndesc + 1,
                                                  s->stream));
-        TRY(dalloc(s, &s->d_gf_desc, 2 * (size_t)ndesc));
         TRY(dalloc(s, &s->d_gf_kept, (size_t)ndesc + 1));
         TRY(dalloc(s, &s->d_gf_pos, (size_t)ndesc + 1));
         TRY(dalloc(s, &s->d_gf_pbval, pb.size()));
         TRY(dalloc(s, &s->d_gf_scan, std::max<size_t>(s->gf_scan_bytes, 1)));
     }
+    // cones in group order (a group's workgroups contiguous), counted, placed
+    // and written
+    TRY(dalloc(s, &desc, 2 * (size_t)ndesc));
+    TRY(dalloc(s, &perm, ndesc));
+    HIP_TRY(hipMemcpyAsync(perm, hperm.data(), hperm.size() * 4, hipMemcpyHostToDevice, s->stream));
+    k_permute_desc<<<grid_for(ndesc), kBlock, 0, s->stream>>>(desc_rm, perm, desc, ndesc);
+    std::vector<uint32_t> hk0(ng), hw(ng);
+    for (size_t i = 0; i < ng; i++) hk0[i] = (uint32_t)s->groups[i].k0;
+    TRY(dalloc(s, &k0s, ng));
+    TRY(dalloc(s, &words, ng));
+    HIP_TRY(hipMemcpyAsync(k0s, hk0.data(), ng * 4, hipMemcpyHostToDevice, s->stream));
+    k_fill_u32<<<grid_for((int64_t)ng), kBlock, 0, s->stream>>>(words, 0u, (int64_t)ng);
+    TRY(dalloc(s, &ct, (size_t)ndesc + 1));
+    TRY(dalloc(s, &ts, (size_t)ndesc + 1));
+    TRY(dalloc(s, &cu, (size_t)ndesc + 1));
+    TRY(dalloc(s, &us, (size_t)ndesc + 1));
+    HIP_TRY(hipMemsetAsync(ct + ndesc, 0, 4, s->stream));
+    HIP_TRY(hipMemsetAsync(cu + ndesc, 0, 8, s->stream));
+    const double inv_aref = 1.0 / s->aref;
+    const uint32_t waves = (uint32_t)ConeShape<R>::waves(T);
+    TRY(dalloc(s, &fars, (size_t)hctl[0]));
+    k_cone_tiles<R, false><<<ndesc, 64, 0, s->stream>>>(g, inv_aref, sorted, s->d_xpos, uoff, up, s->d_fstart,
+                                                        s->d_nup, fars, desc, list, s->d_gmap, k0s, ct, cu, words,
+                                                        nullptr, nullptr, waves, nullptr, nullptr, nullptr);
+    HIP_TRY(hipGetLastError());
+    size_t t1 = 0, t2 = 0;
+    HIP_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, t1, ct, ts, (int)ndesc + 1, s->stream));
+    HIP_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, t2, cu, us, (int)ndesc + 1, s->stream));
+    TRY(dalloc(s, &tmp, std::max(t1, t2)));
+    HIP_TRY(hipcub::DeviceScan::ExclusiveSum(tmp, t1, ct, ts, (int)ndesc + 1, s->stream));
+    HIP_TRY(hipcub::DeviceScan::ExclusiveSum(tmp, t2, cu, us, (int)ndesc + 1, s->stream));
+    uint32_t more = 0;
+    uint64_t units = 0;
+    HIP_TRY(hipMemcpyAsync(hw.data(), words, ng * 4, hipMemcpyDeviceToHost, s->stream));
+    HIP_TRY(hipMemcpyAsync(&more, ts + ndesc, 4, hipMemcpyDeviceToHost, s->stream));
+    HIP_TRY(hipMemcpyAsync(&units, us + ndesc, 8, hipMemcpyDeviceToHost, s->stream));
+    HIP_TRY(hipStreamSynchronize(s->stream));
+    size_t lds = 0, members = 0;
+    for (size_t i = 0; i < ng; i++) {
+        s->groups[i].words = hw[i];
+        members = std::max<size_t>(members, hw[i]);
+        lds = std::max(lds, ConeShape<R>::bytes(T, hw[i]));
+    }
+    if (lds > 65536)  // at most 116 KB (a cone of kConeCap members and 128 roots, FP64)
+        for (const bool general : {false, true}) {
+            HIP_TRY(hipFuncSetAttribute((const void*)SSW_CONE_KERNEL(k_sweep_cone, R, T, general),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 << 10));
+            HIP_TRY(hipFuncSetAttribute((const void*)SSW_CONE_KERNEL(k_sweep_cone_pack, R, T, general),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 << 10));
+        }
+    dfree(s, tmp);
+    dfree(s, desc_rm);
+    dfree(s, up);
+    dfree(s, uoff);
+    dfree(s, cu);
+    dfree(s, ct);
+    TRY(dalloc(s, &s->d_coneblob, (size_t)units));
+    TRY(dalloc(s, &s->d_conetiles, (size_t)ndesc * waves + more));
+    TRY(dalloc(s, &s->d_conemore, (size_t)ndesc));
+    k_cone_tiles<R, true><<<ndesc, 256, members * 4, s->stream>>>(
+        g, inv_aref, sorted, s->d_xpos, nullptr, nullptr, s->d_fstart, s->d_nup, fars, desc, list, s->d_gmap, k0s,
+        nullptr, nullptr, words, ts, us, waves, s->d_coneblob, s->d_conetiles, s->d_conemore);
+    HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(s->stream));
     return SSW_OK;
 }
 
-int build_groups(ssw_sweep* s) {
+// sorted: the tasks in schedule order; s->d_xpos, s->d_fstart and s->d_nup held.
+int group_waves(const ssw_sweep* s) { return ConeShape<float>::waves(s->group_block); }
+
+int build_groups(ssw_sweep* s, const uint32_t* sorted) {
+    return s->fp32 ? build_groups_t<float>(s, sorted) : build_groups_t<double>(s, sorted);
+}
+
+void free_groups(ssw_sweep* s) {
     s->groups.clear();
     s->group_tasks = 0;
     s->group_fallback = false;
-    if (!s->compiled || s->group_request < 2 || s->d_dirinfo) return SSW_OK;  // direction sweeps need no cones
-    return s->fp32 ? build_groups_t<float>(s) : build_groups_t<double>(s);
+    for (uint4** p : {&s->d_coneblob, &s->d_conetiles}) dfree(s, *p);
+    for (uint32_t** p : {&s->d_conemore, &s->d_gmap, &s->d_gcount, &s->d_gbase, &s->d_gblocks, &s->d_pbound, &s->d_gf_kept,
+                         &s->d_gf_pos, &s->d_gf_pbval})
+        dfree(s, *p);
+    dfree(s, s->d_gf_scan);
+    s->gf_scan_bytes = 0;
+    for (uint32_t*& p : s->d_gsel_l) dfree(s, p);
 }
 
 // The direction sweeps' schedule from every task's depth and upwind count:
@@ -3446,12 +3775,14 @@ int build_dir_schedule_t(ssw_sweep* s, uint32_t*& d_depth) {
 }
 
 int init_replay(ssw_sweep* s);
+int setup_overflow(ssw_sweep* s);
 
 // The full schedule, once per grid: Kahn layering of the whole graph, each
 // task's depth, a stable sort by depth of the tasks in (direction, cell)
 // order, then the compiled or geometric per-task data in that order, and the
 // chunk table of the compaction.
 int build_schedule(ssw_sweep* s) {
+    free_groups(s);
     const size_t DN = (size_t)s->D * s->N;
     // sort the tasks by depth, stable over t = d*N + c (double-buffered: four
     // DN-word arrays and a small temporary)
@@ -3498,6 +3829,13 @@ int build_schedule(ssw_sweep* s) {
     if (s->compiled) {
         TRY(dalloc(s, &s->d_xpos, DN));
         k_invert<<<grid_for((int64_t)DN), kBlock, 0, s->stream>>>(d_sorted, s->d_xpos, (uint32_t)DN);
+        HIP_TRY(hipGetLastError());
+        if (s->group_request >= 2) {
+            TRY(build_groups(s, d_sorted));
+            dfree(s, s->d_nup);
+            if (!s->groups.empty()) return init_replay(s);
+        }
+        TRY(setup_overflow(s));
         TRY(dalloc(s, &s->d_hdr, DN));
         TRY(dalloc(s, (uint8_t**)&s->d_A, DN * real_size(s)));
         TRY(dalloc(s, (uint8_t**)&s->d_planes, (size_t)kPlanes * DN * entry_size(s)));
@@ -3546,8 +3884,7 @@ int build_schedule(ssw_sweep* s) {
     return init_replay(s);
 }
 
-// Empty active-set lists, plans and graphs, the cones of the grouped replay,
-// and the full sweep's plan.
+// Empty active-set lists, plans and graphs, and the full sweep's plan.
 int init_replay(ssw_sweep* s) {
     const int L = s->p.num_timestep_levels;
     for (uint32_t*& p : s->d_idx) dfree(s, p);
@@ -3561,15 +3898,12 @@ int init_replay(ssw_sweep* s) {
     s->graphs.assign(L, nullptr);
     for (uint4*& p : s->d_runtab) dfree(s, p);
     s->d_runtab.assign(L, nullptr);
-    for (uint4*& p : s->d_gdesc_l) dfree(s, p);
-    for (uint32_t*& p : s->d_glist_l) dfree(s, p);
-    s->d_gdesc_l.assign(L, nullptr);
-    s->d_glist_l.assign(L, nullptr);
+    for (uint32_t*& p : s->d_gsel_l) dfree(s, p);
+    s->d_gsel_l.assign(L, nullptr);
     s->gcount.assign(L, std::vector<uint32_t>());
     s->gblocks.assign(L, std::vector<uint32_t>());
     s->runtab.assign(L, std::vector<uint4>());
     s->plan.assign(L, std::vector<ssw_sweep::ReplayItem>());
-    TRY(build_groups(s));
     TRY(plan_replay(s, 0));
     return SSW_OK;
 }
@@ -3580,8 +3914,7 @@ const uint4* schedule_tasks(ssw_sweep* s) { return s->compiled ? s->d_hdr : s->d
 // schedule whose cell has level >= lvl, per level set, and its level starts
 // on the host. Sweep level 0 covers every task and needs no list.
 int make_group_list(ssw_sweep* s, int lvl) {
-    if (!s->d_gdesc_l[lvl]) TRY(dalloc(s, &s->d_gdesc_l[lvl], 2 * (size_t)std::max<uint32_t>(1u, s->ndesc)));
-    if (!s->d_glist_l[lvl]) TRY(dalloc(s, &s->d_glist_l[lvl], s->glist_len));
+    if (!s->d_gsel_l[lvl]) TRY(dalloc(s, &s->d_gsel_l[lvl], std::max<uint32_t>(1u, s->ndesc)));
     const size_t ng = std::max<size_t>(1, s->groups.size());
     HIP_TRY(hipMemsetAsync(s->d_gcount, 0, ng * 4, s->stream));
     HIP_TRY(hipMemsetAsync(s->d_gblocks, 0, ng * 4, s->stream));
@@ -3591,22 +3924,19 @@ int make_group_list(ssw_sweep* s, int lvl) {
                                                                           s->groups.back().passes.n + 1);
     std::vector<uint32_t> pbv(npb, 0u);
     if (nd) {
-        // filter, then pack each group's kept descriptors in order (scratch
-        // held since the cone build)
-        uint4* tmp_desc = s->d_gf_desc;
+        // the cones with active tasks, packed in order (scratch held since the
+        // cone build)
         uint32_t *kept = s->d_gf_kept, *pos = s->d_gf_pos, *pbval = s->d_gf_pbval;
         uint8_t* scan_tmp = s->d_gf_scan;
         size_t tb = s->gf_scan_bytes;
-        if (!tmp_desc || !kept || !pos || !pbval || !scan_tmp)
+        if (!kept || !pos || !pbval || !scan_tmp)
             return fail(SSW_ERR_INVALID, "grouped replay: restricted-sweep scratch missing");
         k_fill_u32<<<1, 1, 0, s->stream>>>(kept + nd, 0u, 1);
-        k_group_compact<<<nd, kBlock, 0, s->stream>>>(g, s->d_hdr, lvl, s->d_gdesc, s->d_glist, s->d_gmap, nd,
-                                                       tmp_desc, kept, s->d_glist_l[lvl], s->d_gcount,
-                                                       s->d_gblocks);
+        k_cone_active<<<nd, 64, 0, s->stream>>>(g, lvl, s->d_coneblob, s->d_conetiles, s->d_conemore,
+                                                (uint32_t)group_waves(s), s->d_gmap, kept, s->d_gcount, s->d_gblocks);
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipcub::DeviceScan::ExclusiveSum(scan_tmp, tb, kept, pos, (int)nd + 1, s->stream));
-        k_place_desc<<<grid_for(nd), kBlock, 0, s->stream>>>(tmp_desc, kept, pos, s->d_gmap, s->d_gbase,
-                                                             s->d_gdesc_l[lvl], nd);
+        k_place_cone<<<grid_for(nd), kBlock, 0, s->stream>>>(kept, pos, s->d_gmap, s->d_gbase, s->d_gsel_l[lvl], nd);
         k_gather_u32<<<grid_for((int64_t)npb), kBlock, 0, s->stream>>>(pos, s->d_pbound, pbval, (uint32_t)npb);
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipMemcpyAsync(pbv.data(), pbval, npb * 4, hipMemcpyDeviceToHost, s->stream));
@@ -3619,7 +3949,7 @@ int make_group_list(ssw_sweep* s, int lvl) {
     gb.assign(ng, 0u);
     HIP_TRY(hipMemcpyAsync(gb.data(), s->d_gblocks, ng * 4, hipMemcpyDeviceToHost, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
-    // pass ranges of each group's kept descriptors
+    // pass ranges of each group's kept cones
     if ((int)s->gpass_l.size() <= lvl) s->gpass_l.resize(lvl + 1);
     s->gpass_l[lvl].assign(s->groups.size(), PassTab{});
     for (size_t i = 0; i < s->groups.size(); i++) {
@@ -3631,8 +3961,7 @@ int make_group_list(ssw_sweep* s, int lvl) {
     }
     int64_t kept = 0;
     for (uint32_t v : gc) kept += v;
-    // every list entry kept: the same tasks in the same per-workgroup order as
-    // the full sweep, whose launches (in their die-aware order) are then used
+    // every task active: the full sweep's launches are used
     s->list_full[lvl] = (kept == s->group_tasks) ? 1 : 0;
     s->list_ok[lvl] = 1;
     s->replays[lvl] = 0;
@@ -3701,6 +4030,12 @@ int make_list(ssw_sweep* s, int lvl) {
     return SSW_OK;
 }
 
+template <typename R, typename... Args>
+void launch_cones(int roots, bool general, uint32_t blocks, uint32_t words, hipStream_t st, Args... args) {
+    hipLaunchKernelGGL(SSW_CONE_KERNEL(k_sweep_cone, R, roots, general), dim3(blocks),
+                       dim3(64 * ConeShape<R>::waves(roots)), ConeShape<R>::bytes(roots, words), st, args...);
+}
+
 // Launches one item of sweep level lvl's replay plan on stream st: a group
 // of level sets (its cones one workgroup each), a run of narrow level sets
 // (one workgroup), or one level set.
@@ -3728,32 +4063,10 @@ void launch_item_t(ssw_sweep* s, const Geo& g, const Flux<R>& fl, int lvl, const
     }
     if (it.group) {
         const ssw_sweep::Group& gr = s->groups[it.tab];
-        const uint4* dsc = (all ? s->d_gdesc : s->d_gdesc_l[lvl]) + 2 * (size_t)gr.desc0;
-        const uint32_t* gl = all ? s->d_glist : s->d_glist_l[lvl];
-        const uint32_t nblk = all ? gr.ndesc : s->gblocks[lvl][it.tab];  // restricted: workgroups with active tasks
-        const Entry<R>* pl = (const Entry<R>*)s->d_planes;
-        // full sweeps: die-aware order inside each pass; restricted sweeps
-        // launch their filtered descriptors in order
-        const PassTab pt = all ? gr.passes : s->gpass_l[lvl][it.tab];
-        // groups of exactly 4 level sets (all but the narrow and last ones)
-        // run the kernel that knows its level-set count at compile time
-        using GroupKernel = void (*)(Geo, Flux<R>, const uint4*, const R*, const Entry<R>*, const Entry<R>*,
-                                     const uint32_t*, int, int, const uint4*, const uint32_t*, uint32_t, PassTab);
-        const bool four = gr.levels == 4;
-        GroupKernel kern;
-        int lanes;
-        if (s->group_block == 32) {
-            lanes = 64;
-            kern = four ? k_sweep_group<R, 64, 4> : k_sweep_group<R, 64, 0>;
-        } else if (s->group_block == 64) {
-            lanes = 128;
-            kern = four ? k_sweep_group<R, 128, 4> : k_sweep_group<R, 128, 0>;
-        } else {
-            lanes = 256;
-            kern = four ? k_sweep_group<R, 256, 4> : k_sweep_group<R, 256, 0>;
-        }
-        hipLaunchKernelGGL(kern, dim3(nblk), dim3(lanes), 0, st, g, fl, s->d_hdr, (const R*)s->d_A, pl, ovf,
-                           s->d_fstart, gr.k0, gr.levels, dsc, gl, s->glist_len, pt);
+        launch_cones<R>(s->group_block, !all || fl.offI != nullptr, all ? gr.ndesc : s->gblocks[lvl][it.tab], gr.words,
+                        st, g, fl, s->d_coneblob, s->d_conetiles, s->d_conemore,
+                        all ? nullptr : s->d_gsel_l[lvl] + gr.desc0, gr.desc0, gr.words, all ? 0 : lvl,
+                        all ? gr.passes : s->gpass_l[lvl][it.tab]);
         return;
     }
     if (it.levels > 0) {  // a run of narrow level sets, one workgroup
@@ -3981,7 +4294,7 @@ int run_step(ssw_sweep* s, double* elapsed) {
 
 // ---------------------------------------------------------------------------
 // Packed steps: one step of each of several handles, their grouped launches
-// packed into shared launches (k_sweep_group_pack).
+// packed into shared launches (k_sweep_cone_pack).
 //
 // The handles' sweeps are aligned by index: sweep i of every handle whose
 // step has more than i sweeps runs together. Inside sweep i, the t-th items of
@@ -4006,23 +4319,20 @@ GroupJob<R> group_job(ssw_sweep* s, int lvl, const ssw_sweep::ReplayItem& it, ui
     const Geo g = make_geo(s);
     GroupJob<R> J;
     J.N = g.N;
-    J.Nper = g.Nper;
     J.X = fl.X;
     J.I = fl.I;
     J.P = fl.P;
     J.offI = fl.offI;
     J.sa = fl.sa;
     J.thr = fl.thr;
-    J.hdr = s->d_hdr;
-    J.A = (const R*)s->d_A;
-    J.planes = (const Entry<R>*)s->d_planes;
-    J.ovf = (const Entry<R>*)s->d_ovf;
-    J.fstart = s->d_fstart;
-    J.desc = (all ? s->d_gdesc : s->d_gdesc_l[lvl]) + 2 * (size_t)gr.desc0;
-    J.list = all ? s->d_glist : s->d_glist_l[lvl];
-    J.list_len = s->glist_len;
-    J.k0 = gr.k0;
-    J.phases = gr.levels;
+    J.level = s->d_level;
+    J.blob = s->d_coneblob;
+    J.tiles = s->d_conetiles;
+    J.more = s->d_conemore;
+    J.cone0 = gr.desc0;
+    J.sel = all ? nullptr : s->d_gsel_l[lvl] + gr.desc0;
+    J.words = gr.words;
+    J.lvl = all ? 0 : lvl;
     J.start = 0;
     *nblk = all ? gr.ndesc : s->gblocks[lvl][it.tab];
     J.blocks = *nblk;
@@ -4040,18 +4350,14 @@ struct Pack {
 template <typename R>
 void flush_pack(Pack<R>& p, int roots, hipStream_t st) {
     if (p.a.n <= 0) return;
-    bool four = true;
-    for (int k = 0; k < p.a.n; k++) four = four && p.a.job[k].phases == 4;
-    if (roots == 32) {
-        if (four) k_sweep_group_pack<R, 64, 4><<<p.grid, 64, 0, st>>>(p.a);
-        else k_sweep_group_pack<R, 64, 0><<<p.grid, 64, 0, st>>>(p.a);
-    } else if (roots == 64) {
-        if (four) k_sweep_group_pack<R, 128, 4><<<p.grid, 128, 0, st>>>(p.a);
-        else k_sweep_group_pack<R, 128, 0><<<p.grid, 128, 0, st>>>(p.a);
-    } else {
-        if (four) k_sweep_group_pack<R, 256, 4><<<p.grid, 256, 0, st>>>(p.a);
-        else k_sweep_group_pack<R, 256, 0><<<p.grid, 256, 0, st>>>(p.a);
+    uint32_t words = 0;
+    bool general = false;
+    for (int k = 0; k < p.a.n; k++) {
+        words = std::max(words, p.a.job[k].words);
+        general = general || p.a.job[k].lvl > 0 || p.a.job[k].offI;
     }
+    hipLaunchKernelGGL(SSW_CONE_KERNEL(k_sweep_cone_pack, R, roots, general), dim3(p.grid),
+                       dim3(64 * ConeShape<R>::waves(roots)), ConeShape<R>::bytes(roots, words), st, p.a);
     p.a.n = 0;
     p.grid = 0;
 }
@@ -4497,22 +4803,7 @@ void free_grid(ssw_sweep* s) {
     drop_all_lists(s);
     for (uint32_t*& p : s->d_idx) dfree(s, p);
     for (uint4*& p : s->d_runtab) dfree(s, p);
-    dfree(s, s->d_gdesc);
-    dfree(s, s->d_glist);
-    dfree(s, s->d_gmap);
-    dfree(s, s->d_gcount);
-    dfree(s, s->d_gbase);
-    dfree(s, s->d_gblocks);
-    dfree(s, s->d_pbound);
-    dfree(s, s->d_gf_desc);
-    dfree(s, s->d_gf_kept);
-    dfree(s, s->d_gf_pos);
-    dfree(s, s->d_gf_pbval);
-    dfree(s, s->d_gf_scan);
-    s->gf_scan_bytes = 0;
-    for (uint4*& p : s->d_gdesc_l) dfree(s, p);
-    for (uint32_t*& p : s->d_glist_l) dfree(s, p);
-    s->groups.clear();
+    free_groups(s);
     dfree(s, s->d_off);
     dfree(s, s->d_inv);
     dfree(s, s->d_perm);
@@ -4550,20 +4841,29 @@ void free_grid(ssw_sweep* s) {
     dfree(s, s->d_scan_tmp);
 }
 
-// Overflow entries of the compiled schedule (once per grid).
-int setup_overflow(ssw_sweep* s, uint32_t* d_ovf_count) {
+// Overflow entries of the per-level replay's planes (s->ovf_total of them).
+int setup_overflow(ssw_sweep* s) {
     const size_t DN = (size_t)s->D * s->N;
+    uint32_t *d_cursor = nullptr, *d_count = nullptr;
+    unsigned long long* d_stats = nullptr;
+    Defer cleanup{[&] {
+        dfree(s, d_cursor);
+        dfree(s, d_count);
+        dfree(s, d_stats);
+    }};
+    TRY(dalloc(s, &d_count, DN));
+    TRY(dalloc(s, &d_stats, 4));
+    Geo g = make_geo(s);
+    k_face_stats<<<(unsigned)((s->N + kFluxCells - 1) / kFluxCells),
+                   kFluxCells * ((s->D + kFluxDirs - 1) / kFluxDirs), 0, s->stream>>>(g, d_stats, d_count, nullptr);
+    HIP_TRY(hipGetLastError());
     TRY(dalloc(s, &s->d_ovf_start, DN));
     TRY(dalloc(s, (uint8_t**)&s->d_ovf, (size_t)std::max<int64_t>(1, s->ovf_total) * entry_size(s)));
-    uint32_t* d_cursor = nullptr;
-    Defer cleanup{[&] { dfree(s, d_cursor); }};
     TRY(dalloc(s, &d_cursor, 1));
     HIP_TRY(hipMemsetAsync(d_cursor, 0, 4, s->stream));
-    Geo g = make_geo(s);
-    k_overflow<<<grid_for((int64_t)DN), kBlock, 0, s->stream>>>(g, d_ovf_count, s->d_ovf_start, d_cursor);
+    k_overflow<<<grid_for((int64_t)DN), kBlock, 0, s->stream>>>(g, d_count, s->d_ovf_start, d_cursor);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(s->stream));
-    dfree(s, d_cursor);
     return SSW_OK;
 }
 
@@ -4620,8 +4920,9 @@ int build_direction_graph(ssw_sweep* s, bool choose_mode) {
     HIP_TRY(hipMemsetAsync(d_stats, 0, 5 * 8, s->stream));
     Geo g = make_geo(s);
     if (choose_mode) k_check_mirror<<<grid_for(n), kBlock, 0, s->stream>>>(g, d_stats);
-    const bool dir = s->dir_sweeps && (choose_mode ? s->mode_request != SSW_TRANSPORT_MODE_GEOMETRIC : s->compiled);
-    if (dir) TRY(dalloc(s, &s->d_nup, DN));
+    const bool tiles = (s->dir_sweeps || s->group_request >= 2) &&
+                       (choose_mode ? s->mode_request != SSW_TRANSPORT_MODE_GEOMETRIC : s->compiled);
+    if (tiles) TRY(dalloc(s, &s->d_nup, DN));
     k_face_stats<<<(unsigned)((n + kFluxCells - 1) / kFluxCells),
                    kFluxCells * ((s->D + kFluxDirs - 1) / kFluxDirs), 0, s->stream>>>(g, d_stats + 1, s->d_cnt,
                                                                                       s->d_nup);
@@ -4636,7 +4937,6 @@ int build_direction_graph(ssw_sweep* s, bool choose_mode) {
     for (int k = 0; k < 3; k++) s->dw[k] = (double)hb[k + 1] / ((double)n * s->D);
     s->ovf_total = (int64_t)hb[4];
     if (!choose_mode) {
-        if (s->compiled && !dir) TRY(setup_overflow(s, s->d_cnt));
         return build_schedule(s);
     }
     // transport mode: compiled when, at its peak (schedule arrays, overflow
@@ -4655,7 +4955,6 @@ int build_direction_graph(ssw_sweep* s, bool choose_mode) {
     else if (s->mode_request == SSW_TRANSPORT_MODE_GEOMETRIC) s->compiled = false;
     else s->compiled = (double)comp_need <= 0.85 * (double)free_b;
     if (!s->compiled) dfree(s, s->d_nup);
-    if (s->compiled && !dir) TRY(setup_overflow(s, s->d_cnt));
     return build_schedule(s);
 }
 
@@ -5579,14 +5878,17 @@ int ssw_load_checkpoint(ssw_sweep* s, const void* buf, int64_t bytes) {
 
 extern "C++" {
 namespace {
-// Workgroups of the grouped replay kernel one CU holds at once (0 if unknown).
+// Workgroups of the grouped replay kernel one CU holds at once (0 if unknown),
+// with the LDS of the group of the largest cone.
 template <typename R>
-int group_blocks_per_cu(int roots) {
+int group_blocks_per_cu(const ssw_sweep* s) {
+    uint32_t words = 0;
+    for (const ssw_sweep::Group& gr : s->groups) words = std::max(words, gr.words);
     int n = 0;
-    hipError_t e;
-    if (roots == 32) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_sweep_group<R, 64, 4>, 64, 0);
-    else if (roots == 64) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_sweep_group<R, 128, 4>, 128, 0);
-    else e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_sweep_group<R, 256, 4>, 256, 0);
+    const int roots = s->group_block;
+    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        &n, SSW_CONE_KERNEL(k_sweep_cone, R, roots, false), 64 * ConeShape<R>::waves(roots),
+        ConeShape<R>::bytes(roots, words));
     return e == hipSuccess ? n : 0;
 }
 }  // namespace
@@ -5622,7 +5924,7 @@ int ssw_get_info(ssw_sweep* s, ssw_info* info) {
         info->group_launches = (int64_t)s->groups.size();
         for (const ssw_sweep::Group& gr : s->groups) info->group_workgroups += gr.ndesc;
         info->group_blocks_per_cu =
-            s->fp32 ? group_blocks_per_cu<float>(s->group_block) : group_blocks_per_cu<double>(s->group_block);
+            s->fp32 ? group_blocks_per_cu<float>(s) : group_blocks_per_cu<double>(s);
     }
     {
         int cus = 0;
