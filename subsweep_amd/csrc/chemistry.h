@@ -310,10 +310,10 @@ SSW_HD bool accept(double& value, double change, double safety, double dt, doubl
     return true;
 }
 
-// try_timestep_update (:371-392)
+// try_timestep_update (:371-392) with the rates h at c
 template <typename Ev>
-SSW_HD bool try_step(Cell& c, const Floor& f, double dt, double safety, double& ts, int& proc, const Ev& ev) {
-    const HeatRates h = heat_rates(c, ev);
+SSW_HD bool try_step(Cell& c, const Floor& f, double dt, double safety, double& ts, int& proc, const HeatRates& h,
+                     const Ev& ev) {
     double dT = delta_temperature(c, dt, h);
     double tsT;
     if (!accept(c.T, dT, safety, dt, tsT)) return false;
@@ -340,6 +340,33 @@ struct Walk {
     double dt = 0.0, ts = 0.0;
     int proc = kProcTemperature;
     bool failed = false;
+
+    SSW_HD void overflow(double dt0) {
+        failed = true;
+        proc = kProcTemperature;
+        ts = dt0 / 10.0;
+    }
+    // after an accepted step: true at the end, else on to the deepest pending one
+    SSW_HD bool next(double dt0) {
+        if (lo == 0 && hi == 0) return true;
+        if (hi) {
+            depth = 127 - __builtin_clzll(hi);
+            hi &= ~(1ull << (depth - 64));
+        } else {
+            depth = 63 - __builtin_clzll(lo);
+            lo &= ~(1ull << depth);
+        }
+        dt = dt0;
+        for (int k = 0; k < depth; k++) dt = dt / 2.0;
+        return false;
+    }
+    // after a rejected step: on to the first of its halves
+    SSW_HD void halve() {
+        depth += 1;
+        if (depth < 64) lo |= 1ull << depth;
+        else hi |= 1ull << (depth - 64);
+        dt = dt / 2.0;
+    }
 };
 
 // One attempt of perform_timestep (:394-441); true when the walk has ended,
@@ -349,30 +376,13 @@ SSW_HD bool walk_step(Cell& c, const Floor& f, double dt0, double safety, Walk& 
     clamp_state(c, f);
     double T0 = c.T, x0 = c.x;
     if (w.depth > kMaxDepth) {
-        w.failed = true;
-        w.proc = kProcTemperature;
-        w.ts = dt0 / 10.0;
+        w.overflow(dt0);
         return true;
     }
-    if (try_step(c, f, w.dt, safety, w.ts, w.proc, ev)) {
-        if (w.lo == 0 && w.hi == 0) return true;
-        if (w.hi) {
-            w.depth = 127 - __builtin_clzll(w.hi);
-            w.hi &= ~(1ull << (w.depth - 64));
-        } else {
-            w.depth = 63 - __builtin_clzll(w.lo);
-            w.lo &= ~(1ull << w.depth);
-        }
-        w.dt = dt0;
-        for (int k = 0; k < w.depth; k++) w.dt = w.dt / 2.0;
-    } else {
-        c.T = T0;
-        c.x = x0;
-        w.depth += 1;
-        if (w.depth < 64) w.lo |= 1ull << w.depth;
-        else w.hi |= 1ull << (w.depth - 64);
-        w.dt = w.dt / 2.0;
-    }
+    if (try_step(c, f, w.dt, safety, w.ts, w.proc, heat_rates(c, ev), ev)) return w.next(dt0);
+    c.T = T0;
+    c.x = x0;
+    w.halve();
     return false;
 }
 

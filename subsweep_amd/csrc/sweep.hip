@@ -2486,22 +2486,29 @@ __global__ void __launch_bounds__(kBlock) k_chemistry(const ChemJobs<R, kJobs> j
 // powers (0.4 us each). So a quad of lanes takes a cell and shares them, two
 // rounds of them before the temperature's step and two before the ionised
 // fraction's instead of eleven powers, and a quad that has finished its cell
-// takes the next one while the others of its wave go on. Chemistry of 262144
-// cells with 64 sources: 1.04 -> 0.60 ms (0.19 + 0.41), of 32768 cells in the
-// first two steps 1.96 -> 1.33 ms a step.
+// takes the next one while the others of its wave go on. About half of the
+// attempts are rejected and made again with half the step; so where there are
+// lanes for it (few cells queued, or the queue empty and the quads of a row of
+// 16 lanes idle), `team` = 2 or 4 quads take one cell, quad q its step halved
+// q times, and the first of them that is accepted counts: what they would come
+// to one after the other. First step of 262144 cells with 64 sources: 3.03 ms
+// with a quad a cell, 1.66 like this; of 32768 cells 1.37 and 0.86; both some
+// 0.02 once the gas has settled.
 template <typename R, int kJobs>
 __global__ void __launch_bounds__(64) k_chemistry_tail(const ChemJobs<R, kJobs> jobs) {
     const Geo& g = jobs.mine().g;
     const ChemArgs& ca = jobs.mine().ca;
-    const uint32_t n = ca.queue[0], first = gridDim.x * 16u;
-    const bool lead = (threadIdx.x & 3u) == 0;
-    uint32_t i = blockIdx.x * 16u + threadIdx.x / 4u;
+    const uint32_t n = ca.queue[0], lane = threadIdx.x;
+    uint32_t team = n <= gridDim.x * 4u ? 4u : n <= gridDim.x * 8u ? 2u : 1u;
+    const uint32_t per = 16u / team, first = gridDim.x * per;
+    uint32_t i = blockIdx.x * per + lane / (4u * team);
     int64_t c = 0;
     double dt = 0.0;
     ssw::Cell cell{};
     ssw::Floor floor{};
     ssw::Walk w;
-    bool have = false;
+    ssw::HeatRates h{};
+    bool have = false, hot = false;  // hot: h belongs to the cell's state
     for (;;) {
         if (!have && i < n) {
             c = ca.queue[2 + i];
@@ -2513,14 +2520,81 @@ __global__ void __launch_bounds__(64) k_chemistry_tail(const ChemJobs<R, kJobs> 
             w.lo = 2;
             w.dt = dt / 2.0;
             have = true;
+            hot = false;
         }
-        if (__ballot(have) == 0ull) break;
-        if (have && ssw::walk_step(cell, floor, dt, ca.safety, w, ssw::Quad())) {
-            finish_chemistry<R>(ca, c, cell, ca.change_ts[c], w, lead);
+        const unsigned long long busy = __ballot(have);
+        if (busy == 0ull) break;
+        // a row with idle quads (the queue is empty): fewer, larger teams
+        const uint32_t row = (uint32_t)(busy >> (lane & 48u)) & 0xFFFFu, cells = (uint32_t)__popc(row) / (4u * team);
+        const uint32_t want = cells == 1u ? 4u : cells == 2u ? 2u : team;
+        if (__ballot(want > team)) {
+            uint32_t from = lane;
+            bool moved = want > team;
+            if (moved) {  // the (lane / team's lanes)-th of the row's cells
+                uint32_t left = row;
+                const uint32_t lanes = (1u << (4u * team)) - 1u;
+                if (cells == 2u && (lane & 15u) >= 8u) left &= ~(lanes << (uint32_t)(__ffs((int)left) - 1));
+                from = (lane & 48u) + (uint32_t)(__ffs((int)left) - 1);
+            }
+            auto take = [&](auto v) { return __shfl(v, (int)from); };
+            c = (int64_t)take((long long)c);
+            dt = take(dt);
+            cell.x = take(cell.x);
+            cell.T = take(cell.T);
+            cell.rho = take(cell.rho);
+            cell.vol = take(cell.vol);
+            cell.len = take(cell.len);
+            cell.rate = take(cell.rate);
+            cell.a = ca.scale_factor;
+            floor.on = ca.prevent_cooling != 0;
+            floor.T = take(floor.T);
+            floor.x = take(floor.x);
+            w.lo = (uint64_t)take((unsigned long long)w.lo);
+            w.hi = (uint64_t)take((unsigned long long)w.hi);
+            w.depth = take(w.depth);
+            w.dt = take(w.dt);
+            w.ts = take(w.ts);
+            w.proc = take(w.proc);
+            if (moved) {
+                team = want;
+                have = true;
+                hot = false;
+            }
+        }
+        if (!have) continue;
+        const uint32_t base = lane & ~(4u * team - 1u), q = (lane - base) / 4u;
+        bool ended = false;
+        ssw::clamp_state(cell, floor);
+        if (w.depth > ssw::kMaxDepth) {
+            w.overflow(dt);
+            ended = true;
+        } else {
+            if (!hot) h = ssw::heat_rates(cell, ssw::Quad());
+            ssw::Cell t = cell;
+            double dtq = w.dt, ts = 0.0;
+            for (uint32_t k = 0; k < q; k++) dtq = dtq / 2.0;
+            int proc = 0;
+            const bool ok = w.depth + (int)q <= ssw::kMaxDepth &&
+                            ssw::try_step(t, floor, dtq, ca.safety, ts, proc, h, ssw::Quad());
+            const uint32_t m = (uint32_t)(__ballot(ok) >> base) & ((1u << (4u * team)) - 1u);
+            const uint32_t at = m ? (uint32_t)(__ffs((int)m) - 1) : 0u;
+            const uint32_t rejected = m ? at / 4u : min(team, (uint32_t)(ssw::kMaxDepth + 1 - w.depth));
+            for (uint32_t k = 0; k < rejected; k++) w.halve();
+            hot = m == 0u;
+            if (m) {
+                cell.T = __shfl(t.T, (int)(base + at));
+                cell.x = __shfl(t.x, (int)(base + at));
+                w.ts = __shfl(ts, (int)(base + at));
+                w.proc = __shfl(proc, (int)(base + at));
+                ended = w.next(dt);
+            }
+        }
+        if (ended) {
+            finish_chemistry<R>(ca, c, cell, ca.change_ts[c], w, lane == base);
             have = false;
             uint32_t next = 0;
-            if (lead) next = atomicAdd(&ca.queue[1], 1u);
-            i = first + (uint32_t)__builtin_amdgcn_mov_dpp((int)next, 0, 0xF, 0xF, true);
+            if (lane == base) next = atomicAdd(&ca.queue[1], 1u);
+            i = first + (uint32_t)__shfl((int)next, (int)base);
         }
     }
 }
@@ -4192,7 +4266,7 @@ void launch_chemistry(const ChemJob<R>* j, int n, hipStream_t st) {
     }
     k_periodic<R, kJobs><<<dim3(grid_for(64 * pw), n), kBlock, 0, st>>>(a);
     k_chemistry<R, kJobs><<<dim3(grid_for(cells), n), kBlock, 0, st>>>(a);
-    k_chemistry_tail<R, kJobs><<<dim3((unsigned)std::min<int64_t>((cells + 15) / 16, 2048), n), 64, 0, st>>>(a);
+    k_chemistry_tail<R, kJobs><<<dim3((unsigned)std::min<int64_t>((cells + 3) / 4, 2048), n), 64, 0, st>>>(a);
 }
 
 // ssw_sweep::rates_current after the sweeps of `order`.
