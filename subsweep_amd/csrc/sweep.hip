@@ -96,7 +96,13 @@ constexpr int kConeCap = 3072;             // grouped replay build: cone members
 constexpr int kConeThreads = 256;
 constexpr int kSortCap = 4096;             // grouped replay build: entries of one level set sorted in LDS
 constexpr int kMaxGroup = 8;               // grouped replay: level sets per group
-constexpr uint32_t kNarrowGroup = 2048;    // grouped replay: level sets this narrow go kMaxGroup to a group
+// grouped replay: level sets this narrow go kMaxGroup to a group. Their cones
+// overlap more (1.18 -> 1.41 tasks solved per task on 20000 cells x 84
+// directions), but a launch's first loads are paid half as often: that sweep
+// 1.61 ms with 2048, 1.55 with 4096, 1.56 with 8192; on 117649 x 64 FP32 1.48,
+// 1.47, 1.45; beyond, cones of wide level sets no longer fit.
+constexpr uint32_t kNarrowGroup = 8192;
+constexpr uint32_t kCus = 256;             // MI355X: compute units
 constexpr uint32_t kXcds = 8;              // MI355X: accelerator dies, each with its own L2
 
 // Staging of ssw_download_noalloc, which allocates nothing: a file-scope
@@ -1896,9 +1902,13 @@ __global__ void k_permute_desc(const uint4* in, const uint32_t* perm, uint4* out
 //         sets << 8 | tiles of the cone << 16}
 //   blob  planes, {X index, I index} of the tasks, far list, extra weights,
 //         extra words
-// The first `waves` tiles of cone b are at tiles[b * waves] (those it does not
-// have without tasks), the others from tiles[more[b]] on: no load has to
-// return before a wave's first descriptor is on its way.
+// The first `waves` tiles of a group's b-th cone are at tiles[slot0 + b * waves]
+// (those it does not have without tasks), the others from tiles[more[cone0 +
+// b]] on: no load has to return before a wave's first descriptor is on its way.
+// A group of more than 4 level sets has up to twice the tiles of one of 4;
+// where each CU has one of its cones at most, its workgroups are of twice the
+// waves (up to 16), so that no tile waits for another's end to load
+// (32768 cells x 16 directions FP64, groups of 8: 9.1 -> 7.8 us a launch).
 // A restricted sweep runs the cones with active tasks; a task whose cell is
 // below level lvl is not solved and puts its stored X into its word.
 template <typename R>
@@ -1907,13 +1917,13 @@ struct ConeShape {
     static constexpr uint32_t kFar = 512;                                       // far entries of a tile
     static constexpr uint32_t kBuf = kFar + 128 + 512 / (uint32_t)sizeof(R);    // far, extra weights, extra words
     static constexpr int waves(int roots) { return roots == 32 ? 4 : roots == 64 ? 8 : 16; }
-    static size_t bytes(int roots, uint32_t cone) { return sizeof(R) * (kAt + cone + (size_t)waves(roots) * kBuf); }
+    static size_t bytes(int waves, uint32_t cone) { return sizeof(R) * (kAt + cone + (size_t)waves * kBuf); }
 };
 
 template <typename R, int kWaves, bool kGeneral>
 __device__ __forceinline__ void cone_body(const Geo& g, const Flux<R>& fl, const uint4* __restrict__ blob,
                                           const uint4* __restrict__ tiles, const uint32_t* __restrict__ more,
-                                          uint32_t cone, uint32_t words, int lvl) {
+                                          uint32_t b, uint32_t slot0, uint32_t cone0, uint32_t words, int lvl) {
     using S = DirShape<R>;
     using K = ConeShape<R>;
     extern __shared__ double cone_lds[];
@@ -1922,7 +1932,7 @@ __device__ __forceinline__ void cone_body(const Geo& g, const Flux<R>& fl, const
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     R* const buf = lds + K::kAt + words + w * K::kBuf;
     uint32_t* const bufs = reinterpret_cast<uint32_t*>(buf + K::kFar + 128);
-    uint4 t = tiles[(size_t)cone * kWaves + w];
+    uint4 t = tiles[(size_t)slot0 + (size_t)b * kWaves + w];
     lds[lane] = (R)0;  // by every wave, before its own reads
     auto uni = [](uint32_t v) -> uint32_t { return __builtin_amdgcn_readfirstlane(v); };
     auto rsrc = [&](const uint4* p, uint32_t bytes) {
@@ -1937,7 +1947,7 @@ __device__ __forceinline__ void cone_body(const Geo& g, const Flux<R>& fl, const
     };
     const uint32_t levels = (uni(t.w) >> 8) & 255u, n = uni(t.w) >> 16;
     for (uint32_t i = w; i < n; i += kWaves) {
-        if (i >= kWaves) t = tiles[(size_t)more[cone] + i - kWaves];
+        if (i >= kWaves) t = tiles[(size_t)more[cone0 + b] + i - kWaves];
         const uint64_t off = (uint64_t)uni(t.x) | ((uint64_t)(uni(t.y) & 0xFFFFu) << 32);
         const uint32_t word0 = uni(t.y) >> 16, k = uni(t.w) & 255u, pk = uni(t.z);
         const uint32_t cnt = pk & 127u, np = (pk >> 7) & 15u, nex = (pk >> 11) & 255u, nfar = pk >> 19;
@@ -2045,11 +2055,11 @@ template <typename R, int kWaves, bool kGeneral>
 __global__ void __launch_bounds__(64 * kWaves) k_sweep_cone(Geo g, Flux<R> fl, const uint4* __restrict__ blob,
                                                             const uint4* __restrict__ tiles,
                                                             const uint32_t* __restrict__ more,
-                                                            const uint32_t* __restrict__ sel, uint32_t cone0,
-                                                            uint32_t words, int lvl,
+                                                            const uint32_t* __restrict__ sel, uint32_t slot0,
+                                                            uint32_t cone0, uint32_t words, int lvl,
                                                             PassTab pt) {
     const uint32_t b = pass_item(pt, blockIdx.x);
-    cone_body<R, kWaves, kGeneral>(g, fl, blob, tiles, more, cone0 + (sel ? sel[b] : b), words, lvl);
+    cone_body<R, kWaves, kGeneral>(g, fl, blob, tiles, more, sel ? sel[b] : b, slot0, cone0, words, lvl);
 }
 
 // One problem's grouped launch inside a packed launch: everything the grouped
@@ -2070,7 +2080,7 @@ struct GroupJob {
     const uint4* tiles;
     const uint32_t* more;
     const uint32_t* sel;
-    uint32_t cone0, words;
+    uint32_t slot0, cone0, words;
     int lvl;
     uint32_t start, blocks;
     PassTab pt;
@@ -2105,29 +2115,29 @@ __global__ void __launch_bounds__(64 * kWaves) k_sweep_cone_pack(const PackArgs<
     fl.sa = J.sa;
     fl.thr = J.thr;
     const uint32_t b = pass_item(J.pt, i);
-    cone_body<R, kWaves, kGeneral>(g, fl, J.blob, J.tiles, J.more, J.cone0 + (J.sel ? J.sel[b] : b), J.words, J.lvl);
+    cone_body<R, kWaves, kGeneral>(g, fl, J.blob, J.tiles, J.more, J.sel ? J.sel[b] : b, J.slot0, J.cone0, J.words, J.lvl);
 }
 
 // Tiles of every cone: counted (kFill = false, one wave each: the tiles past
 // the first `waves` and blob units of each cone, the far entries of each task
 // of the list, and the largest cone of each group into words) or written (four
-// waves each, a tile the wave). gk0[gmap[cone]]: first level set of the cone's
-// group.
+// waves each, a tile the wave). ginfo[gmap[cone]]: the cone's group.
 template <typename R, bool kFill>
 __global__ void __launch_bounds__(kFill ? 256 : 64) k_cone_tiles(
     Geo g, double inv_aref, const uint32_t* __restrict__ sorted, const uint32_t* __restrict__ xpos,
     const uint64_t* __restrict__ uoff, const uint32_t* __restrict__ up, const uint32_t* __restrict__ fstart,
     const uint8_t* __restrict__ nups, uint8_t* __restrict__ fars, const uint4* __restrict__ desc,
-    const uint32_t* __restrict__ list, const uint32_t* __restrict__ gmap, const uint32_t* __restrict__ gk0,
+    const uint32_t* __restrict__ list, const uint32_t* __restrict__ gmap, const uint4* __restrict__ ginfo,
     uint32_t* __restrict__ ct, uint64_t* __restrict__ cu, uint32_t* __restrict__ words,
-    const uint32_t* __restrict__ ts, const uint64_t* __restrict__ us, uint32_t waves, uint4* __restrict__ blob,
+    const uint32_t* __restrict__ ts, const uint64_t* __restrict__ us, uint32_t slots, uint4* __restrict__ blob,
     uint4* __restrict__ tiles, uint32_t* __restrict__ more) {
     using K = ConeShape<R>;
     extern __shared__ uint32_t memb[];  // kFill: the cone's tasks
     __shared__ uint32_t fs[kMaxGroup + 1], zs[kMaxGroup + 1];
     const uint32_t w = blockIdx.x, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint4 d0 = desc[2 * (size_t)w], d1 = desc[2 * (size_t)w + 1];
-    const uint32_t k0 = gk0[gmap[w]], levels = d0.y, N = (uint32_t)g.N;
+    const uint4 G = ginfo[gmap[w]];
+    const uint32_t k0 = G.x, waves = G.y, slot = G.z + (w - G.w) * waves, levels = d0.y, N = (uint32_t)g.N;
     uint32_t total = 0;
     for (uint32_t ph = 0; ph < levels; ph++) total += desc_count(d0, d1, (int)ph);
     if (kFill) {
@@ -2143,7 +2153,7 @@ __global__ void __launch_bounds__(kFill ? 256 : 64) k_cone_tiles(
     const uint32_t lo = fstart[k0], cone = d0.x;
     uint32_t seg = 0, nt = 0, all = 0;
     uint64_t off = kFill ? us[w] : 0;
-    const uint32_t more0 = kFill ? gridDim.x * waves + ts[w] : 0u;
+    const uint32_t more0 = kFill ? slots + ts[w] : 0u;
     if (kFill) all = waves + ts[w + 1] - ts[w];  // the tiles, if more than `waves`
     for (uint32_t ph = 0; ph < levels; ph++) {
         const uint32_t m = desc_count(d0, d1, (int)ph);
@@ -2175,7 +2185,7 @@ __global__ void __launch_bounds__(kFill ? 256 : 64) k_cone_tiles(
                     uint4* const lists = base + np * cnt + units16(cnt, 8);
                     uint4* const extra = lists + units16(nf, 4);
                     if (lane == 0)
-                        tiles[nt < waves ? w * (size_t)waves + nt : (size_t)more0 + nt - waves] = make_uint4(
+                        tiles[nt < waves ? slot + nt : (size_t)more0 + nt - waves] = make_uint4(
                             (uint32_t)off, (uint32_t)(off >> 32) | ((K::kAt + seg + b + a) << 16),
                             cnt | (np << 7) | (ne << 11) | (nf << 19), ph | (levels << 8) | (all << 16));
                     if (lane >= a && lane < e) {
@@ -2221,7 +2231,7 @@ __global__ void __launch_bounds__(kFill ? 256 : 64) k_cone_tiles(
     }
     __syncthreads();
     if (threadIdx.x < waves) {
-        uint4* const t = tiles + w * (size_t)waves + threadIdx.x;
+        uint4* const t = tiles + slot + threadIdx.x;
         if (threadIdx.x < nt) t->w = (t->w & 0xFFFFu) | (nt << 16);
         else *t = make_uint4(0u, 0u, 0u, (levels << 8) | (nt << 16));
     }
@@ -2233,13 +2243,15 @@ __global__ void __launch_bounds__(kFill ? 256 : 64) k_cone_tiles(
 // each group are summed into gcount and gblocks (gmap: group of each cone).
 __global__ void __launch_bounds__(64) k_cone_active(Geo g, int lvl, const uint4* __restrict__ blob,
                                                     const uint4* __restrict__ tiles,
-                                                    const uint32_t* __restrict__ more, uint32_t waves,
+                                                    const uint32_t* __restrict__ more,
+                                                    const uint4* __restrict__ ginfo,
                                                     const uint32_t* __restrict__ gmap, uint32_t* kept,
                                                     uint32_t* gcount, uint32_t* gblocks) {
-    const uint32_t tn = tiles[blockIdx.x * (size_t)waves].w >> 16;
+    const uint4 G = ginfo[gmap[blockIdx.x]];
+    const uint32_t waves = G.y, slot = G.z + (blockIdx.x - G.w) * waves, tn = tiles[slot].w >> 16;
     uint32_t n = 0;
     for (uint32_t i = 0; i < tn; i++) {
-        const uint4 t = tiles[i < waves ? blockIdx.x * (size_t)waves + i : (size_t)more[blockIdx.x] + i - waves];
+        const uint4 t = tiles[i < waves ? slot + i : (size_t)more[blockIdx.x] + i - waves];
         const uint32_t cnt = t.z & 127u;
         const uint32_t hdr = blob[((uint64_t)t.x | ((uint64_t)(t.y & 0xFFFFu) << 32)) + min(threadIdx.x, cnt - 1u)].x;
         n += (uint32_t)__popcll(__ballot(threadIdx.x < cnt && g.level[hdr & kCellMask] >= lvl));
@@ -2932,11 +2944,14 @@ struct ssw_sweep {
         uint32_t desc0, ndesc;
         PassTab passes;  // cone ranges of the build passes, relative to desc0
         uint32_t words;  // tasks of its largest cone
+        int waves;       // of its workgroups
+        uint32_t slot0;  // its first tile descriptor
     };
     std::vector<Group> groups;
     uint4 *d_coneblob = nullptr, *d_conetiles = nullptr;
     uint32_t* d_conemore = nullptr;
     uint32_t* d_gmap = nullptr;                     // group of each cone
+    uint4* d_ginfo = nullptr;                       // per group: first level set, waves, first tile, first cone
     uint32_t ndesc = 0;
     // restricted sweeps (level >= 1): kept cones, active tasks per group
     std::vector<uint32_t*> d_gsel_l;
@@ -3411,12 +3426,12 @@ int plan_replay(ssw_sweep* s, int lvl) {
     return SSW_OK;
 }
 
-// A kernel of the grouped replay by roots per workgroup and whether it is a
+// A kernel of the grouped replay by waves per workgroup and whether it is a
 // restricted sweep or has offsets.
-#define SSW_CONE_KERNEL(name, R, roots, general)                                       \
-    ((roots) == 32 ? ((general) ? name<R, 4, true> : name<R, 4, false>)                \
-     : (roots) == 64 ? ((general) ? name<R, 8, true> : name<R, 8, false>)              \
-                     : ((general) ? name<R, 16, true> : name<R, 16, false>))
+#define SSW_CONE_KERNEL(name, R, waves, general)                                       \
+    ((waves) == 4 ? ((general) ? name<R, 4, true> : name<R, 4, false>)                 \
+     : (waves) == 8 ? ((general) ? name<R, 8, true> : name<R, 8, false>)               \
+                    : ((general) ? name<R, 16, true> : name<R, 16, false>))
 
 // The grouped replay of full sweeps (compiled replay, group_request >= 2):
 // groups of m consecutive level sets; in each group, from its last level set
@@ -3447,7 +3462,10 @@ int build_groups_t(ssw_sweep* s, const uint32_t* sorted) {
             if (narrow) mk = kMaxGroup;
         }
         const int lv = std::min(s->kmax, k0 + mk) - k0;
-        s->groups.push_back({k0, lv, 0u, 0u, PassTab{}, 0u});
+        uint32_t widest = 0;
+        for (int k = k0; k < k0 + lv; k++) widest = std::max(widest, fs[k + 1] - fs[k]);
+        const int waves = ConeShape<R>::waves(T) * (lv > kGroupLevels && widest <= (uint32_t)T * kCus ? 2 : 1);
+        s->groups.push_back({k0, lv, 0u, 0u, PassTab{}, 0u, std::min(waves, 16), 0u});
         mmax = std::max(mmax, lv);
         k0 += mk;
     }
@@ -3461,7 +3479,7 @@ int build_groups_t(ssw_sweep* s, const uint32_t* sorted) {
     }
     uint8_t *todo = nullptr, *flags = nullptr, *lvlflag = nullptr, *tmp = nullptr;
     uint32_t *roots = nullptr, *ctl = nullptr, *bounds = nullptr, *perm = nullptr;  // ctl: cursor, fail, selected
-    uint32_t *list = nullptr, *k0s = nullptr, *words = nullptr, *ct = nullptr, *ts = nullptr;
+    uint32_t *list = nullptr, *words = nullptr, *ct = nullptr, *ts = nullptr;
     uint64_t *cu = nullptr, *us = nullptr, *ucnt = nullptr, *uoff = nullptr;
     uint32_t* up = nullptr;
     uint8_t* fars = nullptr;
@@ -3469,7 +3487,7 @@ int build_groups_t(ssw_sweep* s, const uint32_t* sorted) {
     uint4 *meta = nullptr, *desc_rm = nullptr, *desc = nullptr;
     Defer cleanup{[&] {
         for (uint8_t** p : {&todo, &flags, &lvlflag, &tmp}) dfree(s, *p);
-        for (uint32_t** p : {&roots, &ctl, &bounds, &perm, &list, &k0s, &words, &ct, &ts}) dfree(s, *p);
+        for (uint32_t** p : {&roots, &ctl, &bounds, &perm, &list, &words, &ct, &ts}) dfree(s, *p);
         for (uint64_t** p : {&cu, &us, &ucnt, &uoff}) dfree(s, *p);
         dfree(s, up);
         dfree(s, fars);
@@ -3645,11 +3663,18 @@ int build_groups_t(ssw_sweep* s, const uint32_t* sorted) {
     TRY(dalloc(s, &perm, ndesc));
     HIP_TRY(hipMemcpyAsync(perm, hperm.data(), hperm.size() * 4, hipMemcpyHostToDevice, s->stream));
     k_permute_desc<<<grid_for(ndesc), kBlock, 0, s->stream>>>(desc_rm, perm, desc, ndesc);
-    std::vector<uint32_t> hk0(ng), hw(ng);
-    for (size_t i = 0; i < ng; i++) hk0[i] = (uint32_t)s->groups[i].k0;
-    TRY(dalloc(s, &k0s, ng));
+    std::vector<uint32_t> hw(ng);
+    std::vector<uint4> ginfo(ng);
+    uint32_t slots = 0;
+    for (size_t i = 0; i < ng; i++) {
+        ssw_sweep::Group& gr = s->groups[i];
+        gr.slot0 = slots;
+        slots += gr.ndesc * (uint32_t)gr.waves;
+        ginfo[i] = make_uint4((uint32_t)gr.k0, (uint32_t)gr.waves, gr.slot0, gr.desc0);
+    }
+    TRY(dalloc(s, &s->d_ginfo, ng));
     TRY(dalloc(s, &words, ng));
-    HIP_TRY(hipMemcpyAsync(k0s, hk0.data(), ng * 4, hipMemcpyHostToDevice, s->stream));
+    HIP_TRY(hipMemcpyAsync(s->d_ginfo, ginfo.data(), ng * sizeof(uint4), hipMemcpyHostToDevice, s->stream));
     k_fill_u32<<<grid_for((int64_t)ng), kBlock, 0, s->stream>>>(words, 0u, (int64_t)ng);
     TRY(dalloc(s, &ct, (size_t)ndesc + 1));
     TRY(dalloc(s, &ts, (size_t)ndesc + 1));
@@ -3658,11 +3683,10 @@ int build_groups_t(ssw_sweep* s, const uint32_t* sorted) {
     HIP_TRY(hipMemsetAsync(ct + ndesc, 0, 4, s->stream));
     HIP_TRY(hipMemsetAsync(cu + ndesc, 0, 8, s->stream));
     const double inv_aref = 1.0 / s->aref;
-    const uint32_t waves = (uint32_t)ConeShape<R>::waves(T);
     TRY(dalloc(s, &fars, (size_t)hctl[0]));
     k_cone_tiles<R, false><<<ndesc, 64, 0, s->stream>>>(g, inv_aref, sorted, s->d_xpos, uoff, up, s->d_fstart,
-                                                        s->d_nup, fars, desc, list, s->d_gmap, k0s, ct, cu, words,
-                                                        nullptr, nullptr, waves, nullptr, nullptr, nullptr);
+                                                        s->d_nup, fars, desc, list, s->d_gmap, s->d_ginfo, ct, cu,
+                                                        words, nullptr, nullptr, slots, nullptr, nullptr, nullptr);
     HIP_TRY(hipGetLastError());
     size_t t1 = 0, t2 = 0;
     HIP_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, t1, ct, ts, (int)ndesc + 1, s->stream));
@@ -3680,13 +3704,17 @@ int build_groups_t(ssw_sweep* s, const uint32_t* sorted) {
     for (size_t i = 0; i < ng; i++) {
         s->groups[i].words = hw[i];
         members = std::max<size_t>(members, hw[i]);
-        lds = std::max(lds, ConeShape<R>::bytes(T, hw[i]));
+        lds = std::max(lds, ConeShape<R>::bytes(s->groups[i].waves, hw[i]));
     }
     if (lds > 65536)  // at most 116 KB (a cone of kConeCap members and 128 roots, FP64)
         for (const bool general : {false, true}) {
-            HIP_TRY(hipFuncSetAttribute((const void*)SSW_CONE_KERNEL(k_sweep_cone, R, T, general),
+            HIP_TRY(hipFuncSetAttribute((const void*)SSW_CONE_KERNEL(k_sweep_cone, R, 16, general),
                                         hipFuncAttributeMaxDynamicSharedMemorySize, 160 << 10));
-            HIP_TRY(hipFuncSetAttribute((const void*)SSW_CONE_KERNEL(k_sweep_cone_pack, R, T, general),
+            HIP_TRY(hipFuncSetAttribute((const void*)SSW_CONE_KERNEL(k_sweep_cone, R, 8, general),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 << 10));
+            HIP_TRY(hipFuncSetAttribute((const void*)SSW_CONE_KERNEL(k_sweep_cone_pack, R, 16, general),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 << 10));
+            HIP_TRY(hipFuncSetAttribute((const void*)SSW_CONE_KERNEL(k_sweep_cone_pack, R, 8, general),
                                         hipFuncAttributeMaxDynamicSharedMemorySize, 160 << 10));
         }
     dfree(s, tmp);
@@ -3696,19 +3724,17 @@ int build_groups_t(ssw_sweep* s, const uint32_t* sorted) {
     dfree(s, cu);
     dfree(s, ct);
     TRY(dalloc(s, &s->d_coneblob, (size_t)units));
-    TRY(dalloc(s, &s->d_conetiles, (size_t)ndesc * waves + more));
+    TRY(dalloc(s, &s->d_conetiles, (size_t)slots + more));
     TRY(dalloc(s, &s->d_conemore, (size_t)ndesc));
     k_cone_tiles<R, true><<<ndesc, 256, members * 4, s->stream>>>(
-        g, inv_aref, sorted, s->d_xpos, nullptr, nullptr, s->d_fstart, s->d_nup, fars, desc, list, s->d_gmap, k0s,
-        nullptr, nullptr, words, ts, us, waves, s->d_coneblob, s->d_conetiles, s->d_conemore);
+        g, inv_aref, sorted, s->d_xpos, nullptr, nullptr, s->d_fstart, s->d_nup, fars, desc, list, s->d_gmap,
+        s->d_ginfo, nullptr, nullptr, words, ts, us, slots, s->d_coneblob, s->d_conetiles, s->d_conemore);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(s->stream));
     return SSW_OK;
 }
 
 // sorted: the tasks in schedule order; s->d_xpos, s->d_fstart and s->d_nup held.
-int group_waves(const ssw_sweep* s) { return ConeShape<float>::waves(s->group_block); }
-
 int build_groups(ssw_sweep* s, const uint32_t* sorted) {
     return s->fp32 ? build_groups_t<float>(s, sorted) : build_groups_t<double>(s, sorted);
 }
@@ -3717,7 +3743,7 @@ void free_groups(ssw_sweep* s) {
     s->groups.clear();
     s->group_tasks = 0;
     s->group_fallback = false;
-    for (uint4** p : {&s->d_coneblob, &s->d_conetiles}) dfree(s, *p);
+    for (uint4** p : {&s->d_coneblob, &s->d_conetiles, &s->d_ginfo}) dfree(s, *p);
     for (uint32_t** p : {&s->d_conemore, &s->d_gmap, &s->d_gcount, &s->d_gbase, &s->d_gblocks, &s->d_pbound, &s->d_gf_kept,
                          &s->d_gf_pos, &s->d_gf_pbval})
         dfree(s, *p);
@@ -4007,7 +4033,7 @@ int make_group_list(ssw_sweep* s, int lvl) {
             return fail(SSW_ERR_INVALID, "grouped replay: restricted-sweep scratch missing");
         k_fill_u32<<<1, 1, 0, s->stream>>>(kept + nd, 0u, 1);
         k_cone_active<<<nd, 64, 0, s->stream>>>(g, lvl, s->d_coneblob, s->d_conetiles, s->d_conemore,
-                                                (uint32_t)group_waves(s), s->d_gmap, kept, s->d_gcount, s->d_gblocks);
+                                                s->d_ginfo, s->d_gmap, kept, s->d_gcount, s->d_gblocks);
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipcub::DeviceScan::ExclusiveSum(scan_tmp, tb, kept, pos, (int)nd + 1, s->stream));
         k_place_cone<<<grid_for(nd), kBlock, 0, s->stream>>>(kept, pos, s->d_gmap, s->d_gbase, s->d_gsel_l[lvl], nd);
@@ -4105,9 +4131,9 @@ int make_list(ssw_sweep* s, int lvl) {
 }
 
 template <typename R, typename... Args>
-void launch_cones(int roots, bool general, uint32_t blocks, uint32_t words, hipStream_t st, Args... args) {
-    hipLaunchKernelGGL(SSW_CONE_KERNEL(k_sweep_cone, R, roots, general), dim3(blocks),
-                       dim3(64 * ConeShape<R>::waves(roots)), ConeShape<R>::bytes(roots, words), st, args...);
+void launch_cones(int waves, bool general, uint32_t blocks, uint32_t words, hipStream_t st, Args... args) {
+    hipLaunchKernelGGL(SSW_CONE_KERNEL(k_sweep_cone, R, waves, general), dim3(blocks), dim3(64 * waves),
+                       ConeShape<R>::bytes(waves, words), st, args...);
 }
 
 // Launches one item of sweep level lvl's replay plan on stream st: a group
@@ -4137,9 +4163,9 @@ void launch_item_t(ssw_sweep* s, const Geo& g, const Flux<R>& fl, int lvl, const
     }
     if (it.group) {
         const ssw_sweep::Group& gr = s->groups[it.tab];
-        launch_cones<R>(s->group_block, !all || fl.offI != nullptr, all ? gr.ndesc : s->gblocks[lvl][it.tab], gr.words,
+        launch_cones<R>(gr.waves, !all || fl.offI != nullptr, all ? gr.ndesc : s->gblocks[lvl][it.tab], gr.words,
                         st, g, fl, s->d_coneblob, s->d_conetiles, s->d_conemore,
-                        all ? nullptr : s->d_gsel_l[lvl] + gr.desc0, gr.desc0, gr.words, all ? 0 : lvl,
+                        all ? nullptr : s->d_gsel_l[lvl] + gr.desc0, gr.slot0, gr.desc0, gr.words, all ? 0 : lvl,
                         all ? gr.passes : s->gpass_l[lvl][it.tab]);
         return;
     }
@@ -4371,10 +4397,13 @@ int run_step(ssw_sweep* s, double* elapsed) {
 // packed into shared launches (k_sweep_cone_pack).
 //
 // The handles' sweeps are aligned by index: sweep i of every handle whose
-// step has more than i sweeps runs together. Inside sweep i, the t-th items of
+// step has more than i sweeps runs together. Inside sweep i, the next items of
 // the handles' replay plans are launched together: grouped items of handles
-// with the same transport precision and group block go into one packed launch
-// (up to kMaxPack per launch), other items are launched alone. Each handle's
+// with the same transport precision and workgroups go into one packed launch
+// (up to kMaxPack per launch), other items are launched alone. The handle with
+// the most items left says which workgroups are next; taking the t-th items
+// of all, whatever their workgroups, made two launches of many (eight handles,
+// 2.44 ms a step instead of 1.65). Each handle's
 // items still run in its plan's order (everything is on one stream), and a
 // packed workgroup computes exactly what it computes in a launch of its own,
 // so every handle's results are bitwise those of stepping it alone.
@@ -4403,6 +4432,7 @@ GroupJob<R> group_job(ssw_sweep* s, int lvl, const ssw_sweep::ReplayItem& it, ui
     J.blob = s->d_coneblob;
     J.tiles = s->d_conetiles;
     J.more = s->d_conemore;
+    J.slot0 = gr.slot0;
     J.cone0 = gr.desc0;
     J.sel = all ? nullptr : s->d_gsel_l[lvl] + gr.desc0;
     J.words = gr.words;
@@ -4414,7 +4444,7 @@ GroupJob<R> group_job(ssw_sweep* s, int lvl, const ssw_sweep::ReplayItem& it, ui
     return J;
 }
 
-// A packed launch under construction: jobs of one precision and group block.
+// A packed launch under construction: jobs of one precision and workgroup.
 template <typename R>
 struct Pack {
     PackArgs<R> a{};  // value-initialised: no jobs yet
@@ -4422,7 +4452,7 @@ struct Pack {
 };
 
 template <typename R>
-void flush_pack(Pack<R>& p, int roots, hipStream_t st) {
+void flush_pack(Pack<R>& p, int waves, hipStream_t st) {
     if (p.a.n <= 0) return;
     uint32_t words = 0;
     bool general = false;
@@ -4430,31 +4460,31 @@ void flush_pack(Pack<R>& p, int roots, hipStream_t st) {
         words = std::max(words, p.a.job[k].words);
         general = general || p.a.job[k].lvl > 0 || p.a.job[k].offI;
     }
-    hipLaunchKernelGGL(SSW_CONE_KERNEL(k_sweep_cone_pack, R, roots, general), dim3(p.grid),
-                       dim3(64 * ConeShape<R>::waves(roots)), ConeShape<R>::bytes(roots, words), st, p.a);
+    hipLaunchKernelGGL(SSW_CONE_KERNEL(k_sweep_cone_pack, R, waves, general), dim3(p.grid), dim3(64 * waves),
+                       ConeShape<R>::bytes(waves, words), st, p.a);
     p.a.n = 0;
     p.grid = 0;
 }
 
 template <typename R>
-void add_job(Pack<R>& p, const GroupJob<R>& J, int roots, hipStream_t st) {
-    if (p.a.n >= kMaxPack) flush_pack<R>(p, roots, st);
+void add_job(Pack<R>& p, const GroupJob<R>& J, int waves, hipStream_t st) {
+    if (p.a.n >= kMaxPack) flush_pack<R>(p, waves, st);
     GroupJob<R> j = J;
     j.start = p.grid;
     p.grid += (J.blocks + kXcds - 1) / kXcds * kXcds;
     p.a.job[p.a.n++] = j;
 }
 
-// Packs keyed by (precision, group block).
+// Packs keyed by (precision, waves of a workgroup).
 struct Packs {
     Pack<float> f[3];
     Pack<double> d[3];
-    static int slot(int roots) { return roots == 32 ? 0 : roots == 64 ? 1 : 2; }
+    static int slot(int waves) { return waves == 4 ? 0 : waves == 8 ? 1 : 2; }
     void flush(hipStream_t st) {
-        const int roots[3] = {32, 64, 128};
+        const int waves[3] = {4, 8, 16};
         for (int k = 0; k < 3; k++) {
-            flush_pack<float>(f[k], roots[k], st);
-            flush_pack<double>(d[k], roots[k], st);
+            flush_pack<float>(f[k], waves[k], st);
+            flush_pack<double>(d[k], waves[k], st);
         }
     }
 };
@@ -4464,7 +4494,7 @@ void packed_item(ssw_sweep* s, const Geo& g, int lvl, const ssw_sweep::ReplayIte
     if (it.group == 1) {
         uint32_t nblk = 0;
         const GroupJob<R> J = group_job<R>(s, lvl, it, &nblk);
-        if (nblk) add_job<R>(pk, J, s->group_block, st);
+        if (nblk) add_job<R>(pk, J, s->groups[it.tab].waves, st);
         return;
     }
     launch_item_t<R>(s, g, make_flux<R>(s), lvl, it, st);
@@ -4569,23 +4599,30 @@ int step_pack(BatchSweep* bs, int n, double* elapsed) {
     for (int h = 0; h < n; h++) graphs = graphs && bs[h].s->graphs_on;
     const int dev = bs[0].s->device;
     for (size_t i = 0; i < sweeps; i++) {
-        // sweep i of every handle: the t-th plan items together, then the
-        // handles' periodic sources and chemistry together
+        // sweep i of every handle: plan items together where their workgroups
+        // are of the same waves, those of the handle with the most items left
+        // first, then the handles' periodic sources and chemistry together
         const std::function<void()> enqueue = [&]() {
             Packs pk;
-            size_t items = 0;
-            for (int h = 0; h < n; h++)
-                if (i < bs[h].order.size()) items = std::max(items, bs[h].s->plan[bs[h].order[i]].size());
-            for (size_t t = 0; t < items; t++) {
+            std::vector<size_t> at(n, 0);
+            auto left = [&](int h) {
+                return i < bs[h].order.size() ? bs[h].s->plan[bs[h].order[i]].size() - at[h] : (size_t)0;
+            };
+            auto item = [&](int h) -> const ssw_sweep::ReplayItem& { return bs[h].s->plan[bs[h].order[i]][at[h]]; };
+            auto waves = [&](int h) { return item(h).group == 1 ? bs[h].s->groups[item(h).tab].waves : 0; };
+            for (;;) {
+                int lead = 0;
+                for (int h = 1; h < n; h++)
+                    if (left(h) > left(lead)) lead = h;
+                if (!left(lead)) break;
+                const int wv = waves(lead);
                 for (int h = 0; h < n; h++) {
+                    if (!left(h) || waves(h) != wv) continue;
                     BatchSweep& b = bs[h];
-                    if (i >= b.order.size()) continue;
-                    const int lvl = b.order[i];
-                    if (t >= b.s->plan[lvl].size()) continue;
-                    const ssw_sweep::ReplayItem& it = b.s->plan[lvl][t];
-                    const int k = Packs::slot(b.s->group_block);
-                    if (b.s->fp32) packed_item<float>(b.s, b.g, lvl, it, pk.f[k], st);
-                    else packed_item<double>(b.s, b.g, lvl, it, pk.d[k], st);
+                    const int lvl = b.order[i], k = Packs::slot(wv);
+                    if (b.s->fp32) packed_item<float>(b.s, b.g, lvl, item(h), pk.f[k], st);
+                    else packed_item<double>(b.s, b.g, lvl, item(h), pk.d[k], st);
+                    at[h]++;
                 }
                 pk.flush(st);
             }
@@ -5953,16 +5990,16 @@ int ssw_load_checkpoint(ssw_sweep* s, const void* buf, int64_t bytes) {
 extern "C++" {
 namespace {
 // Workgroups of the grouped replay kernel one CU holds at once (0 if unknown),
-// with the LDS of the group of the largest cone.
+// for the group of the most cones.
 template <typename R>
 int group_blocks_per_cu(const ssw_sweep* s) {
-    uint32_t words = 0;
-    for (const ssw_sweep::Group& gr : s->groups) words = std::max(words, gr.words);
+    const ssw_sweep::Group* most = &s->groups[0];
+    for (const ssw_sweep::Group& gr : s->groups)
+        if (gr.ndesc > most->ndesc) most = &gr;
     int n = 0;
-    const int roots = s->group_block;
     const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &n, SSW_CONE_KERNEL(k_sweep_cone, R, roots, false), 64 * ConeShape<R>::waves(roots),
-        ConeShape<R>::bytes(roots, words));
+        &n, SSW_CONE_KERNEL(k_sweep_cone, R, most->waves, false), 64 * most->waves,
+        ConeShape<R>::bytes(most->waves, most->words));
     return e == hipSuccess ? n : 0;
 }
 }  // namespace
