@@ -2297,6 +2297,7 @@ struct ChemArgs {
     double* species_ts;
     double* prev_rate;
     double* change_ts;
+    double* photon;          // sum of the incoming rates (SI); -1: not solved by the last sweep
     const double* vol;
     const double* size;
     double max_ts;
@@ -2453,19 +2454,24 @@ __global__ void __launch_bounds__(kBlock) k_chemistry(const ChemJobs<R, kJobs> j
         if (__lane_id() == __ffsll((long long)__ballot(1)) - 1 && m)
             atomicAdd(ca.active, (unsigned long long)__popcll(m));
     }
-    if (lev < lvl) return;
+    if (lev < lvl) {
+        ca.photon[c] = -1.0;
+        return;
+    }
     const double dt = ca.max_ts * ssw::powi(0.5, lev);
     const uint32_t ps = g.pslot[c];
     const bool has_p = ps != kNone && fl.P;
     const double src = ca.src[c];
-    double rate = 0.0;
+    double rate = 0.0, incoming = 0.0;
 #pragma unroll 6
     for (int d = 0; d < g.D; d++) {
         const double inc = (double)fl.I[iidx(fl, g.N, (uint32_t)d, (uint32_t)c)] * ca.lref;
         // current periodic source (k_periodic ran after the sweep)
         const double per = has_p ? (double)fl.P[(size_t)d * g.Nper + ps] * ca.lref : 0.0;
         rate += (inc + src) + per;  // sum over d of Site::get_rate, in direction order
+        incoming += inc;            // the photon rate, as k_fluxes sums it
     }
+    ca.photon[c] = incoming;
     double rel;
     if (fabs(rate) < fabs(ca.thr)) {
         rel = 0.0;
@@ -2674,12 +2680,15 @@ __global__ void k_levels(Geo g, const double* change_ts, uint8_t* level, double 
 // other, 2.46 ms like this.
 template <typename R, bool kAll>
 __global__ void __launch_bounds__(1024) k_fluxes(Geo g, Flux<R> fl, double lref, double* I_out, double* O_out,
-                                                 double* P_out, double* photon_rate, const uint32_t* rate_idx) {
+                                                 double* P_out, double* photon_rate, const uint32_t* rate_idx,
+                                                 const double* missing) {
     __shared__ double sum[kFluxCells];
     const uint32_t lane = threadIdx.x % kFluxCells;
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / kFluxCells);  // uniform: scalar direction loads
     const int64_t c0 = (int64_t)blockIdx.x * kFluxCells + lane;
     const bool valid = c0 < g.N;
+    // only cells without a rate: where none of the workgroup's is
+    if (missing && !__ballot(valid && missing[c0] < 0.0)) return;
     const uint32_t c = valid ? (uint32_t)c0 : 0u;
     const int d0 = (int)w * kFluxDirs;
     double A[kFluxDirs];
@@ -2737,20 +2746,6 @@ __global__ void __launch_bounds__(1024) k_fluxes(Geo g, Flux<R> fl, double lref,
     }
     // rate_idx: the caller's index of each internal cell (NULL: internal order)
     if (w == 0 && valid) photon_rate[rate_idx ? rate_idx[c] : c] = sum[lane];
-}
-
-// The photon rate from the incoming rates that the last sweep stored, the same
-// sum as k_fluxes': only where that sweep solved every cell and no rate was
-// clamped (ssw_sweep::rates_current). Bound: one read of I, coalesced
-// (262144 cells x 84 directions FP32: 88 MB; the pull takes 2.46 ms).
-template <typename R>
-__global__ void k_rate_sum(Geo g, Flux<R> fl, double lref, double* photon_rate, const uint32_t* rate_idx) {
-    const int64_t c = (int64_t)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-    if (c >= g.N) return;
-    double total = 0.0;
-#pragma unroll 12
-    for (int d = 0; d < g.D; d++) total += (double)fl.I[iidx(fl, g.N, (uint32_t)d, (uint32_t)c)] * lref;
-    photon_rate[rate_idx ? rate_idx[c] : c] = total;
 }
 
 // rotate_directions_system (src/sweep/direction/mod.rs:158-175), state part,
@@ -3138,6 +3133,7 @@ struct ssw_sweep {
     // of the last step: chemistry updates, then the 3 limiting processes' counts
     unsigned long long* d_active = nullptr;
     double* d_photon = nullptr;                     // photon rates of a download (internal order)
+    double* d_rate = nullptr;                       // photon rates from the last sweep's chemistry
     uint32_t* d_chemq = nullptr;                    // k_chemistry's queue (ChemArgs::queue)
     uint8_t* d_level = nullptr;
     void *d_X = nullptr, *d_I = nullptr, *d_P = nullptr;
@@ -3146,11 +3142,12 @@ struct ssw_sweep {
     // every source, and every rate that a checkpoint brought, is >= 0: no
     // incoming rate is negative, so none is clamped when it is stored
     bool nonneg = false;
-    // the stored incoming rates are the pull sums over the current X: the last
-    // sweep solved every cell (a cell solved before its upwind neighbours were
-    // solved again keeps an older sum), nothing was clamped and no rotation
-    // has left offsets
+    // the incoming rates that the last sweep's cells read are the pull sums
+    // over the current X: nothing was clamped and no rotation has left offsets
+    // (other cells may have been solved before their upwind neighbours were
+    // solved again: their d_rate is -1)
     bool rates_current = false;
+    bool rates_partial = false;                     // the last sweep did not solve every cell
     unsigned long long* d_fail = nullptr;
     double lref = 1.0;
     TimestepState ts;
@@ -3346,28 +3343,34 @@ void launch_fluxes(ssw_sweep* s, const Geo& g, double* dI, double* dO, double* d
     const unsigned lanes = (unsigned)(kFluxCells * ((s->D + kFluxDirs - 1) / kFluxDirs));
     if (s->fp32)
         k_fluxes<float, true><<<nb, lanes, 0, s->stream>>>(g, make_flux<float>(s), s->lref, dI, dO, dP, nullptr,
-                                                           nullptr);
+                                                           nullptr, nullptr);
     else
         k_fluxes<double, true><<<nb, lanes, 0, s->stream>>>(g, make_flux<double>(s), s->lref, dI, dO, dP, nullptr,
-                                                            nullptr);
+                                                            nullptr, nullptr);
 }
 
-void launch_photon_rate(ssw_sweep* s, const Geo& g, double* out, const uint32_t* ridx) {
+// The photon rates in d_rate: as the last sweep's chemistry summed them from
+// the incoming rates it read (ssw_sweep::rates_current; 262144 cells x 84
+// directions: a sum of its own from the stored rates took 0.10 ms, a pull of
+// all 2.46), pulled for the cells that sweep did not solve. Without current
+// rates all are pulled, into `out` (at their caller indices with ridx).
+int photon_rates(ssw_sweep* s, const Geo& g, double* out, const uint32_t* ridx) {
     const unsigned nb = (unsigned)((s->N + kFluxCells - 1) / kFluxCells);
     const unsigned lanes = (unsigned)(kFluxCells * ((s->D + kFluxDirs - 1) / kFluxDirs));
+    const double* missing = nullptr;
     if (s->rates_current) {
-        // one wave per workgroup: a small grid still spreads over the CUs
-        if (s->fp32)
-            k_rate_sum<float><<<nb, kFluxCells, 0, s->stream>>>(g, make_flux<float>(s), s->lref, out, ridx);
-        else
-            k_rate_sum<double><<<nb, kFluxCells, 0, s->stream>>>(g, make_flux<double>(s), s->lref, out, ridx);
-    } else if (s->fp32) {
-        k_fluxes<float, false><<<nb, lanes, 0, s->stream>>>(g, make_flux<float>(s), s->lref, nullptr, nullptr,
-                                                            nullptr, out, ridx);
-    } else {
-        k_fluxes<double, false><<<nb, lanes, 0, s->stream>>>(g, make_flux<double>(s), s->lref, nullptr, nullptr,
-                                                             nullptr, out, ridx);
+        if (!s->rates_partial) return SSW_OK;
+        missing = out = s->d_rate;
+        ridx = nullptr;
     }
+    if (s->fp32)
+        k_fluxes<float, false><<<nb, lanes, 0, s->stream>>>(g, make_flux<float>(s), s->lref, nullptr, nullptr, nullptr,
+                                                            out, ridx, missing);
+    else
+        k_fluxes<double, false><<<nb, lanes, 0, s->stream>>>(g, make_flux<double>(s), s->lref, nullptr, nullptr,
+                                                             nullptr, out, ridx, missing);
+    HIP_TRY(hipGetLastError());
+    return SSW_OK;
 }
 
 int set_need_all(ssw_sweep* s, uint32_t v) {
@@ -4378,6 +4381,7 @@ ChemArgs chem_args(ssw_sweep* s) {
     ca.sa = s->d_sa;
     ca.species_ts = s->d_sts;
     ca.prev_rate = s->d_prev;
+    ca.photon = s->d_rate;
     ca.change_ts = s->d_change;
     ca.vol = s->d_vol;
     ca.size = s->d_size;
@@ -4413,10 +4417,11 @@ void launch_chemistry(const ChemJob<R>* j, int n, hipStream_t st) {
     k_chemistry_tail<R, kJobs><<<dim3((unsigned)std::min<int64_t>((cells + 3) / 4, 2048), n), 64, 0, st>>>(a);
 }
 
-// ssw_sweep::rates_current after the sweeps of `order`.
-bool rates_are_current(const ssw_sweep* s, const std::vector<int>& order) {
+// ssw_sweep::rates_current and rates_partial after the sweeps of `order`.
+void rates_after(ssw_sweep* s, const std::vector<int>& order) {
     const int last = order.back();
-    return s->nonneg && !s->rotated && (last == 0 || s->list_full[last]);
+    s->rates_current = s->nonneg && !s->rotated;
+    s->rates_partial = last != 0 && !s->list_full[last];
 }
 
 template <typename R>
@@ -4482,7 +4487,7 @@ int run_step(ssw_sweep* s, double* elapsed) {
         s->sweeps_last++;
     }
     HIP_TRY(hipGetLastError());
-    s->rates_current = rates_are_current(s, order);
+    rates_after(s, order);
     double el = s->ts.current_max_timestep();
     s->ts.advance();
     k_levels<<<gcells, kBlock, 0, s->stream>>>(g, s->d_change, s->d_level, s->p.max_timestep,
@@ -4782,7 +4787,7 @@ int step_pack(BatchSweep* bs, int n, double* elapsed) {
     }
     for (int h = 0; h < n; h++) {
         ssw_sweep* s = bs[h].s;
-        s->rates_current = rates_are_current(s, bs[h].order);
+        rates_after(s, bs[h].order);
         const double el = s->ts.current_max_timestep();
         s->ts.advance();
         k_levels<<<grid_for(s->N), kBlock, 0, st>>>(bs[h].g, s->d_change, s->d_level, s->p.max_timestep,
@@ -5021,6 +5026,7 @@ void free_state(ssw_sweep* s) {
     dfree(s, s->d_change);
     dfree(s, s->d_chemq);
     dfree(s, s->d_photon);
+    dfree(s, s->d_rate);
     dfree(s, s->d_X);
     dfree(s, s->d_I);
     dfree(s, s->d_P);
@@ -5601,6 +5607,7 @@ int ssw_upload_state(ssw_sweep* s, const double* density, const double* xhii, co
     TRY(dalloc(s, (uint8_t**)&s->d_sa, n * sa_size(s)));
     TRY(dalloc(s, &s->d_sts, n));
     TRY(dalloc(s, &s->d_prev, n));
+    TRY(dalloc(s, &s->d_rate, n));
     TRY(dalloc(s, &s->d_change, n));
     TRY(dalloc(s, &s->d_chemq, (size_t)n + 2));
     TRY(dalloc(s, (uint8_t**)&s->d_X, (size_t)s->D * n * es));
@@ -5743,10 +5750,9 @@ int ssw_download(ssw_sweep* s, double* x, double* T, double* sts, double* photon
     want(s->d_sts, sts);
     want(s->d_change, change);
     if (photon) {
-        if (!s->d_photon) TRY(dalloc(s, &s->d_photon, s->N));
-        launch_photon_rate(s, make_geo(s), s->d_photon, nullptr);
-        HIP_TRY(hipGetLastError());
-        want(s->d_photon, photon);
+        if (!s->rates_current && !s->d_photon) TRY(dalloc(s, &s->d_photon, s->N));
+        TRY(photon_rates(s, make_geo(s), s->d_photon, nullptr));
+        want(s->rates_current ? s->d_rate : s->d_photon, photon);
     }
     return fetch_outputs(s, src, dst, s->d_level, level);
 }
@@ -5767,13 +5773,10 @@ int ssw_download_noalloc(ssw_sweep* s, double* x, double* T, double* sts, double
     if (change) TRY(noalloc_out(s, s->d_change, change, stage));
     if (level) TRY(noalloc_out(s, s->d_level, level, stage));
     if (photon) {
-        // the photon rate of every cell lands at its caller index in the staging buffer
-        const Geo g = make_geo(s);
-        double* pr = (double*)stage;
-        const uint32_t* ridx = s->permuted ? s->d_inv : nullptr;
-        launch_photon_rate(s, g, pr, ridx);
-        HIP_TRY(hipGetLastError());
-        HIP_TRY(hipMemcpyAsync(photon, pr, (size_t)n * 8, hipMemcpyDeviceToHost, s->stream));
+        // pulled: the photon rate of every cell lands at its caller index in the staging buffer
+        TRY(photon_rates(s, make_geo(s), (double*)stage, s->permuted ? s->d_inv : nullptr));
+        if (s->rates_current) TRY(noalloc_out(s, s->d_rate, photon, stage));
+        else HIP_TRY(hipMemcpyAsync(photon, stage, (size_t)n * 8, hipMemcpyDeviceToHost, s->stream));
     }
     HIP_TRY(hipStreamSynchronize(s->stream));
     return SSW_OK;
