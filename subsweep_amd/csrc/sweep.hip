@@ -3554,14 +3554,16 @@ int plan_replay(ssw_sweep* s, int lvl) {
      : (waves) == 8 ? ((general) ? name<R, 8, true> : name<R, 8, false>)               \
                     : ((general) ? name<R, 16, true> : name<R, 16, false>))
 
+void free_groups(ssw_sweep* s);
+
 // The grouped replay of full sweeps (compiled replay, group_request >= 2):
 // groups of m consecutive level sets; in each group, from its last level set
 // down to its first, the level set's tasks in no cone yet become roots, in
 // blocks of kGroupT, whose cones are built (k_cone) and compiled into tiles
-// (k_cone_tiles). If a cone exceeds the LDS capacity or the task list its
-// bound, there are no groups, and sweeps keep the per-level replay.
+// (k_cone_tiles). If a cone exceeds the LDS capacity, the task list its bound
+// or the tiles the free memory, there are no groups.
 template <typename R>
-int build_groups_t(ssw_sweep* s, const uint32_t* sorted) {
+int build_groups_t(ssw_sweep* s, const uint32_t* sorted, uint32_t narrow_group) {
     const int m = s->group_request;
     const size_t DN = (size_t)s->D * s->N;
     const std::vector<uint32_t>& fs = s->full_start;
@@ -3569,7 +3571,7 @@ int build_groups_t(ssw_sweep* s, const uint32_t* sorted) {
     const size_t desc_cap = DN / T + (size_t)s->kmax + 1;  // at most ceil(width / T) per level set
     const size_t list_cap = DN + DN / 4 + (1u << 20);
     // groups of m level sets, of kMaxGroup where that many consecutive level
-    // sets hold at most kNarrowGroup tasks each (the narrow ends of the
+    // sets hold at most narrow_group tasks each (the narrow ends of the
     // graph, whose cones stay small); per pass r the level set
     // k0 + levels - 1 - r of each group that has it (pass 0: the last level
     // sets, all tasks roots)
@@ -3579,7 +3581,7 @@ int build_groups_t(ssw_sweep* s, const uint32_t* sorted) {
         int mk = m;
         if (m < kMaxGroup && k0 + kMaxGroup <= s->kmax) {
             bool narrow = true;
-            for (int k = k0; narrow && k < k0 + kMaxGroup; k++) narrow = fs[k + 1] - fs[k] <= kNarrowGroup;
+            for (int k = k0; narrow && k < k0 + kMaxGroup; k++) narrow = fs[k + 1] - fs[k] <= narrow_group;
             if (narrow) mk = kMaxGroup;
         }
         const int lv = std::min(s->kmax, k0 + mk) - k0;
@@ -3652,7 +3654,7 @@ int build_groups_t(ssw_sweep* s, const uint32_t* sorted) {
     }
     // blocks of group g in pass r: [rstart[r][g], rstart[r][g] + rcount[r][g]) of the pass-major descriptors
     std::vector<std::vector<uint32_t>> rstart(mmax, std::vector<uint32_t>(ng, 0u)), rcount(rstart);
-    uint32_t ndesc = 0;
+    uint32_t ndesc = 0, hctl[2] = {0, 0};
     std::vector<uint4> hmeta;
     std::vector<uint8_t> hflag(s->kmax);
     std::vector<int> hlv;
@@ -3711,12 +3713,11 @@ int build_groups_t(ssw_sweep* s, const uint32_t* sorted) {
         k_cone<<<nb, kConeThreads, 0, s->stream>>>(uoff, up, s->d_fstart, meta, rl, todo, list, (uint32_t)list_cap, ctl,
                                                    desc_rm + 2 * (size_t)ndesc, ctl + 1);
         HIP_TRY(hipGetLastError());
+        HIP_TRY(hipMemcpyAsync(hctl, ctl, 8, hipMemcpyDeviceToHost, s->stream));
         HIP_TRY(hipStreamSynchronize(s->stream));  // meta is reallocated by the next pass
         ndesc += nb;
+        if (hctl[1] != 0) break;
     }
-    uint32_t hctl[2] = {0, 0};
-    HIP_TRY(hipMemcpyAsync(hctl, ctl, 8, hipMemcpyDeviceToHost, s->stream));
-    HIP_TRY(hipStreamSynchronize(s->stream));
     dfree(s, meta);
     dfree(s, tmp);
     dfree(s, bounds);
@@ -3726,7 +3727,7 @@ int build_groups_t(ssw_sweep* s, const uint32_t* sorted) {
     dfree(s, flags);
     dfree(s, ctl);
     dfree(s, todo);
-    if (hctl[1] != 0) {  // a cone or the list did not fit: per-level replay
+    if (hctl[1] != 0) {  // a cone or the list did not fit
         s->groups.clear();
         s->group_fallback = true;
         return SSW_OK;
@@ -3844,6 +3845,18 @@ int build_groups_t(ssw_sweep* s, const uint32_t* sorted) {
     dfree(s, uoff);
     dfree(s, cu);
     dfree(s, ct);
+    // The tiles of FP32 cones can take more than the per-level replay's planes
+    // (measured: up to 35 B more per task, clustered cells x 16 directions). Where
+    // they and the state do not fit beside what is held, that replay runs.
+    size_t free_b = 0, total_b = 0;
+    HIP_TRY(hipMemGetInfo(&free_b, &total_b));
+    const size_t tile_bytes = 16 * ((size_t)units + slots + more) + 4 * (size_t)ndesc;
+    const size_t state_bytes = 2 * (DN + (size_t)s->D * s->Nper) * sizeof(R) + 128 * (size_t)s->N;
+    if (tile_bytes + state_bytes + total_b / 32 > free_b) {
+        free_groups(s);
+        s->group_fallback = true;
+        return SSW_OK;
+    }
     TRY(dalloc(s, &s->d_coneblob, (size_t)units));
     TRY(dalloc(s, &s->d_conetiles, (size_t)slots + more));
     TRY(dalloc(s, &s->d_conemore, (size_t)ndesc));
@@ -3855,9 +3868,18 @@ int build_groups_t(ssw_sweep* s, const uint32_t* sorted) {
     return SSW_OK;
 }
 
+// Groups with kNarrowGroup, or, where a cone or the list does not fit, a
+// quarter of it (cones of 8 level sets of few directions reach further: 262144
+// cells x 16 directions fit with 2048 only, 2.07 ms a frame); if that does not
+// fit either, sweeps keep the per-level replay.
 // sorted: the tasks in schedule order; s->d_xpos, s->d_fstart and s->d_nup held.
 int build_groups(ssw_sweep* s, const uint32_t* sorted) {
-    return s->fp32 ? build_groups_t<float>(s, sorted) : build_groups_t<double>(s, sorted);
+    for (uint32_t narrow : {kNarrowGroup, kNarrowGroup / 4}) {
+        s->group_fallback = false;
+        TRY(s->fp32 ? build_groups_t<float>(s, sorted, narrow) : build_groups_t<double>(s, sorted, narrow));
+        if (!s->group_fallback) break;
+    }
+    return SSW_OK;
 }
 
 void free_groups(ssw_sweep* s) {
@@ -6228,7 +6250,7 @@ int64_t ssw_estimate_device_bytes(const ssw_sweep_parameters* p, int64_t n, int6
     // a permuted grid), level starts, chunk table
     const int64_t grid = (n + 1) * 4 + F * 32 + F * 4 + n * 16 + n * 4 + num_periodic_cells * 8 + F * 4 + n +
                          (n + 4) * 4 + n * 8 + DN / kChunk * 40 + (1 << 20);
-    const int64_t sched = comp ? DN * (16 + rs + kPlanes * es + 4) + ovf : DN * 16;  // compiled: + positions
+    int64_t sched = comp ? DN * (16 + rs + kPlanes * es + 4) + ovf : DN * 16;  // compiled: + positions
     // compiled replay with the default grouped replay (4 level sets, 64 roots):
     // group lists instead of active-set lists, and the cone build's scratch
     const int64_t grp = comp ? group_bytes(DN, n, L, kGroupT) : 0;
@@ -6238,7 +6260,14 @@ int64_t ssw_estimate_device_bytes(const ssw_sweep_parameters* p, int64_t n, int6
     // with the sorted order and overflow starts
     const int64_t ostart = comp ? DN * 4 + ovf : 0;
     int64_t build = std::max(DN * 20 + ostart, std::max(DN * 16 + ostart, sched + DN * 4 + ostart));
-    if (comp) build = std::max(build, sched + grp + DN * 5);
+    // the grouped replay's tiles: planes, indices and far list of every solved
+    // task (measured: up to 131 B in FP32, 174 B in FP64) and the
+    // positions, in place of `sched`
+    const int64_t cones = std::min(DN + DN / 4 + (1 << 20), DN + 3 * DN / 4) * (rs == 4 ? 140 : 190) + DN * 4;
+    if (comp) {
+        build = std::max(build, std::max(sched, cones) + grp + DN * 5);
+        sched = std::max(sched, cones);
+    }
     // afterwards: schedule, active-set (or group) lists, state, the photon-rate
     // and the optional outputs' downloads
     const int64_t run = sched + lists + n * 8 * 9 + n * 4 + 2 * DN * rs + D * num_periodic_cells * rs + n * 40;

@@ -38,3 +38,25 @@ def test_cones_bitwise_equal_geometric(name, precision, levels, roots, hip_avail
             for u, v in zip(a.transport_state(), b.transport_state()):
                 assert np.array_equal(u.view(np.uint8), v.view(np.uint8)), f"step {step}"
             assert np.array_equal(a.results().level, b.results().level)
+
+
+def test_cones_of_few_directions_stay_grouped(hip_available):
+    """262144 cells x 16 directions: level sets of 3700 tasks on average, whose
+    cones of 8 level sets do not all fit; the groups are then built with 8 only
+    where level sets are narrow. Its memory stays within the estimate."""
+    from subsweep_amd import workloads as W
+    from subsweep_amd.serve import estimate_device_bytes
+    pb = W.jittered_problem(64, 1.0, "6", 16, periodic=True, steps=2, precision=32)
+    with Sweep(pb.params, pb.grid, *pb.state(), transport_mode=N.TRANSPORT_MODE_GEOMETRIC) as a, \
+         Sweep(pb.params, pb.grid, *pb.state(), transport_mode=N.TRANSPORT_MODE_COMPILED) as b:
+        info = b.info()
+        assert info.group_fallback == 0 and info.group_tasks >= pb.grid.num_cells * 16
+        for step in range(2):
+            assert a.run_sweeps() == b.run_sweeps()
+            for u, v in zip(a.transport_state(), b.transport_state()):
+                assert np.array_equal(u.view(np.uint8), v.view(np.uint8)), f"step {step}"
+        b.results()
+    with Sweep(pb.params, pb.grid, *pb.state(), transport_mode=N.TRANSPORT_MODE_COMPILED) as b:
+        b.run_sweeps()
+        b.results()
+        assert b.info().peak_device_bytes <= estimate_device_bytes(pb, N.TRANSPORT_MODE_COMPILED)
