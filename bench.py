@@ -46,17 +46,17 @@ sys.path.insert(0, ROOT)
 
 PEAK_HBM_GBS = 8000.0
 KERNELS = {3: "k_sweep_rec (geometric replay: one launch per Kahn level set, all directions, 16 lanes per task)",
-           4: "k_sweep_group (compiled replay grouped: one launch per 4 consecutive Kahn level sets, one workgroup per "
-              "block of 64 root tasks solving their upwind cone level set by level set; with group levels 1, "
-              "k_sweep_comp: one launch per level set, one lane per task)"}
+           4: "k_sweep_cone (compiled replay grouped: one launch per 4 to 8 consecutive Kahn level sets, one workgroup "
+              "per block of 64 root tasks solving their upwind cone in tiles of up to 64 tasks, X between its level "
+              "sets through LDS; with group levels 1, k_sweep_comp: one launch per level set, one lane per task)"}
 
 
 def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
-DIR_KERNEL = ("k_sweep_dir (direction sweeps: one launch per sweep, one 512-lane workgroup per direction solving its "
-              "level sets in order with workgroup barriers only, recent upwind values from an LDS ring)")
+DIR_KERNEL = ("k_sweep_dir (direction sweeps: one launch per sweep, one workgroup per direction solving its level sets "
+              "in order in tiles of up to 64 tasks a wave, upwind values from LDS words that the schedule names)")
 
 
 def kernel_name(info) -> str:
@@ -71,26 +71,27 @@ def bytes_per_update(info, precision: int) -> float:
     return base + info.downwind_local * bl + info.downwind_periodic * bp + info.downwind_boundary * bb
 
 
-def occupancy(info) -> dict:
+def occupancy(info, precision: int) -> dict:
     """Waves of the dominant transport kernel per CU: launched (mean
     workgroups per launch x waves per workgroup / CUs) against what one CU
     can hold of this kernel at once (its register and LDS limits). The
-    direction sweeps launch one 8-wave workgroup per direction, and their
-    128 KiB LDS ring admits one workgroup per CU."""
+    direction sweeps launch one workgroup per direction, of 16 waves in FP32
+    and 12 in FP64, and their 128 KiB LDS ring admits one per CU."""
     cus = int(info.compute_units)
     if info.direction_sweeps:
         wg = int(info.num_directions)
-        launched = wg * 8 / cus if cus else None
+        waves = 16 if precision == 32 else 12
+        launched = wg * waves / cus if cus else None
         return {"kernel": "k_sweep_dir", "compute_units": cus, "workgroups_per_launch": wg,
-                "waves_per_workgroup": 8, "launched_waves_per_cu": launched, "limit_waves_per_cu": 8,
-                "frac": launched / 8 if launched else None}
+                "waves_per_workgroup": waves, "launched_waves_per_cu": launched, "limit_waves_per_cu": waves,
+                "frac": launched / waves if launched else None}
     if info.group_launches <= 0:
         return None
-    waves_per_wg = 2 * int(info.group_block) // 64
+    waves_per_wg = int(info.group_block) // 8  # as the widest groups have
     wg = info.group_workgroups / info.group_launches
     limit = int(info.group_blocks_per_cu) * waves_per_wg
     launched = wg * waves_per_wg / cus if cus else None
-    return {"kernel": "k_sweep_group", "compute_units": cus, "workgroups_per_launch": wg,
+    return {"kernel": "k_sweep_cone", "compute_units": cus, "workgroups_per_launch": wg,
             "waves_per_workgroup": waves_per_wg, "launched_waves_per_cu": launched,
             "limit_waves_per_cu": limit, "frac": launched / limit if (limit and launched) else None}
 
@@ -155,7 +156,7 @@ def run_gpu(pb, precision: int, steps: int, warmup: int, profile_steps: int = 3,
         "group_levels": int(info.group_levels),
         "group_block": int(info.group_block),
         "group_tasks_per_full_sweep": int(info.group_tasks),
-        "occupancy": occupancy(info),
+        "occupancy": occupancy(info, precision),
         "transport_mode": int(info.transport_mode),
         "info": info,
         "results": res,
