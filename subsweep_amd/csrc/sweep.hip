@@ -2434,6 +2434,11 @@ __device__ __forceinline__ void finish_chemistry(const ChemArgs& ca, int64_t c, 
 // the rate and the first attempt of the solver; cells whose full step is
 // rejected go to the queue of k_chemistry_tail, else a wave would last as long
 // as its slowest cell's sub-steps, one after the other.
+// The rates of kChemDirs directions are loaded together, the last ones clamped
+// to the last direction: with the loop unrolled six times, and its remainder
+// one dependent gather after the other, a frame of 2 M clustered cells x 84
+// directions took 89.4 ms, with 8, 12 and 16 at once 87.0, 87.4 and 87.5.
+constexpr int kChemDirs = 8;
 template <typename R, int kJobs>
 __global__ void __launch_bounds__(kBlock) k_chemistry(const ChemJobs<R, kJobs> jobs) {
     const ChemJob<R>& J = jobs.mine();
@@ -2463,13 +2468,25 @@ __global__ void __launch_bounds__(kBlock) k_chemistry(const ChemJobs<R, kJobs> j
     const bool has_p = ps != kNone && fl.P;
     const double src = ca.src[c];
     double rate = 0.0, incoming = 0.0;
-#pragma unroll 6
-    for (int d = 0; d < g.D; d++) {
-        const double inc = (double)fl.I[iidx(fl, g.N, (uint32_t)d, (uint32_t)c)] * ca.lref;
+    for (int d0 = 0; d0 < g.D; d0 += kChemDirs) {
+        R inc[kChemDirs], per[kChemDirs];
+#pragma unroll
+        for (int j = 0; j < kChemDirs; j++)
+            inc[j] = fl.I[iidx(fl, g.N, (uint32_t)min(d0 + j, g.D - 1), (uint32_t)c)];
         // current periodic source (k_periodic ran after the sweep)
-        const double per = has_p ? (double)fl.P[(size_t)d * g.Nper + ps] * ca.lref : 0.0;
-        rate += (inc + src) + per;  // sum over d of Site::get_rate, in direction order
-        incoming += inc;            // the photon rate, as k_fluxes sums it
+#pragma unroll
+        for (int j = 0; j < kChemDirs; j++) per[j] = (R)0;
+        if (has_p) {
+#pragma unroll
+            for (int j = 0; j < kChemDirs; j++) per[j] = fl.P[(size_t)min(d0 + j, g.D - 1) * g.Nper + ps];
+        }
+#pragma unroll
+        for (int j = 0; j < kChemDirs; j++) {
+            if (d0 + j >= g.D) break;
+            const double i = (double)inc[j] * ca.lref;
+            rate += (i + src) + (double)per[j] * ca.lref;  // sum over d of Site::get_rate, in direction order
+            incoming += i;                                 // the photon rate, as k_fluxes sums it
+        }
     }
     ca.photon[c] = incoming;
     double rel;
