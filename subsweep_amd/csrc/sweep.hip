@@ -54,6 +54,7 @@
 #include <algorithm>
 #include <array>
 #include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
@@ -3580,7 +3581,7 @@ void free_groups(ssw_sweep* s);
 // (k_cone_tiles). If a cone exceeds the LDS capacity, the task list its bound
 // or the tiles the free memory, there are no groups.
 template <typename R>
-int build_groups_t(ssw_sweep* s, const uint32_t* sorted, uint32_t narrow_group) {
+int build_groups_t(ssw_sweep* s, const uint32_t* sorted, uint32_t narrow_group, bool* retry) {
     const int m = s->group_request;
     const size_t DN = (size_t)s->D * s->N;
     const std::vector<uint32_t>& fs = s->full_start;
@@ -3864,19 +3865,27 @@ int build_groups_t(ssw_sweep* s, const uint32_t* sorted, uint32_t narrow_group) 
     dfree(s, ct);
     // The tiles of FP32 cones can take more than the per-level replay's planes
     // (measured: up to 35 B more per task, clustered cells x 16 directions). Where
-    // they and the state do not fit beside what is held, that replay runs.
+    // they and the state do not fit beside what is held, that replay runs. Freed
+    // memory comes back some time after the frees above (16.8 M cells: 57 GB were
+    // still missing), so where free memory is short, it is waited for, at most 2 s.
     size_t free_b = 0, total_b = 0;
-    HIP_TRY(hipMemGetInfo(&free_b, &total_b));
-    const size_t tile_bytes = 16 * ((size_t)units + slots + more) + 4 * (size_t)ndesc;
-    const size_t state_bytes = 2 * (DN + (size_t)s->D * s->Nper) * sizeof(R) + 128 * (size_t)s->N;
-    if (tile_bytes + state_bytes + total_b / 32 > free_b) {
+    const size_t need = 16 * ((size_t)units + slots + more) + 4 * (size_t)ndesc +
+                        2 * (DN + (size_t)s->D * s->Nper) * sizeof(R) + 128 * (size_t)s->N;
+    for (int k = 0; k < 100; k++) {
+        HIP_TRY(hipMemGetInfo(&free_b, &total_b));
+        if (need + total_b / 64 <= free_b) break;
+        std::this_thread::sleep_for(std::chrono::milliseconds(20));
+    }
+    int rc = need + total_b / 64 <= free_b ? dalloc(s, &s->d_coneblob, (size_t)units) : SSW_ERR_OOM;
+    if (rc == SSW_OK) rc = dalloc(s, &s->d_conetiles, (size_t)slots + more);
+    if (rc == SSW_OK) rc = dalloc(s, &s->d_conemore, (size_t)ndesc);
+    if (rc == SSW_ERR_OOM) {
         free_groups(s);
         s->group_fallback = true;
+        *retry = false;
         return SSW_OK;
     }
-    TRY(dalloc(s, &s->d_coneblob, (size_t)units));
-    TRY(dalloc(s, &s->d_conetiles, (size_t)slots + more));
-    TRY(dalloc(s, &s->d_conemore, (size_t)ndesc));
+    TRY(rc);
     k_cone_tiles<R, true><<<ndesc, 256, members * 4, s->stream>>>(
         g, inv_aref, sorted, s->d_xpos, nullptr, nullptr, s->d_fstart, s->d_nup, fars, desc, list, s->d_gmap,
         s->d_ginfo, nullptr, nullptr, words, ts, us, slots, s->d_coneblob, s->d_conetiles, s->d_conemore);
@@ -3892,9 +3901,11 @@ int build_groups_t(ssw_sweep* s, const uint32_t* sorted, uint32_t narrow_group) 
 // sorted: the tasks in schedule order; s->d_xpos, s->d_fstart and s->d_nup held.
 int build_groups(ssw_sweep* s, const uint32_t* sorted) {
     for (uint32_t narrow : {kNarrowGroup, kNarrowGroup / 4}) {
+        bool retry = true;
         s->group_fallback = false;
-        TRY(s->fp32 ? build_groups_t<float>(s, sorted, narrow) : build_groups_t<double>(s, sorted, narrow));
-        if (!s->group_fallback) break;
+        TRY(s->fp32 ? build_groups_t<float>(s, sorted, narrow, &retry)
+                    : build_groups_t<double>(s, sorted, narrow, &retry));
+        if (!s->group_fallback || !retry) break;
     }
     return SSW_OK;
 }
