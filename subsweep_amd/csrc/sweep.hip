@@ -411,7 +411,11 @@ __device__ __forceinline__ void task_faces(const Geo& g, const Flux<R>& fl, bool
 
 // Every local face c->nb needs a mirror face nb->c with exactly the negated
 // normal, which makes the upwind/downwind classification of the pair agree.
-__global__ void k_check_mirror(Geo g, unsigned long long* bad) {
+// uneven: faces that one side repeats more often than the other. nb's upwind
+// counter is then decremented more often than it counts: it may become ready
+// before another of its upwind neighbours, so that only the replays that read
+// upwind values from memory, one level set at a time, run on such grids.
+__global__ void k_check_mirror(Geo g, unsigned long long* bad, unsigned long long* uneven) {
     int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= g.N) return;
     for (uint32_t f = g.off[c]; f < g.off[c + 1]; f++) {
@@ -423,14 +427,20 @@ __global__ void k_check_mirror(Geo g, unsigned long long* bad) {
             continue;
         }
         double4 a = g.geo[f];
-        bool found = false;
+        uint32_t mirrors = 0, same = 0;
         for (uint32_t h = g.off[nb]; h < g.off[nb + 1]; h++) {
             uint32_t hk = g.nk[h];
             if ((hk >> 30) != kKindLocal || (int64_t)(hk & kNbrMask) != c) continue;
             double4 b = g.geo[h];
-            if (b.x == -a.x && b.y == -a.y && b.z == -a.z) found = true;
+            if (b.x == -a.x && b.y == -a.y && b.z == -a.z) mirrors++;
         }
-        if (!found) atomicAdd(bad, 1ull);
+        if (mirrors == 0) atomicAdd(bad, 1ull);
+        for (uint32_t h = g.off[c]; h < g.off[c + 1]; h++) {
+            if (g.nk[h] != nk) continue;
+            double4 b = g.geo[h];
+            if (b.x == a.x && b.y == a.y && b.z == a.z) same++;
+        }
+        if (mirrors != same) atomicAdd(uneven, 1ull);
     }
 }
 
@@ -541,7 +551,9 @@ __global__ void k_count(Geo g, int lvl) {
 // Bound: the chain of a level set (queue, face range, faces, counters, one
 // barrier). With kLds the counters lie in LDS as bytes (at most 127 upwind
 // faces; an inactive cell's byte starts at 255 and never reaches 0), up to
-// kLayerCells cells; else they are decremented in memory. The queues are in
+// kLayerCells cells; else they are decremented in memory, as on grids whose
+// faces repeat unevenly: a byte decremented below 0 would borrow from the next
+// cell's, a counter in memory only never becomes ready again. The queues are in
 // LDS, longer ones go on in `spill` (2 N entries a direction). A launch for
 // every level set of all directions took 5 to 30 us a level set: 32768 cells x
 // 84 directions 4.5 -> 1.3 ms, 262144 cells 23 -> 9.8 ms, 2 M clustered 184 ->
@@ -3105,6 +3117,7 @@ struct ssw_sweep {
     double aref = 1.0;
     double dw[3] = {0, 0, 0};
     int64_t ovf_total = 0;
+    bool uneven_faces = false;                      // k_check_mirror's `uneven`
     // upwind counters, held only while a layering or a count runs
     uint32_t *d_cnt = nullptr, *d_need = nullptr;
     // full schedule
@@ -3161,7 +3174,8 @@ struct ssw_sweep {
     // incoming rate is negative, so none is clamped when it is stored
     bool nonneg = false;
     // the incoming rates that the last sweep's cells read are the pull sums
-    // over the current X: nothing was clamped and no rotation has left offsets
+    // over the current X: nothing was clamped, no rotation has left offsets,
+    // and no cell was solved before an upwind neighbour (uneven_faces)
     // (other cells may have been solved before their upwind neighbours were
     // solved again: their d_rate is -1)
     bool rates_current = false;
@@ -3463,7 +3477,7 @@ int kahn_layering(ssw_sweep* s, int lvl, int64_t expected, uint32_t* d_depth, in
     const Geo g = make_geo(s);
     k_fill_u32<<<grid_for((int64_t)kcap + 2), kBlock, 0, s->stream>>>(hist, 0u, (int64_t)kcap + 2);
     k_count<<<grid_for((int64_t)DN), kBlock, 0, s->stream>>>(g, lvl);
-    if (s->N <= (int64_t)kLayerCells)
+    if (s->N <= (int64_t)kLayerCells && !s->uneven_faces)
         k_layers<true><<<s->D, 1024, 0, s->stream>>>(g, kcap, d_depth, spill, hist + 2, hist);
     else
         k_layers<false><<<s->D, 1024, 0, s->stream>>>(g, kcap, d_depth, spill, hist + 2, hist);
@@ -4066,7 +4080,7 @@ int build_schedule(ssw_sweep* s) {
     TRY(dalloc(s, &d_depth, DN));
     TRY(kahn_layering(s, 0, (int64_t)DN, d_depth, &s->kmax, &s->full_start));
     Geo g = make_geo(s);
-    if (s->compiled && s->dir_sweeps) {
+    if (s->compiled && s->dir_sweeps && !s->uneven_faces) {
         TRY(s->fp32 ? build_dir_schedule_t<float>(s, d_depth) : build_dir_schedule_t<double>(s, d_depth));
         return init_replay(s);
     }
@@ -4101,7 +4115,10 @@ int build_schedule(ssw_sweep* s) {
         TRY(dalloc(s, &s->d_xpos, DN));
         k_invert<<<grid_for((int64_t)DN), kBlock, 0, s->stream>>>(d_sorted, s->d_xpos, (uint32_t)DN);
         HIP_TRY(hipGetLastError());
-        if (s->group_request >= 2) {
+        if (s->uneven_faces) {
+            dfree(s, s->d_nup);
+            s->group_fallback = s->group_request >= 2;
+        } else if (s->group_request >= 2) {
             TRY(build_groups(s, d_sorted));
             dfree(s, s->d_nup);
             if (!s->groups.empty()) return init_replay(s);
@@ -4470,7 +4487,7 @@ void launch_chemistry(const ChemJob<R>* j, int n, hipStream_t st) {
 // ssw_sweep::rates_current and rates_partial after the sweeps of `order`.
 void rates_after(ssw_sweep* s, const std::vector<int>& order) {
     const int last = order.back();
-    s->rates_current = s->nonneg && !s->rotated;
+    s->rates_current = s->nonneg && !s->rotated && !s->uneven_faces;
     s->rates_partial = last != 0 && !s->list_full[last];
 }
 
@@ -5201,10 +5218,10 @@ int build_direction_graph(ssw_sweep* s, bool choose_mode) {
     const size_t DN = (size_t)s->D * n;
     unsigned long long* d_stats = nullptr;
     Defer cleanup{[&] { dfree(s, d_stats); }};
-    TRY(dalloc(s, &d_stats, 5));
-    HIP_TRY(hipMemsetAsync(d_stats, 0, 5 * 8, s->stream));
+    TRY(dalloc(s, &d_stats, 6));
+    HIP_TRY(hipMemsetAsync(d_stats, 0, 6 * 8, s->stream));
     Geo g = make_geo(s);
-    if (choose_mode) k_check_mirror<<<grid_for(n), kBlock, 0, s->stream>>>(g, d_stats);
+    if (choose_mode) k_check_mirror<<<grid_for(n), kBlock, 0, s->stream>>>(g, d_stats, d_stats + 5);
     const bool tiles = (s->dir_sweeps || s->group_request >= 2) &&
                        (choose_mode ? s->mode_request != SSW_TRANSPORT_MODE_GEOMETRIC : s->compiled);
     if (tiles) TRY(dalloc(s, &s->d_nup, DN));
@@ -5212,13 +5229,14 @@ int build_direction_graph(ssw_sweep* s, bool choose_mode) {
                    kFluxCells * ((s->D + kFluxDirs - 1) / kFluxDirs), 0, s->stream>>>(g, d_stats + 1, s->d_cnt,
                                                                                       s->d_nup);
     HIP_TRY(hipGetLastError());
-    unsigned long long hb[5] = {0, 0, 0, 0, 0};
+    unsigned long long hb[6] = {0, 0, 0, 0, 0, 0};
     HIP_TRY(hipMemcpyAsync(hb, d_stats, sizeof(hb), hipMemcpyDeviceToHost, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
     dfree(s, d_stats);
     if (hb[0] != 0)
         return fail(SSW_ERR_GRID, std::to_string(hb[0]) +
                                       " local faces have no mirror face with the exactly negated normal");
+    if (choose_mode) s->uneven_faces = hb[5] != 0;
     for (int k = 0; k < 3; k++) s->dw[k] = (double)hb[k + 1] / ((double)n * s->D);
     s->ovf_total = (int64_t)hb[4];
     if (!choose_mode) {
