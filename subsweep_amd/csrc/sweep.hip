@@ -3101,6 +3101,7 @@ struct ssw_sweep {
     // grid
     int64_t N = 0, F = 0, Nper = 0;
     bool have_grid = false, have_state = false;
+    bool have_schedule = false;                     // the schedule is whole (a failed rotation may leave none)
     // internal cell order: internal index perm[c] for caller's cell c (Morton
     // order of the positions given with ssw_set_cell_positions), inv = perm^-1
     std::vector<double> pos;
@@ -4061,13 +4062,14 @@ int build_dir_schedule_t(ssw_sweep* s, uint32_t*& d_depth) {
 
 int init_replay(ssw_sweep* s);
 int setup_overflow(ssw_sweep* s);
+void free_schedule(ssw_sweep* s);
 
 // The full schedule, once per grid: Kahn layering of the whole graph, each
 // task's depth, a stable sort by depth of the tasks in (direction, cell)
 // order, then the compiled or geometric per-task data in that order, and the
-// chunk table of the compaction.
+// chunk table of the compaction. A graph with a cycle leaves the schedule that
+// was there as it is (have_schedule); from then on it is replaced.
 int build_schedule(ssw_sweep* s) {
-    free_groups(s);
     const size_t DN = (size_t)s->D * s->N;
     // sort the tasks by depth, stable over t = d*N + c (double-buffered: four
     // DN-word arrays and a small temporary)
@@ -4078,7 +4080,12 @@ int build_schedule(ssw_sweep* s) {
         dfree(s, d_tmp);
     }};
     TRY(dalloc(s, &d_depth, DN));
-    TRY(kahn_layering(s, 0, (int64_t)DN, d_depth, &s->kmax, &s->full_start));
+    int depth = 0;
+    std::vector<uint32_t> starts;
+    TRY(kahn_layering(s, 0, (int64_t)DN, d_depth, &depth, &starts));
+    free_schedule(s);
+    s->kmax = depth;
+    s->full_start = std::move(starts);
     Geo g = make_geo(s);
     if (s->compiled && s->dir_sweeps && !s->uneven_faces) {
         TRY(s->fp32 ? build_dir_schedule_t<float>(s, d_depth) : build_dir_schedule_t<double>(s, d_depth));
@@ -4193,6 +4200,7 @@ int init_replay(ssw_sweep* s) {
     s->runtab.assign(L, std::vector<uint4>());
     s->plan.assign(L, std::vector<ssw_sweep::ReplayItem>());
     TRY(plan_replay(s, 0));
+    s->have_schedule = true;
     return SSW_OK;
 }
 
@@ -5101,11 +5109,37 @@ void free_state(ssw_sweep* s) {
     dfree(s, s->d_offP);
 }
 
-void free_grid(ssw_sweep* s) {
+// Everything that build_schedule makes.
+void free_schedule(ssw_sweep* s) {
+    s->have_schedule = false;
     drop_all_lists(s);
     for (uint32_t*& p : s->d_idx) dfree(s, p);
     for (uint4*& p : s->d_runtab) dfree(s, p);
     free_groups(s);
+    dfree(s, s->d_fstart);
+    dfree(s, s->d_dirblob);
+    dfree(s, s->d_dirtiles);
+    dfree(s, s->d_dirinfo);
+    dfree(s, s->d_dircell);
+    dfree(s, s->d_dirsa);
+    dfree(s, s->d_dirlev);
+    dfree(s, s->d_recs);
+    dfree(s, s->d_hdr);
+    dfree(s, s->d_A);
+    dfree(s, s->d_planes);
+    dfree(s, s->d_ovf_start);
+    dfree(s, s->d_ovf);
+    dfree(s, s->d_xpos);
+    dfree(s, s->d_chunks);
+    dfree(s, s->d_first_chunk);
+    dfree(s, s->d_ccount);
+    dfree(s, s->d_coff);
+    dfree(s, s->d_cstart);
+    dfree(s, s->d_scan_tmp);
+}
+
+void free_grid(ssw_sweep* s) {
+    free_schedule(s);
     dfree(s, s->d_off);
     dfree(s, s->d_inv);
     dfree(s, s->d_perm);
@@ -5120,27 +5154,7 @@ void free_grid(ssw_sweep* s) {
     dfree(s, s->d_pgeo);
     dfree(s, s->d_cnt);
     dfree(s, s->d_level);
-    dfree(s, s->d_fstart);
-    dfree(s, s->d_dirblob);
-    dfree(s, s->d_dirtiles);
-    dfree(s, s->d_dirinfo);
-    dfree(s, s->d_dircell);
-    dfree(s, s->d_dirsa);
-    dfree(s, s->d_dirlev);
     dfree(s, s->d_nup);
-    dfree(s, s->d_recs);
-    dfree(s, s->d_hdr);
-    dfree(s, s->d_A);
-    dfree(s, s->d_planes);
-    dfree(s, s->d_ovf_start);
-    dfree(s, s->d_ovf);
-    dfree(s, s->d_xpos);
-    dfree(s, s->d_chunks);
-    dfree(s, s->d_first_chunk);
-    dfree(s, s->d_ccount);
-    dfree(s, s->d_coff);
-    dfree(s, s->d_cstart);
-    dfree(s, s->d_scan_tmp);
 }
 
 // Overflow entries of the per-level replay's planes (s->ovf_total of them).
@@ -5757,22 +5771,52 @@ int ssw_rotate_directions(ssw_sweep* s, const double* matrix) {
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipStreamSynchronize(s->stream));
     }
+    const std::vector<double> before = s->dirs;
+    const std::array<double, 3> dw{s->dw[0], s->dw[1], s->dw[2]};
+    const int64_t ovf_total = s->ovf_total;
     std::vector<double> kept;
     rotate_table(matrix, s->dirs, kept);
-    HIP_TRY(hipMemcpyAsync(s->d_dirs, s->dirs.data(), s->dirs.size() * 8, hipMemcpyHostToDevice, s->stream));
     // the dependency graph and schedule of the rotated directions
-    drop_all_lists(s);
-    s->rates_current = false;
-    TRY(dalloc(s, &s->d_cnt, DN));
-    TRY(build_direction_graph(s, false));
-    s->rotated = true;
-    if (s->have_state) {
-        TRY(dalloc(s, &d_kept, kept.size()));
-        HIP_TRY(hipMemcpyAsync(d_kept, kept.data(), kept.size() * 8, hipMemcpyHostToDevice, s->stream));
-        TRY(s->fp32 ? rotate_state_t<float>(s, d_kept, dI, dO, dP) : rotate_state_t<double>(s, d_kept, dI, dO, dP));
-        TRY(set_need_all(s, 1u));
+    auto build = [&]() -> int {
+        HIP_TRY(hipMemcpyAsync(s->d_dirs, s->dirs.data(), s->dirs.size() * 8, hipMemcpyHostToDevice, s->stream));
+        TRY(dalloc(s, &s->d_cnt, DN));
+        return build_direction_graph(s, false);
+    };
+    int rc = build();
+    if (rc != SSW_OK && s->have_schedule) {
+        // the rotated graph has a cycle, or its layering did not fit: the
+        // handle stays as it was
+        const std::string why = g_err;
+        dfree(s, s->d_cnt);
+        dfree(s, s->d_nup);
+        s->dirs = before;
+        for (int k = 0; k < 3; k++) s->dw[k] = dw[k];
+        s->ovf_total = ovf_total;
+        HIP_TRY(hipMemcpyAsync(s->d_dirs, s->dirs.data(), s->dirs.size() * 8, hipMemcpyHostToDevice, s->stream));
+        HIP_TRY(hipStreamSynchronize(s->stream));
+        return fail(rc, why);
     }
-    HIP_TRY(hipStreamSynchronize(s->stream));
+    auto turn = [&]() -> int {  // the state with them
+        s->rotated = true;
+        s->rates_current = false;
+        if (s->have_state) {
+            TRY(dalloc(s, &d_kept, kept.size()));
+            HIP_TRY(hipMemcpyAsync(d_kept, kept.data(), kept.size() * 8, hipMemcpyHostToDevice, s->stream));
+            TRY(s->fp32 ? rotate_state_t<float>(s, d_kept, dI, dO, dP) : rotate_state_t<double>(s, d_kept, dI, dO, dP));
+            TRY(set_need_all(s, 1u));
+        }
+        HIP_TRY(hipStreamSynchronize(s->stream));
+        return SSW_OK;
+    };
+    if (rc == SSW_OK) rc = turn();
+    if (rc != SSW_OK) {  // no schedule, or a state that is not its own: later calls are refused
+        const std::string why = g_err;
+        (void)hipStreamSynchronize(s->stream);
+        free_state(s);
+        free_grid(s);
+        s->have_grid = s->have_state = false;
+        return fail(rc, why);
+    }
     return SSW_OK;
 }
 
