@@ -3171,9 +3171,10 @@ struct ssw_sweep {
     void *d_X = nullptr, *d_I = nullptr, *d_P = nullptr;
     void *d_offI = nullptr, *d_offP = nullptr;      // rate offsets after a rotation (Flux::offI / offP)
     bool rotated = false;                           // directions rotated since ssw_create
-    // every source, and every rate that a checkpoint brought, is >= 0: no
-    // incoming rate is negative, so none is clamped when it is stored
-    bool nonneg = false;
+    // every source, and every rate that a checkpoint brought, is >= 0, and so
+    // is every face's area: no incoming rate is negative, so none is clamped
+    // when it is stored
+    bool nonneg = false, areas_nonneg = false;
     // the incoming rates that the last sweep's cells read are the pull sums
     // over the current X: nothing was clamped, no rotation has left offsets,
     // and no cell was solved before an upwind neighbour (uneven_faces)
@@ -4495,7 +4496,7 @@ void launch_chemistry(const ChemJob<R>* j, int n, hipStream_t st) {
 // ssw_sweep::rates_current and rates_partial after the sweeps of `order`.
 void rates_after(ssw_sweep* s, const std::vector<int>& order) {
     const int last = order.back();
-    s->rates_current = s->nonneg && !s->rotated && !s->uneven_faces;
+    s->rates_current = s->nonneg && s->areas_nonneg && !s->rotated && !s->uneven_faces;
     s->rates_partial = last != 0 && !s->list_full[last];
 }
 
@@ -5559,7 +5560,11 @@ int ssw_upload_grid(ssw_sweep* s, int64_t n, const int64_t* off, const int32_t* 
     s->F = F;
     TRY(make_order(s, n));
     double asum = 0.0;
-    for (int64_t f = 0; f < F; f++) asum += area[f];  // caller's order: independent of the internal order
+    s->areas_nonneg = true;
+    for (int64_t f = 0; f < F; f++) {
+        asum += area[f];  // caller's order: independent of the internal order
+        if (!(area[f] >= 0.0)) s->areas_nonneg = false;
+    }
     // Areas are carried in units of a power of two near the mean face area, so
     // that X = O / A keeps the range of O (SI areas reach 1e42 m^2); scaling
     // by a power of two is exact.
