@@ -73,6 +73,7 @@
 #include "chemistry.h"
 #include "direction_bins.h"
 #include "level_math.h"
+#include "memory_plan.h"
 
 namespace {
 
@@ -3186,6 +3187,7 @@ struct ssw_sweep {
     double lref = 1.0;
     TimestepState ts;
     int64_t bytes = 0, peak_bytes = 0;
+    int64_t capacity = 0;                           // expected_free
     std::unordered_map<void*, size_t> alloc;
     int64_t sweeps_last = 0;
     int64_t builds_last = 0;
@@ -3202,6 +3204,30 @@ struct ssw_sweep {
 
 namespace {
 
+std::array<std::atomic<int64_t>, kMaxDevices> g_held{};  // device bytes of all handles, per device
+
+std::atomic<int64_t>& held(const ssw_sweep* s) { return g_held[(size_t)s->device % kMaxDevices]; }
+
+// Device memory that is free once all that the process's handles have freed is
+// back. Freed memory is reported, and can be allocated again, only some time
+// after the free (16.8 M cells: 57 GB were still missing when the tiles were to
+// be allocated), so it is counted from the most that was free and held together
+// since the call began (expect_frees).
+int64_t expected_free(ssw_sweep* s) {
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    s->capacity = std::max(s->capacity, (int64_t)free_b + held(s));
+    return s->capacity - held(s);
+}
+
+void expect_frees(ssw_sweep* s) {
+    s->capacity = 0;
+    (void)expected_free(s);
+}
+
 template <typename T>
 void dfree(ssw_sweep* s, T*& p) {
     if (p) {
@@ -3209,6 +3235,7 @@ void dfree(ssw_sweep* s, T*& p) {
         auto it = s->alloc.find((void*)p);
         if (it != s->alloc.end()) {
             s->bytes -= (int64_t)it->second;
+            held(s) -= (int64_t)it->second;
             s->alloc.erase(it);
         }
         (void)hipFree((void*)p);
@@ -3221,9 +3248,15 @@ int dalloc(ssw_sweep* s, T** p, size_t count) {
     dfree(s, *p);
     if (count == 0) count = 1;
     hipError_t e;
-    {
-        std::shared_lock<std::shared_mutex> lock(g_capture_mu);
-        e = hipMalloc((void**)p, count * sizeof(T));
+    for (int tries = 0;; tries++) {
+        {
+            std::shared_lock<std::shared_mutex> lock(g_capture_mu);
+            e = hipMalloc((void**)p, count * sizeof(T));
+        }
+        // memory that was freed and is not back yet: at most 2 s
+        if (e != hipErrorOutOfMemory || tries == 100 || expected_free(s) < (int64_t)(count * sizeof(T))) break;
+        (void)hipGetLastError();
+        std::this_thread::sleep_for(std::chrono::milliseconds(20));
     }
     if (e != hipSuccess) {
         *p = nullptr;
@@ -3232,6 +3265,7 @@ int dalloc(ssw_sweep* s, T** p, size_t count) {
                                      " bytes failed: " + hipGetErrorString(e));
     }
     s->bytes += (int64_t)(count * sizeof(T));
+    held(s) += (int64_t)(count * sizeof(T));
     s->peak_bytes = std::max(s->peak_bytes, s->bytes);
     s->alloc[(void*)*p] = count * sizeof(T);
     return SSW_OK;
@@ -3881,18 +3915,13 @@ int build_groups_t(ssw_sweep* s, const uint32_t* sorted, uint32_t narrow_group, 
     dfree(s, ct);
     // The tiles of FP32 cones can take more than the per-level replay's planes
     // (measured: up to 35 B more per task, clustered cells x 16 directions). Where
-    // they and the state do not fit beside what is held, that replay runs. Freed
-    // memory comes back some time after the frees above (16.8 M cells: 57 GB were
-    // still missing), so where free memory is short, it is waited for, at most 2 s.
-    size_t free_b = 0, total_b = 0;
-    const size_t need = 16 * ((size_t)units + slots + more) + 4 * (size_t)ndesc +
-                        2 * (DN + (size_t)s->D * s->Nper) * sizeof(R) + 128 * (size_t)s->N;
-    for (int k = 0; k < 100; k++) {
-        HIP_TRY(hipMemGetInfo(&free_b, &total_b));
-        if (need + total_b / 64 <= free_b) break;
-        std::this_thread::sleep_for(std::chrono::milliseconds(20));
-    }
-    int rc = need + total_b / 64 <= free_b ? dalloc(s, &s->d_coneblob, (size_t)units) : SSW_ERR_OOM;
+    // they and what the handle still allocates do not fit, that replay runs.
+    const int64_t DP = (int64_t)s->D * s->Nper;
+    const int64_t later = !s->have_state ? ssw::state_bytes(s->N, (int64_t)DN, DP, sizeof(R))
+                          : !s->d_offI   ? ssw::offset_bytes((int64_t)DN, DP, sizeof(R))
+                                         : 0;
+    const int64_t bytes = 16 * (int64_t)((size_t)units + slots + more) + 4 * (int64_t)ndesc;
+    int rc = ssw::cones_fit(bytes, later, expected_free(s)) ? dalloc(s, &s->d_coneblob, (size_t)units) : SSW_ERR_OOM;
     if (rc == SSW_OK) rc = dalloc(s, &s->d_conetiles, (size_t)slots + more);
     if (rc == SSW_OK) rc = dalloc(s, &s->d_conemore, (size_t)ndesc);
     if (rc == SSW_ERR_OOM) {
@@ -5261,8 +5290,7 @@ int build_direction_graph(ssw_sweep* s, bool choose_mode) {
     // starts and sorted order while the schedule is written; then the
     // active-set lists and the transport state), it needs at most 85% of the
     // free device memory (automatic), else geometric
-    size_t free_b = 0, total_b = 0;
-    HIP_TRY(hipMemGetInfo(&free_b, &total_b));
+    const int64_t free_b = expected_free(s);
     const size_t rs = real_size(s);
     const size_t comp_bytes = DN * (16 + rs + kPlanes * entry_size(s) + 4) + (size_t)s->ovf_total * entry_size(s);
     const bool grouped = s->group_request >= 2;
@@ -5553,6 +5581,7 @@ int ssw_upload_grid(ssw_sweep* s, int64_t n, const int64_t* off, const int32_t* 
     }
     const int64_t F = off[n];
     if (F >= (int64_t)0xFFFFFFFFll) return fail(SSW_ERR_INVALID, "too many faces");
+    expect_frees(s);
     free_state(s);
     free_grid(s);
     s->have_grid = s->have_state = false;
@@ -5760,6 +5789,7 @@ int ssw_rotate_directions(ssw_sweep* s, const double* matrix) {
     if (!s->have_grid) return fail(SSW_ERR_INVALID, "ssw_upload_grid must be called first");
     for (int k = 0; k < 9; k++)
         if (!std::isfinite(matrix[k])) return fail(SSW_ERR_INVALID, "rotation matrix must be finite");
+    expect_frees(s);
     const int64_t n = s->N;
     const size_t DN = (size_t)s->D * n;
     // the rates before the rotation, as the reference's sites hold them
