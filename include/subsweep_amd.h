@@ -401,7 +401,7 @@ double ssw_chemistry_timestep(double* state, double density, double volume, doub
  * the handle's peak from ssw_upload_grid through ssw_step and ssw_download,
  * used for admission against an HBM budget, for handles with the default
  * launch shape (grouped replay of 4 level sets with 64 roots in the compiled
- * mode; the diagnostic downloads of
+ * mode; direction sweeps take less; the diagnostic downloads of
  * counts, level sets, fluxes and transport state allocate transient arrays
  * beyond it). No counterpart in the reference. */
 int64_t ssw_estimate_device_bytes(const ssw_sweep_parameters* params, int64_t num_cells, int64_t num_faces,

@@ -43,6 +43,7 @@
 #include <vector>
 
 #include "../../include/subsweep_amd.h"
+#include "memory_plan.h"
 
 namespace {
 
@@ -55,6 +56,7 @@ struct Req {
     int64_t ticket = 0;
     int64_t estimate = 0;
     int32_t mode = SSW_TRANSPORT_MODE_GEOMETRIC;
+    ssw::Replay replay = ssw::Replay::kGeometric;
     double t_submit = 0, t_start = 0, t_end = 0;
     int32_t status = SSW_OK;
     std::string error;
@@ -72,10 +74,12 @@ double now_s(std::chrono::steady_clock::time_point t0) {
     return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
 }
 
-// An idle handle in the cache and the device memory it holds.
+// An idle handle in the cache, the device memory it holds, and the estimate of
+// the request that made it (one of another launch shape may take it).
 struct Idle {
     ssw_sweep* s = nullptr;
     int64_t bytes = 0;
+    int64_t estimate = 0;
     uint64_t last_use = 0;
 };
 
@@ -159,7 +163,8 @@ ssw_sweep* setup_request(Req* q) {
         }
         rc = ssw_set_transport_mode(s, q->mode);
         if (rc == SSW_OK) rc = ssw_set_replay_block(s, r.replay_block);
-        if (rc == SSW_OK) rc = ssw_set_direction_sweeps(s, r.direction_sweeps ? 1 : 0);
+        if (rc == SSW_OK) rc = ssw_set_direction_sweeps(s, q->replay == ssw::Replay::kDirections ? 1 : 0);
+        if (rc == SSW_OK && q->replay == ssw::Replay::kPerLevel) rc = ssw_set_group_levels(s, 1);
         if (rc == SSW_OK && r.cell_position) rc = ssw_set_cell_positions(s, r.num_cells, r.cell_position);
         if (rc == SSW_OK)
             rc = ssw_upload_grid(s, r.num_cells, r.face_offsets, r.face_neighbour, r.face_kind, r.face_area,
@@ -272,6 +277,31 @@ void stepper(ssw_server* sv) {
     }
 }
 
+// The request's transport mode, launch shape and estimate. A compiled request
+// that asks for no shape gets the grouped replay where as many of them as there
+// are slots fit the budget; its tiles take up to 1.4 times what planes take
+// (FP32), so elsewhere it gets direction sweeps, whose tiles take less than
+// planes (bitwise the same results), then planes. Without a mode, geometric
+// transport where none of them fits the budget shared by the slots.
+void plan_replay(const ssw_server* sv, const ssw_request& r, const ssw::Problem& p, Req* q) {
+    q->mode = r.transport_mode;
+    if (q->mode == SSW_TRANSPORT_MODE_AUTO || q->mode == SSW_TRANSPORT_MODE_COMPILED) {
+        const int64_t share = sv->budget / sv->slots;
+        const bool any = q->mode == SSW_TRANSPORT_MODE_AUTO;
+        const int64_t limit = any ? share : sv->budget;
+        q->replay = r.direction_sweeps ? ssw::Replay::kDirections : ssw::Replay::kGrouped;
+        if (q->replay == ssw::Replay::kGrouped && ssw::handle_bytes(p, q->replay) > share)
+            q->replay = ssw::Replay::kDirections;
+        if (ssw::handle_bytes(p, q->replay) > limit) q->replay = ssw::Replay::kPerLevel;
+        if (any) {
+            const bool fits = ssw::handle_bytes(p, q->replay) <= limit;
+            q->mode = fits ? SSW_TRANSPORT_MODE_COMPILED : SSW_TRANSPORT_MODE_GEOMETRIC;
+            if (!fits) q->replay = ssw::Replay::kGeometric;
+        }
+    }
+    q->estimate = ssw::handle_bytes(p, q->replay);
+}
+
 // Takes idle handles out of the cache, least recently used first, until
 // `need` more bytes fit in the budget or the cache is empty (the caller holds
 // sv->mu and frees the returned handles after releasing it).
@@ -330,8 +360,9 @@ void worker(ssw_server* sv) {
                             if (it->second.empty()) sv->idle.erase(it);
                         }
                     }
-                    evict_for(sv, head->estimate, evicted);
-                    const bool fits = sv->reserved + sv->cached_bytes + head->estimate <= sv->budget;
+                    const int64_t need = std::max(head->estimate, hit.estimate);
+                    evict_for(sv, need, evicted);
+                    const bool fits = sv->reserved + sv->cached_bytes + need <= sv->budget;
                     if (hit.s && !fits) {
                         sv->idle[head->key].push_back(hit);
                         sv->cached_bytes += hit.bytes;
@@ -342,6 +373,7 @@ void worker(ssw_server* sv) {
                     if (fits) {
                         sv->queue.pop_front();
                         q = head;
+                        q->estimate = need;
                         sv->reserved += q->estimate;
                         sv->running++;
                         sv->peak_reserved = std::max(sv->peak_reserved, sv->reserved + sv->cached_bytes);
@@ -377,7 +409,7 @@ void worker(ssw_server* sv) {
             sv->reserved -= q->estimate;
             sv->running--;
             if (keep) {
-                sv->idle[q->key].push_back(Idle{keep, held, ++sv->use_clock});
+                sv->idle[q->key].push_back(Idle{keep, held, q->estimate, ++sv->use_clock});
                 sv->cached_bytes += held;
             }
         }
@@ -432,13 +464,8 @@ int ssw_server_submit(ssw_server* sv, const ssw_request* r, int64_t* ticket) {
                     nper++;
                     break;
                 }
-    q->mode = r->transport_mode;
-    if (q->mode == SSW_TRANSPORT_MODE_AUTO) {
-        // compiled when it fits the budget shared by the slots, else geometric
-        const int64_t comp = ssw_estimate_device_bytes(&r->params, r->num_cells, F, nper, SSW_TRANSPORT_MODE_COMPILED);
-        q->mode = comp <= sv->budget / sv->slots ? SSW_TRANSPORT_MODE_COMPILED : SSW_TRANSPORT_MODE_GEOMETRIC;
-    }
-    q->estimate = ssw_estimate_device_bytes(&r->params, r->num_cells, F, nper, q->mode);
+    plan_replay(sv, *r, {r->num_cells, F, nper, r->params.num_directions, r->params.num_timestep_levels,
+                         r->params.transport_precision == SSW_TRANSPORT_FP32}, q.get());
     q->key = cache_key(*r, q->mode);
     q->r.params.explicit_directions = nullptr;  // read once, into the key; handles copy them at creation
     if (r->params.explicit_directions) {

@@ -1053,10 +1053,7 @@ struct DirShape {
     static constexpr uint32_t kBuf = 256 + 512 / (uint32_t)sizeof(R);    // 128 far, 128 weights, 128 words of 4 bytes
     static constexpr uint32_t kWords = kBufs + kWaves * kBuf;
     // planes that hold up to n entries
-    __host__ __device__ static constexpr uint32_t planes(uint32_t n) {
-        if (sizeof(R) == 4) return n <= 3 ? 2u : n <= 5 ? 3u : n <= 7 ? 4u : n <= 11 ? 5u : 6u;
-        return n <= 1 ? 2u : n <= 3 ? 3u : n <= 5 ? 4u : n <= 7 ? 6u : n <= 9 ? 7u : n <= 11 ? 8u : 9u;
-    }
+    __host__ __device__ static constexpr uint32_t planes(uint32_t n) { return ssw::tile_planes(sizeof(R) == 4, n); }
     // place of weight plane j
     __host__ __device__ static constexpr uint32_t wplane(uint32_t j) { return j + 1 < (uint32_t)kS1 ? j + 1 : j + 2; }
 };
@@ -3537,19 +3534,6 @@ int kahn_layering(ssw_sweep* s, int lvl, int64_t expected, uint32_t* d_depth, in
     return SSW_OK;
 }
 
-// Device bytes of the grouped replay for DN tasks, n cells and L timestep
-// levels with T roots per workgroup: the full graph's task list (bound: DN +
-// DN/4 + 2^20 entries), descriptors and group map, and per restricted sweep
-// level a filtered list and descriptors (replacing the active-set lists).
-int64_t group_bytes(int64_t DN, int64_t n, int64_t L, int64_t T) {
-    const int64_t kmx = std::min<int64_t>(n + 2, 1 << 22);
-    const int64_t dcap = DN / T + kmx + 1;
-    const int64_t list = (DN + DN / 4 + (1 << 20)) * 4;
-    // + the transient scratch of a restricted sweep's filter (descriptors in
-    // place, kept flags, their prefix sum)
-    return list + dcap * 36 + kmx * 4 + (L - 1) * (list + dcap * 32) + (L > 1 ? dcap * 40 + (1 << 20) : 0);
-}
-
 // The replay plan of sweep level lvl from its level starts (the full
 // schedule's for level 0, the active-set list's otherwise): in the compiled
 // replay, each maximal run of at least two consecutive non-empty level sets of
@@ -3637,7 +3621,7 @@ int build_groups_t(ssw_sweep* s, const uint32_t* sorted, uint32_t narrow_group, 
     const std::vector<uint32_t>& fs = s->full_start;
     const int T = s->group_block;
     const size_t desc_cap = DN / T + (size_t)s->kmax + 1;  // at most ceil(width / T) per level set
-    const size_t list_cap = DN + DN / 4 + (1u << 20);
+    const size_t list_cap = (size_t)ssw::cone_list_cap((int64_t)DN);
     // groups of m level sets, of kMaxGroup where that many consecutive level
     // sets hold at most narrow_group tasks each (the narrow ends of the
     // graph, whose cones stay small); per pass r the level set
@@ -5253,12 +5237,16 @@ int noalloc_out(ssw_sweep* s, const T* src, T* dst, uint8_t* stage) {
     return SSW_OK;
 }
 
+ssw::Problem memory_problem(const ssw_sweep_parameters& p, int64_t n, int64_t faces, int64_t periodic_cells) {
+    return {n, faces, periodic_cells, p.num_directions, p.num_timestep_levels,
+            p.transport_precision == SSW_TRANSPORT_FP32};
+}
+
 // The per-direction dependency graph of the uploaded faces under the current
 // directions: mirror check (first build), downwind statistics, overflow
 // counts, the transport mode (choose_mode) and the schedule. d_cnt is held.
 int build_direction_graph(ssw_sweep* s, bool choose_mode) {
     const int64_t n = s->N;
-    const int L = s->p.num_timestep_levels;
     const size_t DN = (size_t)s->D * n;
     unsigned long long* d_stats = nullptr;
     Defer cleanup{[&] { dfree(s, d_stats); }};
@@ -5286,20 +5274,16 @@ int build_direction_graph(ssw_sweep* s, bool choose_mode) {
     if (!choose_mode) {
         return build_schedule(s);
     }
-    // transport mode: compiled when, at its peak (schedule arrays, overflow
-    // starts and sorted order while the schedule is written; then the
-    // active-set lists and the transport state), it needs at most 85% of the
-    // free device memory (automatic), else geometric
-    const int64_t free_b = expected_free(s);
-    const size_t rs = real_size(s);
-    const size_t comp_bytes = DN * (16 + rs + kPlanes * entry_size(s) + 4) + (size_t)s->ovf_total * entry_size(s);
-    const bool grouped = s->group_request >= 2;
-    const size_t lists = grouped ? (size_t)group_bytes((int64_t)DN, n, L, s->group_block) + DN * 5
-                                 : DN * 4 * (size_t)(L - 1);  // grouped: + build scratch
-    const size_t comp_need = comp_bytes + std::max<size_t>(DN * 8, lists + DN * 2 * rs);
+    // transport mode: compiled when the least that a compiled replay needs (planes,
+    // or the directions' tiles; cones are built where they fit as well) is at
+    // most 85% of the free device memory (automatic), else geometric
+    const int64_t need = ssw::replay_bytes(memory_problem(s->p, n, s->F, s->Nper),
+                                           s->dir_sweeps && !s->uneven_faces ? ssw::Replay::kDirections
+                                                                             : ssw::Replay::kPerLevel) +
+                         std::max<int64_t>(0, s->ovf_total - (int64_t)DN / 16) * (int64_t)entry_size(s);
     if (s->mode_request == SSW_TRANSPORT_MODE_COMPILED) s->compiled = true;
     else if (s->mode_request == SSW_TRANSPORT_MODE_GEOMETRIC) s->compiled = false;
-    else s->compiled = (double)comp_need <= 0.85 * (double)free_b;
+    else s->compiled = (double)need <= 0.85 * (double)expected_free(s);
     if (!s->compiled) dfree(s, s->d_nup);
     return build_schedule(s);
 }
@@ -6365,39 +6349,10 @@ double ssw_chemistry_timestep(double* state, double density, double volume, doub
 int64_t ssw_estimate_device_bytes(const ssw_sweep_parameters* p, int64_t n, int64_t F, int64_t num_periodic_cells,
                                   int32_t mode) {
     if (!p || n <= 0) return 0;
-    const int64_t D = p->num_directions, L = p->num_timestep_levels;
-    const int64_t rs = p->transport_precision == SSW_TRANSPORT_FP32 ? 4 : 8;
-    const int64_t es = rs == 4 ? 8 : 16;
-    const int64_t DN = D * n;
-    const bool comp = mode == SSW_TRANSPORT_MODE_COMPILED;
-    const int64_t ovf = comp ? DN * es / 16 : 0;   // overflow entries (bound used for the estimate)
-    // held from the grid upload on: grid arrays (with the caller-order map of
-    // a permuted grid), level starts, chunk table
-    const int64_t grid = (n + 1) * 4 + F * 32 + F * 4 + n * 16 + n * 4 + num_periodic_cells * 8 + F * 4 + n +
-                         (n + 4) * 4 + n * 8 + DN / kChunk * 40 + (1 << 20);
-    int64_t sched = comp ? DN * (16 + rs + kPlanes * es + 4) + ovf : DN * 16;  // compiled: + positions
-    // compiled replay with the default grouped replay (4 level sets, 64 roots):
-    // group lists instead of active-set lists, and the cone build's scratch
-    const int64_t grp = comp ? group_bytes(DN, n, L, kGroupT) : 0;
-    const int64_t lists = comp ? grp : (L - 1) * DN * 4;
-    // transient peak of the schedule build: counters + layering records (+
-    // overflow starts), the four sort arrays, or the schedule being written
-    // with the sorted order and overflow starts
-    const int64_t ostart = comp ? DN * 4 + ovf : 0;
-    int64_t build = std::max(DN * 20 + ostart, std::max(DN * 16 + ostart, sched + DN * 4 + ostart));
-    // the grouped replay's tiles: planes, indices and far list of every solved
-    // task (measured: up to 131 B in FP32, 174 B in FP64) and the
-    // positions, in place of `sched`
-    const int64_t cones = std::min(DN + DN / 4 + (1 << 20), DN + 3 * DN / 4) * (rs == 4 ? 140 : 190) + DN * 4;
-    if (comp) {
-        build = std::max(build, std::max(sched, cones) + grp + DN * 5);
-        sched = std::max(sched, cones);
-    }
-    // afterwards: schedule, active-set (or group) lists, state, the photon-rate
-    // and the optional outputs' downloads
-    const int64_t run = sched + lists + n * 8 * 9 + n * 4 + 2 * DN * rs + D * num_periodic_cells * rs + n * 40;
-    const int64_t b = grid + std::max(build, run);
-    return b + b / 20 + (1 << 20);
+    // compiled: the default launch shape
+    return ssw::handle_bytes(memory_problem(*p, n, F, num_periodic_cells), mode == SSW_TRANSPORT_MODE_COMPILED
+                                                                               ? ssw::Replay::kGrouped
+                                                                               : ssw::Replay::kGeometric);
 }
 
 int ssw_set_timing(ssw_sweep* s, int32_t enabled) {

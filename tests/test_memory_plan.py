@@ -1,39 +1,17 @@
-"""CPU: the decisions of the schedule build on device memory
-(subsweep_amd/csrc/memory_plan.h, compiled here with the host compiler)."""
-
-import ctypes as C
-import pathlib
-import shutil
-import subprocess
+"""CPU: the decisions of the schedule build and of the request loop on device
+memory (subsweep_amd/csrc/memory_plan.h, compiled here with the host compiler)."""
 
 import pytest
 
-HEADER = pathlib.Path(__file__).parent.parent / "subsweep_amd" / "csrc" / "memory_plan.h"
-SOURCE = f"""
-#include "{HEADER}"
-extern "C" {{
-int64_t state_bytes(int64_t n, int64_t dn, int64_t dp, int64_t rs) {{ return ssw::state_bytes(n, dn, dp, rs); }}
-int64_t offset_bytes(int64_t dn, int64_t dp, int64_t rs) {{ return ssw::offset_bytes(dn, dp, rs); }}
-int cones_fit(int64_t tiles, int64_t later, int64_t free) {{ return ssw::cones_fit(tiles, later, free); }}
-}}
-"""
+from memory_plan_util import DIRECTIONS, GEOMETRIC, GROUPED, PER_LEVEL, build_plan
+
 MB = 1 << 20
 GB = 1 << 30
 
 
 @pytest.fixture(scope="module")
 def plan(tmp_path_factory):
-    if shutil.which("g++") is None:
-        pytest.skip("g++ is not available")
-    d = tmp_path_factory.mktemp("plan")
-    (d / "plan.cpp").write_text(SOURCE)
-    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", str(d / "plan.cpp"), "-o", str(d / "plan.so")],
-                   check=True)
-    lib = C.CDLL(str(d / "plan.so"))
-    for f in (lib.state_bytes, lib.offset_bytes):
-        f.restype, f.argtypes = C.c_int64, [C.c_int64] * (4 if f is lib.state_bytes else 3)
-    lib.cones_fit.restype, lib.cones_fit.argtypes = C.c_int, [C.c_int64] * 3
-    return lib
+    return build_plan(tmp_path_factory)
 
 
 @pytest.mark.parametrize("tiles,later,free,fits", [
@@ -55,3 +33,28 @@ def test_later_allocations(plan, rs):
     state = plan.state_bytes(n, n * d, per * d, rs)
     assert state == 2 * n * d * rs + per * d * rs + n * (80 + 2 * rs + 4)
     assert plan.offset_bytes(n * d, per * d, rs) == (n + per) * d * rs
+
+
+# cells, faces, periodic cells, directions, levels, FP32: estimate of a compiled
+# request while all held planes and the group lists of every timestep level
+ADMITTED = [
+    (1000, 6000, 0, 16, 1, False, 11041568),
+    (4096, 63000, 1400, 1, 1, True, 10452023),
+    (8192, 127000, 2000, 16, 1, True, 31806763),
+    (32768, 508000, 6000, 84, 4, True, 491294785),
+    (262144, 4040000, 24000, 84, 1, True, 3326914344),
+    (262144, 4040000, 24000, 84, 4, False, 6291717486),
+    (524288, 8080000, 40000, 32, 2, True, 2950719832),
+    (2097152, 32300000, 100000, 84, 4, True, 30016745761),
+]
+
+
+@pytest.mark.parametrize("case", ADMITTED)
+def test_a_compiled_launch_shape_fits_where_planes_and_lists_did(plan, case):
+    *problem, before = case
+    assert plan.handle_bytes(*problem, DIRECTIONS) <= before
+    assert plan.handle_bytes(*problem, PER_LEVEL) <= before
+    assert plan.handle_bytes(*problem, GEOMETRIC) <= plan.handle_bytes(*problem, PER_LEVEL)
+    # cones that do not fit leave planes
+    assert plan.handle_bytes(*problem, GROUPED) >= plan.handle_bytes(*problem, PER_LEVEL)
+    assert plan.replay_bytes(*problem, GROUPED) < plan.handle_bytes(*problem, GROUPED)
