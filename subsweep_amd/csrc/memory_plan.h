@@ -32,12 +32,13 @@ inline int64_t offset_bytes(int64_t dn, int64_t dp, int64_t rs) { return (dn + d
 
 // Whether the grouped replay's tiles are built: they and what the handle
 // allocates after them have to fit into `free`, the memory that is free once
-// all that was freed has come back. 1/16 and 1 MB for the rounding of the
-// allocations; no part of it belongs to the device's size, since a small grid
-// on a nearly full device has to be grouped as anywhere else.
+// all that was freed has come back. 1 MB and 1/16, at most 1 GB, for the
+// rounding of the allocations and transient downloads; no part of it belongs to
+// the device's size, since a small grid on a nearly full device has to be
+// grouped as anywhere else.
 inline bool cones_fit(int64_t tiles, int64_t later, int64_t free) {
     const int64_t need = tiles + later;
-    return need + need / 16 + (1 << 20) <= free;
+    return need + std::min<int64_t>(need / 16, 1 << 30) + (1 << 20) <= free;
 }
 
 // How a handle replays its sweeps: from the faces, from planes with one launch

@@ -18,9 +18,9 @@ def plan(tmp_path_factory):
     (4 * MB, 1 * MB, 7 * MB, True),             # a small grid on a nearly full device
     (4 * MB, 1 * MB, 5 * MB, False),
     (0, 0, 1 * MB, True),
-    (150 * GB, 20 * GB, 182 * GB, True),        # the largest: 1/16 of what it needs is left
-    (150 * GB, 20 * GB, 180 * GB, False),
-    (150 * GB, 0, 160 * GB, True),              # its state is there already (a rotation)
+    (200 * GB, 20 * GB, 222 * GB, True),        # the largest
+    (200 * GB, 20 * GB, 221 * GB, False),
+    (200 * GB, 0, 202 * GB, True),              # its state is there already (a rotation)
     (150 * GB, 0, 0, False),
 ])
 def test_cones_fit(plan, tiles, later, free, fits):
