@@ -3169,10 +3169,10 @@ struct ssw_sweep {
     void *d_X = nullptr, *d_I = nullptr, *d_P = nullptr;
     void *d_offI = nullptr, *d_offP = nullptr;      // rate offsets after a rotation (Flux::offI / offP)
     bool rotated = false;                           // directions rotated since ssw_create
-    // every source, and every rate that a checkpoint brought, is >= 0, and so
-    // is every face's area: no incoming rate is negative, so none is clamped
-    // when it is stored
-    bool nonneg = false, areas_nonneg = false;
+    // every source and periodic source is >= 0, every face's area, and every X
+    // (not known after a checkpoint was loaded, until a full sweep has solved
+    // them all): no incoming rate is negative, so none is clamped when it is stored
+    bool nonneg = false, areas_nonneg = false, x_nonneg = false;
     // the incoming rates that the last sweep's cells read are the pull sums
     // over the current X: nothing was clamped, no rotation has left offsets,
     // and no cell was solved before an upwind neighbour (uneven_faces)
@@ -4509,8 +4509,12 @@ void launch_chemistry(const ChemJob<R>* j, int n, hipStream_t st) {
 // ssw_sweep::rates_current and rates_partial after the sweeps of `order`.
 void rates_after(ssw_sweep* s, const std::vector<int>& order) {
     const int last = order.back();
-    s->rates_current = s->nonneg && s->areas_nonneg && !s->rotated && !s->uneven_faces;
-    s->rates_partial = last != 0 && !s->list_full[last];
+    auto full = [&](int lvl) { return lvl == 0 || s->list_full[lvl]; };
+    bool x = s->x_nonneg;  // before the last sweep
+    for (size_t i = 0; i + 1 < order.size(); i++) x = x || full(order[i]);
+    s->rates_current = s->nonneg && s->areas_nonneg && x && !s->rotated && !s->uneven_faces;
+    s->x_nonneg = x || full(last);
+    s->rates_partial = !full(last);
 }
 
 template <typename R>
@@ -5692,7 +5696,7 @@ int ssw_upload_state(ssw_sweep* s, const double* density, const double* xhii, co
     std::vector<double> sod(n);
     double lmax = 0.0;
     s->rates_current = false;
-    s->nonneg = true;
+    s->nonneg = s->x_nonneg = true;
     for (int64_t c = 0; c < n; c++) {
         if (!(source[c] >= 0.0)) s->nonneg = false;
         sod[c] = source[c] / (double)s->D;  // Site::source_per_direction_bin
@@ -6176,9 +6180,9 @@ int load_t(ssw_sweep* s, const uint8_t* buf) {
     for (int d = 0; d < s->D; d++)
         for (size_t j = 0; j < order.size(); j++) Pd[(size_t)d * s->Nper + order[j]] = Pc[(size_t)d * s->Nper + j];
     auto negative = [](auto v) { return !(v >= 0); };  // NaN counts
-    s->rates_current = false;
+    s->rates_current = s->x_nonneg = false;
     s->nonneg = std::none_of(cell.begin() + 3 * n, cell.begin() + 4 * n, negative) &&
-                std::none_of(X.begin(), X.end(), negative) && std::none_of(Pd.begin(), Pd.end(), negative);
+                std::none_of(Pd.begin(), Pd.end(), negative);
     s->lref = h.lref;
     std::vector<double2> sa(n);
     for (int64_t c = 0; c < n; c++)
