@@ -6039,11 +6039,11 @@ int ssw_download_transport(ssw_sweep* s, void* X, void* I) {
             in = dtmp;
         }
         HIP_TRY(hipMemcpyAsync(out, in, m, hipMemcpyDeviceToHost, s->stream));
-        HIP_TRY(hipStreamSynchronize(s->stream));
         return SSW_OK;
     };
     TRY(get(X, s->d_X, s->compiled));
-    TRY(get(I, s->d_I, s->d_dirinfo != nullptr));
+    TRY(get(I, s->d_I, s->d_dirinfo != nullptr));  // into dtmp only after X has left it: stream order
+    HIP_TRY(hipStreamSynchronize(s->stream));
     dfree(s, dtmp);
     for (void* a : {X, I}) {
         if (!a) continue;
@@ -6124,8 +6124,7 @@ int save_t(ssw_sweep* s, uint8_t* buf) {
         HIP_TRY(hipGetLastError());
     }
     HIP_TRY(hipMemcpyAsync(X, tmp ? (void*)tmp : s->d_X, DN * sizeof(R), hipMemcpyDeviceToHost, s->stream));
-    if (s->d_dirinfo) {  // I in X's order
-        HIP_TRY(hipStreamSynchronize(s->stream));
+    if (s->d_dirinfo) {  // I in X's order, after the copy of X in stream order
         k_gather_x<R><<<grid_for(DN), kBlock, 0, s->stream>>>((const R*)s->d_I, s->d_xpos, tmp, DN);
         HIP_TRY(hipGetLastError());
     }
