@@ -187,7 +187,10 @@ int ssw_download_chemistry_outputs(ssw_sweep* s, double* photoionization_rate, d
  * maximum of 1 + old_i . new_j, kernel_f :177-188), and with 0 otherwise.
  * Later sweeps add their corrections to these rates, as the reference's
  * accumulated rates do. A handle with rotated directions does not save or
- * load checkpoints. */
+ * load checkpoints.
+ * A rotation into directions with a dependency cycle returns SSW_ERR_CYCLE and
+ * leaves the handle as it was; one that fails later (out of memory) drops grid
+ * and state, so that later calls ask for ssw_upload_grid. */
 int ssw_rotate_directions(ssw_sweep* s, const double* matrix);
 
 /* get_rotation_matrix (src/sweep/direction/mod.rs:112-135): the row-major

@@ -6,16 +6,23 @@
 //              periodic face also a compact list of those faces
 //   cell state rho, x, T, source/D, attenuation, timestep, previous rate,
 //              change timescale (f64[N]); timestep level (u8[N])
-//   fluxes     direction-major [d * N + c]:
-//              X = outgoing rate / downwind effective area (FP64 or scaled FP32)
+//   fluxes     X = outgoing rate / downwind effective area (FP64 or scaled FP32)
 //              I = incoming rate at solve time (FP64 or scaled FP32)
+//              direction-major [d * N + c]; in the compiled replays X in schedule
+//              order (xpos), with direction sweeps I too
 //              P[d * Nper + slot] periodic-source snapshot of the periodic cells
 //   schedule   the (cell, direction) tasks of the full dependency graph in Kahn
 //              order, level-major, within a level sorted by (direction, cell);
-//              full_start[k] is where level set k begins. Two replay forms:
+//              full_start[k] is where level set k begins. Four replay forms:
 //              geometric  task records {cell | face_count << 25, first_face,
 //                         direction, periodic slot} (16 B per task)
-//              compiled   per task a header {cell | direction << 25, periodic
+//              cones      the default: groups of level sets cut into cones,
+//                         compiled into tiles whose entries name LDS words
+//                         (k_sweep_cone)
+//              directions one workgroup per direction, its tasks in tiles
+//                         (k_sweep_dir)
+//              per level  group levels 1, or where cones do not fit:
+//                         per task a header {cell | direction << 25, periodic
 //                         slot, overflow start, upwind count}, the effective area
 //                         A, and its upwind local faces as (neighbour, weight)
 //                         pairs in kPlanes planes: entry q of the task at
@@ -29,9 +36,10 @@
 //              A sweep at timestep level l solves the cells with level >= l.
 //              Restricted to those cells, the full graph's level sets are still
 //              a valid order (an active task's active upwind neighbours are in
-//              earlier level sets), so such a sweep replays the full schedule
+//              earlier level sets), so such a sweep replays the full schedule:
 //              through a per-level list of the active positions (idx[l]),
-//              made by a stream compaction when the active set changes.
+//              made by a stream compaction when the active set changes, or the
+//              cones that hold active tasks, or all tiles of the directions.
 //
 // The transport is the reference's upwind sweep (src/sweep/mod.rs:412-513)
 // restated in pull form. A cell that is solved distributes the change of its
@@ -44,9 +52,9 @@
 // after the other, and A by a fixed 16-way tree, in every kernel, so the
 // geometric and the compiled replay give bitwise the same result, whatever
 // order tasks run in. The level sets (Kahn layering of init_counts' counts,
-// src/sweep/mod.rs:346-386) are built on the device once per grid by counter
-// decrements with block-aggregated appends; the level-set parity hook builds
-// the layering of a restricted active set the same way.
+// src/sweep/mod.rs:346-386) are built on the device once per grid, one workgroup
+// per direction (k_layers); the level-set parity hook builds the layering of a
+// restricted active set the same way.
 
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
@@ -92,7 +100,7 @@ constexpr int kPlanes = 12;                // upwind entries per task held in pl
 static_assert(kPlanes % 2 == 0, "FP32 plane entries are stored in pairs");
 constexpr int kChunk = 4096;               // compaction chunk (tasks, within one level set)
 constexpr int kRunBlock = 1024;            // workgroup of a run of narrow level sets (tasks per level set)
-constexpr int kGroupT = 64;                // grouped replay: root tasks per workgroup (default; 64 or 128)
+constexpr int kGroupT = 64;                // grouped replay: root tasks per workgroup (default; 32, 64 or 128)
 constexpr int kGroupLevels = 4;            // grouped replay: level sets per group (default)
 constexpr int kConeCap = 3072;             // grouped replay build: cone members / pending entries per workgroup
 constexpr int kConeThreads = 256;
@@ -3401,8 +3409,7 @@ void to_caller(const ssw_sweep* s, T* a, int64_t blocks) {
 }
 
 // k_fluxes for the incoming, outgoing and periodic rates of every (cell,
-// direction), and the photon rate of every cell (at its caller index with
-// `ridx`), which needs no pull where the last sweep's stored rates are current.
+// direction).
 void launch_fluxes(ssw_sweep* s, const Geo& g, double* dI, double* dO, double* dP) {
     const unsigned nb = (unsigned)((s->N + kFluxCells - 1) / kFluxCells);
     const unsigned lanes = (unsigned)(kFluxCells * ((s->D + kFluxDirs - 1) / kFluxDirs));
@@ -4488,9 +4495,9 @@ ChemArgs chem_args(ssw_sweep* s) {
 }
 
 // The periodic sources and the chemistry of n handles (at most kChemJobs) after
-// their sweeps. The tail gets a wave per 16 cells, at most two per SIMD (its
-// quads take further cells as they finish); waves that find no queued cell end
-// at once.
+// their sweeps. The tail gets a wave per 4 cells, so that a queue of all of them
+// has four quads a cell, at most two per SIMD (its quads then take further cells
+// as they finish); waves that find no queued cell end at once.
 template <typename R, int kJobs>
 void launch_chemistry(const ChemJob<R>* j, int n, hipStream_t st) {
     ChemJobs<R, kJobs> a;
